@@ -216,6 +216,28 @@ int lutgemm_gemv_block_apot_i8(const uint32_t *bW, const int8_t *alpha_i8, const
                                int M, void *stream);
 
 /*
+ * A quantised linear layer in one call: out[m][n] = fp16(bias[n] + sum), whatever `out` held before
+ * (bias_f16 may be NULL: zero).  The operands and the sum are those of the entry point of the same
+ * format above; the caller need not copy the bias into every row of `out` first, which is a launch of
+ * its own and, at one row, as long as the GEMV.  The reference's module does that copy
+ * (lut_gemm/quant.py:46).
+ *   format     : LUTGEMM_FORMAT_*, see lutgemm_describe_plan below;
+ *   qbias_f16  : uniform format only, NULL otherwise;
+ *   alpha_pow2 : 1 = the promise of lutgemm_gemv_rowwise_pow2_f16 (row-wise format only), else 0.
+ * Errors, capture and workspace rules as everywhere.
+ */
+typedef struct lutgemm_linear {
+    const uint32_t *bW;
+    const void *alpha;
+    const void *qbias_f16;
+    const void *x_f16;
+    const void *bias_f16;
+    void *out_f16;
+    int format, N, K, nb, num_groups, M, alpha_pow2;
+} lutgemm_linear;
+int lutgemm_linear_f16(const lutgemm_linear *layer, void *stream);
+
+/*
  * Algorithmic HBM bytes of one call (signs + alphas + x + out read + out
  * write), the figure throughput is quoted against.  alpha_bytes_per_entry is
  * 2 (fp16, uint16) or 3 (int8 x 3); alpha_entries is the alpha element count.

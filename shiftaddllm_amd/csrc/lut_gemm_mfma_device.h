@@ -366,7 +366,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         if (m < p.M && n < p.N && (p.ksplit == 1 || (int)(old[i] >> 56) == p.ksplit - 1)) {
             __half *dst = p.out + (size_t)m * p.N + n;
             const float y = p.ksplit == 1 ? val[i] : fixed_total((old[i] | contrib[i].flags) + contrib[i].add, p.ksplit);
-            const __half y16 = __float2half_rn((p.overwrite ? 0.0f : __half2float(*dst)) + y);
+            const __half y16 = __float2half_rn((p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y);
             *dst = y16;
             if (p.ksplit > 1)
                 __hip_atomic_store(p.accum + (size_t)m * p.N + n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

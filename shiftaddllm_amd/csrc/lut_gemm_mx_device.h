@@ -401,7 +401,7 @@ __device__ __forceinline__ void mx_tile(const Problem &p, const MxActivations &a
         if (mine[i] && (p.ksplit == 1 || (int)(old[i] >> 56) == p.ksplit - 1)) {
             __half *dst = p.out + (size_t)m * p.N + n;
             const float y = p.ksplit == 1 ? val[i] : fixed_total((old[i] | contrib[i].flags) + contrib[i].add, p.ksplit);
-            *dst = __float2half_rn((p.overwrite ? 0.0f : __half2float(*dst)) + y);
+            *dst = __float2half_rn((p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y);
             if (p.ksplit > 1)
                 __hip_atomic_store(p.accum + (size_t)m * p.N + n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }

@@ -864,7 +864,7 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
                 slot_sum[r] = p.sumsq_in[(size_t)min(m0 + r, p.M - 1) * p.sumsq_slots + min(tid, p.sumsq_slots - 1)];
         }
     }
-    // the caller's output, needed only by whoever completes a sum: fetched early,
+    // the caller's output (or bias), needed only by whoever completes a sum: fetched early,
     // off the critical path (again whenever the range moves on to another tile)
     unsigned short out_prev[MROWS];
     [[maybe_unused]] unsigned short out_prev_twin = 0;
@@ -873,7 +873,7 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
             // t counts tile pairs
             const int na = min(2 * t * kTileCols + own_col_of(kw), p.N - 1);
             const int nb2 = min((2 * t + 1) * kTileCols + own_col_of(kw), p.N - 1);
-            const unsigned short *row = (const unsigned short *)(p.out + (size_t)min(m0, p.M - 1) * p.N);
+            const unsigned short *row = (const unsigned short *)(p.init + (size_t)min(m0, p.M - 1) * p.init_stride);
             out_prev[0] = row[na];
             out_prev_twin = row[nb2];
             return;
@@ -890,7 +890,7 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
         }
 #pragma unroll
         for (int r = 0; r < MROWS; ++r)
-            out_prev[r] = *((const unsigned short *)(p.out + (size_t)min(m0 + r, p.M - 1) * p.N) + n);
+            out_prev[r] = *((const unsigned short *)(p.init + (size_t)min(m0 + r, p.M - 1) * p.init_stride) + n);
     };
     __builtin_amdgcn_sched_barrier(0);  // keep these requests ahead of the sign words
 

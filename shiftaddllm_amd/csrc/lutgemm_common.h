@@ -136,8 +136,12 @@ struct Problem {
     int rows_per_group;  // block modes: N / R
     const __half *norm_w;  // non-null: y = rsqrt(mean(x^2) + norm_eps) * W(fp16(x * norm_w))
     // ---- cache line 2 ----------------------------------------------------------------------
-    const __half *gate;    // non-null [M][K]: the input is fp16(fp16(silu(gate)) * x)
-    const __half *qbias;
+    union {
+        const __half *gate;   // row-wise, non-null [M][K]: the input is fp16(fp16(silu(gate)) * x)
+        const __half *qbias;  // uniform
+    };
+    const __half *init;    // what the sums are added to: row m at init + m * init_stride (out itself, or
+                           // one bias row for all of them: stride 0)
     __half *out;
     unsigned long long *accum;  // [M][N] fixed-point words, zero between launches
     Divisor by_items;        // item / items_per_wg
@@ -145,10 +149,11 @@ struct Problem {
     // Matrix-core kernel: K-steps per K-slice and slices per tile.
     int sets_per_split;
     int ksplit;
+    int init_stride;
+    int overwrite;       // 1: out = y instead of init + y
+    // ---- cache line 3: needed when sums are handed over --------------------------------------
     float norm_eps;
     int twin;            // look-up kernel: 1 = the items are twin items (n_tiles counts tile pairs)
-    // ---- cache line 3: needed when sums are handed over --------------------------------------
-    int overwrite;       // 1: out = y instead of out += y
     // RMSNorm split over two launches (fused entry point only).  The launch that completes
     // a residual row also leaves next_in = fp16(out * next_w) and adds the squares of its
     // outputs, 32 columns at a time, into sumsq_out[m][n / 32]; the launch that consumes
@@ -169,7 +174,7 @@ struct Problem {
     long long stamp_slots;   // capacity in readings
 #endif
 };
-static_assert(offsetof(Problem, by_group_words) == 64 && offsetof(Problem, gate) == 128 && offsetof(Problem, overwrite) == 192,
+static_assert(offsetof(Problem, by_group_words) == 64 && offsetof(Problem, gate) == 128 && offsetof(Problem, norm_eps) == 192,
               "Problem: fields are grouped by cache line");
 
 struct Group {

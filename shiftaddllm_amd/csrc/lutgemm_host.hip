@@ -304,9 +304,11 @@ int fill_problem(Problem &p, int mode, const uint32_t *bW, const void *alpha, co
     p = Problem{};
     p.W = bW;
     p.alpha = alpha;
-    p.qbias = (const __half *)qbias;
+    if (mode == kUniformF16) p.qbias = (const __half *)qbias;
     p.x = (const __half *)x;
     p.out = (__half *)out;
+    p.init = p.out;
+    p.init_stride = N;
     p.N = N;
     p.K = K;
     p.M = M;
@@ -609,12 +611,22 @@ int run_mx(Problem &p, const Accum &acc)
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
+// `bias`: null = accumulate into out; otherwise *bias is the row every output row starts from (null:
+// zeros) and out is written, not read.
 int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, const void *x,
-        void *out, int N, int K, int nb, int num_groups, int M, const Accum &acc, bool alpha_pow2 = false)
+        void *out, int N, int K, int nb, int num_groups, int M, const Accum &acc, bool alpha_pow2 = false,
+        const void *const *bias = nullptr)
 {
     Problem p;
     int rc = fill_problem(p, mode, bW, alpha, qbias, x, out, N, K, nb, num_groups, M);
     if (rc != LUTGEMM_OK) return rc;
+    if (bias && *bias) {
+        if (!aligned(*bias, 2)) return LUTGEMM_EALIGN;
+        p.init = (const __half *)*bias;
+        p.init_stride = 0;
+    } else if (bias) {
+        p.overwrite = 1;
+    }
     if (alpha_pow2 && mode == kRowF16 && mfma_eligible(p, mode) && p.M >= mfma_min_rows() && mx_wanted(p)) return run_mx(p, acc);
     int kernel = kLookup, mrows = 1;
     rc = plan_single(p, mode, &kernel, &mrows);
@@ -1274,6 +1286,14 @@ int lutgemm_gemv_block_apot_i8(const uint32_t *bW, const int8_t *alpha_i8, const
     if (num_apot != 3) return LUTGEMM_EUNSUP;
     return run(kBlockApotI8, bW, alpha_i8, nullptr, x_f16, out_f16, N, K, nb, num_groups, M,
                Accum{(hipStream_t)stream});
+}
+
+int lutgemm_linear_f16(const lutgemm_linear *layer, void *stream)
+{
+    if (!layer || layer->format < LUTGEMM_FORMAT_ROWWISE_F16 || layer->format > LUTGEMM_FORMAT_UNIFORM_F16) return LUTGEMM_EINVAL;
+    const lutgemm_linear &c = *layer;
+    return run(c.format, c.bW, c.alpha, c.qbias_f16, c.x_f16, c.out_f16, c.N, c.K, c.nb, c.num_groups, c.M,
+               Accum{(hipStream_t)stream}, c.alpha_pow2 != 0 && c.format == LUTGEMM_FORMAT_ROWWISE_F16, &c.bias_f16);
 }
 
 size_t lutgemm_algorithmic_bytes(int N, int K, int nb, int M, size_t alpha_entries,

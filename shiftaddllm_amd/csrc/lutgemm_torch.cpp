@@ -11,6 +11,7 @@
 //  * `d_input` may hold M rows ([M, K] or [..., K]); the reference's row-wise
 //    and uniform entry points are batch-1 only.
 #include <torch/extension.h>
+#include <ATen/hip/EmptyTensor.h>
 #include <ATen/hip/impl/HIPGuardImplMasqueradingAsCUDA.h>
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
@@ -187,6 +188,90 @@ void lutgemm_compute_block_shiftInt8(torch::Tensor output, torch::Tensor bWeight
     raise_on_error(rc, "lutgemm_compute_block_shiftInt8");
 }
 
+// ---- LutLinear.forward ------------------------------------------------------------------------
+// linear_forward(x, binaryWeight, alpha, bias, out, format, N, K, nb, num_groups, alpha_pow2) -> y
+// The whole of lut_gemm/quant.py:41-54 in one native call: the activations as contiguous fp16 rows,
+// the output [..., N] (allocated here, or `out`, fp16 [rows, N], where the caller reuses one), ONE launch
+// that adds the bias itself, the result in the activations' dtype.  At one row the layer is bound by the
+// host, not the device: through five framework calls and the checked functions above a forward took
+// 11.9 us of host time around a 4.5 us kernel.  A plain CPython function, because the argument
+// conversions of pybind11 are a tenth of what is left.
+at::Tensor linear_forward(const at::Tensor &x, const at::Tensor &bW, const at::Tensor &alpha, const at::Tensor *bias,
+                          const at::Tensor *out, int64_t format, int64_t N, int64_t K, int64_t nb, int64_t groups,
+                          bool alpha_pow2)
+{
+    TORCH_CHECK(x.is_cuda(), "the input must be a GPU tensor");
+    const auto dims = x.sizes();
+    TORCH_CHECK(!dims.empty() && dims.back() == K && x.numel() > 0, "expected a non-empty input of [..., ", K, "], got ", dims);
+    const int64_t rows = x.numel() / K;
+    const auto device = x.device();
+    const c10::hip::HIPGuardMasqueradingAsCUDA guard(device);
+    const c10::ScalarType dtype = x.scalar_type();
+    const at::Tensor x16 = dtype == at::kHalf && x.is_contiguous() ? x : x.to(at::kHalf).contiguous();
+
+    c10::SmallVector<int64_t, 5> shape(dims.begin(), dims.end());
+    shape.back() = N;
+    at::Tensor y = out ? *out : at::Tensor(at::detail::empty_cuda(shape, at::kHalf, device, c10::nullopt));
+    check_common(y, bW, x16, N, K, nb);
+    int64_t entries;
+    c10::ScalarType type = at::kHalf;
+    switch (format) {
+    case LUTGEMM_FORMAT_ROWWISE_F16:
+        TORCH_CHECK(groups > 0 && K % groups == 0 && (K / groups) % 32 == 0, "K/num_groups must be a multiple of 32");
+        entries = groups * nb * N;
+        break;
+    case LUTGEMM_FORMAT_BLOCK_F16:
+    case LUTGEMM_FORMAT_BLOCK_SHIFT_U16:
+    case LUTGEMM_FORMAT_BLOCK_APOT_I8:
+        check_block(N, groups);
+        entries = (K / 8) * nb * groups * (format == LUTGEMM_FORMAT_BLOCK_APOT_I8 ? 3 : 1);
+        if (format != LUTGEMM_FORMAT_BLOCK_F16) type = format == LUTGEMM_FORMAT_BLOCK_APOT_I8 ? at::kChar : at::kShort;
+        break;
+    default: TORCH_CHECK(false, "unknown alpha format ", format);
+    }
+    check_alpha(alpha, y, type, entries, "alpha");
+    if (bias)
+        TORCH_CHECK(bias->scalar_type() == at::kHalf && bias->device() == device && bias->is_contiguous() && bias->numel() == N,
+                    "bias must be ", N, " contiguous float16 values on the input's device");
+    lutgemm_linear layer{};
+    layer.bW = (const uint32_t *)bW.const_data_ptr();
+    layer.alpha = alpha.const_data_ptr();
+    layer.x_f16 = x16.const_data_ptr();
+    layer.bias_f16 = bias ? bias->const_data_ptr() : nullptr;
+    layer.out_f16 = y.data_ptr();
+    layer.format = (int)format;
+    layer.N = (int)N;
+    layer.K = (int)K;
+    layer.nb = (int)nb;
+    layer.num_groups = (int)groups;
+    layer.M = (int)rows;
+    layer.alpha_pow2 = alpha_pow2;
+    raise_on_error(lutgemm_linear_f16(&layer, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()), "LutLinear.forward");
+    if (dtype != at::kHalf) y = y.to(dtype);
+    return out ? y.view(shape) : y;
+}
+
+PyObject *linear_forward_py(PyObject *, PyObject *const *args, Py_ssize_t n)
+{
+    HANDLE_TH_ERRORS
+    TORCH_CHECK(n == 11, "linear_forward takes 11 arguments");
+    for (int i = 0; i < 5; ++i)
+        TORCH_CHECK(THPVariable_Check(args[i]) || (i >= 3 && args[i] == Py_None), "argument ", i, " of linear_forward must be a tensor");
+    int64_t v[6];
+    for (int i = 0; i < 6; ++i) {
+        v[i] = PyLong_AsLongLong(args[5 + i]);
+        if (v[i] == -1 && PyErr_Occurred()) return nullptr;
+    }
+    const at::Tensor *bias = args[3] == Py_None ? nullptr : &THPVariable_Unpack(args[3]);
+    const at::Tensor *out = args[4] == Py_None ? nullptr : &THPVariable_Unpack(args[4]);
+    return THPVariable_Wrap(linear_forward(THPVariable_Unpack(args[0]), THPVariable_Unpack(args[1]), THPVariable_Unpack(args[2]),
+                                           bias, out, v[0], v[1], v[2], v[3], v[4], v[5] != 0));
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef linear_forward_def = {"linear_forward", (PyCFunction)(void (*)(void))linear_forward_py, METH_FASTCALL,
+                                  "LutLinear.forward in one call"};
+
 // Calibration copy for profiler byte counters (no reference counterpart).
 void copy_bytes(torch::Tensor dst, torch::Tensor src)
 {
@@ -313,5 +398,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
     m.def("makeRandomWeight_int3", &makeRandomWeight_int3, "fill weight_int3[:K_new, :N] with random words");
     m.def("makeRandomWeight", &makeRandomWeight, "fill qW [K, NUM_BITS, N] with +-1 and bW [K/32, NUM_BITS, N] with their packing");
     m.def("parsing", &parsing, "host tensors -> flat device buffers {bWeight, q_bias, alpha}");
+    m.add_object("linear_forward", py::reinterpret_steal<py::object>(PyCFunction_New(&linear_forward_def, nullptr)));
     m.def("copy_bytes", &copy_bytes, "calibration copy kernel");
 }

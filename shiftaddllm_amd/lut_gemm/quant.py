@@ -18,6 +18,8 @@ from .. import native
 APOT_ABSENT = -128  # int8 exponent of an absent additive term
 
 ALPHA_FORMATS = ("apot_int8", "block_fp16", "block_shift_u16", "rowwise_fp16")
+# LUTGEMM_FORMAT_* of include/lutgemm_gfx950.h
+_FORMAT_CODES = {"rowwise_fp16": 0, "block_fp16": 1, "block_shift_u16": 2, "apot_int8": 3}
 
 
 def encode_apot_int8(alpha: torch.Tensor, num_apot: int = 3) -> torch.Tensor:
@@ -109,7 +111,7 @@ class LutLinear(nn.Module):
         self.bias = bias
         self.reuse_output = False      # see _output
         self._pow2_cache = None        # see _alphas_are_powers_of_two
-        self._bias_cache = None
+        self._bias_cache = None        # see _bias_vector
         self._out_cache = {}
 
     def quantize_to_apot(self, x):
@@ -126,14 +128,15 @@ class LutLinear(nn.Module):
             state_dict[key] = a[::8].contiguous()
         super()._load_from_state_dict(state_dict, prefix, *args, **kwargs)
 
-    def _bias_rows(self, rows, device):
-        """The bias as `rows` contiguous fp16 rows on `device`, formed once per (rows, device)
-        and per state of the bias tensor: what every call copies its output from."""
+    def _bias_vector(self, device):
+        """The bias as the fp16 vector on `device` that the kernel adds: the bias itself where it is
+        one, otherwise a copy formed once per device and per state of the bias tensor."""
         b = self.bias
-        key = (rows, device, b.data_ptr(), b._version)
+        if b is None or (b.dtype is torch.float16 and b.device == device and b.is_contiguous()):
+            return b
+        key = (device, b.data_ptr(), b._version)
         if self._bias_cache is None or self._bias_cache[0] != key:
-            t = b.detach().to(device=device, dtype=torch.float16).reshape(1, self.N).expand(rows, self.N).contiguous()
-            self._bias_cache = (key, t)
+            self._bias_cache = (key, b.detach().to(device=device, dtype=torch.float16).reshape(self.N).contiguous())
         return self._bias_cache[1]
 
     def _alphas_are_powers_of_two(self):
@@ -151,56 +154,29 @@ class LutLinear(nn.Module):
         return self._pow2_cache[1]
 
     def _output(self, rows, device):
-        """The tensor the kernel accumulates into, pre-filled with the bias (or zeros): a new
-        one per call like the reference's `bias.clone()` (lut_gemm/quant.py:46), or, with
-        `reuse_output`, one buffer per (rows, device) that every call overwrites (no allocation
+        """With `reuse_output`, the one buffer per (rows, device) that every call overwrites (no allocation
         on the call path, e.g. under HIP graph capture; the caller must be done with the previous
-        result)."""
-        if self.reuse_output:
-            buf = self._out_cache.get((rows, device))
-            if buf is None:
-                buf = self._out_cache[(rows, device)] = torch.empty((rows, self.N), dtype=torch.float16, device=device)
-            if self.bias is None:
-                buf.zero_()
-            else:
-                buf.copy_(self._bias_rows(rows, device))
-            return buf
-        if self.bias is None:
-            return torch.zeros((rows, self.N), dtype=torch.float16, device=device)
-        return self._bias_rows(rows, device).clone()
+        result); otherwise None: a new tensor per call, like the reference's `bias.clone()`
+        (lut_gemm/quant.py:46)."""
+        if not self.reuse_output:
+            return None
+        buf = self._out_cache.get((rows, device))
+        if buf is None:
+            buf = self._out_cache[(rows, device)] = torch.empty((rows, self.N), dtype=torch.float16, device=device)
+        return buf
 
     def forward(self, x):
-        if x.shape[-1] != self.K:
-            raise ValueError(f"expected last dimension {self.K}, got {tuple(x.shape)}")
-        dtype = x.dtype
-        # an fp16, contiguous input (what a half-precision decoder passes) goes to the kernel as it is
-        x2 = x.reshape(-1, self.K)
-        if dtype != torch.float16:
-            x2 = x2.to(torch.float16)
-        if not x2.is_contiguous():
-            x2 = x2.contiguous()
-        output = self._output(x2.shape[0], x2.device)
-
-        ext = native.lutgemm
-        fmt = self.alpha_format
-        if fmt == "apot_int8":
-            ext.lutgemm_compute_block_shiftInt8(output, self.binaryWeight, self.alpha, x2, self.N,
-                                                self.K, self.wbit, self.num_groups, 3)
-        elif fmt == "block_fp16":
-            ext.lutgemm_compute_block(output, self.binaryWeight, self.alpha, x2, self.N, self.K,
-                                      self.wbit, self.num_groups)
-        elif fmt == "block_shift_u16":
-            ext.lutgemm_compute_block_shift(output, self.binaryWeight, self.alpha, x2, self.N,
-                                            self.K, self.wbit, self.num_groups, 3)
-        elif 3 <= x2.shape[0] <= 8 and self._alphas_are_powers_of_two():
-            ext.lutgemm_compute_shift_scale_pow2(output, self.binaryWeight, self.alpha, x2, self.N,
-                                                 self.K, self.wbit, self.num_groups)
-        else:
-            ext.lutgemm_compute_shift_scale(output, self.binaryWeight, self.alpha, x2, self.N,
-                                            self.K, self.wbit, self.num_groups)
-        if dtype != torch.float16:
-            output = output.to(dtype)
-        return output.view(*x.shape[:-1], self.N)
+        K = self.K
+        if x.shape[-1] != K:
+            raise ValueError(f"expected last dimension {K}, got {tuple(x.shape)}")
+        buffers = self._buffers
+        fmt = _FORMAT_CODES[self.alpha_format]
+        rows = x.numel() // K
+        pow2 = fmt == 0 and 3 <= rows <= 8 and self._alphas_are_powers_of_two()
+        device = x.device
+        return native.lutgemm.linear_forward(x, buffers["binaryWeight"], buffers["alpha"], self._bias_vector(device),
+                                             self._output(rows, device) if self.reuse_output else None, fmt, self.N, K,
+                                             self.wbit, self.num_groups, pow2)
 
     def extra_repr(self):
         return "in_features={}, out_features={}, bias={}, wbit={}, group_size={}, alpha_format={}".format(

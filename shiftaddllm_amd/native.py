@@ -36,6 +36,7 @@ C_ABI_SYMBOLS = (
     "lutgemm_gemv_block_f16",
     "lutgemm_gemv_block_shift_u16",
     "lutgemm_gemv_block_apot_i8",
+    "lutgemm_linear_f16",
     "lutgemm_algorithmic_bytes",
     "lutgemm_copy_bytes",
     "lutgemm_workspace_words",
@@ -86,6 +87,14 @@ class FusedProblem(ctypes.Structure):
                 ("next_norm_weight_f16", ctypes.c_void_p), ("next_input_f16", ctypes.c_void_p),
                 ("sumsq_out_f32", ctypes.c_void_p), ("sumsq_in_f32", ctypes.c_void_p),
                 ("sumsq_in_slots", ctypes.c_int)]
+
+
+class Linear(ctypes.Structure):
+    """struct lutgemm_linear of include/lutgemm_gfx950.h."""
+    _fields_ = [("bW", ctypes.c_void_p), ("alpha", ctypes.c_void_p), ("qbias_f16", ctypes.c_void_p),
+                ("x_f16", ctypes.c_void_p), ("bias_f16", ctypes.c_void_p), ("out_f16", ctypes.c_void_p),
+                ("format", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int), ("nb", ctypes.c_int),
+                ("num_groups", ctypes.c_int), ("M", ctypes.c_int), ("alpha_pow2", ctypes.c_int)]
 
 
 class ChainProblem(ctypes.Structure):
@@ -165,6 +174,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     for name in ("lutgemm_gemv_rowwise_f16", "lutgemm_gemv_uniform_f16", "lutgemm_gemv_block_f16",
                  "lutgemm_gemv_block_shift_u16", "lutgemm_gemv_block_apot_i8"):
         getattr(lib, name).restype = ci
+    lib.lutgemm_linear_f16.argtypes = [ctypes.POINTER(Linear), vp]
+    lib.lutgemm_linear_f16.restype = ci
     lib.lutgemm_algorithmic_bytes.argtypes = [ci, ci, ci, ci, sz, ci]
     lib.lutgemm_algorithmic_bytes.restype = sz
     lib.lutgemm_copy_bytes.argtypes = [vp, vp, sz, vp]
