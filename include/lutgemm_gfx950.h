@@ -284,7 +284,7 @@ int lutgemm_reserve_workspace(void *stream, size_t words);
 #define LUTGEMM_FORMAT_UNIFORM_F16 4
 
 typedef struct lutgemm_plan {
-    int kernel;          /* 0: table look-up kernel, 1: matrix-core kernel, 2: block-scaled matrix-core kernel */
+    int kernel;          /* 0: table look-up kernel, 1: matrix-core kernel, 2: block-scaled matrix-core kernel, 3: GEMM kernel */
     int workgroups;      /* of the launch */
     int rows_per_pass;   /* activation rows a workgroup handles together */
     int row_chunks;      /* ceil(M / rows_per_pass) */
@@ -302,6 +302,14 @@ typedef struct lutgemm_plan {
 } lutgemm_plan;
 
 int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
+/* Calls of many rows (33 and more; where the fp16 matrix-core kernel applies as well, large ones), in every format, run on the GEMM
+ * kernel instead, whose plan this returns: kernel 3, rows_per_pass 64 or 128, tiles of 256 columns, k_units
+ * and units_per_slice in steps of 64 inputs, k_slices that a second launch adds up (their sums live in the
+ * per-stream buffer of the split activations; a call under capture whose buffer is too small, and
+ * lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order).  A call that takes
+ * one of the other kernels is described as lutgemm_describe_plan describes it; that function itself
+ * describes the look-up and fp16 matrix-core kernels for any row count. */
+int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
 /* The same for lutgemm_gemv_rowwise_pow2_f16: kernel 2 is the block-scaled matrix-core kernel
  * (rows_per_pass 5, 8 or 16; tiles of 64 columns, steps of 128 inputs); a call that takes one
  * of the other kernels is described as lutgemm_describe_plan describes it. */
@@ -338,6 +346,8 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
  *                   as its scale) instead of a shift and a bit operation per fp16 pair
  *                   1 = where that is faster (up to 16 rows, six or more rounds of K-steps
  *                   per workgroup), 2 = always, 0 = never; default 1
+ *   TILE_MIN_M    : rows from which a call takes the GEMM kernel (0 = by sizes; a large value switches
+ *                   that kernel off)
  *   CHAIN_GRID    : workgroups of a chained launch (0 = as many as the device holds
  *                   at once, which is also the upper limit)
  *   CHAIN_BLOCKS  : ranges the problems of one stage of a chained launch are cut into
@@ -354,7 +364,8 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
 #define LUTGEMM_OPTION_TWIN_ITEMS 8
 #define LUTGEMM_OPTION_BLOCK_SCALED 9
 #define LUTGEMM_OPTION_POW2_CONVERT 10
-#define LUTGEMM_OPTION_COUNT 11
+#define LUTGEMM_OPTION_TILE_MIN_M 11
+#define LUTGEMM_OPTION_COUNT 12
 int lutgemm_set_option(int which, int value);
 int lutgemm_get_option(int which);
 

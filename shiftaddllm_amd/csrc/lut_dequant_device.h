@@ -1,0 +1,233 @@
+// Sign planes -> fp16 weights in matrix-core operand registers, for gfx950 (wave64).
+//
+// With several activation rows a BCQ product is a GEMM, and its weights are worth forming once per
+// row tile instead of once per bit plane: W = sum_b +-alpha_b takes 2^nb values per alpha group, so a
+// lane keeps those values as a byte-wise table in registers and picks four weights at a time with
+// v_perm_b32 by the nb sign bits of each:
+//   * 13 shift / bit-field-insert instructions merge the nb sign words of 32 inputs into nibbles, 8
+//     byte permutes put the nibbles of four consecutive inputs into the bytes of one register;
+//   * per four weights: mask, one v_perm_b32 for the high bytes, one for the low bytes, two that
+//     interleave them into two packed fp16 pairs.
+// About two vector instructions per weight at three planes, where expanding every plane to +-alpha
+// takes one per weight AND PLANE plus a matrix instruction per plane.
+//
+// Precision: the table entries are formed in fp32 (scaled by a power of two that keeps them in the
+// middle of fp16's range) and rounded to fp16 once; what the rounding leaves over is a second table,
+// whose product is added as well wherever an entry is not exact.  Power-of-two alphas, which is what
+// the reference's quantiser emits (quantizers/bcq_quant/bcq_shift.py:15-24), are exact and skip it.
+// Two fp16 pieces hold 22 bits of the largest entry of a wave's first step.
+#ifndef LUT_DEQUANT_DEVICE_H
+#define LUT_DEQUANT_DEVICE_H
+
+#include "lutgemm_common.h"
+
+namespace lutgemm {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Entries of a table as bytes: entry i's high byte is byte i & 3 of hi[i >> 2], its low byte the same of
+// lo[i >> 2].  Four planes: 8 entries for the three planes relative to plane 3, whose sign is applied
+// afterwards; uniform mode (whose q_bias breaks that symmetry): 16 entries.
+template <int NB, bool UNI>
+struct WeightTable {
+    static constexpr int kRegs = NB <= 2 ? 1 : (NB == 4 && UNI) ? 4 : 2;
+    uint32_t hi[kRegs], lo[kRegs];
+};
+
+__device__ __forceinline__ uint32_t pack_halves(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __floats2half2_rn(a, b));
+}
+
+// bytes of four packed halves: high bytes / low bytes in entry order, or in reverse
+__device__ __forceinline__ uint32_t high_bytes(uint32_t p01, uint32_t p23) { return __builtin_amdgcn_perm(p23, p01, 0x07050301u); }
+__device__ __forceinline__ uint32_t low_bytes(uint32_t p01, uint32_t p23) { return __builtin_amdgcn_perm(p23, p01, 0x06040200u); }
+__device__ __forceinline__ uint32_t high_bytes_rev(uint32_t p01, uint32_t p23) { return __builtin_amdgcn_perm(p23, p01, 0x01030507u); }
+__device__ __forceinline__ uint32_t low_bytes_rev(uint32_t p01, uint32_t p23) { return __builtin_amdgcn_perm(p23, p01, 0x00020406u); }
+
+// The distinct fp32 entries of a table, from which the others follow by symmetry.
+//   a[b]: the planes' multipliers; UNI: a[b] = alpha / 2^(b+1) and q = q_bias.
+template <int NB, bool UNI>
+struct TableEntries {
+    static constexpr int kCount = UNI ? (NB == 1 ? 2 : 1 << NB) : NB == 4 ? 8 : NB == 3 ? 4 : NB == 2 ? 2 : 1;
+    float e[kCount];
+};
+
+template <int NB, bool UNI>
+__device__ __forceinline__ TableEntries<NB, UNI> table_entries(const float (&a)[NB], float q)
+{
+    TableEntries<NB, UNI> t;
+    if constexpr (UNI) {
+#pragma unroll
+        for (int i = 0; i < t.kCount; ++i) {
+            float v = q;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) v += ((i >> b) & 1) ? a[b] : -a[b];
+            t.e[i] = v;
+        }
+    } else if constexpr (NB == 1) {
+        t.e[0] = a[0];                          // entry 1
+    } else if constexpr (NB == 2) {
+        t.e[0] = a[1] - a[0];                   // entries 2, 3
+        t.e[1] = a[1] + a[0];
+    } else if constexpr (NB == 3) {
+        const float s = a[0] + a[1], d = a[0] - a[1];
+        t.e[0] = a[2] - s;                      // entries 4..7
+        t.e[1] = a[2] + d;
+        t.e[2] = a[2] - d;
+        t.e[3] = a[2] + s;
+    } else {
+        // entry i: plane 3 negative, plane b of the sign of plane 3 where bit b of i is set
+        const float s = a[0] + a[1], d = a[0] - a[1], u = -a[3] - a[2], v = a[2] - a[3];
+        t.e[0] = v + s;                         // -(a3 - a2 - a1 - a0)
+        t.e[1] = v - d;
+        t.e[2] = v + d;
+        t.e[3] = v - s;
+        t.e[4] = u + s;
+        t.e[5] = u - d;
+        t.e[6] = u + d;
+        t.e[7] = u - s;
+    }
+    return t;
+}
+
+// Entries -> byte table.
+template <int NB, bool UNI>
+__device__ __forceinline__ void pack_table(const TableEntries<NB, UNI> &t, WeightTable<NB, UNI> &w)
+{
+    if constexpr (UNI) {
+        if constexpr (NB == 1) {
+            const uint32_t p = pack_halves(t.e[0], t.e[1]);
+            w.hi[0] = high_bytes(p, p);
+            w.lo[0] = low_bytes(p, p);
+        } else {
+#pragma unroll
+            for (int r = 0; r < w.kRegs; ++r) {
+                const uint32_t p01 = pack_halves(t.e[4 * r], t.e[4 * r + 1]), p23 = pack_halves(t.e[4 * r + 2], t.e[4 * r + 3]);
+                w.hi[r] = high_bytes(p01, p23);
+                w.lo[r] = low_bytes(p01, p23);
+            }
+        }
+    } else if constexpr (NB == 1) {
+        const uint32_t p = pack_halves(t.e[0], t.e[0]);
+        w.hi[0] = high_bytes(p, p) ^ 0x00800080u;      // entry 0 (bytes 0 and 2) negative
+        w.lo[0] = low_bytes(p, p);
+    } else if constexpr (NB == 2) {
+        const uint32_t p = pack_halves(t.e[0], t.e[1]);   // entries 2, 3; 1 = -2, 0 = -3
+        w.hi[0] = __builtin_amdgcn_perm(p, p, 0x03010103u) ^ 0x00008080u;
+        w.lo[0] = __builtin_amdgcn_perm(p, p, 0x02000002u);
+    } else if constexpr (NB == 3) {
+        const uint32_t p45 = pack_halves(t.e[0], t.e[1]), p67 = pack_halves(t.e[2], t.e[3]);
+        w.hi[1] = high_bytes(p45, p67);
+        w.lo[1] = low_bytes(p45, p67);
+        w.hi[0] = high_bytes_rev(p45, p67) ^ 0x80808080u;
+        w.lo[0] = low_bytes_rev(p45, p67);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            const uint32_t p01 = pack_halves(t.e[4 * r], t.e[4 * r + 1]), p23 = pack_halves(t.e[4 * r + 2], t.e[4 * r + 3]);
+            w.hi[r] = high_bytes(p01, p23);
+            w.lo[r] = low_bytes(p01, p23);
+        }
+    }
+}
+
+// What rounding the entries to fp16 leaves over (zero where they are exact, non-zero or NaN otherwise).
+template <int NB, bool UNI>
+__device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntries<NB, UNI> &t)
+{
+    TableEntries<NB, UNI> r;
+#pragma unroll
+    for (int i = 0; i < t.kCount; ++i) r.e[i] = t.e[i] - __half2float(__float2half_rn(t.e[i]));
+    return r;
+}
+
+template <int NB, bool UNI>
+__device__ __forceinline__ bool any_nonzero(const TableEntries<NB, UNI> &t)
+{
+    uint32_t bits = 0;
+#pragma unroll
+    for (int i = 0; i < t.kCount; ++i) bits |= __builtin_bit_cast(uint32_t, t.e[i]);
+    return (bits << 1) != 0u;
+}
+
+// The sign words of 32 inputs of one output, one per plane -> y[c]: byte i of it holds the table indices
+// of inputs 8 c + i (low nibble) and 8 c + 4 + i (high nibble).  Bits above the index are garbage, except
+// bit 3 at four planes (plane 3 itself).
+template <int NB, bool UNI>
+__device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (&y)[4])
+{
+    auto bfi = [](uint32_t m, uint32_t a, uint32_t b) { return (m & a) | (~m & b); };
+    uint32_t n[4];
+    if constexpr (NB == 1) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) n[t] = w[0] >> t;
+    } else {
+        uint32_t w0 = w[0], w1 = w[1], w2 = NB > 2 ? w[NB > 2 ? 2 : 0] : 0u;
+        [[maybe_unused]] const uint32_t w3 = NB > 3 ? w[NB > 3 ? 3 : 0] : 0u;
+        if constexpr (NB == 4 && !UNI) {
+            w0 = ~(w0 ^ w3);
+            w1 = ~(w1 ^ w3);
+            w2 = ~(w2 ^ w3);
+        }
+        const uint32_t even = bfi(0x55555555u, w0, w1 << 1), odd = bfi(0x55555555u, w0 >> 1, w1);
+        n[0] = even;
+        n[1] = odd;
+        n[2] = even >> 2;
+        n[3] = odd >> 2;
+        if constexpr (NB >= 3) {
+            uint32_t up[4] = {w2 << 2, w2 << 1, w2, w2 >> 1};
+            if constexpr (NB == 4) {
+                const uint32_t top[4] = {w3 << 3, w3 << 2, w3 << 1, w3};
+#pragma unroll
+                for (int t = 0; t < 4; ++t) up[t] = bfi(0x44444444u, up[t], top[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) n[t] = bfi(0x33333333u, n[t], up[t]);
+        }
+    }
+    const uint32_t z01a = __builtin_amdgcn_perm(n[1], n[0], 0x05010400u), z01b = __builtin_amdgcn_perm(n[1], n[0], 0x07030602u);
+    const uint32_t z23a = __builtin_amdgcn_perm(n[3], n[2], 0x05010400u), z23b = __builtin_amdgcn_perm(n[3], n[2], 0x07030602u);
+    y[0] = __builtin_amdgcn_perm(z23a, z01a, 0x05040100u);
+    y[1] = __builtin_amdgcn_perm(z23a, z01a, 0x07060302u);
+    y[2] = __builtin_amdgcn_perm(z23b, z01b, 0x05040100u);
+    y[3] = __builtin_amdgcn_perm(z23b, z01b, 0x07060302u);
+}
+
+// Eight weights (inputs 8 c .. 8 c + 7, in order) as a matrix operand.
+template <int NB, bool UNI>
+__device__ __forceinline__ u32x4 pick_weights(uint32_t y, const WeightTable<NB, UNI> &t)
+{
+    constexpr uint32_t kMask = NB == 1 ? 0x01010101u : NB == 2 ? 0x03030303u : 0x07070707u;
+    uint32_t out[4];
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+        const uint32_t sel = (half ? y >> 4 : y) & kMask;
+        uint32_t h, l;
+        if constexpr (NB <= 2) {
+            h = __builtin_amdgcn_perm(t.hi[0], t.hi[0], sel);
+            l = __builtin_amdgcn_perm(t.lo[0], t.lo[0], sel);
+        } else {
+            h = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
+            l = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel);
+            if constexpr (NB == 4 && !UNI) {
+                h ^= (half ? y : y << 4) & 0x80808080u;       // plane 3 positive: the other sign
+            } else if constexpr (NB == 4) {
+                const uint32_t top = ((half ? y >> 7 : y >> 3) & 0x01010101u);
+                const uint32_t mask = (top << 8) - top;       // bytes of 0xff where plane 3 is positive
+                const uint32_t h1 = __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel), l1 = __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel);
+                h = (h & ~mask) | (h1 & mask);
+                l = (l & ~mask) | (l1 & mask);
+            }
+        }
+        out[2 * half] = __builtin_amdgcn_perm(h, l, 0x05010400u);
+        out[2 * half + 1] = __builtin_amdgcn_perm(h, l, 0x07030602u);
+    }
+    return (u32x4){out[0], out[1], out[2], out[3]};
+}
+
+}  // namespace lutgemm
+
+#endif

@@ -1,0 +1,515 @@
+// GEMM kernel templates for BCQ linear layers with many activation rows (prompts, large batches) on
+// MI355X (gfx950, wave64), every alpha format.
+//
+//   out[m][n] = init[m][n] + sum_k x[m][k] * W[n][k],  W formed from the sign planes on the fly.
+//
+// A workgroup of 4 waves owns 256 outputs x 32 * MF activation rows.  Each wave forms the weights of its
+// own 64 outputs in registers (lut_dequant_device.h), directly in the layout of the matrix
+// instruction's A operand (v_mfma_f32_32x32x16_f16: lane l holds output l % 32 and eight inputs), so a
+// weight is formed once per workgroup and never stored; the activations, the B operand, go through LDS
+// and are read by all four waves.  64 outputs per wave is what keeps the LDS reads at half a
+// 16-byte read per matrix instruction.
+//
+// A K-step is 64 inputs = two sign words: lanes 0..31 take the first word, lanes 32..63 the second, and
+// matrix instruction j multiplies byte j of either.  While the matrix cores work on step t the vector
+// ALU forms the weights of step t + 1 from sign words that were requested in step t - 1, and the
+// activations of step t + 2 travel from memory to registers (they enter LDS in step t + 1).
+#ifndef LUT_GEMM_TILE_DEVICE_H
+#define LUT_GEMM_TILE_DEVICE_H
+
+#include <utility>
+
+#include "lut_dequant_device.h"
+
+namespace lutgemm {
+
+constexpr int kTileThreads = 256;
+constexpr int kTileN = 256;            // outputs per workgroup
+constexpr int kTileWaveN = 64;         // outputs per wave
+constexpr int kTileStepK = 64;
+constexpr int kTileMaxRowGroups = 66;  // alpha row groups a tile of 256 outputs can touch (4 outputs each at least)
+
+enum TileFormat : int {
+    kTileRow = 0,        // one alpha per (group of inputs, plane, output)
+    kTileUniform = 1,    // alpha and q_bias per (group of inputs, output)
+    kTileBlock = 2,      // one alpha per (8 inputs, plane, row group)
+    kTileBlockWide = 3,  // the same where 64 outputs never straddle a row group
+};
+
+template <int MF>
+constexpr int kTileXBytes = 32 * MF * kTileStepK * 2;
+template <int FMT>   // scales of one step
+constexpr int kTileStageBytes = FMT == kTileRow ? 2 * kTileN * 8 : FMT == kTileUniform ? 2 * kTileN * 4 : 8 * kTileMaxRowGroups * 16;
+template <int FMT, int MF>
+constexpr int kTileLdsBytes = 2 * kTileXBytes<MF> + 4 * kTileStageBytes<FMT>;
+
+template <int... Is, class F>
+__device__ __forceinline__ void static_for_impl(std::integer_sequence<int, Is...>, F &&f)
+{
+    (f(std::integral_constant<int, Is>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F &&f)
+{
+    static_for_impl(std::make_integer_sequence<int, N>{}, f);
+}
+
+template <int NB, int FMT, int MF>
+__device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int m_tile, int slice, char *lds)
+{
+    constexpr bool UNI = FMT == kTileUniform;
+    constexpr bool BLOCK = FMT >= kTileBlock;
+    constexpr int kTabs = BLOCK ? 4 : 1;                       // tables per 32-output fragment and step
+    constexpr int kFragTabs = FMT == kTileBlockWide ? 1 : 2;   // fragments with tables of their own
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, kh = lane >> 5;
+    const int n0 = __builtin_amdgcn_readfirstlane(n_tile * kTileN + wave * kTileWaveN);
+    const int m0 = m_tile * 32 * MF;
+    int nn[2];
+#pragma unroll
+    for (int f = 0; f < 2; ++f) nn[f] = min(n0 + 32 * f + l32, p.N - 1);
+
+    // ---- activations: global -> registers -> LDS ------------------------------------------------
+    // Thread t carries 16-byte chunk t % 8 of rows t / 8 + 32 i; chunk c of row r sits in slot c ^ (r % 8) of
+    // the row's 128 bytes, which spreads the eight rows a quarter of a wave reads together over all banks.
+    const int xr = tid >> 3, xc = tid & 7;
+    uint32_t xoff[MF];
+#pragma unroll
+    for (int i = 0; i < MF; ++i) xoff[i] = (uint32_t)min(m0 + xr + 32 * i, p.M - 1) * (uint32_t)p.K * 2u;
+    const uint32_t xslot = (uint32_t)(xr * 128 + ((xc ^ (xr & 7)) * 16));
+    u32x4 xreg[MF];
+    auto load_x = [&](int t) {
+        const uint32_t k = (uint32_t)min(t * kTileStepK + xc * 8, p.K - 8) * 2u;
+#pragma unroll
+        for (int i = 0; i < MF; ++i) xreg[i] = *(const u32x4 *)((const char *)p.x + (xoff[i] + k));
+    };
+    auto store_x = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < MF; ++i) *(u32x4 *)(lds + buf * kTileXBytes<MF> + xslot + i * 4096) = xreg[i];
+    };
+    // matrix instruction j reads chunk 4 * kh + j of the lane's row, i.e. slot (4 * kh ^ l32 % 8) ^ j
+    const uint32_t bslot = (uint32_t)(l32 * 128 + ((4 * kh ^ (l32 & 7)) * 16));
+
+    // ---- signs and scales --------------------------------------------------------------------------
+    uint32_t words[2][NB];
+    auto load_words = [&](int t, uint32_t (&w)[2][NB]) {
+        const int wd = min(2 * t + kh, p.kwords - 1);
+        const uint32_t row = (uint32_t)wd * NB * (uint32_t)p.N;
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                w[f][b] = *(const uint32_t *)((const char *)p.W + (row + (uint32_t)b * (uint32_t)p.N + (uint32_t)nn[f]) * 4u);
+    };
+    // The scales of a step go through LDS as well (four steps' worth: while step t runs, those of steps t
+    // and t + 1 are read and those of step t + 2 written), fetched at the start of a step and written at
+    // its end:
+    //   row-wise: [word 0, 1][output 0..255][plane 0..3] fp16;  uniform: [word][output][alpha, q_bias] fp16;
+    //   block formats: the decoded multipliers, [chunk 0..7][row group of the tile][plane 0..3] fp32.
+    char *stage = lds + 2 * kTileXBytes<MF>;
+    auto stage_at = [&](int t) { return stage + (t & 3) * kTileStageBytes<FMT>; };
+    [[maybe_unused]] int rg0 = 0, n_rg = 1;
+    [[maybe_unused]] bool straddles = true;   // the wave's 64 outputs lie in several row groups
+    [[maybe_unused]] uint32_t rgl[2] = {0u, 0u};
+    if constexpr (BLOCK) {
+        const int first = n_tile * kTileN;
+        rg0 = first / p.rows_per_group;
+        n_rg = min(first + kTileN - 1, p.N - 1) / p.rows_per_group - rg0 + 1;
+#pragma unroll
+        for (int f = 0; f < 2; ++f) rgl[f] = (uint32_t)(nn[f] / p.rows_per_group - rg0);
+        straddles = min(n0, p.N - 1) / p.rows_per_group != min(n0 + kTileWaveN - 1, p.N - 1) / p.rows_per_group;
+    }
+    constexpr int kFetched = BLOCK ? 1 : UNI ? 2 : NB;
+    uint32_t fetched[kFetched];
+    // block formats: multiplier i of a step = row group i % n_rg of the tile, (chunk, plane) number i / n_rg
+    struct ScaleSlot {
+        int cb, r, dst;
+    };
+    [[maybe_unused]] auto scale_slot = [&](int i) {
+        ScaleSlot z;
+        z.cb = i / n_rg;
+        z.r = i - z.cb * n_rg;
+        const int c = z.cb / NB;
+        z.dst = (c * kTileMaxRowGroups + z.r) * 4 + (z.cb - c * NB);
+        return z;
+    };
+    [[maybe_unused]] ScaleSlot own{};
+    if constexpr (BLOCK) own = scale_slot(min(tid, 8 * NB * n_rg - 1));
+    [[maybe_unused]] auto raw_scale = [&](int t, const ScaleSlot &z) {
+        const int last = p.K / 8 * NB - 1;
+        const uint32_t at = (uint32_t)min(8 * NB * t + z.cb, last) * (uint32_t)p.R + (uint32_t)(rg0 + z.r);
+        if (p.mode == kBlockApotI8) {   // three bytes, as part of four that lie inside the tensor
+            const uint32_t from = min(3u * at, 3u * (uint32_t)(last + 1) * (uint32_t)p.R - 4u);
+            uint32_t v;
+            __builtin_memcpy(&v, (const char *)p.alpha + from, 4);
+            return v >> (8u * (3u * at - from));
+        }
+        return (uint32_t) * (const uint16_t *)((const char *)p.alpha + 2u * at);
+    };
+    [[maybe_unused]] auto put_scale = [&](int t, const ScaleSlot &z, uint32_t u) {
+        float v = 0.0f;
+        if (p.mode == kBlockF16) {
+            v = half_bits_to_float(u & 0xffffu);
+        } else if (p.mode == kBlockShiftU16) {
+            v = (float)((1u << (u & 7u)) + (1u << ((u >> 3) & 7u)) + (1u << ((u >> 6) & 7u)));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                const int x = (int)(int8_t)(u >> (8 * e));
+                v += x == -128 ? 0.0f : ldexpf(1.0f, x);
+            }
+        }
+        ((float *)stage_at(t))[z.dst] = v;
+    };
+    auto fetch_scales = [&](int t) {
+        if constexpr (BLOCK) {
+            fetched[0] = raw_scale(t, own);
+        } else {
+            // threads 0..127: two outputs each for the step's first word, the others for its second
+            const uint32_t n = (uint32_t)min(n_tile * kTileN + 2 * (tid & 127), p.N - 2);
+            const uint32_t g = (uint32_t)fast_div(min(2 * t + (tid >> 7), p.kwords - 1), p.by_group_words);
+            if constexpr (UNI) {
+                const uint32_t at = (g * (uint32_t)p.N + n) * 2u;
+                fetched[0] = *(const uint32_t *)((const char *)p.alpha + at);
+                fetched[1] = *(const uint32_t *)((const char *)p.qbias + at);
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    fetched[b] = *(const uint32_t *)((const char *)p.alpha + ((g * NB + (uint32_t)b) * (uint32_t)p.N + n) * 2u);
+            }
+        }
+    };
+    auto store_scales = [&](int t) {
+        if constexpr (BLOCK) {
+            const int all = 8 * NB * n_rg;
+            if (tid < all) put_scale(t, own, fetched[0]);
+            for (int i = tid + kTileThreads; i < all; i += kTileThreads) {   // (row groups of a few outputs)
+                const ScaleSlot z = scale_slot(i);
+                put_scale(t, z, raw_scale(t, z));
+            }
+        } else {
+            constexpr int kEach = UNI ? 2 : 4;   // halves per output
+            unsigned short *dst = (unsigned short *)stage_at(t) + 2 * tid * kEach;
+#pragma unroll
+            for (int b = 0; b < kFetched; ++b) {
+                dst[b] = (unsigned short)fetched[b];
+                dst[kEach + b] = (unsigned short)(fetched[b] >> 16);
+            }
+        }
+    };
+    // multipliers of fragment f (and, block formats, chunk c of the lane's word) in step t, unscaled
+    auto multipliers = [&](int t, int f, int c, float (&a)[NB], float &q) {
+        q = 0.0f;
+        if constexpr (BLOCK) {
+            const f32x4 v = *(const f32x4 *)(stage_at(t) + ((4 * kh + c) * kTileMaxRowGroups + rgl[f]) * 16);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) a[b] = v[b];
+        } else {
+            const int at = kh * kTileN + wave * kTileWaveN + 32 * f + l32;
+            if constexpr (UNI) {
+                const uint32_t v = ((const uint32_t *)stage_at(t))[at];
+                const float alpha = half_bits_to_float(v & 0xffffu);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) a[b] = alpha * (1.0f / (float)(2 << b));
+                q = half_bits_to_float(v >> 16);
+            } else {
+                const u32x2 v = ((const u32x2 *)stage_at(t))[at];
+                const uint32_t v2[2] = {v.x, v.y};
+#pragma unroll
+                for (int b = 0; b < NB; ++b) a[b] = half_bits_to_float((v2[b >> 1] >> (16 * (b & 1))) & 0xffffu);
+            }
+        }
+    };
+
+    // ---- the step's weights -----------------------------------------------------------------------
+    u32x4 A[2][4][2];            // [step parity][matrix instruction][fragment]
+    bool lo_cur = false;         // rounding the current step's weights to fp16 left something over (uniform over the wave)
+    WeightTable<NB, UNI> tab[kFragTabs][kTabs];
+    float unit = 1.0f;           // weights are formed as W * unit, a power of two
+    auto wave_max_bits = [&](float v) {
+        uint32_t m = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+        if (m >= 0x7f800000u) m = 0u;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d));
+        return __builtin_bit_cast(float, m);
+    };
+    auto largest = [&](int t) {   // upper bound of |W| in the step
+        float most = 0.0f;
+#pragma unroll
+        for (int f = 0; f < kFragTabs; ++f)
+#pragma unroll
+            for (int c = 0; c < kTabs; ++c) {
+                float a[NB], q, s;
+                multipliers(t, f, c, a, q);
+                s = fabsf(q);
+#pragma unroll
+                for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
+                most = fmaxf(most, s);
+            }
+        return wave_max_bits(most);
+    };
+    auto unit_for = [](float most) {   // power of two that brings `most` to 2^8 .. 2^9
+        const int e = most > 0.0f ? (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127 : 8;
+        return ldexpf(1.0f, min(max(8 - e, -120), 120));
+    };
+    // One table of step t, or of what its rounding leaves over; true when some entry is
+    // not an fp16 number.
+    auto make_table = [&](int t, bool lo, int f, int c) {
+        const float u = 2 * t + kh < p.kwords ? unit : 0.0f;   // a word beyond K has no weight
+        float a[NB], q;
+        multipliers(t, f, c, a, q);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) a[b] *= u;
+        const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u), r = table_residual(e);
+        if (lo)
+            pack_table(r, tab[f][c]);
+        else
+            pack_table(e, tab[f][c]);
+        return any_nonzero(r);
+    };
+    auto make_tables = [&](int t, bool lo) {
+        bool inexact = false;
+#pragma unroll
+        for (int f = 0; f < kFragTabs; ++f)
+#pragma unroll
+            for (int c = 0; c < kTabs; ++c) inexact = make_table(t, lo, f, c) || inexact;
+        return inexact;
+    };
+    auto pick = [&](int f, int c, const uint32_t (&y)[4]) {
+        return pick_weights<NB, UNI>(y[c], tab[FMT == kTileBlockWide ? 0 : f][BLOCK ? c : 0]);
+    };
+
+    f32x16 acc[2][MF];
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < MF; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[f][i][r] = 0.0f;
+
+    auto activations = [&](int buf, int j, int i) {
+        return __builtin_bit_cast(f16x8, *(const u32x4 *)(lds + buf * kTileXBytes<MF> + i * 4096 + (bslot ^ (uint32_t)(16 * j))));
+    };
+    auto multiply = [&](int buf, int j, const u32x4 (&a)[2]) {
+#pragma unroll
+        for (int i = 0; i < MF; ++i) {
+            const f16x8 b = activations(buf, j, i);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+                acc[f][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a[f]), b, acc[f][i], 0, 0, 0);
+        }
+    };
+
+    uint32_t words_lo[2][NB];
+    // Some weight of step t (in A[set]) is no fp16 number: a second piece is due in that step, after a change
+    // of unit if it is out of fp16's range.
+    auto second_piece = [&](int t, int set) {
+        load_words(t, words_lo);
+        const float most = largest(t);
+        if (most * unit > 32768.0f) {
+            const float fresh = unit_for(most), by = fresh / unit;
+            unit = fresh;
+            (void)make_tables(t, false);
+#pragma unroll
+            for (int f = 0; f < 2; ++f) {
+                uint32_t y[4];
+                sign_indices<NB, UNI>(words_lo[f], y);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) A[set][c][f] = pick(f, c, y);
+#pragma unroll
+                for (int i = 0; i < MF; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[f][i][r] *= by;
+            }
+        }
+    };
+
+    // step t with parity P: buffer P of LDS holds its activations, A[P] its weights; `words` belong to step t + 1,
+    // words_lo, where a second piece is due, to step t.
+    auto step = [&](int t, auto parity) {
+        constexpr int P = decltype(parity)::value;
+        store_x(P ^ 1);
+        fetch_scales(t + 2);
+        load_x(t + 2);
+        if (lo_cur) {
+            (void)make_tables(t, true);
+            uint32_t y[2][4];
+#pragma unroll
+            for (int f = 0; f < 2; ++f) sign_indices<NB, UNI>(words_lo[f], y[f]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const u32x4 a[2] = {pick(0, j, y[0]), pick(1, j, y[1])};
+                multiply(P, j, a);
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // The matrix instructions of step t, two at a time (one activation fragment against both weight
+        // fragments), each pair with its share of the vector work on step t + 1 and the request for the
+        // next activation fragment.  (Left to itself the compiler puts all vector work in front of all
+        // matrix work and waits for every fragment right behind its request.)
+        bool inexact = false;
+        uint32_t y[2][4];
+        // (block formats: a chunk's tables, then its weights, so that few tables are live at a time)
+        constexpr int kPer = kFragTabs + 2, kItems = BLOCK ? 3 + 4 * kPer : 3 + 2 + 8, kSlots = 4 * MF;
+        auto item = [&](auto k_c) {
+            constexpr int k = decltype(k_c)::value, r = k - 3;
+            constexpr bool table = BLOCK ? r % kPer < kFragTabs : r < 2;
+            constexpr int c = BLOCK ? r / kPer : table ? 0 : (r - 2) >> 1;
+            constexpr int f = BLOCK ? (table ? r % kPer : r % kPer - kFragTabs) : r & 1;
+            if constexpr (k < 2)
+                sign_indices<NB, UNI>(words[k], y[k]);
+            else if constexpr (k == 2)
+                load_words(t + 2, words);
+            else if constexpr (table && FMT == kTileBlock && f == 1) {
+                // (where the wave's outputs lie in one row group, as most waves' do, the tables are the same)
+                if (straddles)
+                    inexact = make_table(t + 1, false, 1, c) || inexact;
+                else
+                    tab[1][c] = tab[0][c];
+            } else if constexpr (table)
+                inexact = make_table(t + 1, false, f, c) || inexact;
+            else
+                A[P ^ 1][c][f] = pick(f, c, y[f]);
+        };
+        f16x8 b = activations(P, 0, 0);
+        static_for<kSlots>([&](auto s_c) {
+            constexpr int s = decltype(s_c)::value, j = s / MF, i = s % MF;
+            f16x8 next = b;
+            if constexpr (s + 1 < kSlots) next = activations(P, (s + 1) / MF, (s + 1) % MF);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+                acc[f][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, A[P][j][f]), b, acc[f][i], 0, 0, 0);
+            constexpr int first = s * kItems / kSlots, count = (s + 1) * kItems / kSlots - first;
+            static_for<count>([&](auto c_c) { item(std::integral_constant<int, first + decltype(c_c)::value>()); });
+            b = next;
+            __builtin_amdgcn_sched_barrier(0);
+        });
+        lo_cur = __builtin_amdgcn_ballot_w64(inexact) != 0ull;
+        if (lo_cur) second_piece(t + 1, P ^ 1);
+        store_scales(t + 2);
+        __syncthreads();
+    };
+
+    // ---- prologue: step 0's activations in LDS, its weights in A[0] --------------------------------------
+    const int t0 = slice * p.slice_steps, t1 = min(t0 + p.slice_steps, p.steps);   // (even numbers)
+    load_x(t0);
+    load_words(t0, words);
+    fetch_scales(t0);
+    store_scales(t0);
+    fetch_scales(t0 + 1);
+    store_scales(t0 + 1);
+    store_x(0);
+    load_x(t0 + 1);
+    __syncthreads();
+    unit = unit_for(largest(t0));
+    lo_cur = __builtin_amdgcn_ballot_w64(make_tables(t0, false)) != 0ull;
+    if (lo_cur) load_words(t0, words_lo);
+#pragma unroll
+    for (int f = 0; f < 2; ++f) {
+        uint32_t y[4];
+        sign_indices<NB, UNI>(words[f], y);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) A[0][c][f] = pick(f, c, y);
+    }
+    load_words(t0 + 1, words);
+#pragma clang loop unroll(disable)
+    for (int t = t0; t < t1; t += 2) {
+        step(t, std::integral_constant<int, 0>());
+        step(t + 1, std::integral_constant<int, 1>());
+    }
+
+    const float back = 1.0f / unit;
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int i = 0; i < MF; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[f][i][r] *= back;
+
+    // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
+    // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
+    float *sums = p.ksplit > 1 ? p.partial + (size_t)slice * p.M * p.N : nullptr;
+#pragma unroll
+    for (int i = 0; i < MF; ++i) {
+        const int m = m0 + 32 * i + l32;
+        if (m >= p.M) continue;
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int g = 0; g < 4; ++g) {
+                const int n = n0 + 32 * f + 8 * g + 4 * kh;
+                if (n >= p.N) continue;
+                float v[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[r] = acc[f][i][4 * g + r];
+                if (sums) {
+                    *(f32x4 *)(sums + (size_t)m * p.N + n) = (f32x4){v[0], v[1], v[2], v[3]};
+                    continue;
+                }
+                if (!p.overwrite) {
+                    const u32x2 old = *(const u32x2 *)(p.init + (size_t)m * p.init_stride + n);
+                    v[0] += half_bits_to_float(old.x & 0xffffu);
+                    v[1] += half_bits_to_float(old.x >> 16);
+                    v[2] += half_bits_to_float(old.y & 0xffffu);
+                    v[3] += half_bits_to_float(old.y >> 16);
+                }
+                *(u32x2 *)(p.out + (size_t)m * p.N + n) = (u32x2){pack_halves(v[0], v[1]), pack_halves(v[2], v[3])};
+            }
+    }
+}
+
+// Flat workgroup index -> (output tile, row tile, K-slice).  Workgroups go to the 8 XCDs in turn: the row
+// tiles of an output tile, which stream the same sign words, sit on one XCD, behind one L2.
+__device__ __forceinline__ void decode_tile(const TileProblem &p, int b, int &n_tile, int &m_tile, int &slice)
+{
+    const int q = b >> 3;
+    m_tile = q % p.m_tiles;
+    const int strip = (q / p.m_tiles) * 8 + (b & 7);   // output tile and slice
+    n_tile = strip % p.n_tiles;
+    slice = strip / p.n_tiles;
+}
+
+// Four outputs per thread: the slices' sums, in slice order, and what they are added to.  One launch behind
+// the tiles rather than the last slice's workgroup of each tile: that one alone reads at 60 GB/s
+// (4096 x 4096, 128 rows, 16 slices: 32 us, most of them this tail).
+__global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
+{
+    const uint32_t quads = (uint32_t)p.N / 4u;
+    const uint32_t at = blockIdx.x * 256u + threadIdx.x;
+    if (at >= quads * (uint32_t)p.M) return;
+    const size_t stride = (size_t)p.M * p.N;
+    const float *src = p.partial + (size_t)at * 4u;
+    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    int sl = 0;
+    for (; sl + 4 <= p.ksplit; sl += 4) {
+        f32x4 q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) q[u] = *(const f32x4 *)(src + (size_t)(sl + u) * stride);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v += q[u];
+    }
+    for (; sl < p.ksplit; ++sl) v += *(const f32x4 *)(src + (size_t)sl * stride);
+    const uint32_t m = at / quads, n = 4u * (at - m * quads);
+    if (!p.overwrite) {
+        const u32x2 old = *(const u32x2 *)(p.init + (size_t)m * p.init_stride + n);
+        v[0] += half_bits_to_float(old.x & 0xffffu);
+        v[1] += half_bits_to_float(old.x >> 16);
+        v[2] += half_bits_to_float(old.y & 0xffffu);
+        v[3] += half_bits_to_float(old.y >> 16);
+    }
+    *(u32x2 *)(p.out + (size_t)m * p.N + n) = (u32x2){pack_halves(v[0], v[1]), pack_halves(v[2], v[3])};
+}
+
+template <int NB, int FMT, int MF>
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+lut_gemm_tile_kernel(const TileProblem p)
+{
+    __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
+    int n_tile, m_tile, slice;
+    decode_tile(p, (int)blockIdx.x, n_tile, m_tile, slice);
+    if (slice >= p.ksplit) return;
+    gemm_tile<NB, FMT, MF>(p, n_tile, m_tile, slice, lds);
+}
+
+}  // namespace lutgemm
+
+#endif

@@ -177,6 +177,24 @@ struct Problem {
 static_assert(offsetof(Problem, by_group_words) == 64 && offsetof(Problem, gate) == 128 && offsetof(Problem, norm_eps) == 192,
               "Problem: fields are grouped by cache line");
 
+// One problem of the GEMM kernel for many activation rows (lut_gemm_tile_device.h).
+struct TileProblem {
+    const uint32_t *W;
+    const void *alpha;
+    const __half *qbias;
+    const __half *x;
+    const __half *init;
+    __half *out;
+    int N, K, M, kwords;
+    Divisor by_group_words;
+    int R, rows_per_group, mode;     // block formats; mode: AlphaMode
+    int n_tiles, m_tiles, tile_rows;
+    int steps;                       // K-steps, rounded up to an even number
+    int ksplit, slice_steps;         // K-slices and steps of each (even; the last one may have fewer)
+    float *partial;                  // ksplit > 1: [slice][M][N] partial sums
+    int init_stride, overwrite;
+};
+
 struct Group {
     int count;
     Problem p[kMaxGroup];

@@ -23,6 +23,7 @@ constexpr int kMfmaWaves = 8;       // waves of a matrix-core workgroup: K-steps
 constexpr int kMfmaTileCols = 64;   // outputs per matrix-core workgroup
 constexpr int kMfmaStepK = 128;
 constexpr int kMaxDevices = 64;
+constexpr size_t kTileSumBytes = 64u << 20;   // GEMM kernel: sums of the K-slices of a launch, at most
 
 thread_local int g_last_hip_error = 0;
 
@@ -179,6 +180,7 @@ constexpr Option kOptions[LUTGEMM_OPTION_COUNT] = {
     {"LUTGEMM_MFMA_BLOCKS", 0},   {"LUTGEMM_PAIR_TABLES", 1},  {"LUTGEMM_SINGLE_ITEM", 1},
     {"LUTGEMM_CHAIN_BLOCKS", 0}, {"LUTGEMM_CHAIN_GRID", 0},  {"LUTGEMM_TWIN_ITEMS", 4},
     {"LUTGEMM_BLOCK_SCALED", 1}, {"LUTGEMM_POW2_CONVERT", 1},
+    {"LUTGEMM_TILE_MIN_M", 0},
 };
 std::atomic<int> g_option[LUTGEMM_OPTION_COUNT];
 std::once_flag g_option_once;
@@ -611,6 +613,104 @@ int run_mx(Problem &p, const Accum &acc)
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
+// ---- GEMM kernel for many activation rows ------------------------------------------------------------
+// Whether a call takes the GEMM kernel.  The fp16 matrix-core kernel, which row-wise problems of fitting sizes have
+// beside it, expands every plane again for every 32 rows, but has tiles of 64 outputs and meets its K-slices
+// in the accumulator words.  Measured (us, that kernel vs this one): 4096x4096x3 at 64 / 128 / 256 rows 14.4 / 18.8,
+// 17.1 / 26.4, 32.1 / 34.7; 11008x4096x2 27.4 / 23.6, 40.3 / 31.2, 79 / 43.5; 8192x8192x4 35.1 / 28.6, 67.7 / 44.4, 135 / 69;
+// 1024x28672x4 23.9 / 37.7, 34.6 / 59, 58 / 61.  The look-up kernel, the only other one of the other formats, takes four
+// rows at a time: 4096x4096x3 at 33 rows of int8 exponents 48 / 17.6, 13824x5120x2 104 / 33.
+bool tile_wanted(const Problem &p, int mode)
+{
+    const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
+    // (32-bit byte offsets into the operands)
+    const unsigned long long limit = 1ull << 32;
+    if ((unsigned long long)p.kwords * p.nb * p.N * 4 >= limit || (unsigned long long)p.M * p.K * 2 >= limit) return false;
+    if (is_block(mode) && (unsigned long long)p.K / 8 * p.nb * p.R * 3 >= limit) return false;
+    if (least > 0) return p.M >= least;
+    if (p.M < 33) return false;
+    if (p.M > 256) return true;
+    if (mfma_eligible(p, mode)) return (long)p.N * p.K >= 40000000 && p.N >= 4096;
+    return is_block(mode) || (long)p.M * p.N * p.K >= 200000000;
+}
+
+// K-slices a call may be cut into: none where their sums have no place (the entry point that allocates
+// nothing; a stream under capture whose buffer would have to grow is left uncut as well, so that reserved
+// accumulator words are all that a captured call needs).
+size_t tile_slices_allowed(const Accum &acc)
+{
+    if (acc.fixed) return 0;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(acc.stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return kTileSumBytes;
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    std::lock_guard<std::mutex> lock(g_ws_mutex);
+    return g_workspaces[std::make_pair(dev, acc.stream)].split_bytes;
+}
+
+// Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices: a workgroup each, two per CU.
+// `room`: bytes for the slices' sums.
+// Costs in microseconds, measured at three planes: a step of a 128-row tile takes 1.2 alone on its CU and
+// 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 4; the sums of the slices
+// are written and read at about 4 TB/s, by a second launch that costs another 4.
+void plan_tile(TileProblem &t, size_t room)
+{
+    constexpr long kCUs = 256;
+    t.tile_rows = t.M <= 64 ? 64 : 128;
+    t.n_tiles = (t.N + 255) / 256;
+    t.m_tiles = (t.M + t.tile_rows - 1) / t.tile_rows;
+    t.steps = (t.kwords + 3) / 4 * 2;
+    const long tiles = (long)t.n_tiles * t.m_tiles;
+    const double alone = t.tile_rows == 128 ? 1.2 : 0.9, beside = t.tile_rows == 128 ? 2.1 : 1.6;
+    double best_cost = 0.0;
+    for (int ks = 1; ks <= 16 && (ks == 1 || 2 * ks <= t.steps); ++ks) {
+        const int steps = ((t.steps + ks - 1) / ks + 1) & ~1;
+        const int slices = (t.steps + steps - 1) / steps;
+        if (slices != ks) continue;
+        const long wgs = tiles * slices;
+        if (ks > 1 && (wgs > 2 * kCUs || (size_t)ks * t.M * t.N * 4 > room)) break;
+        const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;
+        double cost = (double)rounds * (steps * beside + 4.0);
+        if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 4.0;
+        if (ks > 1) cost += 4.0 + 2.0 * (double)((size_t)ks * t.M * t.N * 4) / 4e6;
+        if (ks == 1 || cost < best_cost * 0.99) {
+            best_cost = cost;
+            t.ksplit = slices;
+            t.slice_steps = steps;
+        }
+    }
+}
+
+int run_tile(const Problem &p, int mode, const Accum &acc)
+{
+    TileProblem t{};
+    t.W = p.W;
+    t.alpha = p.alpha;
+    if (mode == kUniformF16) t.qbias = p.qbias;
+    t.x = p.x;
+    t.init = p.init;
+    t.out = p.out;
+    t.N = p.N;
+    t.K = p.K;
+    t.M = p.M;
+    t.kwords = p.kwords;
+    t.by_group_words = p.by_group_words;
+    t.R = p.R;
+    t.rows_per_group = p.rows_per_group;
+    t.mode = mode;
+    plan_tile(t, tile_slices_allowed(acc));
+    t.init_stride = p.init_stride;
+    t.overwrite = p.overwrite;
+    if (t.ksplit > 1) {
+        void *sums = nullptr;
+        const int rc = stream_split_buffer(acc.stream, (size_t)t.ksplit * t.M * t.N * 4, &sums);
+        if (rc != LUTGEMM_OK) return rc;
+        t.partial = (float *)sums;
+    }
+    const hipError_t e = launch_tile(t, p.nb, acc.stream);
+    return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
+}
+
 // `bias`: null = accumulate into out; otherwise *bias is the row every output row starts from (null:
 // zeros) and out is written, not read.
 int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, const void *x,
@@ -627,6 +727,7 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     } else if (bias) {
         p.overwrite = 1;
     }
+    if (tile_wanted(p, mode)) return run_tile(p, mode, acc);
     if (alpha_pow2 && mode == kRowF16 && mfma_eligible(p, mode) && p.M >= mfma_min_rows() && mx_wanted(p)) return run_mx(p, acc);
     int kernel = kLookup, mrows = 1;
     rc = plan_single(p, mode, &kernel, &mrows);
@@ -1363,6 +1464,33 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
     plan->k_slices = p.ksplit;
     plan->units_per_slice = p.sets_per_split;
     plan->needs_workspace = p.ksplit > 1;
+    return LUTGEMM_OK;
+}
+
+int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
+{
+    int rc = lutgemm_describe_plan(format, N, K, nb, groups, M, plan);
+    if (rc != LUTGEMM_OK) return rc;
+    alignas(16) static const uint64_t dummy[2] = {0, 0};
+    Problem p;
+    rc = fill_problem(p, format, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
+    if (rc != LUTGEMM_OK) return rc;
+    if (!tile_wanted(p, format)) return LUTGEMM_OK;
+    TileProblem t{};
+    t.N = N;
+    t.M = M;
+    t.kwords = p.kwords;
+    plan_tile(t, kTileSumBytes);
+    *plan = lutgemm_plan{};
+    plan->kernel = 3;
+    plan->workgroups = t.n_tiles * t.m_tiles * t.ksplit;
+    plan->rows_per_pass = t.tile_rows;
+    plan->row_chunks = t.m_tiles;
+    plan->tiles = t.n_tiles;
+    plan->tile_columns = 256;
+    plan->k_units = t.steps;
+    plan->k_slices = t.ksplit;
+    plan->units_per_slice = t.slice_steps;
     return LUTGEMM_OK;
 }
 

@@ -35,6 +35,10 @@ hipError_t launch_mx(const Problem &p, void *split, hipStream_t stream);
 inline int mx_chunk_rows(int M) { return M <= 5 ? 5 : M <= 8 ? 8 : 16; }
 inline size_t mx_split_bytes(int M, int K) { return (size_t)M * K * 3 + (size_t)K + (size_t)M * (K / 32) * 4; }
 
+// GEMM kernel for many activation rows, every alpha format; one wave per SIMD and 256 outputs per workgroup
+struct TileProblem;
+hipError_t launch_tile(const TileProblem &p, int nb, hipStream_t stream);
+
 }  // namespace lutgemm
 
 #endif

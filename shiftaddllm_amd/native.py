@@ -43,6 +43,7 @@ C_ABI_SYMBOLS = (
     "lutgemm_reserve_workspace",
     "lutgemm_describe_plan",
     "lutgemm_describe_pow2_plan",
+    "lutgemm_describe_tile_plan",
     "lutgemm_set_option",
     "lutgemm_set_timestamp_buffer",
     "lutgemm_get_option",
@@ -57,7 +58,7 @@ C_ABI_SYMBOLS = (
 
 MAX_GROUP = 8
 OPTIONS = {"TARGET_BLOCKS": 0, "FIRST_SHARE": 1, "MFMA_MIN_M": 2, "MFMA_BLOCKS": 3, "PAIR_TABLES": 4, "SINGLE_ITEM": 5,
-           "CHAIN_BLOCKS": 6, "CHAIN_GRID": 7, "TWIN_ITEMS": 8, "BLOCK_SCALED": 9, "POW2_CONVERT": 10}
+           "CHAIN_BLOCKS": 6, "CHAIN_GRID": 7, "TWIN_ITEMS": 8, "BLOCK_SCALED": 9, "POW2_CONVERT": 10, "TILE_MIN_M": 11}
 CHAIN_MAX_ROWS = 4
 CHAIN_MAX_TAG = 65534
 NOALLOC_MAX_WORDS = 1 << 18
@@ -182,6 +183,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.lutgemm_copy_bytes.restype = ci
     lib.lutgemm_describe_plan.argtypes = [ci, ci, ci, ci, ci, ci, ctypes.POINTER(Plan)]
     lib.lutgemm_describe_plan.restype = ci
+    lib.lutgemm_describe_tile_plan.argtypes = [ci, ci, ci, ci, ci, ci, ctypes.POINTER(Plan)]
+    lib.lutgemm_describe_tile_plan.restype = ci
     lib.lutgemm_describe_pow2_plan.argtypes = [ci, ci, ci, ci, ci, ctypes.POINTER(Plan)]
     lib.lutgemm_describe_pow2_plan.restype = ci
     lib.lutgemm_set_option.argtypes = [ci, ci]
