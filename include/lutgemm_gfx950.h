@@ -112,11 +112,7 @@ int lutgemm_gemv_rowwise_f16(const uint32_t *bW, const void *alpha_f16, const vo
  * largest of its 32; smaller ones are cut off at 2^-25 of it); the three pieces of up to
  * 5 rows share the 16 columns of one instruction.  Accumulation is fp32, one rounding to
  * fp16 at the end, as in every other entry point.  An infinity or NaN among the activations
- * gives NaN in every output of its row.  Calls of up to 16 rows that take the fp16
- * matrix-core kernel with long K extents per workgroup form their sign operands through
- * the same kind of table and gfx950's scaled fp4 -> fp16 conversion (option
- * LUTGEMM_OPTION_POW2_CONVERT): the same exact products as lutgemm_gemv_rowwise_f16,
- * summed in another order.  Other calls run exactly as lutgemm_gemv_rowwise_f16 does.  With an alpha that breaks the promise the result is that
+ * gives NaN in every output of its row.  Other calls run exactly as lutgemm_gemv_rowwise_f16 does.  With an alpha that breaks the promise the result is that
  * of the alpha with its mantissa bits cleared (zero counts as 2^-15).
  * The split activations (3 * M * K + K + M * K / 8 bytes) live in a second per-stream
  * buffer that grows like the accumulator workspace: make one call of each size before
@@ -302,13 +298,15 @@ typedef struct lutgemm_plan {
 } lutgemm_plan;
 
 int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
-/* Calls of many rows (33 and more; where the fp16 matrix-core kernel applies as well, large ones), in every format, run on the GEMM
- * kernel instead, whose plan this returns: kernel 3, rows_per_pass 64 or 128, tiles of 256 columns, k_units
- * and units_per_slice in steps of 64 inputs, k_slices that a second launch adds up (their sums live in the
- * per-stream buffer of the split activations; a call under capture whose buffer is too small, and
- * lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order).  A call that takes
- * one of the other kernels is described as lutgemm_describe_plan describes it; that function itself
- * describes the look-up and fp16 matrix-core kernels for any row count. */
+/* What a call of two rows and more takes, in every format.  lutgemm_describe_plan describes the look-up
+ * kernel and, for row-wise problems whose sizes fit it (K a multiple of 128, groups of a multiple of 128
+ * inputs, N a multiple of 16), the matrix-core kernel; beyond those, from two or three rows on, the
+ * matrix-core kernel takes every problem whose tiles of 64 columns touch at most four alpha row groups
+ * (kernel 1), and calls of many rows run on the GEMM kernel (kernel 3: rows_per_pass 64 or 128, tiles of
+ * 256 columns, k_units and units_per_slice in steps of 64 inputs, k_slices that a second launch adds up;
+ * their sums live in the per-stream buffer of the split activations; a call under capture whose buffer is
+ * too small, and lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order).
+ * A call that neither takes is described as lutgemm_describe_plan describes it. */
 int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
 /* The same for lutgemm_gemv_rowwise_pow2_f16: kernel 2 is the block-scaled matrix-core kernel
  * (rows_per_pass 5, 8 or 16; tiles of 64 columns, steps of 128 inputs); a call that takes one
@@ -340,12 +338,8 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
  *                   kernel 1 = where it is the faster one (few rows, large matrices),
  *                   2 = wherever it applies, 0 = never (the call then behaves like
  *                   lutgemm_gemv_rowwise_f16); default 1
- *   POW2_CONVERT  : calls of lutgemm_gemv_rowwise_pow2_f16 that take the fp16 matrix-core
- *                   kernel form its sign operands through an LDS table and the scaled
- *                   fp4 -> fp16 conversion instruction (which applies a power-of-two alpha
- *                   as its scale) instead of a shift and a bit operation per fp16 pair
- *                   1 = where that is faster (up to 16 rows, six or more rounds of K-steps
- *                   per workgroup), 2 = always, 0 = never; default 1
+ *   POW2_CONVERT  : no effect (it chose between two ways of expanding sign planes, which the
+ *                   matrix-core kernel no longer does)
  *   TILE_MIN_M    : rows from which a call takes the GEMM kernel (0 = by sizes; a large value switches
  *                   that kernel off)
  *   CHAIN_GRID    : workgroups of a chained launch (0 = as many as the device holds

@@ -19,9 +19,18 @@
 #ifndef LUT_DEQUANT_DEVICE_H
 #define LUT_DEQUANT_DEVICE_H
 
+#include <type_traits>
+
 #include "lutgemm_common.h"
 
 namespace lutgemm {
+
+// how alphas are laid out, as far as forming weights goes
+enum WeightFormat : int {
+    kWeightRow = 0,      // one alpha per (group of inputs, plane, output)
+    kWeightUniform = 1,  // alpha and q_bias per (group of inputs, output)
+    kWeightBlock = 2,    // one alpha per (8 inputs, plane, row group)
+};
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -226,6 +235,55 @@ __device__ __forceinline__ u32x4 pick_weights(uint32_t y, const WeightTable<NB, 
         out[2 * half + 1] = __builtin_amdgcn_perm(h, l, 0x07030602u);
     }
     return (u32x4){out[0], out[1], out[2], out[3]};
+}
+
+// ---- block formats: one multiplier, as it lies in memory and decoded --------------------------------------
+// `at`: its index, below `count`, the multipliers of the tensor (at least four).
+__device__ __forceinline__ uint32_t raw_multiplier(const void *alpha, int mode, uint32_t at, uint32_t count)
+{
+    if (mode == kBlockApotI8) {   // three bytes, as part of four that lie inside the tensor
+        const uint32_t from = min(3u * at, 3u * count - 4u);
+        uint32_t v;
+        __builtin_memcpy(&v, (const char *)alpha + from, 4);
+        return v >> (8u * (3u * at - from));
+    }
+    return (uint32_t) * (const uint16_t *)((const char *)alpha + 2u * at);
+}
+
+__device__ __forceinline__ float decode_multiplier(uint32_t u, int mode)
+{
+    if (mode == kBlockF16) return half_bits_to_float(u & 0xffffu);
+    if (mode == kBlockShiftU16) return (float)((1u << (u & 7u)) + (1u << ((u >> 3) & 7u)) + (1u << ((u >> 6) & 7u)));
+    float v = 0.0f;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {
+        const int x = (int)(int8_t)(u >> (8 * e));
+        v += x == -128 ? 0.0f : ldexpf(1.0f, x);
+    }
+    return v;
+}
+
+// ---- the power of two that keeps a wave's weights in the middle of fp16's range ---------------------------
+__device__ __forceinline__ float wave_max_finite(float v)   // of |v| over the 64 lanes; NaN and inf count as 0
+{
+    uint32_t m = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+    if (m >= 0x7f800000u) m = 0u;
+    auto other = [](uint32_t x, auto ctrl) {
+        return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, decltype(ctrl)::value, 0xf, 0xf, false);
+    };
+    m = max(m, other(m, std::integral_constant<int, 0xb1>()));    // quad_perm [1,0,3,2]
+    m = max(m, other(m, std::integral_constant<int, 0x4e>()));    // quad_perm [2,3,0,1]
+    m = max(m, other(m, std::integral_constant<int, 0x141>()));   // row_half_mirror
+    m = max(m, other(m, std::integral_constant<int, 0x140>()));   // row_mirror
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)m, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)m, 16);
+    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)m, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)m, 48);
+    return __builtin_bit_cast(float, max(max(a, b), max(c, d)));
+}
+
+__device__ __forceinline__ float unit_for(float most)   // brings `most` to 2^8 .. 2^9
+{
+    const int e = most > 0.0f ? (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127 : 8;
+    return ldexpf(1.0f, min(max(8 - e, -120), 120));
 }
 
 }  // namespace lutgemm

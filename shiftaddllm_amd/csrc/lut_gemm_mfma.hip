@@ -1,28 +1,36 @@
-// Matrix-core kernel instances (row-wise alpha, several activation rows).
+// Matrix-core kernel instances (a few activation rows, every alpha format).
 #include "lut_gemm_mfma_device.h"
 #include "lutgemm_launch.h"
 
 namespace lutgemm {
 namespace {
 
-template <int NB>
-hipError_t launch_nb(const Problem &p, int mt, bool pow2, hipStream_t stream)
+template <int NB, int FMT, bool OWN>
+hipError_t launch_fmt(const Problem &p, int mt, hipStream_t stream)
 {
     const dim3 grid((unsigned)p.n_blocks), block(kMfmaThreads);
-    const bool one = mt == 1 && p.sets_per_split == kMfmaWaves;  // one round per K-slice
-    if (pow2 && one)
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1, true, true>), grid, block, 0, stream, p);
-    else if (pow2 && mt == 2)
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 2, false, true>), grid, block, 0, stream, p);
-    else if (pow2)
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1, false, true>), grid, block, 0, stream, p);
-    else if (one)
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1, true>), grid, block, 0, stream, p);
+    const bool one = p.sets_per_split == kMfmaWaves;  // one round per K-slice
+    if (mt == 2 && one)
+        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 2, FMT, OWN, true>), grid, block, 0, stream, p);
     else if (mt == 2)
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 2>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 2, FMT, OWN, false>), grid, block, 0, stream, p);
+    else if (one)
+        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1, FMT, OWN, true>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((lut_gemm_mfma_kernel<NB, 1, FMT, OWN, false>), grid, block, 0, stream, p);
     return hipGetLastError();
+}
+
+template <int NB>
+hipError_t launch_nb(const Problem &p, int mt, hipStream_t stream)
+{
+    // tables shared by the wave need steps of 128 inputs inside one alpha group
+    const bool own = p.K % kMfmaStepK != 0 || p.group_words % 4 != 0;
+    if (p.alpha_mode == kRowF16)
+        return own ? launch_fmt<NB, kWeightRow, true>(p, mt, stream) : launch_fmt<NB, kWeightRow, false>(p, mt, stream);
+    if (p.alpha_mode == kUniformF16)
+        return own ? launch_fmt<NB, kWeightUniform, true>(p, mt, stream) : launch_fmt<NB, kWeightUniform, false>(p, mt, stream);
+    return launch_fmt<NB, kWeightBlock, false>(p, mt, stream);
 }
 
 template <int NB>
@@ -50,13 +58,13 @@ hipError_t launch_mfma_fused(const Problem &p, int mt, hipStream_t stream)
     }
 }
 
-hipError_t launch_mfma(const Problem &p, int mt, bool pow2, hipStream_t stream)
+hipError_t launch_mfma(const Problem &p, int mt, hipStream_t stream)
 {
     switch (p.nb) {
-    case 1: return launch_nb<1>(p, mt, pow2, stream);
-    case 2: return launch_nb<2>(p, mt, pow2, stream);
-    case 3: return launch_nb<3>(p, mt, pow2, stream);
-    default: return launch_nb<4>(p, mt, pow2, stream);
+    case 1: return launch_nb<1>(p, mt, stream);
+    case 2: return launch_nb<2>(p, mt, stream);
+    case 3: return launch_nb<3>(p, mt, stream);
+    default: return launch_nb<4>(p, mt, stream);
     }
 }
 

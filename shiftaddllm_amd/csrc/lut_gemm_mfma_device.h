@@ -1,125 +1,74 @@
-// Matrix-core kernel templates for BCQ linear layers with several activation rows on
-// MI355X (gfx950, wave64): row-wise alpha, the semantics of lut_gemm/mv_fp16_bias.hpp:
-// 498-579 in the ShiftAddLLM checkout extended to M rows.
+// Matrix-core kernel templates for BCQ linear layers with a few activation rows (2 to about 128) on MI355X
+// (gfx950, wave64), every alpha format: the semantics of lut_gemm/mv_fp16_bias.hpp:8-579 in the ShiftAddLLM
+// checkout extended to M rows.
 #ifndef LUT_GEMM_MFMA_DEVICE_H
 #define LUT_GEMM_MFMA_DEVICE_H
 
-#include "lutgemm_common.h"
+#include "lut_dequant_device.h"
 
 namespace lutgemm {
 
 // ---------------------------------------------------------------------------
-// Small-batch path (row-wise alpha, several activation rows): matrix cores.
+// A table look-up costs one LDS read and two VALU operations per sign byte PER ROW, so beyond a row or
+// two the look-up kernel is VALU/LDS bound.  Here every weight is formed once as fp16
+// (lut_dequant_device.h) and multiplied with 16 activation rows at a time by v_mfma_f32_16x16x32_f16.
+// Forming it costs about two to three vector instructions per weight, whatever the row count, which is
+// what bounds the kernel up to 32 rows; expanding each plane to +-alpha, as this kernel did before, cost
+// one per weight and plane and a matrix instruction per plane instead of one per weight.
 //
-// Table look-ups cost one LDS read and two VALU operations per sign byte PER
-// ROW, so beyond a couple of rows the look-up kernel is VALU/LDS bound
-// (measured: ~21 us per extra row on a 132 MB matrix whose stream takes 18 us).
-// Here the sign bits are expanded to +-alpha fp16 in registers (one VALU
-// operation per two signs plus the shift that brings them into place) and
-// multiplied with 16 activation rows at a time by v_mfma_f32_16x16x32_f16, fp32
-// accumulation over all bit planes and groups: alpha is an fp16 number, so
-// +-alpha is exact and the products are the reference's alpha * (+-x).
+// Work split: a workgroup of 8 waves owns 64 outputs; its waves take different K-steps (128 inputs = 4
+// sign words) and their accumulators meet in LDS at the end, so that the number of cross-workgroup
+// atomics does not grow with the K parallelism.  Lane l (li = l&15, kb = l>>4) loads the sign words of
+// outputs n = base + 4*li .. +3 for word kb of its step (256-byte runs per row).  Matrix instruction
+// (e, c) takes from every lane the eight weights of byte c of its word of output e: its A rows are
+// outputs base + 4*i + e and its K block kb is byte c of word kb.
 //
-// Work split: a workgroup of 8 waves owns 64 outputs; its waves take different
-// K-steps (128 inputs = 4 sign words, inside one alpha group) and their
-// accumulators meet in LDS at the end, so that the number of cross-workgroup
-// atomics does not grow with the K parallelism.  Lane l (li = l&15, kb = l>>4)
-// loads the four sign words of outputs n = base + 4*li .. +3 for word kb of its
-// step (256-byte runs per row).  MFMA instance (e, beta) takes from every lane 8
-// signs of its word e: bits 4*beta+i and 16+4*beta+i, i < 4 -- two bits 16 apart
-// land in the sign positions of a packed fp16 pair with ONE shift and ONE
-// three-input bit operation.  So the instance's A rows are outputs base + 4*i + e
-// and its K block kb is word kb.
+// Tables.  Where the step lies in one alpha group, or the alphas are per block, a step needs 64 tables for
+// a wave (one per output) or 16 (one per 8 inputs and row group): lane (li, kb) forms the one of output
+// base + 4*li + kb, or of chunk li and row group kb, and the lanes hand them round by ds_bpermute.
+// Shorter groups (OWN) leave every lane with four tables of its own.
 //
-// Nothing is staged through LDS in the main loop and there is no barrier in it: a
-// lane's B operands of a step are the 32 activations of row li under its word kb,
-// 64 contiguous bytes that it loads itself (L2 hits: the activations are M*K*2
-// bytes in all), and instance beta's operand is halves 4*beta+i and 16+4*beta+i of
-// them, paired like the signs by four byte permutes.  Each wave runs its own
-// two-deep pipeline of (signs, alphas, activations) and the waves of a workgroup
-// drift freely until the final reduction.
+// Nothing is staged through LDS in the main loop and there is no barrier in it: a lane's B operands of a
+// step are the 32 activations of row li under its word kb, 64 contiguous bytes that it loads itself
+// (L2 hits).  Each wave runs its own two-deep pipeline of (signs, scales, activations) and the waves of
+// a workgroup drift freely until the final reduction.
 // ---------------------------------------------------------------------------
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-
 constexpr int kMfmaThreads = 512;
 constexpr int kMfmaWaves = kMfmaThreads / 64;
 constexpr int kMfmaTileCols = 64;     // outputs per workgroup
 constexpr int kMfmaStepK = 128;
+constexpr int kMfmaMaxRowGroups = 4;  // alpha row groups 64 outputs may touch (block formats)
 constexpr int kRedRow = 65;           // the final reduction's LDS rows, padded against bank conflicts
 template <int MT>
 constexpr int kMfmaRedBytes = kMfmaWaves * 16 * MT * kRedRow * 4;
-// POW2 instances keep a 64 KiB table in front (sign byte -> eight 4-bit floats, see mfma_tile); the
-// final reduction takes its place afterwards, the rows' reciprocal RMS sit behind both.
-constexpr int kSignLutBytes = 256 * 64 * 4;   // 256 entries x 64 copies: copy l for lane l, one bank per lane of a half-wave
-template <int MT, bool POW2 = false>
-constexpr int kMfmaScaleOffset = (POW2 && kSignLutBytes > kMfmaRedBytes<MT>) ? kSignLutBytes : kMfmaRedBytes<MT>;
-template <int MT, bool POW2 = false>
-constexpr int kMfmaLdsBytes = kMfmaScaleOffset<MT, POW2> + 16 * MT * 4;
+// the rows' reciprocal RMS sit behind the final reduction
+template <int MT>
+constexpr int kMfmaLdsBytes = kMfmaRedBytes<MT> + 16 * MT * 4;
 
-// Operands of one K-step of a wave: per bit plane word kb of 4 outputs; the alphas of
-// those 4 outputs for bit plane kb (one load covers all planes: lane group kb of the wave
-// takes plane kb, and hands them to the other groups by lane permutes when the plane's
-// turn comes); per 16-row tile the lane's 32 activations.
-template <int NB, int MT>
+// Operands of one K-step of a wave: per bit plane word kb of 4 outputs; per 16-row tile the lane's 32
+// activations; the scales of the lane's table(s), as they lie in memory.
+template <int NB, int MT, int FMT, bool OWN>
 struct MfmaOperands {
+    static constexpr int kScales = FMT == kWeightUniform ? (OWN ? 4 : 2) : (OWN ? 2 * NB : NB);
     u32x4 w[NB];
-    u32x2 alpha;
     u32x4 x[MT][4];
+    uint32_t s[kScales];
 };
 
-template <int NB, int MT>
-__device__ __forceinline__ void mfma_load(MfmaOperands<NB, MT> &r, const Problem &p, int step, int kb, uint32_t wcol4,
-                                          const __half *const (&xlane)[MT])
-{
-    const uint32_t row_bytes = (uint32_t)p.N * 4u;
-    const char *wbase = (const char *)p.W + (size_t)step * 4 * NB * row_bytes;
-    const uint32_t wrow = (uint32_t)kb * (NB * row_bytes);
-#pragma unroll
-    for (int b = 0; b < NB; ++b)
-        r.w[b] = __builtin_nontemporal_load((const u32x4 *)(wbase + (size_t)b * row_bytes + (wrow + wcol4)));
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) r.x[mt][c] = *(const u32x4 *)(xlane[mt] + step * kMfmaStepK + 8 * c);
-    const int g = fast_div(step * 4, p.by_group_words);
-    const char *abase = (const char *)p.alpha + (size_t)g * NB * (p.N * 2u) + (wcol4 >> 1);
-    r.alpha = *(const u32x2 *)(abase + (size_t)min(kb, NB - 1) * (p.N * 2u));
-}
-
-// 8 signs of sign word `w` -> 8 fp16 values +-alpha (bit set = +alpha): pair i holds
-// bit 4*beta+i (low half) and bit 16+4*beta+i (high half).  `alpha2` is the output's
-// alpha in both halves; the sign rides on it, so the matrix cores multiply and add
-// alpha * sign * x directly and no per-plane scaling of partial sums is left over.
-__device__ __forceinline__ f16x8 expand_signs(uint32_t w, int beta, uint32_t alpha2)
-{
-    // (~shifted & 0x80008000) ^ alpha2 as ONE three-input bit operation (truth table
-    // 0xa6 = (~a & b) ^ c); the compiler otherwise emits not + and + xor.
-    const uint32_t sign = 0x80008000u;
-    u32x4 r;
-    r.x = __builtin_amdgcn_bitop3_b32(w << (15 - (4 * beta + 0)), sign, alpha2, 0xa6);
-    r.y = __builtin_amdgcn_bitop3_b32(w << (15 - (4 * beta + 1)), sign, alpha2, 0xa6);
-    r.z = __builtin_amdgcn_bitop3_b32(w << (15 - (4 * beta + 2)), sign, alpha2, 0xa6);
-    r.w = __builtin_amdgcn_bitop3_b32(w << (15 - (4 * beta + 3)), sign, alpha2, 0xa6);
-    return __builtin_bit_cast(f16x8, r);
-}
-
-// xs: kMfmaLdsBytes<MT, POW2> bytes of LDS for the final reduction (and, behind them, the
-// reciprocal RMS of the tile's rows).
+// xs: kMfmaLdsBytes<MT> bytes of LDS for the final reduction (and, behind them, the reciprocal RMS of the
+// tile's rows).
+// OWN: every lane forms its own four tables (per-column alphas with groups that are no multiple of 128
+//      inputs, or K no multiple of 128).
 // EXTRA: the launch honours the split-RMSNorm fields of the problem (next_in, sumsq_*).
 // ONE: every K-slice of the launch is a single round, i.e. a wave takes at most one step (the
 //      host's choice): nothing is requested beyond that step.
-// POW2: the caller promises that every alpha is a positive normal fp16 power of two.  Sign bits then
-//      become fp16 +-alpha without the per-pair shift and bit operation: a byte of the sign word
-//      (eight signs) indexes a table in LDS whose entries hold eight 4-bit floats +-1 (e2m1 codes
-//      0x2 / 0xA), and v_cvt_scalef32_pk_f16_fp4 turns two of them into a packed fp16 pair times a
-//      scale of which the hardware uses the exponent only (measured: scale 3.0 gives +-2), which for
-//      a power of two is the alpha itself.  One table read and four conversions per matrix
-//      instruction instead of eight vector operations, the eight signs come out in input order, so
-//      the activations need no permutes either.
-template <int NB, int MT, bool EXTRA = false, bool ONE = false, bool POW2 = false>
+template <int NB, int MT, int FMT = kWeightRow, bool OWN = false, bool EXTRA = false, bool ONE = false>
 __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, char *xs)
 {
+    constexpr bool UNI = FMT == kWeightUniform;
+    static_assert(!OWN || FMT != kWeightBlock, "block formats share their tables");
+    typedef MfmaOperands<NB, MT, FMT, OWN> Operands;
+    typedef WeightTable<NB, UNI> Table;
     const int tid = threadIdx.x;
     const int lane = tid & 63;
     const int wave = tid >> 6;
@@ -138,17 +87,76 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     const int step_end = min(step_begin + p.sets_per_split, p.nsets);
 
     // the lane's activations: row li of each 16-row tile (rows beyond M are clamped to
-    // the last one: computed twice, written once), the 32 inputs under word kb
+    // the last one: computed twice, written once)
     const __half *xlane[MT];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xlane[mt] = p.x + (size_t)min(m0 + 16 * mt + li, p.M - 1) * p.K + 32 * kb;
+    for (int mt = 0; mt < MT; ++mt) xlane[mt] = p.x + (size_t)min(m0 + 16 * mt + li, p.M - 1) * p.K;
+
+    // block formats: the tile's row groups; this lane forms tables of group rg and looks its own outputs up
+    // among those of lane group rg_of
+    [[maybe_unused]] int rg = 0, rg_of = 0;
+    if constexpr (FMT == kWeightBlock) {
+        const int rg0 = n_base / p.rows_per_group, n_rg = min(n_base + kMfmaTileCols - 1, p.N - 1) / p.rows_per_group - rg0 + 1;
+        rg = rg0 + min(kb, n_rg - 1);
+        rg_of = (int)(wcol4 >> 2) / p.rows_per_group - rg0;
+    }
+
+    auto load = [&](Operands &r, int step) {
+        // (a word beyond K, in the last step only: clamped; its weights are zero)
+        const int kbc = OWN || FMT == kWeightBlock ? min(kb, p.kwords - 1 - 4 * step) : kb;
+        const uint32_t row_bytes = (uint32_t)p.N * 4u;
+        const char *wbase = (const char *)p.W + (size_t)step * 4 * NB * row_bytes;
+        const uint32_t wrow = (uint32_t)kbc * (NB * row_bytes);
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+            r.w[b] = __builtin_nontemporal_load((const u32x4 *)(wbase + (size_t)b * row_bytes + (wrow + wcol4)));
+        if constexpr (FMT == kWeightBlock) {
+            const int rows = p.K / 8 * NB;
+#pragma unroll
+            for (int b = 0; b < NB; ++b)
+                r.s[b] = raw_multiplier(p.alpha, p.alpha_mode, (uint32_t)(min(16 * step + li, p.K / 8 - 1) * NB + b) * (uint32_t)p.R + (uint32_t)rg,
+                                        (uint32_t)rows * (uint32_t)p.R);
+        } else if constexpr (OWN) {
+            const uint32_t g = (uint32_t)fast_div(4 * step + kbc, p.by_group_words);
+            if constexpr (UNI) {
+                const uint32_t at = g * (p.N * 2u) + (wcol4 >> 1);
+                const u32x2 a = *(const u32x2 *)((const char *)p.alpha + at), q = *(const u32x2 *)((const char *)p.qbias + at);
+                r.s[0] = a.x;
+                r.s[1] = a.y;
+                r.s[2] = q.x;
+                r.s[3] = q.y;
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b) {
+                    const u32x2 a = *(const u32x2 *)((const char *)p.alpha + ((g * NB + (uint32_t)b) * (p.N * 2u) + (wcol4 >> 1)));
+                    r.s[2 * b] = a.x;
+                    r.s[2 * b + 1] = a.y;
+                }
+            }
+        } else {
+            const int g = fast_div(step * 4, p.by_group_words);
+            const uint32_t col2 = (wcol4 >> 1) + 2u * (uint32_t)kb;
+            if constexpr (UNI) {
+                r.s[0] = *(const unsigned short *)((const char *)p.alpha + (size_t)g * (p.N * 2u) + col2);
+                r.s[1] = *(const unsigned short *)((const char *)p.qbias + (size_t)g * (p.N * 2u) + col2);
+            } else {
+#pragma unroll
+                for (int b = 0; b < NB; ++b)
+                    r.s[b] = *(const unsigned short *)((const char *)p.alpha + (size_t)(g * NB + b) * (p.N * 2u) + col2);
+            }
+        }
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) r.x[mt][c] = *(const u32x4 *)(xlane[mt] + (4 * step + kbc) * 32 + 8 * c);
+    };
 
     // split RMSNorm, consuming side: wave w sums the slots of rows w, w + 8, ... and leaves
     // their reciprocal RMS in LDS for the hand-over
     // The slots are requested here, ahead of everything else, and summed once the first
     // step's operands have been requested behind them (see the main loop): loads return in
     // order, so that wait is for the slots alone.
-    float *row_scale = (float *)(xs + kMfmaScaleOffset<MT, POW2>);
+    float *row_scale = (float *)(xs + kMfmaRedBytes<MT>);
     typedef float f32x4v __attribute__((ext_vector_type(4)));
     constexpr int kScaleRows = 2 * MT;  // rows per wave
     bool scaled = false;
@@ -187,86 +195,119 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[e][mt] = (f32x4){0.0f, 0.0f, 0.0f, 0.0f};
 
-    // POW2: the sign table.  Entry i, copy c at byte i * 256 + 4 * c; lane l reads copy l, so one
-    // v_perm_b32 of (sign word, per-lane constant) is the address: index byte in bits 8..15, the
-    // lane's copy offset in bits 0..7.
-    [[maybe_unused]] const uint32_t lane_off = (uint32_t)(4 * lane) * 0x01010101u;
-    if constexpr (POW2) {
-        uint32_t *lut = (uint32_t *)xs;
-#pragma unroll 4
-        for (int idx = tid; idx < kSignLutBytes / 4; idx += kMfmaThreads) {   // a wave writes one entry's 64 copies
-            // (the entry index is the same for the whole wave: scalar arithmetic)
-            uint32_t v = (uint32_t)__builtin_amdgcn_readfirstlane(idx >> 6);   // bit j of it -> bit 4 * j + 3
-            v = (v | (v << 12)) & 0x000f000fu;
-            v = (v | (v << 6)) & 0x03030303u;
-            v = (v | (v << 3)) & 0x11111111u;
-            lut[idx] = 0xaaaaaaaau ^ (v << 3);
+    // ---- one K-step ---------------------------------------------------------------------------------
+    constexpr int kTables = OWN ? 4 : 1;   // tables this lane forms
+    float unit = 0.0f;                     // weights are formed as W * unit, a power of two; 0: not chosen yet
+    // multipliers of this lane's table i
+    auto multipliers = [&](const Operands &ops, int i, float (&a)[NB], float &q) {
+        q = 0.0f;
+        auto half_of = [&](int r) { return half_bits_to_float((ops.s[r + (i >> 1)] >> (16 * (i & 1))) & 0xffffu); };   // (OWN)
+        if constexpr (FMT == kWeightBlock) {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) a[b] = decode_multiplier(ops.s[b], p.alpha_mode);
+        } else if constexpr (UNI) {
+            const float alpha = OWN ? half_of(0) : half_bits_to_float(ops.s[0]);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) a[b] = alpha * (1.0f / (float)(2 << b));
+            q = OWN ? half_of(2) : half_bits_to_float(ops.s[1]);
+        } else {
+#pragma unroll
+            for (int b = 0; b < NB; ++b) a[b] = OWN ? half_of(2 * b) : half_bits_to_float(ops.s[b]);
         }
-        __syncthreads();
-    }
-
-    auto compute = [&](const MfmaOperands<NB, MT> &ops) {
+    };
+    auto largest = [&](const Operands &ops) {   // upper bound of |W| in the step
+        float most = 0.0f;
 #pragma unroll
-        for (int b = 0; b < NB; ++b) {
-            const uint32_t w4[4] = {ops.w[b].x, ops.w[b].y, ops.w[b].z, ops.w[b].w};
-            const int from = 4 * (16 * b + li);   // the lane of group b that holds this lane's outputs
-            const u32x2 al = {(uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)ops.alpha.x),
-                              (uint32_t)__builtin_amdgcn_ds_bpermute(from, (int)ops.alpha.y)};
-            if constexpr (POW2) {
-                // the alpha of output e as the conversion's fp32 scale
-                const float scale[4] = {half_bits_to_float(al.x & 0xffffu), half_bits_to_float(al.x >> 16),
-                                        half_bits_to_float(al.y & 0xffffu), half_bits_to_float(al.y >> 16)};
-                constexpr uint32_t sel[4] = {0x0c0c0400u, 0x0c0c0501u, 0x0c0c0602u, 0x0c0c0703u};
+        for (int i = 0; i < kTables; ++i) {
+            float a[NB], q, s;
+            multipliers(ops, i, a, q);
+            s = fabsf(q);
 #pragma unroll
-                for (int beta = 0; beta < 4; ++beta) {
-                    // byte beta of the sign word = inputs 8 * beta .. + 7 of the lane's 32, in order
-                    f16x8 bx[MT];
+            for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
+            most = fmaxf(most, s);
+        }
+        return wave_max_finite(most);
+    };
+    // The lane's tables of a step, or of what rounding their entries leaves over; true when some entry is
+    // not an fp16 number.
+    auto make_tables = [&](const Operands &ops, int step, bool lo, Table (&tab)[kTables]) {
+        float u = unit;
+        if constexpr (FMT == kWeightBlock) u = 16 * step + li < p.K / 8 ? u : 0.0f;
+        if constexpr (OWN) u = 4 * step + kb < p.kwords ? u : 0.0f;
+        bool inexact = false;
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) bx[mt] = __builtin_bit_cast(f16x8, ops.x[mt][beta]);
+        for (int i = 0; i < kTables; ++i) {
+            float a[NB], q;
+            multipliers(ops, i, a, q);
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const uint32_t nib = *(const uint32_t *)(xs + __builtin_amdgcn_perm(w4[e], lane_off, sel[beta]));
-                        typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-                        const f16x2 p0 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib, scale[e], 0);
-                        const f16x2 p1 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib, scale[e], 1);
-                        const f16x2 p2 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib, scale[e], 2);
-                        const f16x2 p3 = __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(nib, scale[e], 3);
-                        const f16x8 a = {p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+            for (int b = 0; b < NB; ++b) a[b] *= u;
+            const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u), r = table_residual(e);
+            inexact = inexact || any_nonzero(r);
+            if (lo)
+                pack_table(r, tab[i]);
+            else
+                pack_table(e, tab[i]);
+        }
+        return inexact;
+    };
+    auto from_lane = [&](const Table &t, int src) {
+        Table r;
 #pragma unroll
-                        for (int mt = 0; mt < MT; ++mt)
-                            acc[e][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bx[mt], acc[e][mt], 0, 0, 0);
-                    }
-                }
-                continue;
+        for (int i = 0; i < Table::kRegs; ++i) {
+            r.hi[i] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)t.hi[i]);
+            r.lo[i] = (uint32_t)__builtin_amdgcn_ds_bpermute(4 * src, (int)t.lo[i]);
+        }
+        return r;
+    };
+    auto multiply = [&](const Operands &ops, const Table (&tab)[kTables]) {
+        Table t4[4];   // per output, or (block formats) per byte of the word
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            if constexpr (OWN)
+                t4[i] = tab[i];
+            else if constexpr (FMT == kWeightBlock)
+                t4[i] = from_lane(tab[0], 16 * rg_of + 4 * kb + i);
+            else
+                t4[i] = from_lane(tab[0], 16 * i + li);
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            uint32_t w[NB], y[4];
+#pragma unroll
+            for (int b = 0; b < NB; ++b) {
+                w[b] = ops.w[b][e];
+                asm volatile("" : "+v"(w[b]));   // (opaque: or the indices are kept for a second piece)
             }
-            // the alpha of output e in both halves of a register
-            const uint32_t a2[4] = {__builtin_amdgcn_perm(al.x, al.x, 0x01000100u), __builtin_amdgcn_perm(al.x, al.x, 0x03020302u),
-                                    __builtin_amdgcn_perm(al.y, al.y, 0x01000100u), __builtin_amdgcn_perm(al.y, al.y, 0x03020302u)};
+            sign_indices<NB, UNI>(w, y);
 #pragma unroll
-            for (int beta = 0; beta < 4; ++beta) {
-                f16x8 bx[MT];
+            for (int c = 0; c < 4; ++c) {
+                const f16x8 a = __builtin_bit_cast(f16x8, pick_weights<NB, UNI>(y[c], t4[FMT == kWeightBlock ? c : e]));
 #pragma unroll
-                for (int mt = 0; mt < MT; ++mt) {
-                    // halves 4*beta+i and 16+4*beta+i of the lane's 32 activations, interleaved
-                    // like the sign pairs
-                    const u32x4 lo4 = ops.x[mt][beta >> 1], hi4 = ops.x[mt][2 + (beta >> 1)];
-                    const uint32_t lo0 = (beta & 1) ? lo4.z : lo4.x, lo1 = (beta & 1) ? lo4.w : lo4.y;
-                    const uint32_t hi0 = (beta & 1) ? hi4.z : hi4.x, hi1 = (beta & 1) ? hi4.w : hi4.y;
-                    u32x4 v;
-                    v.x = __builtin_amdgcn_perm(hi0, lo0, 0x05040100u);
-                    v.y = __builtin_amdgcn_perm(hi0, lo0, 0x07060302u);
-                    v.z = __builtin_amdgcn_perm(hi1, lo1, 0x05040100u);
-                    v.w = __builtin_amdgcn_perm(hi1, lo1, 0x07060302u);
-                    bx[mt] = __builtin_bit_cast(f16x8, v);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const f16x8 a = expand_signs(w4[e], beta, a2[e]);
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt)
-                        acc[e][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, bx[mt], acc[e][mt], 0, 0, 0);
-                }
+                for (int mt = 0; mt < MT; ++mt)
+                    acc[e][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(f16x8, ops.x[mt][c]), acc[e][mt], 0, 0, 0);
             }
+        }
+    };
+    auto compute = [&](const Operands &ops, int step) {
+        if (unit == 0.0f) unit = unit_for(largest(ops));
+        Table tab[kTables];
+        const bool inexact = __builtin_amdgcn_ballot_w64(make_tables(ops, step, false, tab)) != 0ull;
+        if (inexact) {
+            const float most = largest(ops);
+            if (most * unit > 32768.0f) {   // out of fp16's range: another unit first
+                const float fresh = unit_for(most), by = fresh / unit;
+                unit = fresh;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int mt = 0; mt < MT; ++mt) acc[e][mt] *= by;
+                (void)make_tables(ops, step, false, tab);
+            }
+        }
+        multiply(ops, tab);
+        if (inexact) {
+            (void)make_tables(ops, step, true, tab);
+            multiply(ops, tab);
         }
     };
 
@@ -277,21 +318,21 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // iteration skips its first compute at run time, and a load beyond the wave's last
     // step re-reads that last step (the lines the wave has just asked for) and is
     // discarded, so that the waits can count it.
-    MfmaOperands<NB, MT> opA, opB;
+    Operands opA, opB;
     const int last_step = p.nsets - 1;
-    const int first_step = step_begin + wave;
+    const int first_step = step_begin + wave_s;
     const int n_steps = first_step < step_end ? (step_end - first_step + kMfmaWaves - 1) / kMfmaWaves : 0;
     const int own_last = n_steps > 0 ? first_step + kMfmaWaves * (n_steps - 1) : last_step;
     const int pairs = ONE ? 0 : (n_steps + 1) / 2;
     if constexpr (ONE) {
         // One round per slice: the general loop would request a second, discarded step behind
         // the first one, and a wave cannot end before those loads have come back.
-        mfma_load<NB, MT>(opA, p, min(first_step, last_step), kb, wcol4, xlane);
+        load(opA, min(first_step, last_step));
         __builtin_amdgcn_sched_barrier(0);
         if constexpr (EXTRA)
             if (scaled) row_scales();
         __builtin_amdgcn_sched_barrier(0);
-        if (n_steps > 0) compute(opA);
+        if (n_steps > 0) compute(opA, first_step);
     }
 #pragma clang loop unroll(disable)
     for (int j = 0; j < pairs; ++j) {
@@ -299,24 +340,28 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         int first = __builtin_amdgcn_readfirstlane(j == 0);
         asm volatile("" : "+s"(first));
         const int s = first_step + 2 * kMfmaWaves * j;
-        mfma_load<NB, MT>(opA, p, min(s, own_last), kb, wcol4, xlane);
+        load(opA, min(s, own_last));
         __builtin_amdgcn_sched_barrier(0);
-        if (!first) compute(opB);
+        if (!first) compute(opB, s - kMfmaWaves);
         if constexpr (EXTRA)
             if (first && scaled) row_scales();
         __builtin_amdgcn_sched_barrier(0);
-        mfma_load<NB, MT>(opB, p, min(s + kMfmaWaves, own_last), kb, wcol4, xlane);
+        load(opB, min(s + kMfmaWaves, own_last));
         __builtin_amdgcn_sched_barrier(0);
-        compute(opA);
+        compute(opA, s);
     }
-    if (!ONE && n_steps > 0 && (n_steps & 1) == 0) compute(opB);
+    if (!ONE && n_steps > 0 && (n_steps & 1) == 0) compute(opB, own_last);
     if constexpr (EXTRA && !ONE)
         if (n_steps == 0 && scaled) row_scales();  // (a wave without steps still owes its rows)
+    const float back = unit == 0.0f ? 1.0f : 1.0f / unit;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[e][mt] *= back;
 
     // ---- the 8 waves' accumulators meet in LDS -----------------------------------
     // red[wave][j = (e*MT + mt)*4 + r][lane], rows padded to 65 words so that the
     // read-out below (consecutive threads = consecutive outputs) spreads over the banks
-    if constexpr (POW2) __syncthreads();   // (the table's memory: every wave is done with it)
     float *red = (float *)xs;
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -387,24 +432,27 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     }
 }
 
-template <int NB, int MT, bool ONE = false, bool POW2 = false>
-__global__ void __launch_bounds__(kMfmaThreads) lut_gemm_mfma_kernel(const Problem p)
-{
-    __shared__ __attribute__((aligned(16))) char xs[kMfmaLdsBytes<MT, POW2>];
-    mfma_tile<NB, MT, false, ONE, POW2>(p, (int)blockIdx.x, xs);
-}
-
-// One problem with the split-RMSNorm fields honoured.
-template <int NB, int MT, bool ONE = false>
-__global__ void __launch_bounds__(kMfmaThreads) lut_gemm_mfma_fused_kernel(const Problem p)
+template <int NB, int MT, int FMT, bool OWN, bool ONE>
+__global__ void __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 4 : 2, MT == 1 ? 4 : 2)))
+lut_gemm_mfma_kernel(const Problem p)
 {
     __shared__ __attribute__((aligned(16))) char xs[kMfmaLdsBytes<MT>];
-    mfma_tile<NB, MT, true, ONE>(p, (int)blockIdx.x, xs);
+    mfma_tile<NB, MT, FMT, OWN, false, ONE>(p, (int)blockIdx.x, xs);
 }
 
-// Several problems in one launch; bit widths may differ.
+// One row-wise problem with the split-RMSNorm fields honoured.
+template <int NB, int MT, bool ONE = false>
+__global__ void __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 4 : 2, MT == 1 ? 4 : 2)))
+lut_gemm_mfma_fused_kernel(const Problem p)
+{
+    __shared__ __attribute__((aligned(16))) char xs[kMfmaLdsBytes<MT>];
+    mfma_tile<NB, MT, kWeightRow, false, true, ONE>(p, (int)blockIdx.x, xs);
+}
+
+// Several row-wise problems in one launch; bit widths may differ.
 template <int MT>
-__global__ void __launch_bounds__(kMfmaThreads) lut_gemm_mfma_group_kernel(const Group g)
+__global__ void __launch_bounds__(kMfmaThreads) __attribute__((amdgpu_waves_per_eu(MT == 1 ? 4 : 2, MT == 1 ? 4 : 2)))
+lut_gemm_mfma_group_kernel(const Group g)
 {
     __shared__ __attribute__((aligned(16))) char xs[kMfmaLdsBytes<MT>];
     // grid = (workgroups of the largest problem, problems)
@@ -414,10 +462,10 @@ __global__ void __launch_bounds__(kMfmaThreads) lut_gemm_mfma_group_kernel(const
     const int b = blockIdx.x;
     if (b >= p.n_blocks) return;
     switch (p.nb) {
-    case 1: mfma_tile<1, MT, true>(p, b, xs); break;
-    case 2: mfma_tile<2, MT, true>(p, b, xs); break;
-    case 3: mfma_tile<3, MT, true>(p, b, xs); break;
-    default: mfma_tile<4, MT, true>(p, b, xs); break;
+    case 1: mfma_tile<1, MT, kWeightRow, false, true>(p, b, xs); break;
+    case 2: mfma_tile<2, MT, kWeightRow, false, true>(p, b, xs); break;
+    case 3: mfma_tile<3, MT, kWeightRow, false, true>(p, b, xs); break;
+    default: mfma_tile<4, MT, kWeightRow, false, true>(p, b, xs); break;
     }
 }
 

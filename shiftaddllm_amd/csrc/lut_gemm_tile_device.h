@@ -30,10 +30,10 @@ constexpr int kTileStepK = 64;
 constexpr int kTileMaxRowGroups = 66;  // alpha row groups a tile of 256 outputs can touch (4 outputs each at least)
 
 enum TileFormat : int {
-    kTileRow = 0,        // one alpha per (group of inputs, plane, output)
-    kTileUniform = 1,    // alpha and q_bias per (group of inputs, output)
-    kTileBlock = 2,      // one alpha per (8 inputs, plane, row group)
-    kTileBlockWide = 3,  // the same where 64 outputs never straddle a row group
+    kTileRow = kWeightRow,
+    kTileUniform = kWeightUniform,
+    kTileBlock = kWeightBlock,
+    kTileBlockWide = 3,  // block format where 64 outputs never straddle a row group
 };
 
 template <int MF>
@@ -135,30 +135,12 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     [[maybe_unused]] ScaleSlot own{};
     if constexpr (BLOCK) own = scale_slot(min(tid, 8 * NB * n_rg - 1));
     [[maybe_unused]] auto raw_scale = [&](int t, const ScaleSlot &z) {
-        const int last = p.K / 8 * NB - 1;
-        const uint32_t at = (uint32_t)min(8 * NB * t + z.cb, last) * (uint32_t)p.R + (uint32_t)(rg0 + z.r);
-        if (p.mode == kBlockApotI8) {   // three bytes, as part of four that lie inside the tensor
-            const uint32_t from = min(3u * at, 3u * (uint32_t)(last + 1) * (uint32_t)p.R - 4u);
-            uint32_t v;
-            __builtin_memcpy(&v, (const char *)p.alpha + from, 4);
-            return v >> (8u * (3u * at - from));
-        }
-        return (uint32_t) * (const uint16_t *)((const char *)p.alpha + 2u * at);
+        const int rows = p.K / 8 * NB;
+        const uint32_t at = (uint32_t)min(8 * NB * t + z.cb, rows - 1) * (uint32_t)p.R + (uint32_t)(rg0 + z.r);
+        return raw_multiplier(p.alpha, p.mode, at, (uint32_t)rows * (uint32_t)p.R);
     };
     [[maybe_unused]] auto put_scale = [&](int t, const ScaleSlot &z, uint32_t u) {
-        float v = 0.0f;
-        if (p.mode == kBlockF16) {
-            v = half_bits_to_float(u & 0xffffu);
-        } else if (p.mode == kBlockShiftU16) {
-            v = (float)((1u << (u & 7u)) + (1u << ((u >> 3) & 7u)) + (1u << ((u >> 6) & 7u)));
-        } else {
-#pragma unroll
-            for (int e = 0; e < 3; ++e) {
-                const int x = (int)(int8_t)(u >> (8 * e));
-                v += x == -128 ? 0.0f : ldexpf(1.0f, x);
-            }
-        }
-        ((float *)stage_at(t))[z.dst] = v;
+        ((float *)stage_at(t))[z.dst] = decode_multiplier(u, p.mode);
     };
     auto fetch_scales = [&](int t) {
         if constexpr (BLOCK) {
@@ -225,13 +207,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     bool lo_cur = false;         // rounding the current step's weights to fp16 left something over (uniform over the wave)
     WeightTable<NB, UNI> tab[kFragTabs][kTabs];
     float unit = 1.0f;           // weights are formed as W * unit, a power of two
-    auto wave_max_bits = [&](float v) {
-        uint32_t m = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-        if (m >= 0x7f800000u) m = 0u;
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) m = max(m, (uint32_t)__shfl_xor((int)m, d));
-        return __builtin_bit_cast(float, m);
-    };
     auto largest = [&](int t) {   // upper bound of |W| in the step
         float most = 0.0f;
 #pragma unroll
@@ -245,11 +220,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                 for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
                 most = fmaxf(most, s);
             }
-        return wave_max_bits(most);
-    };
-    auto unit_for = [](float most) {   // power of two that brings `most` to 2^8 .. 2^9
-        const int e = most > 0.0f ? (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127 : 8;
-        return ldexpf(1.0f, min(max(8 - e, -120), 120));
+        return wave_max_finite(most);
     };
     // One table of step t, or of what its rounding leaves over; true when some entry is
     // not an fp16 number.

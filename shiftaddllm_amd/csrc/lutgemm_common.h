@@ -165,7 +165,7 @@ struct Problem {
     // x / gate / out point at TAGGED rows, one 32-bit word per value = fp16 bits | tag << 16
     // (see tagged_word below), x and gate are waited for, out is written with its tag.
     int x_tag, gate_tag, out_tag;
-    int reserved2_;
+    int alpha_mode;         // AlphaMode (matrix-core kernel, block formats)
 #ifdef LUTGEMM_TIMESTAMPS
     // Build with per-wave time stamps (the library variant bench.py --profile-phases loads):
     // kStampsPerWave readings of the 100 MHz wall clock per wave, at fixed points of the

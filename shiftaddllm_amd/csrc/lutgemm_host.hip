@@ -315,6 +315,7 @@ int fill_problem(Problem &p, int mode, const uint32_t *bW, const void *alpha, co
     p.K = K;
     p.M = M;
     p.nb = nb;
+    p.alpha_mode = mode;
     p.kwords = K / 32;
     p.nsets = (p.kwords + kSetWords - 1) / kSetWords;
     p.group_words = 1;
@@ -368,8 +369,8 @@ void plan_mfma(Problem &p, int mt, long want)
 {
     p.n_tiles = (p.N + kMfmaTileCols - 1) / kMfmaTileCols;
     p.mchunks = (p.M + 16 * mt - 1) / (16 * mt);
-    p.nsets = p.K / kMfmaStepK;  // K-steps
-    if (want > p.nsets / kMfmaWaves) want = p.nsets / kMfmaWaves;
+    p.nsets = (p.K + kMfmaStepK - 1) / kMfmaStepK;  // K-steps
+    if (want > (p.nsets + kMfmaWaves - 1) / kMfmaWaves) want = (p.nsets + kMfmaWaves - 1) / kMfmaWaves;
     if (want < 1) want = 1;
     if (want > kMaxSlices) want = kMaxSlices;
     p.sets_per_split = (p.nsets + (int)want - 1) / (int)want;
@@ -408,7 +409,7 @@ int mfma_slices(const Group &g, int mt)
     for (int i = 0; i < g.count; ++i) {
         const Problem &p = g.p[i];
         tiles += (long)((p.N + kMfmaTileCols - 1) / kMfmaTileCols) * ((p.M + 16 * mt - 1) / (16 * mt));
-        const int rounds = p.K / kMfmaStepK / kMfmaWaves;
+        const int rounds = ((p.K + kMfmaStepK - 1) / kMfmaStepK + kMfmaWaves - 1) / kMfmaWaves;
         if (rounds > max_rounds) max_rounds = rounds;
         if (p.M > rows) rows = p.M;
     }
@@ -437,9 +438,20 @@ int mfma_slices(const Group &g, int mt)
     return best;
 }
 
+// 16-row tiles per workgroup of a lone problem.  Two of them form each weight once for 32 rows; a call that fits
+// the chip as single rounds of 16-row tiles, two workgroups per CU, is bound by latencies and better spread
+// (us, one against two, 32 rows: 4096x4096x3 8.9 / 10.4, 768x3072x3 6.9 / 8.9, 3072x768x3 6.1 / 7.1;
+// 11008x4096x3, which does not fit, 17.3 / 15.2).
+int mfma_row_tiles(const Problem &p)
+{
+    if (p.M <= 16) return 1;
+    const long tiles = (p.N + kMfmaTileCols - 1) / kMfmaTileCols, steps = (p.K + kMfmaStepK - 1) / kMfmaStepK;
+    return p.M <= 64 && tiles * ((p.M + 15) / 16) * ((steps + kMfmaWaves - 1) / kMfmaWaves) <= 512 ? 1 : 2;
+}
+
 int run_mfma(Problem &p, const Accum &acc)
 {
-    const int mt = p.M > 16 ? 2 : 1;
+    const int mt = mfma_row_tiles(p);
     Group one{};
     one.count = 1;
     one.p[0] = p;
@@ -448,7 +460,7 @@ int run_mfma(Problem &p, const Accum &acc)
         int rc = accum_words(acc, (size_t)p.M * p.N, &p.accum);
         if (rc != LUTGEMM_OK) return rc;
     }
-    const hipError_t e = launch_mfma(p, mt, false, acc.stream);
+    const hipError_t e = launch_mfma(p, mt, acc.stream);
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
@@ -485,10 +497,31 @@ int run_mfma_group(Group &g, const Accum &acc)
 // Which kernel a lone problem runs on and how it is cut up (no device work).
 enum Kernel : int { kLookup = 0, kMatrixCore = 1 };
 
-int plan_single(Problem &p, int mode, int *kernel, int *mrows)
+// The matrix-core kernel also takes the other formats, alpha groups of any length and any K; 64 outputs may
+// touch four row groups at most.
+bool mfma_any(const Problem &p, int mode)
 {
-    if (mfma_eligible(p, mode)) {
-        const int mt = p.M > 16 ? 2 : 1;
+    // (two rows: the look-up kernel, whose time is that of the sign stream, wins on longer streams; us, look-up
+    // against this kernel: int8 exponents 4096x4096x3 7.5 / 6.5, 13824x5120x2 11.7 / 14.7; uniform 768x768x3
+    // 6.4 / 6.1, 4096x4096x4 7.3 / 9.5, where q_bias makes every weight two pieces)
+    // One row as well where a look-up tile of 256 outputs touches more than two row groups and every lane would
+    // fetch its own multipliers: int8 exponents 768x768x3 in 8 groups 10.3 / 5.1, 4096x4096x3 in 32 groups
+    // 14.8 / 6.8, 1600x28672x4 in 8 groups 35.7 / 18.8.
+    const int least = mfma_min_rows();
+    if (p.M < least) {
+        const long two_rows = mode == kUniformF16 ? 2l << 20 : 8l << 20;
+        const bool scattered = is_block(mode) && p.rows_per_group < kTileCols;
+        if (least != 3 || !(scattered || (p.M == 2 && (long)p.N * (p.K / 8) * p.nb <= two_rows))) return false;
+    }
+    if (is_block(mode))
+        return p.rows_per_group >= 24 && (unsigned long long)p.K / 8 * p.nb * p.R * 3 < (1ull << 32);
+    return (unsigned long long)p.kwords * p.nb * p.N * 2 < (1ull << 32);
+}
+
+int plan_single(Problem &p, int mode, int *kernel, int *mrows, bool any = true)
+{
+    if (mfma_eligible(p, mode) || (any && mfma_any(p, mode))) {
+        const int mt = mfma_row_tiles(p);
         Group one{};
         one.count = 1;
         one.p[0] = p;
@@ -579,22 +612,6 @@ bool mx_wanted(const Problem &p)
     return (p.M <= 5 && sign_bytes >= (48l << 20)) || (p.M <= 8 && sign_bytes >= (96l << 20));
 }
 
-// Whether a planned fp16 matrix-core launch whose alphas are powers of two should form its sign
-// operands through the LDS table and the scaled fp4 -> fp16 conversion (5 vector instructions per
-// matrix instruction instead of 10) rather than by shift and bit operation.  The table costs every
-// workgroup a 64 KiB build and a barrier (1 to 2 us), which pays from about six rounds of K-steps per
-// workgroup on; the 32-row tile would drop to one workgroup per CU with the table and loses.
-// Measured (us, shift-and-bit form vs converted form, 16 rows): 28672x8192x4 48.9 / 42.6,
-// 8192x28672x4 48.2 / 42.8, 28672x8192x2 30.0 / 28.6 (8 rows 28.4 / 25.0); 8192x8192x4 (2 rounds) 19.6 / 19.4,
-// 11008x4096x3 (4 rounds) 15.0 / 15.8, 4096x4096x3 (1 round) 8.8 / 11.0; 32 rows 28672x8192x4 74.1 / 77.6.
-// Option POW2_CONVERT: 1 = by this rule, 2 = whenever the promise is given, 0 = never.
-bool convert_wanted(const Problem &p, int mt)
-{
-    const int how = option(LUTGEMM_OPTION_POW2_CONVERT);
-    if (how != 1) return how == 2;
-    return mt == 1 && p.sets_per_split >= 6 * kMfmaWaves;
-}
-
 // Row-wise problem whose alphas are powers of two, with enough rows for the matrix cores: the
 // block-scaled kernel (16-row tiles; more rows are further row chunks that stream the same sign
 // words side by side).
@@ -614,26 +631,6 @@ int run_mx(Problem &p, const Accum &acc)
 }
 
 // ---- GEMM kernel for many activation rows ------------------------------------------------------------
-// Whether a call takes the GEMM kernel.  The fp16 matrix-core kernel, which row-wise problems of fitting sizes have
-// beside it, expands every plane again for every 32 rows, but has tiles of 64 outputs and meets its K-slices
-// in the accumulator words.  Measured (us, that kernel vs this one): 4096x4096x3 at 64 / 128 / 256 rows 14.4 / 18.8,
-// 17.1 / 26.4, 32.1 / 34.7; 11008x4096x2 27.4 / 23.6, 40.3 / 31.2, 79 / 43.5; 8192x8192x4 35.1 / 28.6, 67.7 / 44.4, 135 / 69;
-// 1024x28672x4 23.9 / 37.7, 34.6 / 59, 58 / 61.  The look-up kernel, the only other one of the other formats, takes four
-// rows at a time: 4096x4096x3 at 33 rows of int8 exponents 48 / 17.6, 13824x5120x2 104 / 33.
-bool tile_wanted(const Problem &p, int mode)
-{
-    const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
-    // (32-bit byte offsets into the operands)
-    const unsigned long long limit = 1ull << 32;
-    if ((unsigned long long)p.kwords * p.nb * p.N * 4 >= limit || (unsigned long long)p.M * p.K * 2 >= limit) return false;
-    if (is_block(mode) && (unsigned long long)p.K / 8 * p.nb * p.R * 3 >= limit) return false;
-    if (least > 0) return p.M >= least;
-    if (p.M < 33) return false;
-    if (p.M > 256) return true;
-    if (mfma_eligible(p, mode)) return (long)p.N * p.K >= 40000000 && p.N >= 4096;
-    return is_block(mode) || (long)p.M * p.N * p.K >= 200000000;
-}
-
 // K-slices a call may be cut into: none where their sums have no place (the entry point that allocates
 // nothing; a stream under capture whose buffer would have to grow is left uncut as well, so that reserved
 // accumulator words are all that a captured call needs).
@@ -649,11 +646,11 @@ size_t tile_slices_allowed(const Accum &acc)
 }
 
 // Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices: a workgroup each, two per CU.
-// `room`: bytes for the slices' sums.
+// `room`: bytes for the slices' sums.  Returns the time the plan should take.
 // Costs in microseconds, measured at three planes: a step of a 128-row tile takes 1.2 alone on its CU and
-// 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 4; the sums of the slices
+// 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 5; the sums of the slices
 // are written and read at about 4 TB/s, by a second launch that costs another 4.
-void plan_tile(TileProblem &t, size_t room)
+double plan_tile(TileProblem &t, size_t room)
 {
     constexpr long kCUs = 256;
     t.tile_rows = t.M <= 64 ? 64 : 128;
@@ -670,8 +667,8 @@ void plan_tile(TileProblem &t, size_t room)
         const long wgs = tiles * slices;
         if (ks > 1 && (wgs > 2 * kCUs || (size_t)ks * t.M * t.N * 4 > room)) break;
         const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;
-        double cost = (double)rounds * (steps * beside + 4.0);
-        if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 4.0;
+        double cost = (double)rounds * (steps * beside + 5.0);
+        if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 5.0;
         if (ks > 1) cost += 4.0 + 2.0 * (double)((size_t)ks * t.M * t.N * 4) / 4e6;
         if (ks == 1 || cost < best_cost * 0.99) {
             best_cost = cost;
@@ -679,6 +676,31 @@ void plan_tile(TileProblem &t, size_t room)
             t.slice_steps = steps;
         }
     }
+    return best_cost;
+}
+
+// Whether a call takes the GEMM kernel rather than the matrix-core kernel, from what either should take (in
+// microseconds; the slowest term only).  The matrix-core kernel forms the weights of a 32-row chunk in rounds of
+// 64 outputs x 1024 inputs, about 3 us each with one workgroup per CU.
+// Measured (us, matrix-core kernel / this one): 4096x4096x3 at 128 rows 15.4 / 25.9, 512 rows 54 / 42; 11008x4096x3 at
+// 48 rows 26 / 22, 256 rows 83 / 47; 8192x8192x4 at 64 rows 28 / 28.5, 128 rows 54 / 42; 1024x28672x4 at 256 rows
+// 45 / 56, 512 rows 77 / 62; int8 exponents 13824x5120x2 at 128 rows 74 / 42, 768x3072x3 at 512 rows 17 / 34.
+bool tile_wanted(const Problem &p, int mode)
+{
+    const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
+    // (32-bit byte offsets into the operands)
+    const unsigned long long limit = 1ull << 32;
+    if ((unsigned long long)p.kwords * p.nb * p.N * 4 >= limit || (unsigned long long)p.M * p.K * 2 >= limit) return false;
+    if (is_block(mode) && (unsigned long long)p.K / 8 * p.nb * p.R * 3 >= limit) return false;
+    if (least > 0) return p.M >= least;
+    if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
+    if (p.M <= 32) return false;
+    TileProblem t{};
+    t.N = p.N;
+    t.M = p.M;
+    t.kwords = p.kwords;
+    const double rounds = (double)((p.N + 63) / 64) * (double)((p.M + 31) / 32) * (double)((p.K + 1023) / 1024);
+    return plan_tile(t, kTileSumBytes) < 5.0 + 3.0 * rounds / 256.0;
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)
@@ -738,7 +760,7 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     }
     hipError_t e;
     if (kernel == kMatrixCore)
-        e = launch_mfma(p, mrows / 16, alpha_pow2 && convert_wanted(p, mrows / 16), acc.stream);
+        e = launch_mfma(p, mrows / 16, acc.stream);
     else if (mode == kRowF16 || mode == kUniformF16)
         e = launch_gemv_rowwise(p, mode, mrows, acc.stream);
     else if (p.rows_per_group >= kTileCols)  // a tile spans at most two row groups
@@ -1407,7 +1429,7 @@ size_t lutgemm_algorithmic_bytes(int N, int K, int nb, int M, size_t alpha_entri
     return signs + alphas + xin + yio;
 }
 
-int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
+static int describe_plan(int format, int N, int K, int nb, int groups, int M, bool any, lutgemm_plan *plan)
 {
     if (!plan || format < LUTGEMM_FORMAT_ROWWISE_F16 || format > LUTGEMM_FORMAT_UNIFORM_F16) return LUTGEMM_EINVAL;
     // (nothing is dereferenced while planning: any aligned non-null address will do)
@@ -1416,7 +1438,7 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
     int rc = fill_problem(p, format, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
     if (rc != LUTGEMM_OK) return rc;
     int kernel = kLookup, mrows = 1;
-    rc = plan_single(p, format, &kernel, &mrows);
+    rc = plan_single(p, format, &kernel, &mrows, any);
     if (rc != LUTGEMM_OK) return rc;
     *plan = lutgemm_plan{};
     plan->kernel = kernel;
@@ -1441,6 +1463,11 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
         plan->needs_workspace = lookup_splits_k(p);
     }
     return LUTGEMM_OK;
+}
+
+int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
+{
+    return describe_plan(format, N, K, nb, groups, M, false, plan);
 }
 
 int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
@@ -1469,7 +1496,7 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
 
 int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
 {
-    int rc = lutgemm_describe_plan(format, N, K, nb, groups, M, plan);
+    int rc = describe_plan(format, N, K, nb, groups, M, true, plan);
     if (rc != LUTGEMM_OK) return rc;
     alignas(16) static const uint64_t dummy[2] = {0, 0};
     Problem p;
