@@ -143,7 +143,7 @@ __device__ __forceinline__ void pack_table(const TableEntries<NB, UNI> &t, Weigh
     }
 }
 
-// What rounding the entries to fp16 leaves over (zero where they are exact, non-zero or NaN otherwise).
+// What rounding the entries to fp16 leaves over (zero where they are exact).
 template <int NB, bool UNI>
 __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntries<NB, UNI> &t)
 {
@@ -153,13 +153,26 @@ __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntri
     return r;
 }
 
+// Whether some signed sum of the multipliers may be no fp16 number.  They all are multiples of u, the
+// smallest of the multipliers' lowest set bits, and at most the sum of magnitudes, so they have eleven bits
+// where that is at most 2048 u.  (bits & bits - 1 clears the lowest mantissa bit; on a power of two it
+// clears an exponent bit instead, which halves u at worst.)  A third of the instructions of rounding every
+// entry and looking at the difference.  A zero multiplier counts for nothing; NaN and infinity are inexact.
 template <int NB, bool UNI>
-__device__ __forceinline__ bool any_nonzero(const TableEntries<NB, UNI> &t)
+__device__ __forceinline__ bool may_round(const float (&a)[NB], float q)
 {
-    uint32_t bits = 0;
+    float sum = 0.0f, least = 3.0e38f;
+    auto take = [&](float v) {
+        const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
+        const float mag = __builtin_bit_cast(float, bits);
+        const float u = mag - __builtin_bit_cast(float, bits & (bits - 1u));
+        sum += mag;
+        least = fminf(least, u > 0.0f ? u : 3.0e38f);
+    };
 #pragma unroll
-    for (int i = 0; i < t.kCount; ++i) bits |= __builtin_bit_cast(uint32_t, t.e[i]);
-    return (bits << 1) != 0u;
+    for (int b = 0; b < NB; ++b) take(a[b]);
+    if constexpr (UNI) take(q);
+    return !(sum <= least * 2048.0f) || sum > 32768.0f;
 }
 
 // The sign words of 32 inputs of one output, one per plane -> y[c]: byte i of it holds the table indices
@@ -168,7 +181,8 @@ __device__ __forceinline__ bool any_nonzero(const TableEntries<NB, UNI> &t)
 template <int NB, bool UNI>
 __device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (&y)[4])
 {
-    auto bfi = [](uint32_t m, uint32_t a, uint32_t b) { return (m & a) | (~m & b); };
+    // (as one three-input bit operation, truth table (m & a) | (~m & b): the compiler takes a chain of them apart)
+    auto bfi = [](uint32_t m, uint32_t a, uint32_t b) { return __builtin_amdgcn_bitop3_b32(m, a, b, 0xca); };
     uint32_t n[4];
     if constexpr (NB == 1) {
 #pragma unroll
@@ -181,20 +195,23 @@ __device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (
             w1 = ~(w1 ^ w3);
             w2 = ~(w2 ^ w3);
         }
+        // pairs of planes as two-bit fields of the even and of the odd inputs, then nibbles
         const uint32_t even = bfi(0x55555555u, w0, w1 << 1), odd = bfi(0x55555555u, w0 >> 1, w1);
         n[0] = even;
         n[1] = odd;
         n[2] = even >> 2;
         n[3] = odd >> 2;
-        if constexpr (NB >= 3) {
-            uint32_t up[4] = {w2 << 2, w2 << 1, w2, w2 >> 1};
-            if constexpr (NB == 4) {
-                const uint32_t top[4] = {w3 << 3, w3 << 2, w3 << 1, w3};
-#pragma unroll
-                for (int t = 0; t < 4; ++t) up[t] = bfi(0x44444444u, up[t], top[t]);
-            }
-#pragma unroll
-            for (int t = 0; t < 4; ++t) n[t] = bfi(0x33333333u, n[t], up[t]);
+        if constexpr (NB == 3) {
+            n[0] = bfi(0x33333333u, n[0], w2 << 2);
+            n[1] = bfi(0x33333333u, n[1], w2 << 1);
+            n[2] = bfi(0x33333333u, n[2], w2);
+            n[3] = bfi(0x33333333u, n[3], w2 >> 1);
+        } else if constexpr (NB == 4) {
+            const uint32_t even2 = bfi(0x55555555u, w2, w3 << 1), odd2 = bfi(0x55555555u, w2 >> 1, w3);
+            n[0] = bfi(0x33333333u, n[0], even2 << 2);
+            n[1] = bfi(0x33333333u, n[1], odd2 << 2);
+            n[2] = bfi(0x33333333u, n[2], even2);
+            n[3] = bfi(0x33333333u, n[3], odd2);
         }
     }
     const uint32_t z01a = __builtin_amdgcn_perm(n[1], n[0], 0x05010400u), z01b = __builtin_amdgcn_perm(n[1], n[0], 0x07030602u);
@@ -222,7 +239,8 @@ __device__ __forceinline__ u32x4 pick_weights(uint32_t y, const WeightTable<NB, 
             h = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
             l = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel);
             if constexpr (NB == 4 && !UNI) {
-                h ^= (half ? y : y << 4) & 0x80808080u;       // plane 3 positive: the other sign
+                // plane 3 positive: the other sign (h ^ (bits & mask))
+                h = __builtin_amdgcn_bitop3_b32(half ? y : y << 4, 0x80808080u, h, 0x6a);
             } else if constexpr (NB == 4) {
                 const uint32_t top = ((half ? y >> 7 : y >> 3) & 0x01010101u);
                 const uint32_t mask = (top << 8) - top;       // bytes of 0xff where plane 3 is positive

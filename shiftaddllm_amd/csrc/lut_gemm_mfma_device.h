@@ -88,9 +88,9 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 
     // the lane's activations: row li of each 16-row tile (rows beyond M are clamped to
     // the last one: computed twice, written once)
-    const __half *xlane[MT];
+    uint32_t xlane[MT];   // (byte offsets: the host keeps M * K * 2 below 2^32)
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xlane[mt] = p.x + (size_t)min(m0 + 16 * mt + li, p.M - 1) * p.K;
+    for (int mt = 0; mt < MT; ++mt) xlane[mt] = (uint32_t)min(m0 + 16 * mt + li, p.M - 1) * (uint32_t)p.K * 2u;
 
     // block formats: the tile's row groups; this lane forms tables of group rg and looks its own outputs up
     // among those of lane group rg_of
@@ -148,7 +148,8 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) r.x[mt][c] = *(const u32x4 *)(xlane[mt] + (4 * step + kbc) * 32 + 8 * c);
+            for (int c = 0; c < 4; ++c)
+                r.x[mt][c] = *(const u32x4 *)((const char *)p.x + (xlane[mt] + (uint32_t)(4 * step + kbc) * 64u) + 16 * c);
     };
 
     // split RMSNorm, consuming side: wave w sums the slots of rows w, w + 8, ... and leaves
@@ -228,8 +229,8 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         }
         return wave_max_finite(most);
     };
-    // The lane's tables of a step, or of what rounding their entries leaves over; true when some entry is
-    // not an fp16 number.
+    // The lane's tables of a step, or of what rounding their entries leaves over; true when some entry may
+    // not be an fp16 number.
     auto make_tables = [&](const Operands &ops, int step, bool lo, Table (&tab)[kTables]) {
         float u = unit;
         if constexpr (FMT == kWeightBlock) u = 16 * step + li < p.K / 8 ? u : 0.0f;
@@ -241,12 +242,13 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             multipliers(ops, i, a, q);
 #pragma unroll
             for (int b = 0; b < NB; ++b) a[b] *= u;
-            const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u), r = table_residual(e);
-            inexact = inexact || any_nonzero(r);
-            if (lo)
-                pack_table(r, tab[i]);
-            else
+            const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u);
+            if (lo) {
+                pack_table(table_residual(e), tab[i]);
+            } else {
+                inexact = may_round<NB, UNI>(a, q * u) || inexact;
                 pack_table(e, tab[i]);
+            }
         }
         return inexact;
     };

@@ -108,7 +108,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     char *stage = lds + 2 * kTileXBytes<MF>;
     auto stage_at = [&](int t) { return stage + (t & 3) * kTileStageBytes<FMT>; };
     [[maybe_unused]] int rg0 = 0, n_rg = 1;
-    [[maybe_unused]] bool straddles = true;   // the wave's 64 outputs lie in several row groups
     [[maybe_unused]] uint32_t rgl[2] = {0u, 0u};
     if constexpr (BLOCK) {
         const int first = n_tile * kTileN;
@@ -116,7 +115,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         n_rg = min(first + kTileN - 1, p.N - 1) / p.rows_per_group - rg0 + 1;
 #pragma unroll
         for (int f = 0; f < 2; ++f) rgl[f] = (uint32_t)(nn[f] / p.rows_per_group - rg0);
-        straddles = min(n0, p.N - 1) / p.rows_per_group != min(n0 + kTileWaveN - 1, p.N - 1) / p.rows_per_group;
     }
     constexpr int kFetched = BLOCK ? 1 : UNI ? 2 : NB;
     uint32_t fetched[kFetched];
@@ -222,20 +220,21 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
             }
         return wave_max_finite(most);
     };
-    // One table of step t, or of what its rounding leaves over; true when some entry is
-    // not an fp16 number.
+    // One table of step t, or of what its rounding leaves over; true when some entry may not
+    // be an fp16 number.
     auto make_table = [&](int t, bool lo, int f, int c) {
         const float u = 2 * t + kh < p.kwords ? unit : 0.0f;   // a word beyond K has no weight
         float a[NB], q;
         multipliers(t, f, c, a, q);
 #pragma unroll
         for (int b = 0; b < NB; ++b) a[b] *= u;
-        const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u), r = table_residual(e);
-        if (lo)
-            pack_table(r, tab[f][c]);
-        else
-            pack_table(e, tab[f][c]);
-        return any_nonzero(r);
+        const TableEntries<NB, UNI> e = table_entries<NB, UNI>(a, q * u);
+        if (lo) {
+            pack_table(table_residual(e), tab[f][c]);
+            return false;
+        }
+        pack_table(e, tab[f][c]);
+        return may_round<NB, UNI>(a, q * u);
     };
     auto make_tables = [&](int t, bool lo) {
         bool inexact = false;
@@ -330,13 +329,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                 sign_indices<NB, UNI>(words[k], y[k]);
             else if constexpr (k == 2)
                 load_words(t + 2, words);
-            else if constexpr (table && FMT == kTileBlock && f == 1) {
-                // (where the wave's outputs lie in one row group, as most waves' do, the tables are the same)
-                if (straddles)
-                    inexact = make_table(t + 1, false, 1, c) || inexact;
-                else
-                    tab[1][c] = tab[0][c];
-            } else if constexpr (table)
+            else if constexpr (table)
                 inexact = make_table(t + 1, false, f, c) || inexact;
             else
                 A[P ^ 1][c][f] = pick(f, c, y[f]);
@@ -478,6 +471,19 @@ lut_gemm_tile_kernel(const TileProblem p)
     int n_tile, m_tile, slice;
     decode_tile(p, (int)blockIdx.x, n_tile, m_tile, slice);
     if (slice >= p.ksplit) return;
+    if constexpr (FMT == kTileBlock) {
+        // most tiles have no wave whose outputs lie in two row groups, and need half the tables
+        bool straddles = false;
+#pragma unroll
+        for (int w = 0; w < kTileN / kTileWaveN; ++w) {
+            const int first = n_tile * kTileN + w * kTileWaveN, last = min(first + kTileWaveN, p.N) - 1;
+            straddles = straddles || (first < p.N && first / p.rows_per_group != last / p.rows_per_group);
+        }
+        if (!straddles) {
+            gemm_tile<NB, kTileBlockWide, MF>(p, n_tile, m_tile, slice, lds);
+            return;
+        }
+    }
     gemm_tile<NB, FMT, MF>(p, n_tile, m_tile, slice, lds);
 }
 

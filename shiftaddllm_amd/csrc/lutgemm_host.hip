@@ -355,6 +355,7 @@ bool mfma_eligible(const Problem &p, int mode)
 {
     if (!(mode == kRowF16 && p.K % kMfmaStepK == 0 && p.group_words % 4 == 0 && p.N % 16 == 0 && p.N >= 16))
         return false;
+    if ((unsigned long long)p.M * p.K * 2 >= (1ull << 32)) return false;   // (32-bit byte offsets)
     if (p.M >= mfma_min_rows()) return true;
     // two rows: the look-up kernel (one table set for both rows, fp16 entry pairs) wins from
     // about 12 MB of sign words on (measured, look-up vs matrix core: 4096x4096x3 7.3 us vs 6.4;
@@ -513,6 +514,7 @@ bool mfma_any(const Problem &p, int mode)
         const bool scattered = is_block(mode) && p.rows_per_group < kTileCols;
         if (least != 3 || !(scattered || (p.M == 2 && (long)p.N * (p.K / 8) * p.nb <= two_rows))) return false;
     }
+    if ((unsigned long long)p.M * p.K * 2 >= (1ull << 32)) return false;
     if (is_block(mode))
         return p.rows_per_group >= 24 && (unsigned long long)p.K / 8 * p.nb * p.R * 3 < (1ull << 32);
     return (unsigned long long)p.kwords * p.nb * p.N * 2 < (1ull << 32);
