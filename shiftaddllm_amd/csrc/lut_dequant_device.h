@@ -149,18 +149,26 @@ __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntri
 {
     TableEntries<NB, UNI> r;
 #pragma unroll
-    for (int i = 0; i < t.kCount; ++i) r.e[i] = t.e[i] - __half2float(__float2half_rn(t.e[i]));
+    for (int i = 0; i < t.kCount; ++i) r.e[i] = __builtin_fmaf(__half2float(__float2half_rn(t.e[i])), -1.0f, t.e[i]);   // one mixed-precision instruction
     return r;
 }
 
-// Whether some signed sum of the multipliers may be no fp16 number.  They all are multiples of u, the
-// smallest of the multipliers' lowest set bits, and at most the sum of magnitudes, so they have eleven bits
-// where that is at most 2048 u.  (bits & bits - 1 clears the lowest mantissa bit; on a power of two it
-// clears an exponent bit instead, which halves u at worst.)  A third of the instructions of rounding every
-// entry and looking at the difference.  A zero multiplier counts for nothing; NaN and infinity are inexact.
+// Whether some entry may be no fp16 number.  The entries of up to three planes are looked at themselves.
+// More of them are bounded by the multipliers: all are multiples of u, the smallest of the multipliers' lowest
+// set bits, and at most the sum of magnitudes, so they have eleven bits where that is at most 2048 u: a third
+// of the instructions.  (bits & bits - 1 clears the lowest mantissa bit; on a power of two it clears an
+// exponent bit instead, which halves u at worst.)  A zero multiplier counts for nothing; NaN and infinity
+// are inexact.
 template <int NB, bool UNI>
-__device__ __forceinline__ bool may_round(const float (&a)[NB], float q)
+__device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const float (&a)[NB], float q)
 {
+    if constexpr (TableEntries<NB, UNI>::kCount <= 4) {
+        const TableEntries<NB, UNI> r = table_residual(t);
+        uint32_t bits = 0;
+#pragma unroll
+        for (int i = 0; i < t.kCount; ++i) bits |= __builtin_bit_cast(uint32_t, r.e[i]);
+        return (bits << 1) != 0u;
+    }
     float sum = 0.0f, least = 3.0e38f;
     auto take = [&](float v) {
         const uint32_t bits = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;

@@ -234,7 +234,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
             return false;
         }
         pack_table(e, tab[f][c]);
-        return may_round<NB, UNI>(a, q * u);
+        return may_round<NB, UNI>(e, a, q * u);
     };
     auto make_tables = [&](int t, bool lo) {
         bool inexact = false;
