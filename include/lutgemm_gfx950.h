@@ -212,24 +212,32 @@ int lutgemm_gemv_block_apot_i8(const uint32_t *bW, const int8_t *alpha_i8, const
                                int M, void *stream);
 
 /*
- * A quantised linear layer in one call: out[m][n] = fp16(bias[n] + sum), whatever `out` held before
+ * A quantised linear layer in one call: out[m][n] = bias[n] + sum, whatever `out` held before
  * (bias_f16 may be NULL: zero).  The operands and the sum are those of the entry point of the same
  * format above; the caller need not copy the bias into every row of `out` first, which is a launch of
  * its own and, at one row, as long as the GEMV.  The reference's module does that copy
  * (lut_gemm/quant.py:46).
  *   format     : LUTGEMM_FORMAT_*, see lutgemm_describe_plan below;
  *   qbias_f16  : uniform format only, NULL otherwise;
- *   alpha_pow2 : 1 = the promise of lutgemm_gemv_rowwise_pow2_f16 (row-wise format only), else 0.
+ *   alpha_pow2 : 1 = the promise of lutgemm_gemv_rowwise_pow2_f16 (row-wise format only), else 0;
+ *   x_type, out_type : LUTGEMM_TYPE_* of x and out.  x is rounded to fp16 first, the sum is rounded once, to
+ *                out_type (out 16-byte aligned for LUTGEMM_TYPE_F32).  Types other than fp16 are taken where
+ *                a conversion of its own would be a large part of the call: one or two rows, up to some
+ *                tens of rows for bf16 x; LUTGEMM_EUNSUP, and no launch, for the others.
  * Errors, capture and workspace rules as everywhere.
  */
+#define LUTGEMM_TYPE_F16 0
+#define LUTGEMM_TYPE_BF16 1
+#define LUTGEMM_TYPE_F32 2
 typedef struct lutgemm_linear {
     const uint32_t *bW;
     const void *alpha;
     const void *qbias_f16;
-    const void *x_f16;
+    const void *x;
     const void *bias_f16;
-    void *out_f16;
+    void *out;
     int format, N, K, nb, num_groups, M, alpha_pow2;
+    int x_type, out_type;
 } lutgemm_linear;
 int lutgemm_linear_f16(const lutgemm_linear *layer, void *stream);
 
@@ -300,7 +308,8 @@ typedef struct lutgemm_plan {
 int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
 /* What a call of two rows and more takes, in every format.  lutgemm_describe_plan describes the look-up
  * kernel and, for row-wise problems whose sizes fit it (K a multiple of 128, groups of a multiple of 128
- * inputs, N a multiple of 16), the matrix-core kernel; beyond those, from two or three rows on, the
+ * inputs, N a multiple of 16), the matrix-core kernel with the row tiles that grouped problems have (32 rows
+ * from 17 rows on; a lone call may take 16-row tiles there); beyond those, from two or three rows on, the
  * matrix-core kernel takes every problem whose tiles of 64 columns touch at most four alpha row groups
  * (kernel 1), and calls of many rows run on the GEMM kernel (kernel 3: rows_per_pass 64 or 128, tiles of
  * 256 columns, k_units and units_per_slice in steps of 64 inputs, k_slices that a second launch adds up;

@@ -33,7 +33,6 @@ enum WeightFormat : int {
 };
 
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 
 // Entries of a table as bytes: entry i's high byte is byte i & 3 of hi[i >> 2], its low byte the same of
@@ -44,11 +43,6 @@ struct WeightTable {
     static constexpr int kRegs = NB <= 2 ? 1 : (NB == 4 && UNI) ? 4 : 2;
     uint32_t hi[kRegs], lo[kRegs];
 };
-
-__device__ __forceinline__ uint32_t pack_halves(float a, float b)
-{
-    return __builtin_bit_cast(uint32_t, __floats2half2_rn(a, b));
-}
 
 // bytes of four packed halves: high bytes / low bytes in entry order, or in reverse
 __device__ __forceinline__ uint32_t high_bytes(uint32_t p01, uint32_t p23) { return __builtin_amdgcn_perm(p23, p01, 0x07050301u); }

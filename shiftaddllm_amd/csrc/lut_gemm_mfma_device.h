@@ -158,10 +158,9 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // step's operands have been requested behind them (see the main loop): loads return in
     // order, so that wait is for the slots alone.
     float *row_scale = (float *)(xs + kMfmaRedBytes<MT>);
-    typedef float f32x4v __attribute__((ext_vector_type(4)));
     constexpr int kScaleRows = 2 * MT;  // rows per wave
     bool scaled = false;
-    [[maybe_unused]] f32x4v slot4[kScaleRows];
+    [[maybe_unused]] f32x4 slot4[kScaleRows];
     // (the wave index as a scalar, so that the rows' addresses are a scalar base plus one lane offset)
     const int wave_s = __builtin_amdgcn_readfirstlane(wave);
     if constexpr (EXTRA) {
@@ -173,7 +172,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
             for (int i = 0; i < kScaleRows; ++i) {
                 const float *slots = p.sumsq_in + (size_t)min(m0 + wave_s + kMfmaWaves * i, p.M - 1) * p.sumsq_slots;
-                slot4[i] = *((const f32x4v *)slots + min(lane, quads - 1));
+                slot4[i] = *((const f32x4 *)slots + min(lane, quads - 1));
             }
         }
     }
@@ -290,7 +289,16 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             }
         }
     };
-    auto compute = [&](const Operands &ops, int step) {
+    auto compute = [&](Operands &ops, int step) {
+        if constexpr (!EXTRA)
+            if (p.x_type == kIoBF16) {
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int c = 0; c < 4; ++c)
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) ops.x[mt][c][j] = halves_of_bf16(ops.x[mt][c][j]);
+            }
         if (unit == 0.0f) unit = unit_for(largest(ops));
         Table tab[kTables];
         const bool inexact = __builtin_amdgcn_ballot_w64(make_tables(ops, step, false, tab)) != 0ull;
@@ -411,10 +419,13 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         const int m = m0 + (tid >> 6) + 8 * i;
         [[maybe_unused]] float sq = 0.0f;  // square of the output this thread completed
         if (m < p.M && n < p.N && (p.ksplit == 1 || (int)(old[i] >> 56) == p.ksplit - 1)) {
-            __half *dst = p.out + (size_t)m * p.N + n;
             const float y = p.ksplit == 1 ? val[i] : fixed_total((old[i] | contrib[i].flags) + contrib[i].add, p.ksplit);
-            const __half y16 = __float2half_rn((p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y);
-            *dst = y16;
+            const float sum = (p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y;
+            const __half y16 = __float2half_rn(sum);
+            if constexpr (EXTRA)
+                p.out[(size_t)m * p.N + n] = y16;
+            else
+                store_result(p.out, (size_t)m * p.N + n, sum, p.out_type);
             if (p.ksplit > 1)
                 __hip_atomic_store(p.accum + (size_t)m * p.N + n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             if constexpr (EXTRA) {

@@ -32,7 +32,7 @@ hipError_t launch_mx(const Problem &p, void *split, hipStream_t stream)
     const long threads = (long)p.M * (p.K / 32) * 8;   // eight threads per block of 32
     unsigned char *pieces = (unsigned char *)split;
     uint32_t *scales = (uint32_t *)(pieces + (size_t)p.M * p.K * kMxPieces + p.K);
-    hipLaunchKernelGGL(mx_split_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p.x, pieces, scales, p.M,
+    hipLaunchKernelGGL(mx_split_kernel, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, p.x, p.x_type, pieces, scales, p.M,
                        p.K);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;

@@ -75,7 +75,7 @@ __device__ __forceinline__ uint32_t e4m3_encode(float v, float *decoded)
 
 // Eight threads per block of 32 (four values each); the block's largest magnitude is found across
 // the eight by lane exchanges.
-__global__ void __launch_bounds__(256) mx_split_kernel(const __half *__restrict__ x, unsigned char *__restrict__ pieces,
+__global__ void __launch_bounds__(256) mx_split_kernel(const void *__restrict__ x, int x_type, unsigned char *__restrict__ pieces,
                                                        uint32_t *__restrict__ scales, int M, int K)
 {
     const uint32_t blocks_per_row = (uint32_t)K / 32u;
@@ -86,7 +86,15 @@ __global__ void __launch_bounds__(256) mx_split_kernel(const __half *__restrict_
     const uint32_t bid = cid >> 3;
     const int m = (int)(bid / blocks_per_row), blk = (int)(bid % blocks_per_row);
     const int step = blk >> 2, q = blk & 3;
-    const u32x2 w = *(const u32x2 *)(x + (size_t)m * K + 32 * blk + 4 * part);
+    const size_t first = (size_t)m * K + 32 * blk + 4 * part;
+    u32x2 w;
+    if (x_type == kIoF32) {
+        const u32x4 f = *(const u32x4 *)((const float *)x + first);
+        w = (u32x2){halves_of_floats(f.x, f.y), halves_of_floats(f.z, f.w)};
+    } else {
+        w = *(const u32x2 *)((const unsigned short *)x + first);
+        if (x_type == kIoBF16) w = (u32x2){halves_of_bf16(w.x), halves_of_bf16(w.y)};
+    }
     const uint32_t h[4] = {w.x & 0xffffu, w.x >> 16, w.y & 0xffffu, w.y >> 16};
     // largest magnitude as fp16 bits (they order like the values; NaN and inf on top)
     uint32_t mxbits = max(max(h[0] & 0x7fffu, h[1] & 0x7fffu), max(h[2] & 0x7fffu, h[3] & 0x7fffu));
@@ -399,9 +407,9 @@ __device__ __forceinline__ void mx_tile(const Problem &p, const MxActivations &a
     for (int i = 0; i < kRowsPerThread; ++i) {
         const int m = m0 + (tid >> 6) + 8 * i;
         if (mine[i] && (p.ksplit == 1 || (int)(old[i] >> 56) == p.ksplit - 1)) {
-            __half *dst = p.out + (size_t)m * p.N + n;
             const float y = p.ksplit == 1 ? val[i] : fixed_total((old[i] | contrib[i].flags) + contrib[i].add, p.ksplit);
-            *dst = __float2half_rn((p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y);
+            store_result(p.out, (size_t)m * p.N + n, (p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y,
+                         p.out_type);
             if (p.ksplit > 1)
                 __hip_atomic_store(p.accum + (size_t)m * p.N + n, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }

@@ -416,7 +416,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                     v[2] += half_bits_to_float(old.y & 0xffffu);
                     v[3] += half_bits_to_float(old.y >> 16);
                 }
-                *(u32x2 *)(p.out + (size_t)m * p.N + n) = (u32x2){pack_halves(v[0], v[1]), pack_halves(v[2], v[3])};
+                store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
             }
     }
 }
@@ -442,16 +442,17 @@ __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
     if (at >= quads * (uint32_t)p.M) return;
     const size_t stride = (size_t)p.M * p.N;
     const float *src = p.partial + (size_t)at * 4u;
-    f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+    f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
     int sl = 0;
     for (; sl + 4 <= p.ksplit; sl += 4) {
         f32x4 q[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) q[u] = *(const f32x4 *)(src + (size_t)(sl + u) * stride);
 #pragma unroll
-        for (int u = 0; u < 4; ++u) v += q[u];
+        for (int u = 0; u < 4; ++u) sum += q[u];
     }
-    for (; sl < p.ksplit; ++sl) v += *(const f32x4 *)(src + (size_t)sl * stride);
+    for (; sl < p.ksplit; ++sl) sum += *(const f32x4 *)(src + (size_t)sl * stride);
+    float v[4] = {sum[0], sum[1], sum[2], sum[3]};
     const uint32_t m = at / quads, n = 4u * (at - m * quads);
     if (!p.overwrite) {
         const u32x2 old = *(const u32x2 *)(p.init + (size_t)m * p.init_stride + n);
@@ -460,7 +461,7 @@ __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
         v[2] += half_bits_to_float(old.y & 0xffffu);
         v[3] += half_bits_to_float(old.y >> 16);
     }
-    *(u32x2 *)(p.out + (size_t)m * p.N + n) = (u32x2){pack_halves(v[0], v[1]), pack_halves(v[2], v[3])};
+    store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
 }
 
 template <int NB, int FMT, int MF>

@@ -13,6 +13,13 @@ template <int NB, int MODE>
 hipError_t launch_nb(const Problem &p, int mrows, hipStream_t stream)
 {
     const dim3 grid((unsigned)p.wgs_per_chunk, (unsigned)p.mchunks), block(kThreads);
+    if (p.x_type != kIoF16 || p.out_type != kIoF16) {   // (one or two rows: the host sees to it)
+        if (mrows == 2)
+            hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 2, false, false, false, kXConvert>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 1, false, false, false, kXConvert>), grid, block, 0, stream, p);
+        return hipGetLastError();
+    }
     if (mrows == 4)
         hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 4>), grid, block, 0, stream, p);
     else if (mrows == 2)

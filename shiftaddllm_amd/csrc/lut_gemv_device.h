@@ -213,8 +213,16 @@ __device__ __forceinline__ WindowChunk fetch_window(const Problem &p, int m0, in
 {
     const WindowIndex i = window_index<MROWS>(p, m0, set0, first_rel, n_items, tid);
     WindowChunk w;
-    w.x = *(const u32x4 *)(p.x + i.base);
-    w.other = (u32x4){0u, 0u, 0u, 0u};
+    if constexpr (XF == kXConvert) {
+        // (two requests whatever the type, so that nothing branches ahead of the sign words)
+        const bool wide = p.x_type == kIoF32;
+        const char *at = (const char *)p.x + (i.base << (wide ? 2 : 1));
+        w.x = *(const u32x4 *)at;
+        w.other = *(const u32x4 *)(at + (wide ? 16 : 0));
+    } else {
+        w.x = *(const u32x4 *)(p.x + i.base);
+        w.other = (u32x4){0u, 0u, 0u, 0u};
+    }
     if constexpr (XF == kXGate) w.other = *(const u32x4 *)(p.gate + i.base);
     if constexpr (XF == kXNorm) w.other = *(const u32x4 *)(p.norm_w + i.kc);
     w.kc = i.kc;
@@ -329,6 +337,7 @@ __device__ __forceinline__ bool poll_tagged(const uint32_t *const (&src)[NCH], c
 // instead (flush_tile) and the reduction that yields it is not waited for here.
 // (x * weight is held as fp16: it must stay below 65504.)
 // XF == kXDynamic: the transform is `xf`, known at run time (uniform over the workgroup).
+// XF == kXConvert: the chunk is of IoType `xf`.
 template <int MROWS, int XF>
 __device__ __forceinline__ void store_window(const WindowChunk &w, float *window, int tid, int xf = XF)
 {
@@ -356,6 +365,13 @@ __device__ __forceinline__ void store_window(const WindowChunk &w, float *window
             }
             xr = (u32x4){o[0], o[1], o[2], o[3]};
         }
+    } else if constexpr (XF == kXConvert) {
+        const u32x4 other = w.other;
+        if (xf == kIoF32)
+            xr = (u32x4){halves_of_floats(xr.x, xr.y), halves_of_floats(xr.z, xr.w), halves_of_floats(other.x, other.y),
+                         halves_of_floats(other.z, other.w)};
+        else if (xf == kIoBF16)
+            xr = (u32x4){halves_of_bf16(xr.x), halves_of_bf16(xr.y), halves_of_bf16(xr.z), halves_of_bf16(xr.w)};
     } else if constexpr (XF != kXNone) {
         const u32x4 other = w.other;
         const uint32_t a[4] = {xr.x, xr.y, xr.z, xr.w};
@@ -696,7 +712,7 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
     // the transform: a compile-time constant except for chained problems (one kernel holds them
     // all, and an instance per bit width and transform is more than the compiler digests: from
     // eight instances of this function on, it emits an empty kernel)
-    [[maybe_unused]] const int xf = XF != kXDynamic ? XF : p.norm_w ? kXNorm : p.gate ? kXGate : kXNone;
+    [[maybe_unused]] const int xf = XF == kXConvert ? p.x_type : XF != kXDynamic ? XF : p.norm_w ? kXNorm : p.gate ? kXGate : kXNone;
     constexpr bool kMayNorm = XF == kXNorm || XF == kXDynamic;
     stamp(p, kStampEntry);
     const int tid = threadIdx.x;
@@ -1004,18 +1020,24 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
                 if (!mine[member]) continue;
                 __half *dst = p.out + (size_t)m0 * p.N + n2[member];
                 const float prev = p.overwrite ? 0.0f : half_bits_to_float(member ? out_prev_twin : out_prev[0]);
+                auto write = [&](float y) {
+                    if constexpr (XF == kXConvert)
+                        store_result(p.out, (size_t)(dst - p.out), y, p.out_type);
+                    else
+                        *dst = __float2half_rn(y);
+                };
                 if (count == 1) {
-                    *dst = __float2half_rn(prev + v2[member]);
+                    write(prev + v2[member]);
                     continue;
                 }
                 if ((int)(old2[member] >> 56) != count - 1) continue;
-                *dst = __float2half_rn(prev + fixed_total((old2[member] | c2[member].flags) + c2[member].add, count));
+                write(prev + fixed_total((old2[member] | c2[member].flags) + c2[member].add, count));
                 __hip_atomic_store(p.accum + (size_t)m0 * p.N + n2[member], 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             return;
         }
         const int n = t * kTileCols + own_col_of(kw2);
-        bool scaled = xf == kXNorm;
+        bool scaled = kMayNorm && xf == kXNorm;
         if constexpr (EXTRA) scaled = scaled || p.sumsq_in != nullptr;
         // the next norm's weight for this lane's column: requested here, used once the
         // sums are complete
@@ -1026,6 +1048,10 @@ __device__ __forceinline__ bool gemv_range(const Problem &p, int range, int mchu
         // An output is complete: round it, write it and, with a split RMSNorm, its product
         // with the next norm's weight beside it.
         auto complete = [&](int r, __half *dst, float y) {
+            if constexpr (XF == kXConvert) {
+                store_result(p.out, (size_t)(dst - p.out), y, p.out_type);
+                return;
+            }
             const __half y16 = __float2half_rn(y);
             if constexpr (DEP) {
                 if (p.out_tag) {
@@ -1324,13 +1350,14 @@ __device__ __forceinline__ void decode_block(const Problem &p, int local, int &r
 // (at most 128 registers, so that two workgroups share a CU)
 // SINGLE: every range of the launch holds exactly one item (see ALONE == 2 in gemv_range).
 // TWIN: the launch's items are twin items (two output tiles per table build, see gemv_range).
-template <int NB, int MODE, int MROWS, bool PAIR = false, bool SINGLE = false, bool TWIN = false>
+// XF: kXNone, or kXConvert where x and out are of the problem's types.
+template <int NB, int MODE, int MROWS, bool PAIR = false, bool SINGLE = false, bool TWIN = false, int XF = kXNone>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 lut_gemv_kernel(const Problem p)
 {
     __shared__ __attribute__((aligned(16))) float lut[kLutDwords + kStageDwords + kWindowDwords];
     // grid = (ranges, row chunks)
-    gemv_range<NB, MODE, MROWS, kXNone, false, SINGLE ? 2 : (MROWS == 1 && !is_block(MODE)), PAIR, false, TWIN>(
+    gemv_range<NB, MODE, MROWS, XF, false, SINGLE ? 2 : (MROWS == 1 && !is_block(MODE)), PAIR, false, TWIN>(
         p, (int)blockIdx.x, (int)blockIdx.y, lut);
 }
 

@@ -18,6 +18,16 @@ hipError_t launch_nb(const Problem &p, int mrows, hipStream_t stream)
     const bool pair_tables = option(LUTGEMM_OPTION_PAIR_TABLES) != 0;
     const bool single_item = option(LUTGEMM_OPTION_SINGLE_ITEM) != 0;
     const dim3 grid((unsigned)p.wgs_per_chunk, (unsigned)p.mchunks), block(kThreads);
+    if (p.x_type != kIoF16 || p.out_type != kIoF16) {
+        // (one or two rows, the latter through pair tables: the host sees to it)
+        if (mrows == 2)
+            hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 2, true, false, false, kXConvert>), grid, block, 0, stream, p);
+        else if (p.twin)
+            hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 1, false, false, true, kXConvert>), grid, block, 0, stream, p);
+        else
+            hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 1, false, false, false, kXConvert>), grid, block, 0, stream, p);
+        return hipGetLastError();
+    }
     if (mrows == 4 && pair_tables)
         hipLaunchKernelGGL((lut_gemv_kernel<NB, MODE, 4, true>), grid, block, 0, stream, p);
     else if (mrows == 2 && pair_tables)

@@ -14,6 +14,7 @@ namespace lutgemm {
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
@@ -63,8 +64,12 @@ constexpr bool is_block(int mode) { return mode == kBlockF16 || mode == kBlockSh
 constexpr bool is_staged(int mode) { return mode >= kBlockF16Staged; }
 constexpr int base_mode(int mode) { return is_staged(mode) ? mode - 4 : mode; }
 
+// type of the activations and of the result (LUTGEMM_TYPE_* of the public header)
+enum IoType : int { kIoF16 = 0, kIoBF16 = 1, kIoF32 = 2 };
+
 // compile-time input transform of a kernel instance
 constexpr int kXNone = 0, kXNorm = 1, kXGate = 2;
+constexpr int kXConvert = 4;  // x (and out) of the problem's x_type (out_type), rounded to fp16 first
 constexpr int kXDynamic = 3;  // chained problems: one of the three, chosen at run time
 
 // Division by a run-time constant without a divide: n / d == umulhi((2 * n) >> shift,
@@ -166,6 +171,7 @@ struct Problem {
     // (see tagged_word below), x and gate are waited for, out is written with its tag.
     int x_tag, gate_tag, out_tag;
     int alpha_mode;         // AlphaMode (matrix-core kernel, block formats)
+    int x_type, out_type;   // IoType of x and out (everything else is fp16)
 #ifdef LUTGEMM_TIMESTAMPS
     // Build with per-wave time stamps (the library variant bench.py --profile-phases loads):
     // kStampsPerWave readings of the 100 MHz wall clock per wave, at fixed points of the
@@ -193,6 +199,7 @@ struct TileProblem {
     int ksplit, slice_steps;         // K-slices and steps of each (even; the last one may have fewer)
     float *partial;                  // ksplit > 1: [slice][M][N] partial sums
     int init_stride, overwrite;
+    int out_type;                    // IoType
 };
 
 struct Group {
@@ -268,6 +275,40 @@ __device__ __forceinline__ float half_bits_to_float(uint32_t bits16)
 __device__ __forceinline__ uint32_t float_to_half_bits(float f)
 {
     return (uint32_t)__half_as_ushort(__float2half_rn(f));
+}
+
+__device__ __forceinline__ uint32_t pack_halves(float a, float b)
+{
+    return __builtin_bit_cast(uint32_t, __floats2half2_rn(a, b));
+}
+
+// two activations of another type as fp16 pairs, and a result in its type
+__device__ __forceinline__ uint32_t halves_of_floats(uint32_t a, uint32_t b)
+{
+    return pack_halves(__builtin_bit_cast(float, a), __builtin_bit_cast(float, b));
+}
+
+__device__ __forceinline__ uint32_t halves_of_bf16(uint32_t two) { return halves_of_floats(two << 16, two & 0xffff0000u); }
+
+__device__ __forceinline__ uint32_t bf16_bits(float v) { return (uint32_t)__builtin_bit_cast(unsigned short, (__bf16)v); }
+
+__device__ __forceinline__ void store_result(void *out, size_t i, float v, int type)
+{
+    if (type == kIoF32)
+        ((float *)out)[i] = v;
+    else
+        ((unsigned short *)out)[i] = (unsigned short)(type == kIoBF16 ? bf16_bits(v) : float_to_half_bits(v));
+}
+
+// four consecutive ones
+__device__ __forceinline__ void store_results(void *out, size_t i, const float (&v)[4], int type)
+{
+    if (type == kIoF32)
+        *(f32x4 *)((float *)out + i) = (f32x4){v[0], v[1], v[2], v[3]};
+    else if (type == kIoBF16)
+        *(u32x2 *)((unsigned short *)out + i) = (u32x2){bf16_bits(v[0]) | bf16_bits(v[1]) << 16, bf16_bits(v[2]) | bf16_bits(v[3]) << 16};
+    else
+        *(u32x2 *)((unsigned short *)out + i) = (u32x2){pack_halves(v[0], v[1]), pack_halves(v[2], v[3])};
 }
 
 // The value of another lane of the same row of 16, by a data-parallel-primitive move.

@@ -523,7 +523,7 @@ bool mfma_any(const Problem &p, int mode)
 int plan_single(Problem &p, int mode, int *kernel, int *mrows, bool any = true)
 {
     if (mfma_eligible(p, mode) || (any && mfma_any(p, mode))) {
-        const int mt = mfma_row_tiles(p);
+        const int mt = any ? mfma_row_tiles(p) : p.M > 16 ? 2 : 1;
         Group one{};
         one.count = 1;
         one.p[0] = p;
@@ -725,6 +725,7 @@ int run_tile(const Problem &p, int mode, const Accum &acc)
     plan_tile(t, tile_slices_allowed(acc));
     t.init_stride = p.init_stride;
     t.overwrite = p.overwrite;
+    t.out_type = p.out_type;
     if (t.ksplit > 1) {
         void *sums = nullptr;
         const int rc = stream_split_buffer(acc.stream, (size_t)t.ksplit * t.M * t.N * 4, &sums);
@@ -736,10 +737,12 @@ int run_tile(const Problem &p, int mode, const Accum &acc)
 }
 
 // `bias`: null = accumulate into out; otherwise *bias is the row every output row starts from (null:
-// zeros) and out is written, not read.
+// zeros) and out is written, not read.  `x_type`, `out_type`: IoType of x and of out (then written, not read);
+// the kernels that take other activations than fp16 themselves are the ones whose few rows make a launch of
+// its own for the conversion dear, LUTGEMM_EUNSUP otherwise (which a caller answers by converting).
 int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, const void *x,
         void *out, int N, int K, int nb, int num_groups, int M, const Accum &acc, bool alpha_pow2 = false,
-        const void *const *bias = nullptr)
+        const void *const *bias = nullptr, int x_type = kIoF16, int out_type = kIoF16)
 {
     Problem p;
     int rc = fill_problem(p, mode, bW, alpha, qbias, x, out, N, K, nb, num_groups, M);
@@ -751,11 +754,21 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     } else if (bias) {
         p.overwrite = 1;
     }
-    if (tile_wanted(p, mode)) return run_tile(p, mode, acc);
+    p.x_type = x_type;
+    p.out_type = out_type;
+    if (tile_wanted(p, mode)) return x_type == kIoF16 ? run_tile(p, mode, acc) : LUTGEMM_EUNSUP;
     if (alpha_pow2 && mode == kRowF16 && mfma_eligible(p, mode) && p.M >= mfma_min_rows() && mx_wanted(p)) return run_mx(p, acc);
     int kernel = kLookup, mrows = 1;
     rc = plan_single(p, mode, &kernel, &mrows);
     if (rc != LUTGEMM_OK) return rc;
+    if (kernel == kMatrixCore) {
+        if (x_type == kIoF32) return LUTGEMM_EUNSUP;   // (a step's operands would not fit the registers)
+    } else if (x_type != kIoF16 || out_type != kIoF16) {
+        const bool per_column = mode == kRowF16 || mode == kUniformF16;
+        if (mrows > 2 || (mrows == 2 && per_column && option(LUTGEMM_OPTION_PAIR_TABLES) == 0) ||
+            (!per_column && p.rows_per_group < kTileCols))
+            return LUTGEMM_EUNSUP;
+    }
     if (kernel == kMatrixCore ? p.ksplit > 1 : lookup_splits_k(p)) {
         rc = accum_words(acc, (size_t)M * N, &p.accum);
         if (rc != LUTGEMM_OK) return rc;
@@ -1417,8 +1430,11 @@ int lutgemm_linear_f16(const lutgemm_linear *layer, void *stream)
 {
     if (!layer || layer->format < LUTGEMM_FORMAT_ROWWISE_F16 || layer->format > LUTGEMM_FORMAT_UNIFORM_F16) return LUTGEMM_EINVAL;
     const lutgemm_linear &c = *layer;
-    return run(c.format, c.bW, c.alpha, c.qbias_f16, c.x_f16, c.out_f16, c.N, c.K, c.nb, c.num_groups, c.M,
-               Accum{(hipStream_t)stream}, c.alpha_pow2 != 0 && c.format == LUTGEMM_FORMAT_ROWWISE_F16, &c.bias_f16);
+    if (c.x_type < kIoF16 || c.x_type > kIoF32 || c.out_type < kIoF16 || c.out_type > kIoF32) return LUTGEMM_EINVAL;
+    if (c.out_type == kIoF32 && !aligned(c.out, 16)) return LUTGEMM_EALIGN;
+    return run(c.format, c.bW, c.alpha, c.qbias_f16, c.x, c.out, c.N, c.K, c.nb, c.num_groups, c.M,
+               Accum{(hipStream_t)stream}, c.alpha_pow2 != 0 && c.format == LUTGEMM_FORMAT_ROWWISE_F16, &c.bias_f16,
+               c.x_type, c.out_type);
 }
 
 size_t lutgemm_algorithmic_bytes(int N, int K, int nb, int M, size_t alpha_entries,

@@ -23,15 +23,15 @@
 namespace {
 
 void check_common(const torch::Tensor &output, const torch::Tensor &bWeight,
-                  const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb)
+                  const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb, bool any_type = false)
 {
     TORCH_CHECK(output.is_cuda(), "output must be a GPU tensor");
     TORCH_CHECK(bWeight.is_cuda() && d_input.is_cuda(), "bWeight and d_input must be GPU tensors");
     TORCH_CHECK(bWeight.get_device() == output.get_device() &&
                     d_input.get_device() == output.get_device(),
                 "all operands must live on the same device");
-    TORCH_CHECK(output.scalar_type() == torch::kHalf, "output must be float16");
-    TORCH_CHECK(d_input.scalar_type() == torch::kHalf, "d_input must be float16");
+    TORCH_CHECK(any_type || output.scalar_type() == torch::kHalf, "output must be float16");
+    TORCH_CHECK(any_type || d_input.scalar_type() == torch::kHalf, "d_input must be float16");
     TORCH_CHECK(bWeight.scalar_type() == torch::kInt32, "bWeight must be int32");
     TORCH_CHECK(output.is_contiguous() && bWeight.is_contiguous() && d_input.is_contiguous(),
                 "operands must be contiguous");
@@ -189,30 +189,41 @@ void lutgemm_compute_block_shiftInt8(torch::Tensor output, torch::Tensor bWeight
 }
 
 // ---- LutLinear.forward ------------------------------------------------------------------------
+int io_type(c10::ScalarType t)
+{
+    return t == at::kHalf ? LUTGEMM_TYPE_F16 : t == at::kBFloat16 ? LUTGEMM_TYPE_BF16 : t == at::kFloat ? LUTGEMM_TYPE_F32 : -1;
+}
+
 // linear_forward(x, binaryWeight, alpha, bias, out, format, N, K, nb, num_groups, alpha_pow2) -> y
-// The whole of lut_gemm/quant.py:41-54 in one native call: the activations as contiguous fp16 rows,
-// the output [..., N] (allocated here, or `out`, fp16 [rows, N], where the caller reuses one), ONE launch
-// that adds the bias itself, the result in the activations' dtype.  At one row the layer is bound by the
-// host, not the device: through five framework calls and the checked functions above a forward took
-// 11.9 us of host time around a 4.5 us kernel.  A plain CPython function, because the argument
-// conversions of pybind11 are a tenth of what is left.
+// The whole of lut_gemm/quant.py:41-54 in one native call: the activations as contiguous rows, the output
+// [..., N] in their dtype (allocated here, or `out`, fp16 [rows, N], where the caller reuses one), ONE launch
+// that adds the bias itself.  At one row the layer is bound by the host, not the device: through five
+// framework calls and the checked functions above a forward took 11.9 us of host time around a 4.5 us
+// kernel.  A plain CPython function, because the argument conversions of pybind11 are a tenth of what is left.
+// bf16 and fp32 activations are converted by the kernel itself where it does that (the call says
+// LUTGEMM_EUNSUP otherwise), and by a launch ahead of it elsewhere; the result is written in the caller's type.
+// (A conversion is 4 us of host time and 3 of the device: bf16 rows of a 2208 x 2964 layer 14.5 -> 7.9 us.)
 at::Tensor linear_forward(const at::Tensor &x, const at::Tensor &bW, const at::Tensor &alpha, const at::Tensor *bias,
                           const at::Tensor *out, int64_t format, int64_t N, int64_t K, int64_t nb, int64_t groups,
                           bool alpha_pow2)
 {
-    TORCH_CHECK(x.is_cuda(), "the input must be a GPU tensor");
     const auto dims = x.sizes();
-    TORCH_CHECK(!dims.empty() && dims.back() == K && x.numel() > 0, "expected a non-empty input of [..., ", K, "], got ", dims);
+    TORCH_CHECK_VALUE(!dims.empty() && dims.back() == K, "expected last dimension ", K, ", got ", dims);
+    TORCH_CHECK(x.is_cuda(), "the input must be a GPU tensor");
+    TORCH_CHECK(x.numel() > 0, "the input is empty");
     const int64_t rows = x.numel() / K;
     const auto device = x.device();
     const c10::hip::HIPGuardMasqueradingAsCUDA guard(device);
     const c10::ScalarType dtype = x.scalar_type();
-    const at::Tensor x16 = dtype == at::kHalf && x.is_contiguous() ? x : x.to(at::kHalf).contiguous();
+    c10::ScalarType out_dtype = out || io_type(dtype) < 0 ? at::kHalf : dtype;
+    at::Tensor in = x.is_contiguous() ? x : x.contiguous();
+    if (io_type(dtype) < 0 || (dtype != at::kHalf && (uintptr_t)in.const_data_ptr() % 16 != 0)) in = in.to(at::kHalf);
 
     c10::SmallVector<int64_t, 5> shape(dims.begin(), dims.end());
     shape.back() = N;
-    at::Tensor y = out ? *out : at::Tensor(at::detail::empty_cuda(shape, at::kHalf, device, c10::nullopt));
-    check_common(y, bW, x16, N, K, nb);
+    auto allocate = [&]() { return at::Tensor(at::detail::empty_cuda(shape, out_dtype, device, c10::nullopt)); };
+    at::Tensor y = out ? *out : allocate();
+    check_common(y, bW, in, N, K, nb, out == nullptr);
     int64_t entries;
     c10::ScalarType type = at::kHalf;
     switch (format) {
@@ -236,9 +247,7 @@ at::Tensor linear_forward(const at::Tensor &x, const at::Tensor &bW, const at::T
     lutgemm_linear layer{};
     layer.bW = (const uint32_t *)bW.const_data_ptr();
     layer.alpha = alpha.const_data_ptr();
-    layer.x_f16 = x16.const_data_ptr();
     layer.bias_f16 = bias ? bias->const_data_ptr() : nullptr;
-    layer.out_f16 = y.data_ptr();
     layer.format = (int)format;
     layer.N = (int)N;
     layer.K = (int)K;
@@ -246,8 +255,26 @@ at::Tensor linear_forward(const at::Tensor &x, const at::Tensor &bW, const at::T
     layer.num_groups = (int)groups;
     layer.M = (int)rows;
     layer.alpha_pow2 = alpha_pow2;
-    raise_on_error(lutgemm_linear_f16(&layer, c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream()), "LutLinear.forward");
-    if (dtype != at::kHalf) y = y.to(dtype);
+    const auto stream = c10::hip::getCurrentHIPStreamMasqueradingAsCUDA().stream();
+    auto launch = [&]() {
+        layer.x = in.const_data_ptr();
+        layer.x_type = io_type(in.scalar_type());
+        layer.out = y.data_ptr();
+        layer.out_type = io_type(out_dtype);
+        return lutgemm_linear_f16(&layer, stream);
+    };
+    int rc = launch();
+    if (rc == LUTGEMM_EUNSUP && layer.x_type != LUTGEMM_TYPE_F16) {
+        in = in.to(at::kHalf);
+        rc = launch();
+    }
+    if (rc == LUTGEMM_EUNSUP && layer.out_type != LUTGEMM_TYPE_F16) {
+        out_dtype = at::kHalf;
+        y = allocate();
+        rc = launch();
+    }
+    raise_on_error(rc, "LutLinear.forward");
+    if (out_dtype != dtype) y = y.to(dtype);
     return out ? y.view(shape) : y;
 }
 

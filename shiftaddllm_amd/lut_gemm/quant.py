@@ -166,16 +166,16 @@ class LutLinear(nn.Module):
         return buf
 
     def forward(self, x):
+        # (at one row the host bounds the layer: what can be checked natively is)
         K = self.K
-        if x.shape[-1] != K:
-            raise ValueError(f"expected last dimension {K}, got {tuple(x.shape)}")
         buffers = self._buffers
         fmt = _FORMAT_CODES[self.alpha_format]
-        rows = x.numel() // K
-        pow2 = fmt == 0 and 3 <= rows <= 8 and self._alphas_are_powers_of_two()
-        device = x.device
-        return native.lutgemm.linear_forward(x, buffers["binaryWeight"], buffers["alpha"], self._bias_vector(device),
-                                             self._output(rows, device) if self.reuse_output else None, fmt, self.N, K,
+        pow2 = fmt == 0 and 3 * K <= x.numel() <= 8 * K and self._alphas_are_powers_of_two()
+        bias = self.bias
+        if bias is not None:
+            bias = self._bias_vector(x.device)
+        out = self._output(x.numel() // K, x.device) if self.reuse_output else None
+        return native.lutgemm.linear_forward(x, buffers["binaryWeight"], buffers["alpha"], bias, out, fmt, self.N, K,
                                              self.wbit, self.num_groups, pow2)
 
     def extra_repr(self):

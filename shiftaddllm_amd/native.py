@@ -93,9 +93,10 @@ class FusedProblem(ctypes.Structure):
 class Linear(ctypes.Structure):
     """struct lutgemm_linear of include/lutgemm_gfx950.h."""
     _fields_ = [("bW", ctypes.c_void_p), ("alpha", ctypes.c_void_p), ("qbias_f16", ctypes.c_void_p),
-                ("x_f16", ctypes.c_void_p), ("bias_f16", ctypes.c_void_p), ("out_f16", ctypes.c_void_p),
+                ("x", ctypes.c_void_p), ("bias_f16", ctypes.c_void_p), ("out", ctypes.c_void_p),
                 ("format", ctypes.c_int), ("N", ctypes.c_int), ("K", ctypes.c_int), ("nb", ctypes.c_int),
-                ("num_groups", ctypes.c_int), ("M", ctypes.c_int), ("alpha_pow2", ctypes.c_int)]
+                ("num_groups", ctypes.c_int), ("M", ctypes.c_int), ("alpha_pow2", ctypes.c_int),
+                ("x_type", ctypes.c_int), ("out_type", ctypes.c_int)]
 
 
 class ChainProblem(ctypes.Structure):
