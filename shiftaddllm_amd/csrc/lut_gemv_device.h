@@ -1364,12 +1364,12 @@ lut_gemv_kernel(const Problem p)
 // Several row-wise problems in one launch.  Bit widths may differ between the
 // problems of a group.
 // XF: the input transform shared by all problems of the launch.
-// (Up to three bit planes take the first item on its own, like a lone problem; four planes
-// keep the loop that requests two items up front: with the peeled first item as well the
-// kernel, whose register count is that of its largest bit width, spills 10-19 registers per
-// lane, and everything slows down: q,k,v of a 7B block 10.3 us per launch with the spills,
-// 9.6 with the old loop throughout, 9.1 this way; gate,up 14.4 / 13.4 / 12.8.)
-template <int XF>
+// EXTRA: some problem has split-RMSNorm fields.
+// Every width takes its first item on its own, like a lone problem.  The widths' bodies are kept apart (what
+// the compiler hoists out of them ahead of the switch lives through all of them, and four planes spilled 16 to
+// 19 registers per lane for it, or, without the peeled first item, waited for two items before the first
+// table): XXX.
+template <int XF, bool EXTRA>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 lut_gemv_group_kernel(const Group g)
 {
@@ -1380,13 +1380,18 @@ lut_gemv_group_kernel(const Group g)
     // then scalar loads that may be repeated at will instead of values to keep in registers)
     const Problem &p = *(const Problem *)((const __attribute__((address_space(4))) Problem *)&g.p[0] + blockIdx.y);
     if ((int)blockIdx.x >= p.n_blocks) return;
-    int range, m;
-    decode_block(p, (int)blockIdx.x, range, m);
+    auto run = [&](auto planes) {
+        constexpr int NB = decltype(planes)::value;
+        asm volatile("; %0 planes" ::"n"(NB));   // (differs from case to case: nothing is hoisted past it)
+        int range, m;
+        decode_block(p, (int)blockIdx.x, range, m);
+        gemv_range<NB, kRowF16, 1, XF, EXTRA, true>(p, range, m, lut);
+    };
     switch (p.nb) {
-    case 1: gemv_range<1, kRowF16, 1, XF, true, true>(p, range, m, lut); break;
-    case 2: gemv_range<2, kRowF16, 1, XF, true, true>(p, range, m, lut); break;
-    case 3: gemv_range<3, kRowF16, 1, XF, true, true>(p, range, m, lut); break;
-    default: gemv_range<4, kRowF16, 1, XF, true, false>(p, range, m, lut); break;
+    case 1: run(std::integral_constant<int, 1>{}); break;
+    case 2: run(std::integral_constant<int, 2>{}); break;
+    case 3: run(std::integral_constant<int, 3>{}); break;
+    default: run(std::integral_constant<int, 4>{}); break;
     }
 }
 

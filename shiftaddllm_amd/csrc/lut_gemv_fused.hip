@@ -12,35 +12,38 @@ namespace lutgemm {
 namespace {
 
 // SINGLE: every range of the launch holds exactly one item.
-template <int NB, int XF, bool SINGLE = false>
+// EXTRA: the problem has split-RMSNorm fields.
+template <int NB, int XF, bool EXTRA, bool SINGLE>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 lut_gemv_fused_kernel(const Problem p)
 {
     __shared__ __attribute__((aligned(16))) float lut[kLutDwords + kStageDwords + kWindowDwords];
-    gemv_range<NB, kRowF16, 1, XF, true, SINGLE ? 2 : 1>(p, (int)blockIdx.x, (int)blockIdx.y, lut);  // grid = (ranges, rows)
+    gemv_range<NB, kRowF16, 1, XF, EXTRA, SINGLE ? 2 : 1>(p, (int)blockIdx.x, (int)blockIdx.y, lut);  // grid = (ranges, rows)
+}
+
+template <int NB, int XF, bool EXTRA>
+hipError_t launch_extra(const Problem &p, hipStream_t stream)
+{
+    const dim3 grid((unsigned)p.wgs_per_chunk, (unsigned)p.mchunks), block(kThreads);
+    if (p.items_per_wg == 1 && p.short_items == 1 && option(LUTGEMM_OPTION_SINGLE_ITEM) != 0)
+        hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, XF, EXTRA, true>), grid, block, 0, stream, p);
+    else
+        hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, XF, EXTRA, false>), grid, block, 0, stream, p);
+    return hipGetLastError();
+}
+
+template <int NB, int XF>
+hipError_t launch_xform(const Problem &p, hipStream_t stream)
+{
+    const bool extra = p.next_w || p.sumsq_out || p.sumsq_in;
+    return extra ? launch_extra<NB, XF, true>(p, stream) : launch_extra<NB, XF, false>(p, stream);
 }
 
 template <int NB>
 hipError_t launch_nb(const Problem &p, int xform, hipStream_t stream)
 {
-    const dim3 grid((unsigned)p.wgs_per_chunk, (unsigned)p.mchunks), block(kThreads);
-    const bool single_item = option(LUTGEMM_OPTION_SINGLE_ITEM) != 0;
-    if (p.items_per_wg == 1 && p.short_items == 1 && single_item) {
-        if (xform == kXNorm)
-            hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXNorm, true>), grid, block, 0, stream, p);
-        else if (xform == kXGate)
-            hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXGate, true>), grid, block, 0, stream, p);
-        else
-            hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXNone, true>), grid, block, 0, stream, p);
-        return hipGetLastError();
-    }
-    if (xform == kXNorm)
-        hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXNorm>), grid, block, 0, stream, p);
-    else if (xform == kXGate)
-        hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXGate>), grid, block, 0, stream, p);
-    else
-        hipLaunchKernelGGL((lut_gemv_fused_kernel<NB, kXNone>), grid, block, 0, stream, p);
-    return hipGetLastError();
+    return xform == kXNorm ? launch_xform<NB, kXNorm>(p, stream)
+           : xform == kXGate ? launch_xform<NB, kXGate>(p, stream) : launch_xform<NB, kXNone>(p, stream);
 }
 
 }  // namespace

@@ -16,6 +16,8 @@
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 
 #include <string>
+#include <type_traits>
+#include <utility>
 #include <vector>
 
 #include "lutgemm_gfx950.h"
@@ -72,8 +74,8 @@ int rows_of(const torch::Tensor &d_input, int64_t kSize) { return (int)(d_input.
 }  // namespace
 
 // lutgemm_cuda.cpp:43-52
-void lutgemm_compute_shift_scale(torch::Tensor output, torch::Tensor bWeight, torch::Tensor alpha,
-                                 torch::Tensor d_input, int64_t mSize, int64_t kSize, int64_t nb,
+void lutgemm_compute_shift_scale(const torch::Tensor &output, const torch::Tensor &bWeight, const torch::Tensor &alpha,
+                                 const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb,
                                  int64_t num_groups)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -91,8 +93,8 @@ void lutgemm_compute_shift_scale(torch::Tensor output, torch::Tensor bWeight, to
 // lutgemm_compute_shift_scale for alphas the caller knows to be powers of two (what the
 // reference's quantiser produces, quantizers/bcq_quant/bcq_shift.py:15-24): a few rows on a large
 // matrix take the block-scaled matrix-core kernel.  No counterpart in the reference's extension.
-void lutgemm_compute_shift_scale_pow2(torch::Tensor output, torch::Tensor bWeight, torch::Tensor alpha,
-                                      torch::Tensor d_input, int64_t mSize, int64_t kSize, int64_t nb,
+void lutgemm_compute_shift_scale_pow2(const torch::Tensor &output, const torch::Tensor &bWeight, const torch::Tensor &alpha,
+                                      const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb,
                                       int64_t num_groups)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -108,8 +110,8 @@ void lutgemm_compute_shift_scale_pow2(torch::Tensor output, torch::Tensor bWeigh
 }
 
 // lutgemm_cuda.cpp:88-98
-void lutgemm_compute(torch::Tensor output, torch::Tensor bWeight, torch::Tensor alpha,
-                     torch::Tensor q_bias, torch::Tensor d_input, int64_t mSize, int64_t kSize,
+void lutgemm_compute(const torch::Tensor &output, const torch::Tensor &bWeight, const torch::Tensor &alpha,
+                     const torch::Tensor &q_bias, const torch::Tensor &d_input, int64_t mSize, int64_t kSize,
                      int64_t nb, int64_t num_groups)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -133,8 +135,8 @@ static void check_block(int64_t mSize, int64_t num_groups)
 }
 
 // lutgemm_cuda.cpp:54-63
-void lutgemm_compute_block(torch::Tensor output, torch::Tensor bWeight, torch::Tensor alpha,
-                           torch::Tensor d_input, int64_t mSize, int64_t kSize, int64_t nb,
+void lutgemm_compute_block(const torch::Tensor &output, const torch::Tensor &bWeight, const torch::Tensor &alpha,
+                           const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb,
                            int64_t num_groups)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -150,8 +152,8 @@ void lutgemm_compute_block(torch::Tensor output, torch::Tensor bWeight, torch::T
 }
 
 // lutgemm_cuda.cpp:65-74
-void lutgemm_compute_block_shift(torch::Tensor output, torch::Tensor bWeight, torch::Tensor alpha,
-                                 torch::Tensor d_input, int64_t mSize, int64_t kSize, int64_t nb,
+void lutgemm_compute_block_shift(const torch::Tensor &output, const torch::Tensor &bWeight, const torch::Tensor &alpha,
+                                 const torch::Tensor &d_input, int64_t mSize, int64_t kSize, int64_t nb,
                                  int64_t num_groups, int64_t num_apot)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -170,8 +172,8 @@ void lutgemm_compute_block_shift(torch::Tensor output, torch::Tensor bWeight, to
 }
 
 // lutgemm_cuda.cpp:76-85
-void lutgemm_compute_block_shiftInt8(torch::Tensor output, torch::Tensor bWeight,
-                                     torch::Tensor alpha, torch::Tensor d_input, int64_t mSize,
+void lutgemm_compute_block_shiftInt8(const torch::Tensor &output, const torch::Tensor &bWeight,
+                                     const torch::Tensor &alpha, const torch::Tensor &d_input, int64_t mSize,
                                      int64_t kSize, int64_t nb, int64_t num_groups, int64_t num_apot)
 {
     check_common(output, bWeight, d_input, mSize, kSize, nb);
@@ -406,18 +408,56 @@ std::vector<torch::Tensor> parsing(torch::Tensor bW, torch::Tensor A, int64_t ro
     return {bWeight, p_q_bias.contiguous(), p_alpha.contiguous()};
 }
 
+// The compute functions as plain CPython functions of positional arguments: tensors, then whole numbers.
+// (pybind11's conversions of nine arguments take 1 us, the kernel of one row of 4096 x 4096 five.)
+template <auto Fn>
+struct Positional;
+
+template <typename... Args, void (*Fn)(Args...)>
+struct Positional<Fn> {
+    template <typename T>
+    static T convert(PyObject *o, const char *name)
+    {
+        if constexpr (std::is_same_v<T, int64_t>) {
+            const int64_t v = PyLong_AsLongLong(o);
+            if (v == -1 && PyErr_Occurred()) throw python_error();
+            return v;
+        } else {
+            TORCH_CHECK_TYPE(THPVariable_Check(o), name, ": expected a tensor, got ", Py_TYPE(o)->tp_name);
+            return THPVariable_Unpack(o);
+        }
+    }
+    template <size_t... I>
+    static void spread(PyObject *const *args, const char *name, std::index_sequence<I...>)
+    {
+        Fn(convert<Args>(args[I], name)...);
+    }
+    static PyObject *call(PyObject *self, PyObject *const *args, Py_ssize_t n)
+    {
+        HANDLE_TH_ERRORS
+        const char *name = (const char *)PyCapsule_GetPointer(self, nullptr);
+        TORCH_CHECK_TYPE(n == (Py_ssize_t)sizeof...(Args), name, " takes ", sizeof...(Args), " arguments, got ", n);
+        spread(args, name, std::index_sequence_for<Args...>{});
+        Py_RETURN_NONE;
+        END_HANDLE_TH_ERRORS
+    }
+    static void define(py::module_ &m, const char *name, const char *doc)
+    {
+        static PyMethodDef def;
+        def = {name, (PyCFunction)(void (*)(void))call, METH_FASTCALL, doc};
+        m.add_object(name, py::reinterpret_steal<py::object>(PyCFunction_New(&def, py::capsule((const void *)name).ptr())));
+    }
+};
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.doc() = "MI355X (gfx950) LUT-GEMM engine behind the ShiftAddLLM `lutgemm` call signatures";
-    m.def("lutgemm_compute", &lutgemm_compute, "uniform-quant LUT-GEMV (alpha, q_bias)");
-    m.def("lutgemm_compute_shift_scale", &lutgemm_compute_shift_scale, "row-wise alpha LUT-GEMV");
-    m.def("lutgemm_compute_shift_scale_pow2", &lutgemm_compute_shift_scale_pow2,
-          "row-wise alpha LUT-GEMV, alphas promised to be powers of two");
-    m.def("lutgemm_compute_block", &lutgemm_compute_block, "block alpha LUT-GEMV (fp16 alpha)");
-    m.def("lutgemm_compute_block_shift", &lutgemm_compute_block_shift,
-          "block alpha LUT-GEMV (uint16 shift fields)");
-    m.def("lutgemm_compute_block_shiftInt8", &lutgemm_compute_block_shiftInt8,
-          "block alpha LUT-GEMV (int8 exponents)");
+    Positional<&lutgemm_compute>::define(m, "lutgemm_compute", "uniform-quant LUT-GEMV (alpha, q_bias)");
+    Positional<&lutgemm_compute_shift_scale>::define(m, "lutgemm_compute_shift_scale", "row-wise alpha LUT-GEMV");
+    Positional<&lutgemm_compute_shift_scale_pow2>::define(m, "lutgemm_compute_shift_scale_pow2", "row-wise alpha LUT-GEMV, alphas promised to be powers of two");
+    Positional<&lutgemm_compute_block>::define(m, "lutgemm_compute_block", "block alpha LUT-GEMV (fp16 alpha)");
+    Positional<&lutgemm_compute_block_shift>::define(m, "lutgemm_compute_block_shift", "block alpha LUT-GEMV (uint16 shift fields)");
+    Positional<&lutgemm_compute_block_shiftInt8>::define(m, "lutgemm_compute_block_shiftInt8", "block alpha LUT-GEMV (int8 exponents)");
     m.def("makeRandomInput", &makeRandomInput, "fill inp[:M, :K] with the reference's random activations");
     m.def("makeRandomAlpha", &makeRandomAlpha, "fill alpha [num_groups, NUM_BITS, N] and q_bias [num_groups, N]");
     m.def("makeRandomBias", &makeRandomBias, "fill bias[:N]");
