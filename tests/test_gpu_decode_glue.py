@@ -98,6 +98,48 @@ def test_attention_step(gpu_device, B, H, KV, hd, max_pos, positions):
         assert torch.allclose(out.float(), want, rtol=5e-3, atol=5e-3), (pos, (out.float() - want).abs().max())
 
 
+@pytest.mark.parametrize("B,H,KV,hd,max_pos,pos,offset", [
+    (2, 16, 4, 128, 600, 255, 0),    # heads of a kv head placed together (8 kv heads); one row short of a block
+    (2, 16, 4, 128, 600, 257, 0),    # a block and one row
+    (3, 9, 3, 64, 700, 640, 0),      # 9 kv heads: not placed
+    (16, 16, 16, 128, 300, 129, 0),  # 256 workgroups: four waves each, one row beyond their block
+    (16, 32, 8, 64, 300, 256, 0),    # the same at the other head size, grouped
+    (1, 4, 2, 128, 80, 70, 1),       # operands off 16-byte alignment: the general kernel
+])
+def test_attention_step_routes(gpu_device, B, H, KV, hd, max_pos, pos, offset):
+    """Workgroup sizes, head placement and alignment, against fp64 attention over the same fp16 caches.  The kernel
+    rounds only its result (fp16, 2^-11) and the rotated q and k; rotation in another order may turn one of those
+    roundings: 2^-11 of a score of a few units, hence 4e-3 of the value scale."""
+    lib = native.cabi()
+    g = torch.Generator(device=gpu_device).manual_seed(B * 100 + H + pos)
+    mk = lambda *s: torch.randn(s, generator=g, device=gpu_device).half()
+
+    def flat(rows, cols):      # a row-major operand `offset` halves behind a 16-byte boundary
+        t = mk(rows * cols + 8)
+        return t[offset:offset + rows * cols].view(rows, cols)
+    q, k, v = flat(B, H * hd), flat(B, KV * hd), flat(B, KV * hd)
+    ang = torch.rand((max_pos, hd // 2), generator=g, device=gpu_device) * 6.28
+    cos, sin = torch.cat([ang.cos()] * 2, -1).half(), torch.cat([ang.sin()] * 2, -1).half()
+    kc, vc = mk(B, KV, max_pos, hd), mk(B, KV, max_pos, hd)
+    kc[:, :, pos + 1:], vc[:, :, pos + 1:] = float("nan"), float("inf")     # never read
+    out = torch.zeros((B, H * hd), dtype=torch.float16, device=gpu_device)
+    p = torch.tensor([pos], dtype=torch.long, device=gpu_device)
+    _ok(lib.lutgemm_decode_attention_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), cos.data_ptr(), sin.data_ptr(), kc.data_ptr(),
+                                         vc.data_ptr(), p.data_ptr(), out.data_ptr(), B, H, KV, hd, max_pos, _sp()))
+    torch.cuda.synchronize()
+    c, s = cos[pos].float().cpu(), sin[pos].float().cpu()
+    qr = _rope(q.float().cpu().view(B, H, hd), c, s).half().double()
+    kr = _rope(k.float().cpu().view(B, KV, hd), c, s).half()
+    keys, vals = kc[:, :, :pos + 1].cpu(), vc[:, :, :pos + 1].cpu()
+    assert torch.equal(vals[:, :, pos], v.cpu().view(B, KV, hd))
+    assert torch.allclose(keys[:, :, pos].float(), kr.float(), rtol=1e-3, atol=1e-3)
+    keys = keys.double().repeat_interleave(H // KV, dim=1)
+    vals = vals.double().repeat_interleave(H // KV, dim=1)
+    att = torch.softmax((keys * qr[:, :, None]).sum(-1) / math.sqrt(hd), dim=-1)
+    want = (att[..., None] * vals).sum(2).reshape(B, H * hd)
+    assert torch.allclose(out.cpu().double(), want, rtol=4e-3, atol=4e-3)
+
+
 def test_attention_rejects_bad_arguments(gpu_device):
     lib = native.cabi()
     t = torch.zeros((4096,), dtype=torch.float16, device=gpu_device)
