@@ -15,7 +15,14 @@
 // middle of fp16's range) and rounded to fp16 once; what the rounding leaves over is a second table,
 // whose product is added as well wherever an entry is not exact.  Power-of-two alphas, which is what
 // the reference's quantiser emits (quantizers/bcq_quant/bcq_shift.py:15-24), are exact and skip it.
-// Two fp16 pieces hold 22 bits of the largest entry of a wave's first step.
+// The power of two (the unit) belongs to ONE output, or to one alpha row group of a block format, and
+// follows that output's weights along K: it is chosen anew wherever an inexact step has left the window
+// [64, 32768] (outputs of one wave may be any number of binades apart, and so may the groups of an output).
+// Two pieces then hold a weight to 2^-23 of itself or 2^-31 of the largest weight of the same output in
+// the same K-step (64 or 128 inputs), whichever is larger.  One unit for all 64 outputs of a wave, as these kernels had at
+// first, lost a bit per binade beyond the tenth and every bit beyond the thirty-third.  Units of their own
+// cost 0 to 2 % (11008x4096x3, 2048 rows 199.0 -> 202.7 us; 5120x13824x2, 512 rows 105.0 -> 106.1), on short
+// calls whose lanes form four tables each 0.3 us (2964x2208x3 in groups of 96, 7 rows 7.5 -> 7.85).
 #ifndef LUT_DEQUANT_DEVICE_H
 #define LUT_DEQUANT_DEVICE_H
 
@@ -149,10 +156,10 @@ __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntri
 
 // Whether some entry may be no fp16 number.  The entries of up to three planes are looked at themselves.
 // More of them are bounded by the multipliers: all are multiples of u, the smallest of the multipliers' lowest
-// set bits, and at most the sum of magnitudes, so they have eleven bits where that is at most 2048 u: a third
-// of the instructions.  (bits & bits - 1 clears the lowest mantissa bit; on a power of two it clears an
-// exponent bit instead, which halves u at worst.)  A zero multiplier counts for nothing; NaN and infinity
-// are inexact.
+// set bits, and at most the sum of magnitudes, so they are fp16 numbers where that is at most 2048 u (eleven
+// bits) and u is no less than 2^-24 (the smallest fp16 number): a third of the instructions.  (bits & bits - 1
+// clears the lowest mantissa bit; on a power of two it clears an exponent bit instead, which halves u at
+// worst.)  A zero multiplier counts for nothing; NaN and infinity are inexact.
 template <int NB, bool UNI>
 __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const float (&a)[NB], float q)
 {
@@ -174,7 +181,7 @@ __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const 
 #pragma unroll
     for (int b = 0; b < NB; ++b) take(a[b]);
     if constexpr (UNI) take(q);
-    return !(sum <= least * 2048.0f) || sum > 32768.0f;
+    return !(sum <= least * 2048.0f) || sum > 32768.0f || least < 0x1p-24f;
 }
 
 // The sign words of 32 inputs of one output, one per plane -> y[c]: byte i of it holds the table indices
@@ -283,27 +290,61 @@ __device__ __forceinline__ float decode_multiplier(uint32_t u, int mode)
     return v;
 }
 
-// ---- the power of two that keeps a wave's weights in the middle of fp16's range ---------------------------
-__device__ __forceinline__ float wave_max_finite(float v)   // of |v| over the 64 lanes; NaN and inf count as 0
+// ---- the power of two that keeps an output's weights in the middle of fp16's range -------------------------
+// (`from`: opaque, so that a loop does not keep the many sums of it and constants in registers of their own)
+__device__ __forceinline__ int opaque(int from)
 {
-    uint32_t m = __builtin_bit_cast(uint32_t, v) & 0x7fffffffu;
-    if (m >= 0x7f800000u) m = 0u;
-    auto other = [](uint32_t x, auto ctrl) {
-        return (uint32_t)__builtin_amdgcn_update_dpp((int)x, (int)x, decltype(ctrl)::value, 0xf, 0xf, false);
-    };
-    m = max(m, other(m, std::integral_constant<int, 0xb1>()));    // quad_perm [1,0,3,2]
-    m = max(m, other(m, std::integral_constant<int, 0x4e>()));    // quad_perm [2,3,0,1]
-    m = max(m, other(m, std::integral_constant<int, 0x141>()));   // row_half_mirror
-    m = max(m, other(m, std::integral_constant<int, 0x140>()));   // row_mirror
-    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)m, 0), b = (uint32_t)__builtin_amdgcn_readlane((int)m, 16);
-    const uint32_t c = (uint32_t)__builtin_amdgcn_readlane((int)m, 32), d = (uint32_t)__builtin_amdgcn_readlane((int)m, 48);
-    return __builtin_bit_cast(float, max(max(a, b), max(c, d)));
+    asm volatile("" : "+v"(from));
+    return from;
 }
 
-__device__ __forceinline__ float unit_for(float most)   // brings `most` to 2^8 .. 2^9
+__device__ __forceinline__ float lane_value(float v, int src)
 {
-    const int e = most > 0.0f ? (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127 : 8;
-    return ldexpf(1.0f, min(max(8 - e, -120), 120));
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * src, __builtin_bit_cast(int, v)));
+}
+
+// Maximum over the 64 lanes, as a scalar (v is not negative).
+__device__ __forceinline__ float wave_max(float v)
+{
+    v = fmaxf(v, dpp_move<0xb1>(v));    // quad_perm [1,0,3,2]
+    v = fmaxf(v, dpp_move<0x4e>(v));    // quad_perm [2,3,0,1]
+    v = fmaxf(v, dpp_move<0x141>(v));   // row_half_mirror
+    v = fmaxf(v, dpp_move<0x140>(v));   // row_mirror
+    const int vi = __builtin_bit_cast(int, v);
+    auto row = [&](int l) { return (uint32_t)__builtin_amdgcn_readlane(vi, l); };
+    return __builtin_bit_cast(float, max(max(row(0), row(16)), max(row(32), row(48))));
+}
+
+// Upper bound of |W| from the multipliers; NaN and infinity count as 0 (no unit helps them).
+template <int NB>
+__device__ __forceinline__ float finite_magnitude(const float (&a)[NB], float q)
+{
+    float s = fabsf(q);
+#pragma unroll
+    for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
+    return s < __builtin_inff() ? s : 0.0f;
+}
+
+// The unit that brings `most` to 2^12 .. 2^13: room to grow by eight and to shrink by 64 before another one is
+// needed.  At most 2^60, where a weight is held to 2^-85, which no sum of 2^17 products with fp16 activations
+// shows in units of 2^-31; sums on the scale of the unit stay finite in fp32.
+__device__ __forceinline__ float unit_for(float most)
+{
+    const int e = most > 0.0f ? (int)(__builtin_bit_cast(uint32_t, most) >> 23) - 127 : 12;
+    return __builtin_bit_cast(float, (uint32_t)(127 + min(max(12 - e, -115), 60)) << 23);
+}
+
+__device__ __forceinline__ float inverse_unit(float unit)   // exact: a unit is a power of two
+{
+    return __builtin_bit_cast(float, 0x7f000000u - __builtin_bit_cast(uint32_t, unit));
+}
+
+// Whether two pieces of weights of magnitude `most` (0: none) call for another unit: beyond 32768 fp16
+// overflows, below 64 the second piece loses bits under 2^-24.
+__device__ __forceinline__ bool outside_window(float most, float unit)
+{
+    const float m = most * unit;
+    return m > 32768.0f || (m < 64.0f && m > 0.0f && unit < 0x1p60f);
 }
 
 }  // namespace lutgemm

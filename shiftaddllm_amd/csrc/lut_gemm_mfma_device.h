@@ -197,7 +197,13 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 
     // ---- one K-step ---------------------------------------------------------------------------------
     constexpr int kTables = OWN ? 4 : 1;   // tables this lane forms
-    float unit = 0.0f;                     // weights are formed as W * unit, a power of two; 0: not chosen yet
+    // Weights are formed as W * unit, a power of two per output (block formats: per row group), held by the lane
+    // whose table it scales (OWN: by the four lanes whose tables they are).
+    float unit[kTables];
+    bool chosen = false;
+    bool same = OWN;                       // all units of the wave are one
+#pragma unroll
+    for (int i = 0; i < kTables; ++i) unit[i] = 1.0f;
     // multipliers of this lane's table i
     auto multipliers = [&](const Operands &ops, int i, float (&a)[NB], float &q) {
         q = 0.0f;
@@ -215,28 +221,63 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             for (int b = 0; b < NB; ++b) a[b] = OWN ? half_of(2 * b) : half_bits_to_float(ops.s[b]);
         }
     };
-    auto largest = [&](const Operands &ops) {   // upper bound of |W| in the step
-        float most = 0.0f;
+    auto magnitude = [&](const Operands &ops, int i) {   // upper bound of |W| in the lane's table i
+        float a[NB], q;
+        multipliers(ops, i, a, q);
+        return finite_magnitude(a, q);
+    };
+    // its maximum over the tables that share a unit
+    auto largest = [&](const Operands &ops, int i) {
+        float m = magnitude(ops, i);
+        if constexpr (OWN) {   // the step's four words
+            m = fmaxf(m, lane_value(m, opaque(lane) ^ 16));
+            m = fmaxf(m, lane_value(m, opaque(lane) ^ 32));
+        } else if constexpr (FMT == kWeightBlock) {   // the step's sixteen chunks: a row of 16 lanes
+            m = fmaxf(m, dpp_move<0xb1>(m));
+            m = fmaxf(m, dpp_move<0x4e>(m));
+            m = fmaxf(m, dpp_move<0x141>(m));
+            m = fmaxf(m, dpp_move<0x140>(m));
+        }
+        return m;
+    };
+    // Accumulators times a factor per unit: register r of acc[e] is output 4 * (4 * kb + r) + e of the tile.
+    // In the main loop the factors are fetched a few at a time (all sixteen in flight are registers that the
+    // operands of the steps need).
+    auto scale_sums = [&](const float (&by)[kTables], auto in_loop) {
+        [[maybe_unused]] const float of_quad = FMT == kWeightBlock ? lane_value(by[0], 16 * rg_of) : 0.0f;
+        const int quad = opaque(4 * kb);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            [[maybe_unused]] const float of_group = FMT == kWeightBlock ? lane_value(of_quad, quad + r) : 0.0f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float f = FMT == kWeightBlock ? of_group : OWN ? lane_value(by[e % kTables], quad + r) : lane_value(by[0], 16 * e + quad + r);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) acc[e][mt][r] *= f;
+            }
+            if constexpr (decltype(in_loop)::value) __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    auto refit = [&](const Operands &ops) {   // units that suit this step
+        float by[kTables];
 #pragma unroll
         for (int i = 0; i < kTables; ++i) {
-            float a[NB], q, s;
-            multipliers(ops, i, a, q);
-            s = fabsf(q);
-#pragma unroll
-            for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
-            most = fmaxf(most, s);
+            const float most = largest(ops, i), fresh = outside_window(most, unit[i]) ? unit_for(most) : unit[i];
+            by[i] = fresh * inverse_unit(unit[i]);
+            unit[i] = fresh;
         }
-        return wave_max_finite(most);
+        same = false;
+        scale_sums(by, std::true_type());
     };
     // The lane's tables of a step, or of what rounding their entries leaves over; true when some entry may
     // not be an fp16 number.
     auto make_tables = [&](const Operands &ops, int step, bool lo, Table (&tab)[kTables]) {
-        float u = unit;
-        if constexpr (FMT == kWeightBlock) u = 16 * step + li < p.K / 8 ? u : 0.0f;
-        if constexpr (OWN) u = 4 * step + kb < p.kwords ? u : 0.0f;
         bool inexact = false;
 #pragma unroll
         for (int i = 0; i < kTables; ++i) {
+            float u = unit[i];
+            if constexpr (FMT == kWeightBlock) u = 16 * step + li < p.K / 8 ? u : 0.0f;
+            if constexpr (OWN) u = 4 * step + kb < p.kwords ? u : 0.0f;
             float a[NB], q;
             multipliers(ops, i, a, q);
 #pragma unroll
@@ -299,23 +340,41 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
                         for (int j = 0; j < 4; ++j) ops.x[mt][c][j] = halves_of_bf16(ops.x[mt][c][j]);
             }
-        if (unit == 0.0f) unit = unit_for(largest(ops));
+        if (!chosen) {
+            chosen = true;
+            if constexpr (OWN) {
+                float most = 0.0f;
+#pragma unroll
+                for (int i = 0; i < kTables; ++i) most = fmaxf(most, magnitude(ops, i));
+                most = wave_max(most);
+#pragma unroll
+                for (int i = 0; i < kTables; ++i) unit[i] = unit_for(most);
+            } else {
+                unit[0] = unit_for(largest(ops, 0));
+            }
+        }
         Table tab[kTables];
-        const bool inexact = __builtin_amdgcn_ballot_w64(make_tables(ops, step, false, tab)) != 0ull;
+        bool inexact = __builtin_amdgcn_ballot_w64(make_tables(ops, step, false, tab)) != 0ull;
+        auto forget = [&]() {   // (the scales as new values: or the multipliers are kept for a second piece)
+            if constexpr (OWN)
+#pragma unroll
+                for (int r = 0; r < Operands::kScales; ++r) asm volatile("" : "+v"(ops.s[r]));
+        };
         if (inexact) {
-            const float most = largest(ops);
-            if (most * unit > 32768.0f) {   // out of fp16's range: another unit first
-                const float fresh = unit_for(most), by = fresh / unit;
-                unit = fresh;
+            forget();
+            bool outside = false;
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) acc[e][mt] *= by;
-                (void)make_tables(ops, step, false, tab);
+            for (int i = 0; i < kTables; ++i) outside = outside_window(magnitude(ops, i), unit[i]) || outside;
+            if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
+                forget();
+                refit(ops);
+                forget();
+                inexact = __builtin_amdgcn_ballot_w64(make_tables(ops, step, false, tab)) != 0ull;
             }
         }
         multiply(ops, tab);
         if (inexact) {
+            forget();
             (void)make_tables(ops, step, true, tab);
             multiply(ops, tab);
         }
@@ -363,11 +422,18 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     if (!ONE && n_steps > 0 && (n_steps & 1) == 0) compute(opB, own_last);
     if constexpr (EXTRA && !ONE)
         if (n_steps == 0 && scaled) row_scales();  // (a wave without steps still owes its rows)
-    const float back = unit == 0.0f ? 1.0f : 1.0f / unit;
+    if (same) {
+        const float back = inverse_unit(unit[0]);
 #pragma unroll
-    for (int e = 0; e < 4; ++e)
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[e][mt] *= back;
+            for (int mt = 0; mt < MT; ++mt) acc[e][mt] *= back;
+    } else {
+        float back[kTables];
+#pragma unroll
+        for (int i = 0; i < kTables; ++i) back[i] = inverse_unit(unit[i]);
+        scale_sums(back, std::false_type());
+    }
 
     // ---- the 8 waves' accumulators meet in LDS -----------------------------------
     // red[wave][j = (e*MT + mt)*4 + r][lane], rows padded to 65 words so that the

@@ -204,26 +204,26 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     u32x4 A[2][4][2];            // [step parity][matrix instruction][fragment]
     bool lo_cur = false;         // rounding the current step's weights to fp16 left something over (uniform over the wave)
     WeightTable<NB, UNI> tab[kFragTabs][kTabs];
-    float unit = 1.0f;           // weights are formed as W * unit, a power of two
-    auto largest = [&](int t) {   // upper bound of |W| in the step
+    // weights are formed as W * unit, a power of two per output (block formats: per row group)
+    float unit[kFragTabs];       // (of this lane's outputs)
+    auto magnitude = [&](int t, int f) {   // upper bound of |W| in this lane's tables of fragment f
         float most = 0.0f;
 #pragma unroll
-        for (int f = 0; f < kFragTabs; ++f)
-#pragma unroll
-            for (int c = 0; c < kTabs; ++c) {
-                float a[NB], q, s;
-                multipliers(t, f, c, a, q);
-                s = fabsf(q);
-#pragma unroll
-                for (int b = 0; b < NB; ++b) s += fabsf(a[b]);
-                most = fmaxf(most, s);
-            }
-        return wave_max_finite(most);
+        for (int c = 0; c < kTabs; ++c) {
+            float a[NB], q;
+            multipliers(t, f, c, a, q);
+            most = fmaxf(most, finite_magnitude(a, q));
+        }
+        return most;
+    };
+    auto largest = [&](int t, int f) {   // of the step's two words
+        const float m = magnitude(t, f);
+        return fmaxf(m, lane_value(m, opaque(lane) ^ 32));
     };
     // One table of step t, or of what its rounding leaves over; true when some entry may not
     // be an fp16 number.
     auto make_table = [&](int t, bool lo, int f, int c) {
-        const float u = 2 * t + kh < p.kwords ? unit : 0.0f;   // a word beyond K has no weight
+        const float u = 2 * t + kh < p.kwords ? unit[f] : 0.0f;   // a word beyond K has no weight
         float a[NB], q;
         multipliers(t, f, c, a, q);
 #pragma unroll
@@ -269,15 +269,40 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         }
     };
 
+    // Sums times a factor per unit: register 4 g + r of a fragment is its output 8 g + 4 kh + r.  (In the main loop
+    // the factors are fetched a few at a time: registers are short there.)
+    auto scale_sums = [&](const float (&by)[kFragTabs], auto in_loop) {
+        const int first = opaque(4 * kh);
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const float v = by[f % kFragTabs];
+                const float x = FMT == kTileBlockWide ? v : lane_value(v, first + 8 * (r >> 2) + (r & 3));
+#pragma unroll
+                for (int i = 0; i < MF; ++i) acc[f][i][r] *= x;
+                if constexpr (decltype(in_loop)::value)
+                    if (r % 4 == 3) __builtin_amdgcn_sched_barrier(0);
+            }
+    };
+
     uint32_t words_lo[2][NB];
     // Some weight of step t (in A[set]) is no fp16 number: a second piece is due in that step, after a change
-    // of unit if it is out of fp16's range.
+    // of the units that do not suit it.
     auto second_piece = [&](int t, int set) {
         load_words(t, words_lo);
-        const float most = largest(t);
-        if (most * unit > 32768.0f) {
-            const float fresh = unit_for(most), by = fresh / unit;
-            unit = fresh;
+        bool outside = false;
+#pragma unroll
+        for (int f = 0; f < kFragTabs; ++f) outside = outside_window(magnitude(t, f), unit[f]) || outside;
+        if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
+            float by[kFragTabs];
+#pragma unroll
+            for (int f = 0; f < kFragTabs; ++f) {
+                const float most = largest(t, f), fresh = outside_window(most, unit[f]) ? unit_for(most) : unit[f];
+                by[f] = fresh * inverse_unit(unit[f]);
+                unit[f] = fresh;
+            }
+            scale_sums(by, std::true_type());
             (void)make_tables(t, false);
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
@@ -285,10 +310,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                 sign_indices<NB, UNI>(words_lo[f], y);
 #pragma unroll
                 for (int c = 0; c < 4; ++c) A[set][c][f] = pick(f, c, y);
-#pragma unroll
-                for (int i = 0; i < MF; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[f][i][r] *= by;
             }
         }
     };
@@ -364,7 +385,8 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     store_x(0);
     load_x(t0 + 1);
     __syncthreads();
-    unit = unit_for(largest(t0));
+#pragma unroll
+    for (int f = 0; f < kFragTabs; ++f) unit[f] = unit_for(largest(t0, f));
     lo_cur = __builtin_amdgcn_ballot_w64(make_tables(t0, false)) != 0ull;
     if (lo_cur) load_words(t0, words_lo);
 #pragma unroll
@@ -381,13 +403,10 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         step(t + 1, std::integral_constant<int, 1>());
     }
 
-    const float back = 1.0f / unit;
+    float back[kFragTabs];
 #pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[f][i][r] *= back;
+    for (int f = 0; f < kFragTabs; ++f) back[f] = inverse_unit(unit[f]);
+    scale_sums(back, std::false_type());
 
     // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
     // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
