@@ -756,8 +756,9 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     }
     p.x_type = x_type;
     p.out_type = out_type;
-    if (tile_wanted(p, mode)) return x_type == kIoF16 ? run_tile(p, mode, acc) : LUTGEMM_EUNSUP;
+    // (ahead of the GEMM kernel: LUTGEMM_OPTION_BLOCK_SCALED = 2 means any number of rows)
     if (alpha_pow2 && mode == kRowF16 && mfma_eligible(p, mode) && p.M >= mfma_min_rows() && mx_wanted(p)) return run_mx(p, acc);
+    if (tile_wanted(p, mode)) return x_type == kIoF16 ? run_tile(p, mode, acc) : LUTGEMM_EUNSUP;
     int kernel = kLookup, mrows = 1;
     rc = plan_single(p, mode, &kernel, &mrows);
     if (rc != LUTGEMM_OK) return rc;

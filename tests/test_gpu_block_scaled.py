@@ -243,3 +243,22 @@ def test_random_shapes_of_the_pow2_entry_against_a_dense_product(gpu_device, blo
         kernels.add(plan.kernel)
         assert rel <= 5e-4 and mad <= 2.5e-3, (N, K, nb, gs, M, rel, mad)
     assert kernels == ({2} if block_scaled == 2 else {1}), kernels
+
+
+@pytest.mark.parametrize("N,K,nb,M", [(11008, 4096, 1, 200), (8192, 8192, 2, 100)])
+def test_forced_block_scaled_kernel_is_not_displaced_by_the_gemm_kernel(gpu_device, N, K, nb, M):
+    """Option BLOCK_SCALED = 2 holds for any number of rows: calls that would otherwise take the GEMM kernel give
+    the same bits whether or not that kernel is switched off."""
+    lib = native.cabi()
+    bW, alpha, x, bias = _problem(N, K, nb, M, seed=N + M)
+    plan = native.Plan()
+    assert lib.lutgemm_describe_tile_plan(0, N, K, nb, K // 128, M, ctypes.byref(plan)) == 0 and plan.kernel == 3
+    lib.lutgemm_set_option(native.OPTIONS["BLOCK_SCALED"], 2)
+    got = _run(lib.lutgemm_gemv_rowwise_pow2_f16, gpu_device, bW, alpha, x, bias, 128)
+    lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 65536)
+    try:
+        want = _run(lib.lutgemm_gemv_rowwise_pow2_f16, gpu_device, bW, alpha, x, bias, 128)
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+        lib.lutgemm_set_option(native.OPTIONS["BLOCK_SCALED"], -1)
+    assert torch.equal(got, want)
