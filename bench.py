@@ -743,7 +743,7 @@ def main():
             if pow2:
                 plan = native.Plan()
                 check(lib.lutgemm_describe_pow2_plan(N, K, nb, K // GROUP, M, ctypes.byref(plan)))
-                e["kernel"] = ("lookup", "matrix_core_fp16", "matrix_core_block_scaled")[plan.kernel]
+                e["kernel"] = ("lookup", "matrix_core_fp16", "matrix_core_block_scaled", "gemm_fp16")[plan.kernel]
             if with_oracle:
                 g = gp[0]
                 with torch.cuda.stream(stream):

@@ -276,8 +276,11 @@ int lutgemm_reserve_workspace(void *stream, size_t words);
  * `format` is one of LUTGEMM_FORMAT_*; `groups` is num_groups for the row-wise
  * and uniform formats and the number of row groups R for the block formats.
  * Returns what the compute entry point would return for the same sizes
- * (LUTGEMM_EINVAL, LUTGEMM_EUNSUP) without launching anything.  The tuning knobs
- * of the environment apply as they do to the compute calls.  No counterpart in
+ * (LUTGEMM_EINVAL, LUTGEMM_EUNSUP) without launching anything.  The tuning options
+ * apply as they do to the compute calls.  The K-slices of the GEMM kernel (rows_per_pass
+ * 64 or 128) are added up by a second launch; their sums live in the per-stream buffer of
+ * the split activations, and a call under capture whose buffer is too small, and
+ * lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order.  No counterpart in
  * the reference, whose launch geometry is fixed at compile time
  * (mv_fp16_bias.hpp:726-774).
  */
@@ -293,31 +296,23 @@ typedef struct lutgemm_plan {
     int rows_per_pass;   /* activation rows a workgroup handles together */
     int row_chunks;      /* ceil(M / rows_per_pass) */
     int tiles;           /* output tiles of tile_columns columns */
-    int k_units;         /* sets of 256 inputs (look-up), steps of 128 (matrix cores) */
+    int k_units;         /* sets of 256 inputs (look-up), steps of 128 (matrix cores), of 64 (GEMM; an even number) */
     /* look-up kernel: the tiles x k_units items of a row chunk, tile-major, are cut into
      * `ranges` contiguous ranges: the first `long_ranges` of `items_per_long_range`
      * items, the others of `items_per_short_range` (the last one may be shorter) */
     int ranges, long_ranges, items_per_long_range, items_per_short_range;
-    /* matrix-core kernel: every tile is cut into `k_slices` slices of
+    /* matrix-core and GEMM kernels: every tile is cut into `k_slices` slices of
      * `units_per_slice` steps (the last one may be shorter) */
     int k_slices, units_per_slice;
     int needs_workspace; /* 1: the launch uses lutgemm_workspace_words(N, M) accumulator words */
-    int tile_columns;    /* output columns per tile: 256 (look-up), 512 (look-up, twin items), 64 (matrix cores) */
+    int tile_columns;    /* output columns per tile: 256 (look-up, GEMM), 512 (look-up, twin items), 64 (matrix cores) */
 } lutgemm_plan;
 
 int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
-/* What a call of two rows and more takes, in every format.  lutgemm_describe_plan describes the look-up
- * kernel and, for row-wise problems whose sizes fit it (K a multiple of 128, groups of a multiple of 128
- * inputs, N a multiple of 16), the matrix-core kernel with the row tiles that grouped problems have (32 rows
- * from 17 rows on; a lone call may take 16-row tiles there); beyond those, from two or three rows on, the
- * matrix-core kernel takes every problem whose tiles of 64 columns touch at most four alpha row groups
- * (kernel 1), and calls of many rows run on the GEMM kernel (kernel 3: rows_per_pass 64 or 128, tiles of
- * 256 columns, k_units and units_per_slice in steps of 64 inputs, k_slices that a second launch adds up;
- * their sums live in the per-stream buffer of the split activations; a call under capture whose buffer is
- * too small, and lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order).
- * A call that neither takes is described as lutgemm_describe_plan describes it. */
+/* The same function under the name it had while it alone described kernels 1 (formats other than whole groups of
+ * 128 inputs) and 3. */
 int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan);
-/* The same for lutgemm_gemv_rowwise_pow2_f16: kernel 2 is the block-scaled matrix-core kernel
+/* What lutgemm_gemv_rowwise_pow2_f16 takes: kernel 2 is the block-scaled matrix-core kernel
  * (rows_per_pass 5, 8 or 16; tiles of 64 columns, steps of 128 inputs); a call that takes one
  * of the other kernels is described as lutgemm_describe_plan describes it. */
 int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_plan *plan);

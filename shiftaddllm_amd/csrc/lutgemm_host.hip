@@ -520,10 +520,10 @@ bool mfma_any(const Problem &p, int mode)
     return (unsigned long long)p.kwords * p.nb * p.N * 2 < (1ull << 32);
 }
 
-int plan_single(Problem &p, int mode, int *kernel, int *mrows, bool any = true)
+int plan_single(Problem &p, int mode, int *kernel, int *mrows)
 {
-    if (mfma_eligible(p, mode) || (any && mfma_any(p, mode))) {
-        const int mt = any ? mfma_row_tiles(p) : p.M > 16 ? 2 : 1;
+    if (mfma_eligible(p, mode) || mfma_any(p, mode)) {
+        const int mt = mfma_row_tiles(p);
         Group one{};
         one.count = 1;
         one.p[0] = p;
@@ -1448,33 +1448,54 @@ size_t lutgemm_algorithmic_bytes(int N, int K, int nb, int M, size_t alpha_entri
     return signs + alphas + xin + yio;
 }
 
-static int describe_plan(int format, int N, int K, int nb, int groups, int M, bool any, lutgemm_plan *plan)
+// The problem of a describe call, without operands (nothing is dereferenced while planning: any aligned
+// non-null address will do).
+static int fill_described(Problem &p, int format, int N, int K, int nb, int groups, int M)
+{
+    alignas(16) static const uint64_t dummy[2] = {0, 0};
+    return fill_problem(p, format, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
+}
+
+int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
 {
     if (!plan || format < LUTGEMM_FORMAT_ROWWISE_F16 || format > LUTGEMM_FORMAT_UNIFORM_F16) return LUTGEMM_EINVAL;
-    // (nothing is dereferenced while planning: any aligned non-null address will do)
-    alignas(16) static const uint64_t dummy[2] = {0, 0};
     Problem p;
-    int rc = fill_problem(p, format, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
-    if (rc != LUTGEMM_OK) return rc;
-    int kernel = kLookup, mrows = 1;
-    rc = plan_single(p, format, &kernel, &mrows, any);
+    int rc = fill_described(p, format, N, K, nb, groups, M);
     if (rc != LUTGEMM_OK) return rc;
     *plan = lutgemm_plan{};
+    if (tile_wanted(p, format)) {
+        TileProblem t{};
+        t.N = N;
+        t.M = M;
+        t.kwords = p.kwords;
+        plan_tile(t, kTileSumBytes);
+        plan->kernel = 3;
+        plan->workgroups = t.n_tiles * t.m_tiles * t.ksplit;
+        plan->rows_per_pass = t.tile_rows;
+        plan->row_chunks = t.m_tiles;
+        plan->tiles = t.n_tiles;
+        plan->tile_columns = 256;
+        plan->k_units = t.steps;
+        plan->k_slices = t.ksplit;
+        plan->units_per_slice = t.slice_steps;
+        return LUTGEMM_OK;
+    }
+    int kernel = kLookup, mrows = 1;
+    rc = plan_single(p, format, &kernel, &mrows);
+    if (rc != LUTGEMM_OK) return rc;
     plan->kernel = kernel;
     plan->workgroups = p.n_blocks;
     plan->rows_per_pass = mrows;
     plan->row_chunks = p.mchunks;
+    plan->tiles = p.n_tiles;
+    plan->k_units = p.nsets;
     if (kernel == kMatrixCore) {
-        plan->tiles = p.n_tiles;
         plan->tile_columns = kMfmaTileCols;
-        plan->k_units = p.nsets;
         plan->k_slices = p.ksplit;
         plan->units_per_slice = p.sets_per_split;
         plan->needs_workspace = p.ksplit > 1;
     } else {
-        plan->tiles = p.n_tiles;
         plan->tile_columns = p.twin ? 2 * kTileCols : kTileCols;
-        plan->k_units = p.nsets;
         plan->long_ranges = p.long_ranges;
         plan->items_per_long_range = p.items_per_wg;
         plan->items_per_short_range = p.short_items;
@@ -1484,20 +1505,14 @@ static int describe_plan(int format, int N, int K, int nb, int groups, int M, bo
     return LUTGEMM_OK;
 }
 
-int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
-{
-    return describe_plan(format, N, K, nb, groups, M, false, plan);
-}
-
 int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
 {
-    int rc = lutgemm_describe_plan(LUTGEMM_FORMAT_ROWWISE_F16, N, K, nb, groups, M, plan);
-    if (rc != LUTGEMM_OK) return rc;
-    alignas(16) static const uint64_t dummy[2] = {0, 0};
+    if (!plan) return LUTGEMM_EINVAL;
     Problem p;
-    rc = fill_problem(p, kRowF16, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
+    const int rc = fill_described(p, kRowF16, N, K, nb, groups, M);
     if (rc != LUTGEMM_OK) return rc;
-    if (!(mfma_eligible(p, kRowF16) && p.M >= mfma_min_rows() && mx_wanted(p))) return LUTGEMM_OK;
+    if (!(mfma_eligible(p, kRowF16) && p.M >= mfma_min_rows() && mx_wanted(p)))
+        return lutgemm_describe_plan(LUTGEMM_FORMAT_ROWWISE_F16, N, K, nb, groups, M, plan);
     plan_mx(p);
     *plan = lutgemm_plan{};
     plan->kernel = 2;
@@ -1515,29 +1530,7 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
 
 int lutgemm_describe_tile_plan(int format, int N, int K, int nb, int groups, int M, lutgemm_plan *plan)
 {
-    int rc = describe_plan(format, N, K, nb, groups, M, true, plan);
-    if (rc != LUTGEMM_OK) return rc;
-    alignas(16) static const uint64_t dummy[2] = {0, 0};
-    Problem p;
-    rc = fill_problem(p, format, (const uint32_t *)dummy, dummy, dummy, dummy, (void *)dummy, N, K, nb, groups, M);
-    if (rc != LUTGEMM_OK) return rc;
-    if (!tile_wanted(p, format)) return LUTGEMM_OK;
-    TileProblem t{};
-    t.N = N;
-    t.M = M;
-    t.kwords = p.kwords;
-    plan_tile(t, kTileSumBytes);
-    *plan = lutgemm_plan{};
-    plan->kernel = 3;
-    plan->workgroups = t.n_tiles * t.m_tiles * t.ksplit;
-    plan->rows_per_pass = t.tile_rows;
-    plan->row_chunks = t.m_tiles;
-    plan->tiles = t.n_tiles;
-    plan->tile_columns = 256;
-    plan->k_units = t.steps;
-    plan->k_slices = t.ksplit;
-    plan->units_per_slice = t.slice_steps;
-    return LUTGEMM_OK;
+    return lutgemm_describe_plan(format, N, K, nb, groups, M, plan);
 }
 
 size_t lutgemm_workspace_words(int N, int M)

@@ -264,7 +264,8 @@ def test_random_shapes_against_a_dense_product(gpu_device):
         seen.add((plan.kernel, plan.rows_per_pass))
         # against an un-rounded reference: a quarter of the bars (the final fp16 rounding alone is 2e-4)
         assert rel <= REL_L2_BAR * 0.25 and mad <= MAX_ABS_BAR * 0.25, (N, K, nb, gs, M, rel, mad)
-    assert seen == {(0, 1), (0, 2), (0, 4), (1, 16), (1, 32)}, seen
+    # (four rows per pass on the look-up kernel: with the matrix cores switched off, test_gpu_options.py)
+    assert seen == {(0, 1), (0, 2), (1, 16), (1, 32), (3, 64)}, seen
 
 
 def test_batch_rows_agree_with_single_row_calls(gpu_device):

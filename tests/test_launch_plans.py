@@ -5,14 +5,16 @@ random ones.  What a kernel relies on (and cannot check itself):
                    and no output tile receives more than 40 contributions (the count field
                    of an accumulator word, lutgemm_common.h);
   matrix cores     the K-slices cover every step, none is empty, each is a whole number of
-                   eight-step rounds, and there are at most 32 of them per tile."""
+                   eight-step rounds, and there are at most 32 of them per tile;
+  GEMM kernel      the K-slices cover every step, none is empty, each is an even number of steps,
+                   and their sums fit the 64 MB a stream keeps for them."""
 import ctypes
 import os
 import random
 
 import pytest
 
-LOOKUP, MATRIX_CORE = 0, 1
+LOOKUP, MATRIX_CORE, GEMM = 0, 1, 3
 ROWWISE, BLOCK_F16, BLOCK_U16, BLOCK_I8, UNIFORM = range(5)
 MAX_CONTRIB = 40
 MAX_SLICES = 32
@@ -62,8 +64,15 @@ def check_plan(p, N, K, M):
             split = split or c > 1
         assert worst <= MAX_CONTRIB, worst
         assert bool(p.needs_workspace) >= split, "a tile shared between ranges needs accumulator words"
+    elif p.kernel == GEMM:
+        assert p.tiles == -(-N // 256) and p.tile_columns == 256 and p.rows_per_pass == (64 if M <= 64 else 128)
+        assert p.k_units == -(-K // 128) * 2 and p.units_per_slice % 2 == 0
+        assert (p.k_slices - 1) * p.units_per_slice < p.k_units <= p.k_slices * p.units_per_slice
+        assert p.workgroups == p.tiles * p.k_slices * p.row_chunks and not p.needs_workspace
+        if p.k_slices > 1:      # one round of two workgroups per CU; the sums of the slices have a place
+            assert p.workgroups <= 512 and p.k_slices <= 16 and p.k_slices * M * N * 4 <= 64 << 20
     else:
-        assert p.tiles == -(-N // 64) and p.k_units == K // 128
+        assert p.kernel == MATRIX_CORE and p.tiles == -(-N // 64) and p.tile_columns == 64 and p.k_units == -(-K // 128)
         assert p.rows_per_pass in (16, 32)
         assert 1 <= p.k_slices <= MAX_SLICES and p.units_per_slice % 8 == 0
         assert p.k_slices * p.units_per_slice >= p.k_units, "slices must cover every K-step"
@@ -86,7 +95,8 @@ def test_benchmark_shapes_every_bit_width_and_batch(lib, N, K):
         for fmt in (BLOCK_F16, BLOCK_U16, BLOCK_I8):
             for M in (1, 2, 5):
                 rc, p = describe(lib, fmt, N, K, nb, 8, M)
-                assert rc == 0 and p.kernel == LOOKUP
+                # one row: the look-up kernel, where a tile of 256 columns touches two row groups at most
+                assert rc == 0 and (M == 2 or p.kernel == (LOOKUP if M == 1 and N // 8 >= 256 else MATRIX_CORE))
                 check_plan(p, N, K, M)
 
 
@@ -94,15 +104,27 @@ def test_which_kernel_takes_what(lib):
     # one row: always the look-up kernel; three rows and more of an eligible problem: matrix cores
     assert describe(lib, ROWWISE, 4096, 4096, 3, 32, 1)[1].kernel == LOOKUP
     assert describe(lib, ROWWISE, 4096, 4096, 3, 32, 3)[1].kernel == MATRIX_CORE
-    assert describe(lib, ROWWISE, 4096, 4096, 3, 32, 32)[1].rows_per_pass == 32
+    # 17 rows and more: 32-row tiles, unless 16-row tiles are single rounds that fit the chip
+    assert describe(lib, ROWWISE, 11008, 4096, 3, 32, 32)[1].rows_per_pass == 32
+    assert describe(lib, ROWWISE, 4096, 4096, 3, 32, 32)[1].rows_per_pass == 16
+    # many rows: the GEMM kernel, in 64- or 128-row tiles
+    assert describe(lib, ROWWISE, 11008, 4096, 3, 32, 2048)[1].kernel == GEMM
+    assert describe(lib, BLOCK_I8, 5120, 13824, 2, 8, 512)[1].kernel == GEMM
+    assert describe(lib, ROWWISE, 28672, 8192, 4, 64, 64)[1].rows_per_pass == 64
     # two rows: matrix cores on short sign streams, the look-up kernel (both rows per pass) on long ones
     assert describe(lib, ROWWISE, 4096, 4096, 3, 32, 2)[1].kernel == MATRIX_CORE
     big = describe(lib, ROWWISE, 28672, 8192, 4, 64, 2)[1]
     assert big.kernel == LOOKUP and big.rows_per_pass == 2 and big.row_chunks == 1
-    # not eligible for the matrix cores: K not a multiple of 128, groups of 32 inputs, other formats
-    assert describe(lib, ROWWISE, 1024, 288, 3, 9, 8)[1].kernel == LOOKUP
-    assert describe(lib, ROWWISE, 1024, 1024, 3, 32, 8)[1].kernel == LOOKUP
-    assert describe(lib, UNIFORM, 1024, 1024, 3, 8, 8)[1].kernel == LOOKUP
+    # the matrix cores take any K, groups of any length and the other formats
+    assert describe(lib, ROWWISE, 1024, 288, 3, 9, 8)[1].kernel == MATRIX_CORE
+    assert describe(lib, ROWWISE, 1024, 1024, 3, 32, 8)[1].kernel == MATRIX_CORE
+    assert describe(lib, UNIFORM, 1024, 1024, 3, 8, 8)[1].kernel == MATRIX_CORE
+    # but not row groups of a few outputs
+    assert describe(lib, BLOCK_F16, 1024, 1024, 3, 64, 8)[1].kernel == LOOKUP
+    # calls whose description once left out the accumulator words they use
+    for fmt, N, K, nb, groups, M in ((ROWWISE, 7716, 2304, 1, 4, 32), (UNIFORM, 7948, 2432, 1, 2, 32)):
+        p = describe(lib, fmt, N, K, nb, groups, M)[1]
+        assert p.kernel == MATRIX_CORE and p.k_slices > 1 and p.needs_workspace == 1
     # the 70B shapes at one row run two workgroups per CU with unequal ranges
     p = describe(lib, ROWWISE, 28672, 8192, 4, 64, 1)[1]
     assert p.ranges == 512 and p.long_ranges == 256 and p.items_per_long_range > p.items_per_short_range
@@ -111,26 +133,33 @@ def test_which_kernel_takes_what(lib):
 
 
 def test_random_shapes(lib):
+    from shiftaddllm_amd import native
     rng = random.Random(1234)
-    seen = {LOOKUP: 0, MATRIX_CORE: 0}
-    for i in range(4000):
-        if i % 2:                                    # shapes the matrix-core kernel takes at three rows and more
+    seen = {LOOKUP: 0, MATRIX_CORE: 0, GEMM: 0}
+    for i in range(6000):
+        if i % 2:                                    # the sizes of published networks
             K = 128 * rng.randint(1, 300)
             N = 16 * rng.randint(1, 2250)
         else:
             K = 32 * rng.randint(1, 1200)
             N = 4 * rng.randint(1, 9000)
         nb = rng.randint(1, 4)
-        M = rng.choice((1, 1, 1, 2, 3, 4, 7, 16, 17, 40, 100))
-        divisors = [g for g in ((128, 256, 512, K) if i % 2 else (32, 64, 96, 128, 256, 512, K)) if K % g == 0]
-        gs = rng.choice(divisors)
-        rc, p = describe(lib, ROWWISE, N, K, nb, K // gs, M)
+        M = rng.choice((1, 1, 1, 2, 3, 4, 7, 16, 17, 33, 40, 65, 100, 300, 2048))
+        fmt = rng.choice((ROWWISE, ROWWISE, BLOCK_F16, BLOCK_U16, BLOCK_I8, UNIFORM))
+        if fmt in (ROWWISE, UNIFORM):
+            groups = K // rng.choice([g for g in ((128, 256, 512, K) if i % 2 else (32, 64, 96, 128, 256, 512, K)) if K % g == 0])
+        else:
+            groups = rng.choice([r for r in (1, 2, 5, 8, 16, N // 4) if N % (4 * r) == 0])
+        rc, p = describe(lib, fmt, N, K, nb, groups, M)
         if rc != 0:
-            assert rc == -3, (N, K, nb, gs, M, rc)      # LUTGEMM_EUNSUP: beyond the exact-division bounds
+            assert rc == -3, (fmt, N, K, nb, groups, M, rc)      # LUTGEMM_EUNSUP: beyond the exact-division bounds
             continue
         check_plan(p, N, K, M)
         seen[p.kernel] += 1
-    assert seen[LOOKUP] > 500 and seen[MATRIX_CORE] > 100
+        other = native.Plan()
+        assert lib.lutgemm_describe_tile_plan(fmt, N, K, nb, groups, M, ctypes.byref(other)) == 0
+        assert bytes(other) == bytes(p)
+    assert min(seen.values()) > 500, seen
 
 
 def test_bad_arguments(lib):
@@ -171,10 +200,16 @@ def test_tuning_options_change_plans_and_keep_their_invariants(lib):
         _, p = describe(lib, ROWWISE, 8192, 8192, 4, 64, 2)
         assert p.kernel == MATRIX_CORE
         lib.lutgemm_set_option(opt["MFMA_MIN_M"], 1000)
-        _, p = describe(lib, ROWWISE, 8192, 8192, 4, 64, 16)
+        _, p = describe(lib, ROWWISE, 8192, 8192, 4, 64, 8)
         assert p.kernel == LOOKUP and p.rows_per_pass == 4
-        check_plan(p, 8192, 8192, 16)
+        check_plan(p, 8192, 8192, 8)
         lib.lutgemm_set_option(opt["MFMA_MIN_M"], -1)
+        # rows from which the GEMM kernel takes over
+        lib.lutgemm_set_option(opt["TILE_MIN_M"], 5)
+        _, p = describe(lib, ROWWISE, 8192, 8192, 4, 64, 5)
+        assert p.kernel == GEMM
+        check_plan(p, 8192, 8192, 5)
+        lib.lutgemm_set_option(opt["TILE_MIN_M"], -1)
         # workgroups aimed at per matrix-core launch
         lib.lutgemm_set_option(opt["MFMA_BLOCKS"], 1024)
         _, p = describe(lib, ROWWISE, 8192, 8192, 4, 64, 16)
