@@ -279,8 +279,9 @@ int lutgemm_reserve_workspace(void *stream, size_t words);
  * (LUTGEMM_EINVAL, LUTGEMM_EUNSUP) without launching anything.  The tuning options
  * apply as they do to the compute calls.  The K-slices of the GEMM kernel (rows_per_pass
  * 64 or 128) are added up by a second launch; their sums live in the per-stream buffer of
- * the split activations, and a call under capture whose buffer is too small, and
- * lutgemm_gemv_rowwise_f16_noalloc, run uncut: the same sums added in another order.  No counterpart in
+ * the split activations.  Where they have no place there (a call under capture whose
+ * buffer is too small, lutgemm_gemv_rowwise_f16_noalloc) a workgroup takes the slices of
+ * its tile in turn: the same bits, more slowly.  No counterpart in
  * the reference, whose launch geometry is fixed at compile time
  * (mv_fp16_bias.hpp:726-774).
  */

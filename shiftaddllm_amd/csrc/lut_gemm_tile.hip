@@ -31,6 +31,7 @@ hipError_t launch_nb(const TileProblem &p, hipStream_t stream)
 
 hipError_t launch_tile(const TileProblem &p, int nb, hipStream_t stream)
 {
+    if (p.ksplit > 1 && !p.partial) return launch_tile_serial(p, nb, stream);
     switch (nb) {
     case 1: return launch_nb<1>(p, stream);
     case 2: return launch_nb<2>(p, stream);

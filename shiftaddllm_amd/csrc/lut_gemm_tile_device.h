@@ -54,7 +54,9 @@ __device__ __forceinline__ void static_for(F &&f)
     static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-template <int NB, int FMT, int MF>
+// SERIAL: the workgroup takes all K-slices of its tile, one after the other, and adds their sums up as
+// tile_sum_kernel does: the bits are those of slices that run side by side, and no memory is needed.
+template <int NB, int FMT, int MF, bool SERIAL>
 __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int m_tile, int slice, char *lds)
 {
     constexpr bool UNI = FMT == kTileUniform;
@@ -249,13 +251,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     };
 
     f32x16 acc[2][MF];
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int i = 0; i < MF; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) acc[f][i][r] = 0.0f;
-
     auto activations = [&](int buf, int j, int i) {
         return __builtin_bit_cast(f16x8, *(const u32x4 *)(lds + buf * kTileXBytes<MF> + i * 4096 + (bslot ^ (uint32_t)(16 * j))));
     };
@@ -374,43 +369,76 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         __syncthreads();
     };
 
-    // ---- prologue: step 0's activations in LDS, its weights in A[0] --------------------------------------
-    const int t0 = slice * p.slice_steps, t1 = min(t0 + p.slice_steps, p.steps);   // (even numbers)
-    load_x(t0);
-    load_words(t0, words);
-    fetch_scales(t0);
-    store_scales(t0);
-    fetch_scales(t0 + 1);
-    store_scales(t0 + 1);
-    store_x(0);
-    load_x(t0 + 1);
-    __syncthreads();
+    auto take_slice = [&](int sl) {
 #pragma unroll
-    for (int f = 0; f < kFragTabs; ++f) unit[f] = unit_for(largest(t0, f));
-    lo_cur = __builtin_amdgcn_ballot_w64(make_tables(t0, false)) != 0ull;
-    if (lo_cur) load_words(t0, words_lo);
+        for (int f = 0; f < 2; ++f)
 #pragma unroll
-    for (int f = 0; f < 2; ++f) {
-        uint32_t y[4];
-        sign_indices<NB, UNI>(words[f], y);
+            for (int i = 0; i < MF; ++i)
 #pragma unroll
-        for (int c = 0; c < 4; ++c) A[0][c][f] = pick(f, c, y);
-    }
-    load_words(t0 + 1, words);
+                for (int r = 0; r < 16; ++r) acc[f][i][r] = 0.0f;
+        // ---- prologue: step 0's activations in LDS, its weights in A[0] --------------------------------------
+        const int t0 = sl * p.slice_steps, t1 = min(t0 + p.slice_steps, p.steps);   // (even numbers)
+        load_x(t0);
+        load_words(t0, words);
+        fetch_scales(t0);
+        store_scales(t0);
+        fetch_scales(t0 + 1);
+        store_scales(t0 + 1);
+        store_x(0);
+        load_x(t0 + 1);
+        __syncthreads();
+#pragma unroll
+        for (int f = 0; f < kFragTabs; ++f) unit[f] = unit_for(largest(t0, f));
+        lo_cur = __builtin_amdgcn_ballot_w64(make_tables(t0, false)) != 0ull;
+        if (lo_cur) load_words(t0, words_lo);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+            uint32_t y[4];
+            sign_indices<NB, UNI>(words[f], y);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) A[0][c][f] = pick(f, c, y);
+        }
+        load_words(t0 + 1, words);
 #pragma clang loop unroll(disable)
-    for (int t = t0; t < t1; t += 2) {
-        step(t, std::integral_constant<int, 0>());
-        step(t + 1, std::integral_constant<int, 1>());
-    }
+        for (int t = t0; t < t1; t += 2) {
+            step(t, std::integral_constant<int, 0>());
+            step(t + 1, std::integral_constant<int, 1>());
+        }
 
-    float back[kFragTabs];
+        float back[kFragTabs];
 #pragma unroll
-    for (int f = 0; f < kFragTabs; ++f) back[f] = inverse_unit(unit[f]);
-    scale_sums(back, std::false_type());
+        for (int f = 0; f < kFragTabs; ++f) back[f] = inverse_unit(unit[f]);
+        scale_sums(back, std::false_type());
+    };
+    if constexpr (SERIAL) {
+        f32x16 total[2][MF];
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) total[f][i][r] = 0.0f;
+#pragma clang loop unroll(disable)
+        for (int sl = 0; sl < p.ksplit; ++sl) {   // (every wave has left the LDS of a slice behind the barrier of its last step)
+            take_slice(sl);
+#pragma unroll
+            for (int f = 0; f < 2; ++f)
+#pragma unroll
+                for (int i = 0; i < MF; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) total[f][i][r] += acc[f][i][r];
+        }
+#pragma unroll
+        for (int f = 0; f < 2; ++f)
+#pragma unroll
+            for (int i = 0; i < MF; ++i) acc[f][i] = total[f][i];
+    } else {
+        take_slice(slice);
+    }
 
     // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
     // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
-    float *sums = p.ksplit > 1 ? p.partial + (size_t)slice * p.M * p.N : nullptr;
+    float *sums = !SERIAL && p.ksplit > 1 ? p.partial + (size_t)slice * p.M * p.N : nullptr;
 #pragma unroll
     for (int i = 0; i < MF; ++i) {
         const int m = m0 + 32 * i + l32;
@@ -454,7 +482,7 @@ __device__ __forceinline__ void decode_tile(const TileProblem &p, int b, int &n_
 // Four outputs per thread: the slices' sums, in slice order, and what they are added to.  One launch behind
 // the tiles rather than the last slice's workgroup of each tile: that one alone reads at 60 GB/s
 // (4096 x 4096, 128 rows, 16 slices: 32 us, most of them this tail).
-__global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
+static __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
 {
     const uint32_t quads = (uint32_t)p.N / 4u;
     const uint32_t at = blockIdx.x * 256u + threadIdx.x;
@@ -483,14 +511,12 @@ __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem p)
     store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
 }
 
-template <int NB, int FMT, int MF>
-__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
-lut_gemm_tile_kernel(const TileProblem p)
+template <int NB, int FMT, int MF, bool SERIAL>
+__device__ __forceinline__ void gemm_workgroup(const TileProblem &p, char *lds)
 {
-    __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
     int n_tile, m_tile, slice;
     decode_tile(p, (int)blockIdx.x, n_tile, m_tile, slice);
-    if (slice >= p.ksplit) return;
+    if (slice >= (SERIAL ? 1 : p.ksplit)) return;
     if constexpr (FMT == kTileBlock) {
         // most tiles have no wave whose outputs lie in two row groups, and need half the tables
         bool straddles = false;
@@ -500,11 +526,28 @@ lut_gemm_tile_kernel(const TileProblem p)
             straddles = straddles || (first < p.N && first / p.rows_per_group != last / p.rows_per_group);
         }
         if (!straddles) {
-            gemm_tile<NB, kTileBlockWide, MF>(p, n_tile, m_tile, slice, lds);
+            gemm_tile<NB, kTileBlockWide, MF, SERIAL>(p, n_tile, m_tile, slice, lds);
             return;
         }
     }
-    gemm_tile<NB, FMT, MF>(p, n_tile, m_tile, slice, lds);
+    gemm_tile<NB, FMT, MF, SERIAL>(p, n_tile, m_tile, slice, lds);
+}
+
+template <int NB, int FMT, int MF>
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+lut_gemm_tile_kernel(const TileProblem p)
+{
+    __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
+    gemm_workgroup<NB, FMT, MF, false>(p, lds);
+}
+
+// One workgroup per tile and per CU (a call that is cut has at most 256 tiles): two sets of accumulators fit.
+template <int NB, int FMT, int MF>
+__global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
+lut_gemm_tile_serial_kernel(const TileProblem p)
+{
+    __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
+    gemm_workgroup<NB, FMT, MF, true>(p, lds);
 }
 
 }  // namespace lutgemm

@@ -633,26 +633,13 @@ int run_mx(Problem &p, const Accum &acc)
 }
 
 // ---- GEMM kernel for many activation rows ------------------------------------------------------------
-// K-slices a call may be cut into: none where their sums have no place (the entry point that allocates
-// nothing; a stream under capture whose buffer would have to grow is left uncut as well, so that reserved
-// accumulator words are all that a captured call needs).
-size_t tile_slices_allowed(const Accum &acc)
-{
-    if (acc.fixed) return 0;
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(acc.stream, &cap) == hipSuccess && cap == hipStreamCaptureStatusNone) return kTileSumBytes;
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
-    std::lock_guard<std::mutex> lock(g_ws_mutex);
-    return g_workspaces[std::make_pair(dev, acc.stream)].split_bytes;
-}
-
 // Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices: a workgroup each, two per CU.
-// `room`: bytes for the slices' sums.  Returns the time the plan should take.
+// The cut depends on the sizes alone, so that a call gives the same bits eagerly, under capture and through the
+// entry point that allocates nothing.  Returns the time the plan should take.
 // Costs in microseconds, measured at three planes: a step of a 128-row tile takes 1.2 alone on its CU and
 // 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 5; the sums of the slices
 // are written and read at about 4 TB/s, by a second launch that costs another 4.
-double plan_tile(TileProblem &t, size_t room)
+double plan_tile(TileProblem &t)
 {
     constexpr long kCUs = 256;
     t.tile_rows = t.M <= 64 ? 64 : 128;
@@ -667,7 +654,7 @@ double plan_tile(TileProblem &t, size_t room)
         const int slices = (t.steps + steps - 1) / steps;
         if (slices != ks) continue;
         const long wgs = tiles * slices;
-        if (ks > 1 && (wgs > 2 * kCUs || (size_t)ks * t.M * t.N * 4 > room)) break;
+        if (ks > 1 && (wgs > 2 * kCUs || (size_t)ks * t.M * t.N * 4 > kTileSumBytes)) break;
         const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;
         double cost = (double)rounds * (steps * beside + 5.0);
         if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 5.0;
@@ -702,7 +689,7 @@ bool tile_wanted(const Problem &p, int mode)
     t.M = p.M;
     t.kwords = p.kwords;
     const double rounds = (double)((p.N + 63) / 64) * (double)((p.M + 31) / 32) * (double)((p.K + 1023) / 1024);
-    return plan_tile(t, kTileSumBytes) < 5.0 + 3.0 * rounds / 256.0;
+    return plan_tile(t) < 5.0 + 3.0 * rounds / 256.0;
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)
@@ -722,14 +709,16 @@ int run_tile(const Problem &p, int mode, const Accum &acc)
     t.R = p.R;
     t.rows_per_group = p.rows_per_group;
     t.mode = mode;
-    plan_tile(t, tile_slices_allowed(acc));
+    plan_tile(t);
     t.init_stride = p.init_stride;
     t.overwrite = p.overwrite;
     t.out_type = p.out_type;
-    if (t.ksplit > 1) {
+    // Where the slices' sums have no place (a stream under capture whose buffer would have to grow, the entry
+    // point that allocates nothing) a workgroup takes the slices of its tile in turn.
+    if (t.ksplit > 1 && !acc.fixed) {
         void *sums = nullptr;
         const int rc = stream_split_buffer(acc.stream, (size_t)t.ksplit * t.M * t.N * 4, &sums);
-        if (rc != LUTGEMM_OK) return rc;
+        if (rc != LUTGEMM_OK && rc != LUTGEMM_ECAPTURE) return rc;
         t.partial = (float *)sums;
     }
     const hipError_t e = launch_tile(t, p.nb, acc.stream);
@@ -1468,7 +1457,7 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
         t.N = N;
         t.M = M;
         t.kwords = p.kwords;
-        plan_tile(t, kTileSumBytes);
+        plan_tile(t);
         plan->kernel = 3;
         plan->workgroups = t.n_tiles * t.m_tiles * t.ksplit;
         plan->rows_per_pass = t.tile_rows;

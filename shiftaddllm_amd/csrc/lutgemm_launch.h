@@ -37,6 +37,7 @@ inline size_t mx_split_bytes(int M, int K) { return (size_t)M * K * 3 + (size_t)
 // GEMM kernel for many activation rows, every alpha format; one wave per SIMD and 256 outputs per workgroup
 struct TileProblem;
 hipError_t launch_tile(const TileProblem &p, int nb, hipStream_t stream);
+hipError_t launch_tile_serial(const TileProblem &p, int nb, hipStream_t stream);   // (launch_tile's, where p.partial is null)
 
 }  // namespace lutgemm
 
