@@ -262,8 +262,11 @@ int lutgemm_copy_bytes(void *dst, const void *src, size_t bytes, void *stream);
  * lutgemm_reserve_workspace(stream, w) no call on `stream` whose sizes need at
  * most w words synchronises or allocates, so such calls can be captured into a
  * HIP graph without a warm-up call.  For a grouped or fused call add up the
- * words of its problems.  Reserving synchronises `stream` and may not be done
- * while it is being captured (LUTGEMM_ECAPTURE).  No counterpart in the
+ * words of its problems.  The reservation also covers the sums of K-slices of
+ * calls of many rows (up to 64 bytes per word, 64 MB in all), but not the split
+ * activations of lutgemm_gemv_rowwise_pow2_f16, whose size depends on K.
+ * Reserving synchronises `stream` and may not be done while it is being captured
+ * (LUTGEMM_ECAPTURE).  No counterpart in the
  * reference, whose kernels accumulate with fp16 atomics straight into `out`.
  */
 size_t lutgemm_workspace_words(int N, int M);

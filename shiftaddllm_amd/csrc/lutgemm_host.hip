@@ -1531,7 +1531,11 @@ size_t lutgemm_workspace_words(int N, int M)
 int lutgemm_reserve_workspace(void *stream, size_t words)
 {
     unsigned long long *unused = nullptr;
-    return stream_workspace((hipStream_t)stream, words, &unused);
+    const int rc = stream_workspace((hipStream_t)stream, words, &unused);
+    if (rc != LUTGEMM_OK) return rc;
+    // the sums of the GEMM kernel's K-slices: at most sixteen per output, 64 MB in all (plan_tile)
+    void *sums = nullptr;
+    return stream_split_buffer((hipStream_t)stream, words < kTileSumBytes / 64 ? words * 64 : kTileSumBytes, &sums);
 }
 
 int lutgemm_copy_bytes(void *dst, const void *src, size_t bytes, void *stream)

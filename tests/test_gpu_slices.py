@@ -65,3 +65,32 @@ def test_same_bits_eager_captured_and_without_allocation(gpu_device, fmt, N, K, 
             assert torch.equal(bits(fixed), want)
     finally:
         lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+
+
+@pytest.mark.parametrize("N,K,M", [(2048, 4096, 100), (5120, 13824, 512)])
+def test_a_reserved_stream_allocates_nothing_for_slices(gpu_device, N, K, M):
+    """lutgemm_reserve_workspace(stream, M * N): an eager call of many rows then takes no device memory."""
+    dev, lib = gpu_device, native.cabi()
+    bW = torch.zeros((K // 32, 2, N), dtype=torch.int32, device=dev)
+    alpha = torch.full((K // 128, 2, N), 2.0 ** -6, device=dev).half()
+    x = torch.ones((M, K), device=dev).half()
+    out = torch.zeros((M, N), device=dev).half()
+    stream = torch.cuda.Stream()
+    sp = ctypes.c_void_p(stream.cuda_stream)
+    torch.cuda.synchronize()
+    lib.lutgemm_release_workspaces()
+    assert lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 33) == 0
+    try:
+        plan = native.Plan()
+        assert lib.lutgemm_describe_plan(ROW, N, K, 2, K // 128, M, ctypes.byref(plan)) == 0 and plan.kernel == 3 and plan.k_slices > 1
+        # (the kernel's code object is loaded by a call on another stream)
+        assert lib.lutgemm_gemv_rowwise_f16(bW.data_ptr(), alpha.data_ptr(), x.data_ptr(), out.data_ptr(), N, K, 2, K // 128, M, None) == 0
+        torch.cuda.synchronize()
+        assert lib.lutgemm_reserve_workspace(sp, lib.lutgemm_workspace_words(N, M)) == 0
+        free = torch.cuda.mem_get_info()[0]
+        assert lib.lutgemm_gemv_rowwise_f16(bW.data_ptr(), alpha.data_ptr(), x.data_ptr(), out.data_ptr(), N, K, 2, K // 128, M, sp) == 0
+        torch.cuda.synchronize()
+        assert torch.cuda.mem_get_info()[0] >= free
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+    assert torch.equal(out, torch.full_like(out, -2.0 * K * 2 * 2.0 ** -6))     # all signs -1, two planes, two calls
