@@ -73,7 +73,7 @@ struct Workspace {
     unsigned long long *accum = nullptr;
     size_t words = 0;
     std::vector<unsigned long long *> retired;  // outgrown buffers: captured graphs may still name them
-    // second buffer of the block-scaled matrix-core path: the split activations of the call in flight
+    // second buffer: split activations (block-scaled kernel) or sums of K-slices (GEMM kernel) of the call in flight
     void *split = nullptr;
     size_t split_bytes = 0;
     std::vector<void *> retired_split;
@@ -81,6 +81,15 @@ struct Workspace {
 
 std::mutex g_ws_mutex;
 std::map<std::pair<int, hipStream_t>, Workspace> g_workspaces;
+
+// Sizes of grown buffers are powers of two: calls of rising size cause few growths, and all outgrown buffers of a
+// stream together are smaller than its largest.  (Beyond 2^48 no allocation succeeds, whatever its size.)
+size_t grown(size_t wanted, size_t least)
+{
+    if (wanted > ((size_t)1 << 48)) return (size_t)1 << 48;
+    while (least < wanted) least *= 2;
+    return least;
+}
 
 // Grow-only, zero-initialised accumulator words per (device, stream).  Growing
 // synchronises the stream and allocates, which a stream under capture cannot do: that
@@ -104,7 +113,7 @@ int stream_workspace(hipStream_t stream, size_t words, unsigned long long **out)
         if (ws.accum) ws.retired.push_back(ws.accum);
         ws.accum = nullptr;
         ws.words = 0;
-        const size_t want = words < (1u << 18) ? (1u << 18) : words;
+        const size_t want = grown(words, 1u << 18);
         e = hipMalloc((void **)&ws.accum, want * sizeof(unsigned long long));
         if (e != hipSuccess) {
             g_last_hip_error = (int)e;
@@ -120,8 +129,8 @@ int stream_workspace(hipStream_t stream, size_t words, unsigned long long **out)
     return LUTGEMM_OK;
 }
 
-// The same for the split activations of the block-scaled path (not zeroed: every call writes what it
-// reads).  Calls on one stream are ordered, so they can share the buffer.
+// The same for the split activations of the block-scaled path and the sums of the GEMM kernel's K-slices (not
+// zeroed: every call writes what it reads).  Calls on one stream are ordered, so they can share the buffer.
 int stream_split_buffer(hipStream_t stream, size_t bytes, void **out)
 {
     int dev = 0;
@@ -139,7 +148,7 @@ int stream_split_buffer(hipStream_t stream, size_t bytes, void **out)
         if (ws.split) ws.retired_split.push_back(ws.split);
         ws.split = nullptr;
         ws.split_bytes = 0;
-        const size_t want = bytes < (1u << 20) ? (1u << 20) : bytes;
+        const size_t want = grown(bytes, 1u << 20);
         e = hipMalloc(&ws.split, want);
         if (e != hipSuccess) {
             g_last_hip_error = (int)e;

@@ -94,3 +94,35 @@ def test_a_reserved_stream_allocates_nothing_for_slices(gpu_device, N, K, M):
     finally:
         lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
     assert torch.equal(out, torch.full_like(out, -2.0 * K * 2 * 2.0 ** -6))     # all signs -1, two planes, two calls
+
+
+def test_calls_of_rising_size_keep_a_bounded_amount_of_memory(gpu_device):
+    """Thirty prompts, each longer than the one before: the buffers that a stream outgrows together stay below the
+    largest one, whose size is a power of two."""
+    dev, lib = gpu_device, native.cabi()
+    N, K, most = 2048, 4096, 512
+    bW = torch.zeros((K // 32, 2, N), dtype=torch.int32, device=dev)
+    alpha = torch.full((K // 128, 2, N), 2.0 ** -6, device=dev).half()
+    x = torch.ones((most, K), device=dev).half()
+    out = torch.zeros((most, N), device=dev).half()
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    lib.lutgemm_release_workspaces()
+    assert lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 33) == 0
+    call = lambda M, sp: lib.lutgemm_gemv_rowwise_f16(bW.data_ptr(), alpha.data_ptr(), x.data_ptr(), out.data_ptr(), N, K, 2, K // 128, M, sp)
+    try:
+        plan = native.Plan()
+        assert lib.lutgemm_describe_plan(ROW, N, K, 2, K // 128, most, ctypes.byref(plan)) == 0 and plan.kernel == 3
+        largest = plan.k_slices * most * N * 4
+        assert call(64, None) == 0 and call(128, None) == 0             # (code objects are loaded)
+        torch.cuda.synchronize()
+        lib.lutgemm_release_workspaces()
+        free = torch.cuda.mem_get_info()[0]
+        for M in range(48, most + 1, 16):
+            assert call(M, ctypes.c_void_p(stream.cuda_stream)) == 0
+        torch.cuda.synchronize()
+        taken = free - torch.cuda.mem_get_info()[0]
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+    power = 1 << (largest - 1).bit_length()
+    assert largest <= taken <= 2 * power + (2 << 20), (largest, taken)
