@@ -160,6 +160,10 @@ int stream_split_buffer(hipStream_t stream, size_t bytes, void **out)
     return LUTGEMM_OK;
 }
 
+// Calls that take two launches with the second buffer between them hold this lock over both: a call of another
+// host thread on the same stream would otherwise put its own first launch in between.
+std::mutex g_two_launches_mutex;
+
 // Where a call takes its accumulator words from.
 struct Accum {
     hipStream_t stream;
@@ -634,6 +638,7 @@ int run_mx(Problem &p, const Accum &acc)
         if (rc != LUTGEMM_OK) return rc;
     }
     if (acc.fixed) return LUTGEMM_EUNSUP;
+    std::lock_guard<std::mutex> lock(g_two_launches_mutex);
     void *buf = nullptr;
     int rc = stream_split_buffer(acc.stream, mx_split_bytes(p.M, p.K), &buf);
     if (rc != LUTGEMM_OK) return rc;
@@ -722,10 +727,12 @@ int run_tile(const Problem &p, int mode, const Accum &acc)
     t.init_stride = p.init_stride;
     t.overwrite = p.overwrite;
     t.out_type = p.out_type;
+    std::unique_lock<std::mutex> lock(g_two_launches_mutex, std::defer_lock);
     // Where the slices' sums have no place (a stream under capture whose buffer would have to grow, the entry
     // point that allocates nothing) a workgroup takes the slices of its tile in turn.
     if (t.ksplit > 1 && !acc.fixed) {
         void *sums = nullptr;
+        lock.lock();
         const int rc = stream_split_buffer(acc.stream, (size_t)t.ksplit * t.M * t.N * 4, &sums);
         if (rc != LUTGEMM_OK && rc != LUTGEMM_ECAPTURE) return rc;
         t.partial = (float *)sums;

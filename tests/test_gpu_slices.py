@@ -1,6 +1,7 @@
 """The K-slices of the GEMM kernel depend on the sizes alone: a call gives the same bits eagerly, under capture on a
 stream that holds no memory for the slices' sums, and through the entry point that allocates nothing."""
 import ctypes
+import threading
 
 import pytest
 import torch
@@ -126,3 +127,40 @@ def test_calls_of_rising_size_keep_a_bounded_amount_of_memory(gpu_device):
         lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
     power = 1 << (largest - 1).bit_length()
     assert largest <= taken <= 2 * power + (2 << 20), (largest, taken)
+
+
+def test_two_host_threads_on_one_stream(gpu_device):
+    """A call whose slices are added up by a second launch keeps the two together: calls of another host thread on
+    the same stream share the buffer between them."""
+    dev, lib = gpu_device, native.cabi()
+    N, K, M = 1024, 4096, 64
+    stream = torch.cuda.Stream()
+    sp = ctypes.c_void_p(stream.cuda_stream)
+    alpha = torch.full((K // 128, 2, N), 2.0 ** -6, device=dev).half()
+    x = torch.ones((M, K), device=dev).half()
+    # all signs -1 in one thread, +1 in the other
+    weights = [torch.full((K // 32, 2, N), v, dtype=torch.int32, device=dev) for v in (0, -1)]
+    outs = [[torch.zeros((M, N), device=dev).half() for _ in range(60)] for _ in weights]
+    codes = [[], []]
+    torch.cuda.synchronize()
+    assert lib.lutgemm_reserve_workspace(sp, lib.lutgemm_workspace_words(N, M)) == 0
+    assert lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 33) == 0
+    try:
+        plan = native.Plan()
+        assert lib.lutgemm_describe_plan(ROW, N, K, 2, K // 128, M, ctypes.byref(plan)) == 0 and plan.kernel == 3 and plan.k_slices > 1
+
+        def work(i):
+            for out in outs[i]:        # (ctypes lets the other thread run during the call)
+                codes[i].append(lib.lutgemm_gemv_rowwise_f16(weights[i].data_ptr(), alpha.data_ptr(), x.data_ptr(), out.data_ptr(), N, K, 2,
+                                                             K // 128, M, sp))
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+    assert codes == [[0] * 60] * 2
+    want = 2 * K * 2.0 ** -6
+    assert all(bool((o == -want).all()) for o in outs[0]) and all(bool((o == want).all()) for o in outs[1])
