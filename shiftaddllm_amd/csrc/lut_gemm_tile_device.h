@@ -456,13 +456,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                     *(f32x4 *)(sums + (size_t)m * p.N + n) = (f32x4){v[0], v[1], v[2], v[3]};
                     continue;
                 }
-                if (!p.overwrite) {
-                    const u32x2 old = *(const u32x2 *)(p.init + (size_t)m * p.init_stride + n);
-                    v[0] += half_bits_to_float(old.x & 0xffffu);
-                    v[1] += half_bits_to_float(old.x >> 16);
-                    v[2] += half_bits_to_float(old.y & 0xffffu);
-                    v[3] += half_bits_to_float(old.y >> 16);
-                }
+                if (!p.overwrite) add_halves(v, p.init + (size_t)m * p.init_stride + n);
                 store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
             }
     }
@@ -501,13 +495,7 @@ static __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem 
     for (; sl < p.ksplit; ++sl) sum += *(const f32x4 *)(src + (size_t)sl * stride);
     float v[4] = {sum[0], sum[1], sum[2], sum[3]};
     const uint32_t m = at / quads, n = 4u * (at - m * quads);
-    if (!p.overwrite) {
-        const u32x2 old = *(const u32x2 *)(p.init + (size_t)m * p.init_stride + n);
-        v[0] += half_bits_to_float(old.x & 0xffffu);
-        v[1] += half_bits_to_float(old.x >> 16);
-        v[2] += half_bits_to_float(old.y & 0xffffu);
-        v[3] += half_bits_to_float(old.y >> 16);
-    }
+    if (!p.overwrite) add_halves(v, p.init + (size_t)m * p.init_stride + n);
     store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
 }
 

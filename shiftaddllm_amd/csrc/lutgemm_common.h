@@ -300,7 +300,19 @@ __device__ __forceinline__ void store_result(void *out, size_t i, float v, int t
         ((unsigned short *)out)[i] = (unsigned short)(type == kIoBF16 ? bf16_bits(v) : float_to_half_bits(v));
 }
 
-// four consecutive ones
+// Four consecutive fp16 values of any alignment (a bias row may begin on any of them) added to v.  The vector type
+// says so: the compiler then takes one 8-byte load, which this hardware allows at any address, because it may.
+typedef u32x2 u32x2_of_halves __attribute__((aligned(2)));
+__device__ __forceinline__ void add_halves(float (&v)[4], const __half *from)
+{
+    const u32x2 old = *(const u32x2_of_halves *)from;
+    v[0] += half_bits_to_float(old.x & 0xffffu);
+    v[1] += half_bits_to_float(old.x >> 16);
+    v[2] += half_bits_to_float(old.y & 0xffffu);
+    v[3] += half_bits_to_float(old.y >> 16);
+}
+
+// four consecutive results
 __device__ __forceinline__ void store_results(void *out, size_t i, const float (&v)[4], int type)
 {
     if (type == kIoF32)

@@ -93,3 +93,30 @@ def test_many_rows_against_a_dense_product(gpu_device, fmt, K, N, nb, M, groups,
     ok = want.abs() < 60000
     err = (out.double() - want)[ok]
     assert (err.norm() / want[ok].norm()).item() <= 3e-4 and (err.abs().max() / want[ok].abs().max()).item() <= 1e-3
+
+
+@pytest.mark.parametrize("K,N,M,out_type", [(512, 260, 130, 0), (8192, 512, 64, 0), (8192, 516, 40, 1), (256, 260, 64, 2)])
+def test_bias_that_begins_on_any_value(gpu_device, K, N, M, out_type):
+    """A bias is aligned to its values only, in the kernel itself and where the slices' sums are added up."""
+    dev, lib = gpu_device, native.cabi()
+    g = torch.Generator(device=dev).manual_seed(K + N)
+    bW = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 32, 2, N), generator=g, device=dev, dtype=torch.int32)
+    alpha = _scales(g, dev, K // 128, 2, N, "any").half()
+    x = torch.randn((M, K), generator=g, device=dev).half()
+    room = torch.randn(N + 4, generator=g, device=dev).half()
+    got = []
+    assert lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 33) == 0
+    try:
+        for first in range(4):
+            bias = room[first:first + N]
+            out = torch.empty((M, N), dtype=(torch.float16, torch.bfloat16, torch.float32)[out_type], device=dev)
+            call = native.Linear(bW.data_ptr(), alpha.data_ptr(), None, x.data_ptr(), bias.data_ptr(), out.data_ptr(), ROW, N, K, 2,
+                                 K // 128, M, 0, 0, out_type)
+            rc = lib.lutgemm_linear_f16(ctypes.byref(call), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+            assert rc == 0, lib.lutgemm_strerror(rc).decode()
+            got.append(out.double() - bias.double())
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+    want = x.double() @ _dense(ROW, bW, alpha, None)
+    for y in got:       # (the rounding of the result: 2^-11, bf16 2^-8, of the sum with the bias)
+        assert ((y - want).norm() / want.norm()).item() <= (6e-4, 5e-3, 1e-6)[out_type]
