@@ -169,14 +169,18 @@ class LutLinear(nn.Module):
         # (at one row the host bounds the layer: what can be checked natively is)
         K = self.K
         buffers = self._buffers
+        signs, alpha = buffers.get("binaryWeight"), buffers.get("alpha")
+        if signs is None:              # (replaced by a parameter or a plain attribute)
+            signs = self.binaryWeight
+        if alpha is None:
+            alpha = self.alpha
         fmt = _FORMAT_CODES[self.alpha_format]
         pow2 = fmt == 0 and 3 * K <= x.numel() <= 8 * K and self._alphas_are_powers_of_two()
         bias = self.bias
         if bias is not None:
             bias = self._bias_vector(x.device)
         out = self._output(x.numel() // K, x.device) if self.reuse_output else None
-        return native.lutgemm.linear_forward(x, buffers["binaryWeight"], buffers["alpha"], bias, out, fmt, self.N, K,
-                                             self.wbit, self.num_groups, pow2)
+        return native.lutgemm.linear_forward(x, signs, alpha, bias, out, fmt, self.N, K, self.wbit, self.num_groups, pow2)
 
     def extra_repr(self):
         return "in_features={}, out_features={}, bias={}, wbit={}, group_size={}, alpha_format={}".format(

@@ -217,3 +217,20 @@ def test_forward_without_native_library_fails_loudly(monkeypatch):
     lin = Q_.LutLinear(64, 8, group_size=8, wbit=2)
     with pytest.raises(ImportError):
         lin(torch.zeros(1, 64, dtype=torch.float16))
+
+
+@pytest.mark.parametrize("replace", ["buffer", "parameter", "attribute"])
+def test_forward_takes_the_tensors_the_module_holds(monkeypatch, replace):
+    """binaryWeight and alpha may be buffers, parameters or plain attributes: forward passes on what the module holds."""
+    from shiftaddllm_amd import native
+    lin = Q_.LutLinear(64, 8, group_size=8, wbit=2)
+    signs, alpha = torch.ones_like(lin.binaryWeight), torch.ones_like(lin.alpha)
+    for name, t in (("binaryWeight", signs), ("alpha", alpha)):
+        if replace != "buffer":
+            delattr(lin, name)
+        setattr(lin, name, torch.nn.Parameter(t, requires_grad=False) if replace == "parameter" else t)
+    seen = []
+    monkeypatch.setattr(native.lutgemm, "linear_forward", lambda *a: seen.append(a))
+    lin(torch.zeros((1, 64), dtype=torch.float16))
+    assert len(seen) == 1 and seen[0][1] is lin.binaryWeight and seen[0][2] is lin.alpha
+    assert seen[0][1].data_ptr() == signs.data_ptr() and seen[0][2].data_ptr() == alpha.data_ptr()
