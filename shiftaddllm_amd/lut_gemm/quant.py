@@ -62,6 +62,11 @@ def decode_apot_int8(code: torch.Tensor) -> torch.Tensor:
     return torch.where(e == APOT_ABSENT, torch.zeros_like(val), val).sum(dim=-1)
 
 
+def _same_memory(held, t):
+    """Whether `t` is the memory that `held` keeps alive (an address alone may have been handed out again)."""
+    return held.data_ptr() == t.data_ptr() and held.device == t.device
+
+
 class LutLinear(nn.Module):
     """Drop-in for lut_gemm/quant.py:8-61.
 
@@ -134,10 +139,11 @@ class LutLinear(nn.Module):
         b = self.bias
         if b is None or (b.dtype is torch.float16 and b.device == device and b.is_contiguous()):
             return b
-        key = (device, b.data_ptr(), b._version)
-        if self._bias_cache is None or self._bias_cache[0] != key:
-            self._bias_cache = (key, b.detach().to(device=device, dtype=torch.float16).reshape(self.N).contiguous())
-        return self._bias_cache[1]
+        c = self._bias_cache
+        if c is None or c[0] != (device, b._version) or not _same_memory(c[1], b):
+            c = ((device, b._version), b.detach(), b.detach().to(device=device, dtype=torch.float16).reshape(self.N).contiguous())
+            self._bias_cache = c
+        return c[2]
 
     def _alphas_are_powers_of_two(self):
         """Whether every row-wise alpha is a positive normal fp16 power of two (what the reference's
@@ -145,13 +151,13 @@ class LutLinear(nn.Module):
         alpha tensor (one device synchronisation), and only by calls of three or more rows, which
         can then take the block-scaled matrix-core kernel."""
         a = self.alpha
-        key = (a.data_ptr(), a._version, a.device)
-        if self._pow2_cache is None or self._pow2_cache[0] != key:
+        c = self._pow2_cache
+        if c is None or c[0] != a._version or not _same_memory(c[1], a):
             bits = a.view(torch.int16).to(torch.int32) & 0xffff
             field = (bits >> 10) & 0x1f
             ok = ((bits & 0x83ff) == 0) & (field >= 1) & (field <= 30)
-            self._pow2_cache = (key, bool(ok.all().item()))
-        return self._pow2_cache[1]
+            c = self._pow2_cache = (a._version, a.detach(), bool(ok.all().item()))
+        return c[2]
 
     def _output(self, rows, device):
         """With `reuse_output`, the one buffer per (rows, device) that every call overwrites (no allocation

@@ -234,3 +234,29 @@ def test_forward_takes_the_tensors_the_module_holds(monkeypatch, replace):
     lin(torch.zeros((1, 64), dtype=torch.float16))
     assert len(seen) == 1 and seen[0][1] is lin.binaryWeight and seen[0][2] is lin.alpha
     assert seen[0][1].data_ptr() == signs.data_ptr() and seen[0][2].data_ptr() == alpha.data_ptr()
+
+
+def test_what_forward_keeps_of_alpha_and_bias_is_not_found_again_by_address():
+    """Tensors swapped in and out: memory of the first one that is handed out again is not taken for it."""
+    lin = Q_.LutLinear(1024, 64, group_size=128, wbit=3, alpha_format="rowwise_fp16")
+    shape = tuple(lin.alpha.shape)
+    for _ in range(30):
+        lin.alpha.data = torch.full(shape, 0.25, dtype=torch.float16)
+        assert lin._alphas_are_powers_of_two()
+        lin.alpha.data = torch.full(shape, 0.5, dtype=torch.float16)      # the first one's memory is free
+        other = [torch.full(shape, 0.375, dtype=torch.float16) for _ in range(4)]
+        for a in other:
+            lin.alpha.data = a
+            assert not lin._alphas_are_powers_of_two()
+            lin.alpha.data = torch.full(shape, 0.5, dtype=torch.float16)
+    cpu = torch.device("cpu")
+    lin.bias = torch.nn.Parameter(torch.zeros(64))
+    for i in range(30):
+        lin.bias.data = torch.full((64,), float(i))
+        assert bool((lin._bias_vector(cpu) == i).all())
+        lin.bias.data = torch.zeros(64)
+        other = [torch.full((64,), float(i + 100)) for _ in range(4)]
+        for b in other:
+            lin.bias.data = b
+            assert bool((lin._bias_vector(cpu) == i + 100).all())
+            lin.bias.data = torch.zeros(64)
