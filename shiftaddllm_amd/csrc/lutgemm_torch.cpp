@@ -452,12 +452,19 @@ struct Positional<Fn> {
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m)
 {
     m.doc() = "MI355X (gfx950) LUT-GEMM engine behind the ShiftAddLLM `lutgemm` call signatures";
-    Positional<&lutgemm_compute>::define(m, "lutgemm_compute", "uniform-quant LUT-GEMV (alpha, q_bias)");
-    Positional<&lutgemm_compute_shift_scale>::define(m, "lutgemm_compute_shift_scale", "row-wise alpha LUT-GEMV");
-    Positional<&lutgemm_compute_shift_scale_pow2>::define(m, "lutgemm_compute_shift_scale_pow2", "row-wise alpha LUT-GEMV, alphas promised to be powers of two");
-    Positional<&lutgemm_compute_block>::define(m, "lutgemm_compute_block", "block alpha LUT-GEMV (fp16 alpha)");
-    Positional<&lutgemm_compute_block_shift>::define(m, "lutgemm_compute_block_shift", "block alpha LUT-GEMV (uint16 shift fields)");
-    Positional<&lutgemm_compute_block_shiftInt8>::define(m, "lutgemm_compute_block_shiftInt8", "block alpha LUT-GEMV (int8 exponents)");
+    // (name, arguments and "--" in front of a description are where help() and inspect find the signature)
+    Positional<&lutgemm_compute>::define(m, "lutgemm_compute",
+        "lutgemm_compute(output, bWeight, alpha, q_bias, d_input, mSize, kSize, nb, num_groups, /)\n--\n\nUniform-quant LUT-GEMV (alpha, q_bias).");
+    Positional<&lutgemm_compute_shift_scale>::define(m, "lutgemm_compute_shift_scale",
+        "lutgemm_compute_shift_scale(output, bWeight, alpha, d_input, mSize, kSize, nb, num_groups, /)\n--\n\nRow-wise alpha LUT-GEMV.");
+    Positional<&lutgemm_compute_shift_scale_pow2>::define(m, "lutgemm_compute_shift_scale_pow2",
+        "lutgemm_compute_shift_scale_pow2(output, bWeight, alpha, d_input, mSize, kSize, nb, num_groups, /)\n--\n\nRow-wise alpha LUT-GEMV, alphas promised to be powers of two.");
+    Positional<&lutgemm_compute_block>::define(m, "lutgemm_compute_block",
+        "lutgemm_compute_block(output, bWeight, alpha, d_input, mSize, kSize, nb, num_groups, /)\n--\n\nBlock alpha LUT-GEMV (fp16 alpha).");
+    Positional<&lutgemm_compute_block_shift>::define(m, "lutgemm_compute_block_shift",
+        "lutgemm_compute_block_shift(output, bWeight, alpha, d_input, mSize, kSize, nb, num_groups, num_apot, /)\n--\n\nBlock alpha LUT-GEMV (uint16 shift fields).");
+    Positional<&lutgemm_compute_block_shiftInt8>::define(m, "lutgemm_compute_block_shiftInt8",
+        "lutgemm_compute_block_shiftInt8(output, bWeight, alpha, d_input, mSize, kSize, nb, num_groups, num_apot, /)\n--\n\nBlock alpha LUT-GEMV (int8 exponents).");
     m.def("makeRandomInput", &makeRandomInput, "fill inp[:M, :K] with the reference's random activations");
     m.def("makeRandomAlpha", &makeRandomAlpha, "fill alpha [num_groups, NUM_BITS, N] and q_bias [num_groups, N]");
     m.def("makeRandomBias", &makeRandomBias, "fill bias[:N]");

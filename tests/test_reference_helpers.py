@@ -120,3 +120,23 @@ def test_bcq_quantiser_on_the_device_matches_the_reference_fixture(gpu_device):
         b_ok = np.array_equal(B.cpu().numpy(), d[f"B{c}"])
         assert a_ok and b_ok, (f"case {c}: alpha equal={a_ok}, B equal={b_ok}, "
                               f"B mismatches={int((B.cpu().numpy() != d[f'B{c}']).sum())} of {B.numel()}")
+
+
+@pytest.mark.parametrize("name,extra", [("lutgemm_compute", ()), ("lutgemm_compute_shift_scale", ()), ("lutgemm_compute_shift_scale_pow2", ()),
+                                        ("lutgemm_compute_block", ()), ("lutgemm_compute_block_shift", ("num_apot",)),
+                                        ("lutgemm_compute_block_shiftInt8", ("num_apot",))])
+def test_compute_functions_state_their_arguments(ext, name, extra):
+    import inspect
+    fn = getattr(ext, name)
+    scales = ("alpha", "q_bias") if name == "lutgemm_compute" else ("alpha",)
+    want = ("output", "bWeight", *scales, "d_input", "mSize", "kSize", "nb", "num_groups", *extra)
+    assert tuple(inspect.signature(fn).parameters) == want
+    assert fn.__name__ == name and fn.__doc__ and "LUT-GEMV" in fn.__doc__
+    # whole numbers of other types are taken, anything else and any other count of arguments refused
+    with pytest.raises(TypeError):
+        fn()
+    t = torch.zeros(4)
+    with pytest.raises(TypeError):
+        fn(*[t] * (2 + len(scales) + 1), *[1.5] * (4 + len(extra)))
+    with pytest.raises(RuntimeError, match="GPU tensor"):
+        fn(*[t] * (2 + len(scales) + 1), *[np.int64(32)] * (4 + len(extra)))
