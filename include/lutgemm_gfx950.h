@@ -26,7 +26,14 @@
  *           (mv_fp16_bias.hpp:342-380): one more fp16 rounding per eight
  *           inputs, output error about 3e-4 relative instead of 2e-4.)
  *           A NaN input gives NaN and an infinite input gives an infinity
- *           or NaN in every output it reaches, whatever the launch plan.
+ *           or NaN in every output it reaches, whatever the launch plan
+ *           (calls of several rows multiply by whole weights: NaN where the
+ *           weight is zero or takes two fp16 pieces).  A NaN or infinite
+ *           scale does the same to every output it belongs to.
+ *           Calls of several rows hold a weight, the sum of its planes'
+ *           scales, to 2^-23 of itself or 2^-31 of the largest weight of the
+ *           same output within 64 or 128 inputs, whichever is larger; sums
+ *           of powers of two that span eleven bits are exact.
  *           Finite inputs have a guaranteed range: while every partial sum
  *           over a run of K stays within +-65536, and (calls with two or
  *           more rows on the look-up kernel, whose tables are fp16) every
@@ -36,6 +43,8 @@
  *           as infinite where K is split over workgroups and is carried as
  *           fp32 where it is not, so the same finite problem may give an
  *           infinity for one M or grouping and a finite value for another.
+ *           Where K is split over workgroups, other than by the GEMM kernel
+ *           of many rows, partial sums are rounded to multiples of 2^-31.
  * Shape rules enforced here (the reference checks nothing and reads or writes
  * out of bounds instead): K % 32 == 0, N % 4 == 0, 1 <= nb <= 4,
  * 1 <= M <= 65535, 16-byte aligned bW and x, 8-byte aligned row-wise alpha and out.
@@ -220,8 +229,10 @@ int lutgemm_gemv_block_apot_i8(const uint32_t *bW, const int8_t *alpha_i8, const
  *   format     : LUTGEMM_FORMAT_*, see lutgemm_describe_plan below;
  *   qbias_f16  : uniform format only, NULL otherwise;
  *   alpha_pow2 : 1 = the promise of lutgemm_gemv_rowwise_pow2_f16 (row-wise format only), else 0;
- *   x_type, out_type : LUTGEMM_TYPE_* of x and out.  x is rounded to fp16 first, the sum is rounded once, to
- *                out_type (out 16-byte aligned for LUTGEMM_TYPE_F32).  Types other than fp16 are taken where
+ *   x_type, out_type : LUTGEMM_TYPE_* of x and out.  x is rounded to fp16 first, the sum is rounded to out_type
+ *                (out 16-byte aligned for LUTGEMM_TYPE_F32).  The sum is the same whatever out_type is, with the
+ *                guaranteed range stated above: bf16 and fp32 results hold sums beyond +-65536, and digits below
+ *                2^-31, only where the launch plan does not split K.  Types other than fp16 are taken where
  *                a conversion of its own would be a large part of the call: one or two rows, up to some
  *                tens of rows for bf16 x; LUTGEMM_EUNSUP, and no launch, for the others.
  * Errors, capture and workspace rules as everywhere.
