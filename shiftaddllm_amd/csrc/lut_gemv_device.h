@@ -1368,7 +1368,8 @@ lut_gemv_kernel(const Problem p)
 // Every width takes its first item on its own, like a lone problem.  The widths' bodies are kept apart (what
 // the compiler hoists out of them ahead of the switch lives through all of them, and four planes spilled 16 to
 // 19 registers per lane for it, or, without the peeled first item, waited for two items before the first
-// table): XXX.
+// table): q,k,v of 2, 3 and 4 bits 10.9 -> 10.1 us, of 4 bits 10.9 -> 9.8, gate,up of 2 and 4 bits 12.9 -> 12.1
+// (one row, 4096 wide, 7B sizes).
 template <int XF, bool EXTRA>
 __global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4)))
 lut_gemv_group_kernel(const Group g)
