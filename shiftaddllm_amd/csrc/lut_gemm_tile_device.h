@@ -93,14 +93,16 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 
     // ---- signs and scales --------------------------------------------------------------------------
     uint32_t words[2][NB];
-    auto load_words = [&](int t, uint32_t (&w)[2][NB]) {
+    auto load_fragment = [&](int t, int f, uint32_t (&w)[NB]) {
         const int wd = min(2 * t + kh, p.kwords - 1);
         const uint32_t row = (uint32_t)wd * NB * (uint32_t)p.N;
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int b = 0; b < NB; ++b)
+            w[b] = *(const uint32_t *)((const char *)p.W + (row + (uint32_t)b * (uint32_t)p.N + (uint32_t)nn[f]) * 4u);
+    };
+    auto load_words = [&](int t, uint32_t (&w)[2][NB]) {
 #pragma unroll
-            for (int b = 0; b < NB; ++b)
-                w[f][b] = *(const uint32_t *)((const char *)p.W + (row + (uint32_t)b * (uint32_t)p.N + (uint32_t)nn[f]) * 4u);
+        for (int f = 0; f < 2; ++f) load_fragment(t, f, w[f]);
     };
     // The scales of a step go through LDS as well (four steps' worth: while step t runs, those of steps t
     // and t + 1 are read and those of step t + 2 written), fetched at the start of a step and written at
@@ -298,13 +300,16 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                 unit[f] = fresh;
             }
             scale_sums(by, std::true_type());
-            (void)make_tables(t, false);
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
                 uint32_t y[4];
                 sign_indices<NB, UNI>(words_lo[f], y);
 #pragma unroll
-                for (int c = 0; c < 4; ++c) A[set][c][f] = pick(f, c, y);
+                for (int c = 0; c < 4; ++c) {
+                    if (c < kTabs) (void)make_table(t, false, f % kFragTabs, c);
+                    A[set][c][f] = pick(f, c, y);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
         }
     };
@@ -317,14 +322,17 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         fetch_scales(t + 2);
         load_x(t + 2);
         if (lo_cur) {
-            (void)make_tables(t, true);
             uint32_t y[2][4];
 #pragma unroll
             for (int f = 0; f < 2; ++f) sign_indices<NB, UNI>(words_lo[f], y[f]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                if (j < kTabs)
+#pragma unroll
+                    for (int f = 0; f < kFragTabs; ++f) (void)make_table(t, true, f, j);
                 const u32x4 a[2] = {pick(0, j, y[0]), pick(1, j, y[1])};
                 multiply(P, j, a);
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -334,21 +342,35 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         // matrix work and waits for every fragment right behind its request.)
         bool inexact = false;
         uint32_t y[2][4];
-        // (block formats: a chunk's tables, then its weights, so that few tables are live at a time)
-        constexpr int kPer = kFragTabs + 2, kItems = BLOCK ? 3 + 4 * kPer : 3 + 2 + 8, kSlots = 4 * MF;
+        // (One fragment after the other, and block formats a chunk's table, then its weights, so that few tables and
+        // indices are live at a time; where both fragments share their tables, chunk after chunk.)
+        constexpr bool WIDE = FMT == kTileBlockWide;
+        constexpr int kFragment = BLOCK ? 10 : 7, kItems = WIDE ? 3 + 4 * 3 : 2 * kFragment, kSlots = 4 * MF;
         auto item = [&](auto k_c) {
-            constexpr int k = decltype(k_c)::value, r = k - 3;
-            constexpr bool table = BLOCK ? r % kPer < kFragTabs : r < 2;
-            constexpr int c = BLOCK ? r / kPer : table ? 0 : (r - 2) >> 1;
-            constexpr int f = BLOCK ? (table ? r % kPer : r % kPer - kFragTabs) : r & 1;
-            if constexpr (k < 2)
-                sign_indices<NB, UNI>(words[k], y[k]);
-            else if constexpr (k == 2)
-                load_words(t + 2, words);
-            else if constexpr (table)
-                inexact = make_table(t + 1, false, f, c) || inexact;
-            else
-                A[P ^ 1][c][f] = pick(f, c, y[f]);
+            constexpr int k = decltype(k_c)::value;
+            if constexpr (WIDE) {
+                constexpr int r = k - 3, c = r / 3, f = r % 3 - 1;
+                if constexpr (k < 2)
+                    sign_indices<NB, UNI>(words[k], y[k]);
+                else if constexpr (k == 2)
+                    load_words(t + 2, words);
+                else if constexpr (f < 0)
+                    inexact = make_table(t + 1, false, 0, c) || inexact;
+                else
+                    A[P ^ 1][c][f] = pick(f, c, y[f]);
+            } else {
+                constexpr int f = k / kFragment, r = k % kFragment - 2;
+                constexpr bool table = BLOCK ? r % 2 == 0 : r == 0;
+                constexpr int c = BLOCK ? r / 2 : table ? 0 : r - 1;
+                if constexpr (r == -2)
+                    sign_indices<NB, UNI>(words[f], y[f]);
+                else if constexpr (r == -1)
+                    load_fragment(t + 2, f, words[f]);
+                else if constexpr (table)
+                    inexact = make_table(t + 1, false, f, c) || inexact;
+                else
+                    A[P ^ 1][c][f] = pick(f, c, y[f]);
+            }
         };
         f16x8 b = activations(P, 0, 0);
         static_for<kSlots>([&](auto s_c) {
