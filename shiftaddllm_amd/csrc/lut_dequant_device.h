@@ -19,10 +19,8 @@
 // follows that output's weights along K: it is chosen anew wherever an inexact step has left the window
 // [64, 32768] (outputs of one wave may be any number of binades apart, and so may the groups of an output).
 // Two pieces then hold a weight to 2^-23 of itself or 2^-31 of the largest weight of the same output in
-// the same K-step (64 or 128 inputs), whichever is larger.  One unit for all 64 outputs of a wave, as these kernels had at
-// first, lost a bit per binade beyond the tenth and every bit beyond the thirty-third.  Units of their own
-// cost 0 to 2 % (11008x4096x3, 2048 rows 199.0 -> 202.7 us; 5120x13824x2, 512 rows 105.0 -> 106.1), on short
-// calls whose lanes form four tables each 0.3 us (2964x2208x3 in groups of 96, 7 rows 7.5 -> 7.85).
+// the same K-step (64 or 128 inputs), whichever is larger.  (One unit for all 64 outputs of a wave, as these
+// kernels had at first, lost a bit per binade beyond the tenth and every bit beyond the thirty-third.)
 #ifndef LUT_DEQUANT_DEVICE_H
 #define LUT_DEQUANT_DEVICE_H
 

@@ -198,12 +198,18 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // ---- one K-step ---------------------------------------------------------------------------------
     constexpr int kTables = OWN ? 4 : 1;   // tables this lane forms
     // Weights are formed as W * unit, a power of two per output (block formats: per row group), held by the lane
-    // whose table it scales (OWN: by the four lanes whose tables they are).
-    float unit[kTables];
+    // whose table it scales.  OWN: by the four lanes whose tables they are, the biased exponents of a lane's four as the
+    // bytes of one register (8192x8192x4 in groups of 32, 8 rows 38 us with four registers, 29 with one; 34 when one
+    // unit served the whole wave); all begin with the unit that suits the wave's largest output, which is what
+    // ordinary layers stay with: their sums are scaled back by one number.  A single step (ONE) has the units it
+    // chose and needs no check.
+    typename std::conditional<OWN, uint32_t, float>::type units = OWN ? 0 : 1;
     bool chosen = false;
     bool same = OWN;                       // all units of the wave are one
-#pragma unroll
-    for (int i = 0; i < kTables; ++i) unit[i] = 1.0f;
+    auto unit = [&](int i) {
+        if constexpr (OWN) return __builtin_bit_cast(float, ((units >> (8 * i)) & 0xffu) << 23);
+        else return units;
+    };
     // multipliers of this lane's table i
     auto multipliers = [&](const Operands &ops, int i, float (&a)[NB], float &q) {
         q = 0.0f;
@@ -260,14 +266,23 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     };
     auto refit = [&](const Operands &ops) {   // units that suit this step
         float by[kTables];
+        decltype(units) now = 0;
 #pragma unroll
         for (int i = 0; i < kTables; ++i) {
-            const float most = largest(ops, i), fresh = outside_window(most, unit[i]) ? unit_for(most) : unit[i];
-            by[i] = fresh * inverse_unit(unit[i]);
-            unit[i] = fresh;
+            const float most = largest(ops, i), old = unit(i), fresh = outside_window(most, old) ? unit_for(most) : old;
+            by[i] = fresh * inverse_unit(old);
+            if constexpr (OWN) now |= (__builtin_bit_cast(uint32_t, fresh) >> 23) << (8 * i);
+            else now = fresh;
         }
+        units = now;
         same = false;
-        scale_sums(by, std::true_type());
+        if constexpr (!ONE) scale_sums(by, std::true_type());
+    };
+    auto any_outside = [&](const Operands &ops) {
+        bool outside = false;
+#pragma unroll
+        for (int i = 0; i < kTables; ++i) outside = outside_window(magnitude(ops, i), unit(i)) || outside;
+        return __builtin_amdgcn_ballot_w64(outside) != 0ull;
     };
     // The lane's tables of a step, or of what rounding their entries leaves over; true when some entry may
     // not be an fp16 number.
@@ -275,7 +290,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         bool inexact = false;
 #pragma unroll
         for (int i = 0; i < kTables; ++i) {
-            float u = unit[i];
+            float u = unit(i);
             if constexpr (FMT == kWeightBlock) u = 16 * step + li < p.K / 8 ? u : 0.0f;
             if constexpr (OWN) u = 4 * step + kb < p.kwords ? u : 0.0f;
             float a[NB], q;
@@ -346,11 +361,10 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
                 float most = 0.0f;
 #pragma unroll
                 for (int i = 0; i < kTables; ++i) most = fmaxf(most, magnitude(ops, i));
-                most = wave_max(most);
-#pragma unroll
-                for (int i = 0; i < kTables; ++i) unit[i] = unit_for(most);
+                units = (__builtin_bit_cast(uint32_t, unit_for(wave_max(most))) >> 23) * 0x01010101u;
+                if (ONE && any_outside(ops)) refit(ops);
             } else {
-                unit[0] = unit_for(largest(ops, 0));
+                units = unit_for(largest(ops, 0));
             }
         }
         Table tab[kTables];
@@ -360,12 +374,9 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
                 for (int r = 0; r < Operands::kScales; ++r) asm volatile("" : "+v"(ops.s[r]));
         };
-        if (inexact) {
+        if (!ONE && inexact) {   // (a single step has the units it chose)
             forget();
-            bool outside = false;
-#pragma unroll
-            for (int i = 0; i < kTables; ++i) outside = outside_window(magnitude(ops, i), unit[i]) || outside;
-            if (__builtin_amdgcn_ballot_w64(outside) != 0ull) {
+            if (any_outside(ops)) {
                 forget();
                 refit(ops);
                 forget();
@@ -423,7 +434,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     if constexpr (EXTRA && !ONE)
         if (n_steps == 0 && scaled) row_scales();  // (a wave without steps still owes its rows)
     if (same) {
-        const float back = inverse_unit(unit[0]);
+        const float back = chosen ? inverse_unit(unit(0)) : 1.0f;
 #pragma unroll
         for (int e = 0; e < 4; ++e)
 #pragma unroll
@@ -431,7 +442,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     } else {
         float back[kTables];
 #pragma unroll
-        for (int i = 0; i < kTables; ++i) back[i] = inverse_unit(unit[i]);
+        for (int i = 0; i < kTables; ++i) back[i] = inverse_unit(unit(i));
         scale_sums(back, std::false_type());
     }
 

@@ -343,7 +343,9 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         bool inexact = false;
         uint32_t y[2][4];
         // (One fragment after the other, and block formats a chunk's table, then its weights, so that few tables and
-        // indices are live at a time; where both fragments share their tables, chunk after chunk.)
+        // indices are live at a time; where both fragments share their tables, chunk after chunk.  The loop needs every
+        // register there is: with both fragments' at once it reloaded spilled values behind all loads in flight,
+        // 8192x8192x4 at 128 rows 51 us instead of 41.5, 11008x4096x4 at 2048 rows 294 instead of 242.)
         constexpr bool WIDE = FMT == kTileBlockWide;
         constexpr int kFragment = BLOCK ? 10 : 7, kItems = WIDE ? 3 + 4 * 3 : 2 * kFragment, kSlots = 4 * MF;
         auto item = [&](auto k_c) {

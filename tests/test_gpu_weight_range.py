@@ -16,6 +16,7 @@ MFMA, TILE = 1, 3
 CASES = [  # kernel, format, K, N, planes, groups or row groups
     (MFMA, ROW, 4096, 128, 1, 32), (MFMA, ROW, 4096, 128, 3, 8), (MFMA, ROW, 4096, 192, 4, 32), (MFMA, ROW, 4064, 100, 2, 127),
     (MFMA, ROW, 4064, 128, 4, 127), (MFMA, UNIFORM, 4096, 128, 3, 8), (MFMA, UNIFORM, 4064, 64, 4, 127),
+    (MFMA, ROW, 1024, 128, 3, 8), (MFMA, ROW, 992, 100, 4, 31), (MFMA, UNIFORM, 992, 64, 2, 31), (MFMA, BLOCK_F16, 1024, 256, 4, 8),  # one step a wave
     (MFMA, BLOCK_F16, 4096, 256, 2, 8), (MFMA, BLOCK_I8, 4064, 128, 4, 4), (MFMA, BLOCK_I8, 4096, 256, 3, 1),
     (TILE, ROW, 1024, 320, 1, 8), (TILE, ROW, 1024, 512, 3, 8), (TILE, ROW, 992, 260, 4, 31), (TILE, UNIFORM, 1024, 256, 4, 8),
     (TILE, UNIFORM, 992, 256, 2, 31), (TILE, BLOCK_F16, 1024, 512, 3, 32), (TILE, BLOCK_I8, 992, 512, 4, 4), (TILE, BLOCK_I8, 1024, 512, 2, 16),
@@ -40,7 +41,7 @@ def test_every_output_keeps_its_precision(gpu_device, kernel, fmt, K, N, nb, gro
     per_column = fmt in (ROW, UNIFORM)
     outer, inner = (groups, N) if per_column else (K // 8, groups)
     planes = 1 if fmt == UNIFORM else nb
-    edge = 2048 if kernel == MFMA else 512
+    edge = 2048 if K > 4000 else 512
     first = torch.arange(outer, device=dev) * (K // outer) < edge
     bW = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 32, nb, N), generator=g, device=dev, dtype=torch.int32)
     a = torch.exp2(_exponents(pattern, outer, inner, first, dev).float().view(outer, 1, inner) - torch.arange(planes, device=dev).view(1, planes, 1))
