@@ -354,7 +354,7 @@ int lutgemm_describe_pow2_plan(int N, int K, int nb, int groups, int M, lutgemm_
  *                   many items take twin items instead (one table build per 512 outputs
  *                   instead of per 256; default 4, 0 = never)
  *   BLOCK_SCALED  : lutgemm_gemv_rowwise_pow2_f16 takes the block-scaled matrix-core
- *                   kernel 1 = where it is the faster one (few rows, large matrices),
+ *                   kernel 1 = for few rows of large matrices (see that function),
  *                   2 = wherever it applies, 0 = never (the call then behaves like
  *                   lutgemm_gemv_rowwise_f16); default 1
  *   POW2_CONVERT  : no effect (it chose between two ways of expanding sign planes, which the

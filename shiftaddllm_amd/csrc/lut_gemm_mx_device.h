@@ -7,8 +7,8 @@
 // power-of-two scale (an exponent byte) per row and per block of 32 inputs, applied inside the
 // matrix core.  So here
 //   * a sign bit becomes a 4-bit float +-1 (e2m1 codes 0x2 / 0xA): eight signs = one byte of the
-//     sign word = one 32-bit table entry, one LDS read per eight signs instead of a vector
-//     instruction per sign (which is what bounds the fp16 matrix-core kernel);
+//     sign word = one 32-bit table entry, one LDS read per eight signs where the fp16 matrix-core kernel
+//     forms every weight with two to three vector instructions;
 //   * the alpha of (output, bit plane, group) rides as the A-side block scale: its fp16 exponent
 //     field plus 112 is the exponent byte, no multiplication anywhere;
 //   * the activations are split ahead of the launch into three 8-bit floats (e4m3) per value with
@@ -22,8 +22,8 @@
 // instructions hold them (pieces 0 and 1, then piece 2 beside eight columns of zeros), with up to 16
 // rows three.  Matrix instructions take about the same time whatever their format and depth when
 // every CU issues them (measured: 16 ns for v_mfma_f32_16x16x32_f16, 17 to 20 ns for this one), so
-// what counts is their number: per (bit plane, 16 outputs, 128 inputs) one, two or three here
-// against four of the fp16 instruction, which also needs 128 vector instructions of sign expansion.
+// what counts is their number: per (16 outputs, 128 inputs) and BIT PLANE one, two or three here against
+// four of the fp16 instruction for all planes, behind the vector instructions that form the weights.
 //
 // Operand layout of the instruction (measured on the device, not documented here elsewhere):
 //   A (4-bit): lane l holds row l % 16, inputs 32 * (l / 16) .. + 31, eight per register, low

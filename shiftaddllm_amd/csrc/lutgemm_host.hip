@@ -370,10 +370,10 @@ bool mfma_eligible(const Problem &p, int mode)
         return false;
     if ((unsigned long long)p.M * p.K * 2 >= (1ull << 32)) return false;   // (32-bit byte offsets)
     if (p.M >= mfma_min_rows()) return true;
-    // two rows: the look-up kernel (one table set for both rows, fp16 entry pairs) wins from
-    // about 12 MB of sign words on (measured, look-up vs matrix core: 4096x4096x3 7.3 us vs 6.4;
-    // 11008x4096x2 10.5 vs 9.6; 5120x5120x4 9.8 vs 10.5; 11008x4096x3 11.9 vs 12.8; 8192x8192x4
-    // 14.2 vs 16.6; 28672x8192x4 34.7 vs 52)
+    // two rows: the look-up kernel (one table set for both rows, fp16 entry pairs) wins on long sign streams.  The
+    // line was drawn at 12 MB for an earlier matrix-core kernel; measured with this one (us, look-up / matrix
+    // core, * = taken): 4096x4096x3 6.9 / 5.6*, 11008x4096x2 9.6 / 8.1*, 5120x5120x4 (12.5 MB) 8.7* / 8.1, 11008x4096x3
+    // 10.6* / 9.5, 8192x8192x4 13.5* / 12.6, 28672x8192x4 30.8* / 33.2: it now lies between 32 and 112 MB.
     return p.M == 2 && mfma_min_rows() == 3 && (long)p.N * (p.K / 8) * p.nb <= (12l << 20);
 }
 
@@ -393,8 +393,7 @@ void plan_mfma(Problem &p, int mt, long want)
     p.n_blocks = p.n_tiles * p.ksplit * p.mchunks;
 }
 
-// Workgroups wanted per launch of the 32-row tile: one per CU (its register count allows
-// no second one).  Measured, 8192x8192x4: 36.4 us at 256 and 40.0 at 512.
+// LUTGEMM_OPTION_MFMA_BLOCKS: workgroups a matrix-core launch aims for instead of the rules below.
 int mfma_blocks_override()
 {
     return option(LUTGEMM_OPTION_MFMA_BLOCKS);
@@ -402,19 +401,23 @@ int mfma_blocks_override()
 
 // K-slices per tile for the problems of one launch (all get the same number, each up to
 // its own limit).
-//   32-row tile: as many as reach one workgroup per CU.
-//   16-row tile: the kernel is bound by the vector ALU work of expanding sign bits, two
-//   workgroups share a CU, and the launch ends when the busiest CU does.  With w =
-//   ceil(workgroups / 256) workgroups on that CU and R rounds (one K-step per wave, about
-//   2.2 us at three bit planes) per workgroup, the slice count that minimises
+//   32-row tile: as many as reach one workgroup per CU (its register count allows no second one).  Measured at 32 rows (us, slices -> time):
+//   8192x28672x4: 1 -> 79.6, 2 -> 47.7, 4 -> 55.0; 8192x8192x4: 1 -> 27.4, 2 -> 20.6, 4 -> 24.2; 5120x13824x2: 1 -> 34.5,
+//   3 -> 19.7, 4 -> 24.0; 11008x4096x3: 1 -> 15.5, 2 -> 23.0; 28672x8192x4, whose 448 tiles leave a second round a
+//   quarter empty: 1 -> 55.6, 2 -> 72.3, 4 -> 75.9.
+//   16-row tile: the launch ends when the busiest CU does, two workgroups share a CU.  With w =
+//   ceil(workgroups / 256) workgroups on that CU and R rounds (one K-step per wave) per workgroup, the slice
+//   count that minimises
 //       w * R  +  0.18 * w  +  0.9 * max(0, w - 2)
 //   is taken, the smaller one on ties: a workgroup's start and hand-over cost a fifth of a
 //   round, and one that has to wait for a slot on its CU most of a round.  A lone workgroup
 //   of four or more rounds hides its loads badly when there are many of them (more than
-//   eight activation rows, or nine CUs in ten busy) and is charged 12 % more.  Fitted to
-//   launches at 4 and 16 rows (us, slices -> time): 8192x8192x4: 2 -> 17.9, 4 -> 16.7;
-//   11008x4096x3: 1 -> 13.0, 2 -> 13.4 (16 rows: 16.7, 14.9); 22016x4096x3: 1 -> 21.4, 2 -> 18.3;
-//   28672x8192x2: 1 -> 28.1, 4 -> 32.5; 5120x13824x3: 3 -> 16.2, 5 -> 18.4.
+//   eight activation rows, or nine CUs in ten busy) and is charged 12 % more.  The constants were fitted to a
+//   kernel that expanded every plane by itself; for this one they pick (us at 4 / 16 rows, slices -> time, * = taken):
+//   8192x8192x4: 2 -> 12.9 / 15.4, 4* -> 12.9 / 14.6; 4096x4096x3: 2 -> 7.2 / 8.4, 4* -> 5.8 / 7.1; 5120x13824x3: 3* -> 12.3 /
+//   15.3, 5 -> 14.0 / 18.9; 4096x11008x2: 3 -> 9.1 / 11.3, 4* -> 8.1 / 10.2; 28672x8192x2: 1* -> 22.8 / 27.0, 4 -> 25.4 / 30.0;
+//   28672x8192x4: 1* -> 34.2 / 38.9, 4 -> 36.7 / 40.0; 22016x4096x3: 1 -> 15.6 / 18.4, 2* -> 14.7 / 17.1.  The one miss among
+//   these is 11008x4096x3 at 16 rows: 1 -> 11.8, 2* -> 12.5, 4 -> 11.8 (4 rows: 1* -> 9.6).
 int mfma_slices(const Group &g, int mt)
 {
     constexpr long kCUs = 256;
@@ -454,8 +457,11 @@ int mfma_slices(const Group &g, int mt)
 
 // 16-row tiles per workgroup of a lone problem.  Two of them form each weight once for 32 rows; a call that fits
 // the chip as single rounds of 16-row tiles, two workgroups per CU, is bound by latencies and better spread
-// (us, one against two, 32 rows: 4096x4096x3 8.9 / 10.4, 768x3072x3 6.9 / 8.9, 3072x768x3 6.1 / 7.1;
-// 11008x4096x3, which does not fit, 17.3 / 15.2).
+// (us, one against two, 32 rows: 4096x4096x3 8.9 / 10.6, 768x3072x3 6.3 / 8.7, 3072x768x3 4.8 / 6.3; 64 rows:
+// 768x3072x3 7.7 / 9.8; 11008x4096x3 at 32 rows, which does not fit, 17.5 / 15.6).  Beyond 64 rows two are taken
+// whatever the size, which the same measurements do not bear out everywhere: 768x3072x3 at 96 rows 8.0 / 9.9, at 128
+// rows 10.9 / 10.3, 2048x2048x3 at 128 rows 7.0 / 10.6, 1024x1024x3 at 256 rows 4.8 / 6.3, 1024x8192x4 at 96 rows
+// 13.4 / 13.2.
 int mfma_row_tiles(const Problem &p)
 {
     if (p.M <= 16) return 1;
@@ -516,11 +522,11 @@ enum Kernel : int { kLookup = 0, kMatrixCore = 1 };
 bool mfma_any(const Problem &p, int mode)
 {
     // (two rows: the look-up kernel, whose time is that of the sign stream, wins on longer streams; us, look-up
-    // against this kernel: int8 exponents 4096x4096x3 7.5 / 6.5, 13824x5120x2 11.7 / 14.7; uniform 768x768x3
-    // 6.4 / 6.1, 4096x4096x4 7.3 / 9.5, where q_bias makes every weight two pieces)
+    // against this kernel: int8 exponents 4096x4096x3 7.3 / 6.9, 13824x5120x2 11.6 / 15.0; uniform 768x768x3
+    // 5.7 / 5.1, 2048x2048x3 6.4 / 6.2, 4096x4096x4 7.6 / 8.8, where q_bias makes every weight two pieces)
     // One row as well where a look-up tile of 256 outputs touches more than two row groups and every lane would
-    // fetch its own multipliers: int8 exponents 768x768x3 in 8 groups 10.3 / 5.1, 4096x4096x3 in 32 groups
-    // 14.8 / 6.8, 1600x28672x4 in 8 groups 35.7 / 18.8.
+    // fetch its own multipliers: int8 exponents 768x768x3 in 8 groups 10.0 / 5.2, 4096x4096x3 in 32 groups
+    // 14.8 / 6.9, 1600x28672x4 in 8 groups 35.7 / 17.0.
     const int least = mfma_min_rows();
     if (p.M < least) {
         const long two_rows = mode == kUniformF16 ? 2l << 20 : 8l << 20;
@@ -611,13 +617,15 @@ void plan_mx(Problem &p)
 }
 
 // Whether a problem that may take the block-scaled kernel should.  It needs one, two or three matrix
-// instructions per (bit plane, 16 outputs, 128 inputs) for up to 5, 8 or 16 rows where the fp16 kernel
-// needs four (and its sign expansion), but also a launch of its own that splits the activations
-// (3 to 4 us with the gap between the launches).  Measured (us, fp16 kernel vs block-scaled):
-//   28672x8192x4: 4 rows 50.8 / 33.5, 8 rows 50.1 / 40.2, 16 rows 48.4 / 58.3
-//   28672x8192x2: 4 rows 27.1 / 23.5, 8 rows 29.0 / 30.2
-//   8192x8192x4:  4 rows 17.0 / 16.4, 8 rows 17.8 / 18.6;  8192x8192x2: 4 rows 11.2 / 13.6
-// so: up to 5 rows from 48 MB of sign words on, up to 8 rows from 96 MB on.
+// instructions per (bit plane, 16 outputs, 128 inputs) for up to 5, 8 or 16 rows, and a launch of its own
+// that splits the activations (3 to 4 us with the gap between the launches); the fp16 kernel needs four per
+// weight tile whatever the planes, and forms the weights.  Up to 5 rows from 48 MB of sign words on, up to 8 rows from
+// 96 MB on: drawn for an fp16 kernel that expanded every plane (28672x8192x4: 4 rows 50.8 us).  Measured with the
+// present one (us, fp16 kernel / block-scaled, * = taken):
+//   28672x8192x4: 4 rows 33.7 / 33.8*, 8 rows 34.9 / 41.1*, 16 rows 38.9* / 58.8
+//   28672x8192x2: 4 rows 22.5 / 23.9*, 8 rows 23.3* / 29.0;  8192x28672x4: 4 rows 33.4 / 35.3*, 8 rows 34.2 / 42.1*
+//   8192x8192x4:  4 rows 12.8* / 16.0, 8 rows 13.0* / 18.6;  8192x8192x2: 4 rows 9.3* / 13.5
+// so the rule no longer pays: on a par up to five rows, 20 % behind at eight.
 bool mx_wanted(const Problem &p)
 {
     const int how = option(LUTGEMM_OPTION_BLOCK_SCALED);
@@ -650,9 +658,12 @@ int run_mx(Problem &p, const Accum &acc)
 // Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices: a workgroup each, two per CU.
 // The cut depends on the sizes alone, so that a call gives the same bits eagerly, under capture and through the
 // entry point that allocates nothing.  Returns the time the plan should take.
-// Costs in microseconds, measured at three planes: a step of a 128-row tile takes 1.2 alone on its CU and
-// 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 5; the sums of the slices
+// Costs in microseconds, taken at three planes for all of them: a step of a 128-row tile takes 1.2 alone on its CU
+// and 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 5; the sums of the slices
 // are written and read at about 4 TB/s, by a second launch that costs another 4.
+// Measured at one to four planes (128 rows alone, beside another; 64 rows alone): row-wise 0.88, 0.97, 1.07, 1.36 / 1.63,
+// 1.73, 1.88, 2.19 / 0.66, 0.73, 0.84, 1.04; int8 exponents 1.41, 1.25, 1.40, 1.75 / 1.85, 1.84, 2.06, 2.44 / 1.18, 1.10,
+// 1.25, 1.57.
 double plan_tile(TileProblem &t)
 {
     constexpr long kCUs = 256;
@@ -685,9 +696,12 @@ double plan_tile(TileProblem &t)
 // Whether a call takes the GEMM kernel rather than the matrix-core kernel, from what either should take (in
 // microseconds; the slowest term only).  The matrix-core kernel forms the weights of a 32-row chunk in rounds of
 // 64 outputs x 1024 inputs, about 3 us each with one workgroup per CU.
-// Measured (us, matrix-core kernel / this one): 4096x4096x3 at 128 rows 15.4 / 25.9, 512 rows 54 / 42; 11008x4096x3 at
-// 48 rows 26 / 22, 256 rows 83 / 47; 8192x8192x4 at 64 rows 28 / 28.5, 128 rows 54 / 42; 1024x28672x4 at 256 rows
-// 45 / 56, 512 rows 77 / 62; int8 exponents 13824x5120x2 at 128 rows 74 / 42, 768x3072x3 at 512 rows 17 / 34.
+// Measured (us, matrix-core kernel / this one, * = taken): 4096x4096x3 at 64 rows 13.1* / 19.1, 128 rows 15.0* / 26.1, 512
+// rows 54.7 / 42.1*; 11008x4096x3 at 256 rows 83 / 48.5*; 8192x8192x4 at 64 rows 27.4* / 30.2, 128 rows 52.5 / 41.5*;
+// 28672x8192x4 at 48 rows 97 / 67.5*; 1024x28672x4 at 256 rows 44.3* / 53.6, 512 rows 76.7 / 59.4*; 4096x11008x2 at 128 rows
+// 28.8* / 35.7; int8 exponents 13824x5120x2 at 128 rows 74.5 / 42.6*, 768x3072x3 at 512 rows 15.9* / 27.9.  The estimate of
+// the matrix-core kernel is low where its last round is nearly empty, and the slower kernel is taken by a tenth or so:
+// 11008x4096x3 at 48 rows 25.8* / 24.0, 64 rows 29.1* / 24.6; int8 exponents 13824x5120x2 at 64 rows 38.7* / 35.3.
 bool tile_wanted(const Problem &p, int mode)
 {
     const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
