@@ -202,6 +202,11 @@ struct TileProblem {
     int out_type;                    // IoType
 };
 
+// Floats from one slice's sums to the next.  The odd number of 256-byte blocks between them keeps the same output of all
+// slices, which are read together, off the same memory channels where M * N is a multiple of a large power of two
+// (4096x4096x3, 512 rows in 4 slices 42.6 -> 34.2 us, 1024 rows in 2 slices 60.0 -> 51.6).
+__host__ __device__ constexpr size_t tile_slice_stride(int M, int N) { return (size_t)M * N + 17 * 64; }
+
 struct Group {
     int count;
     Problem p[kMaxGroup];

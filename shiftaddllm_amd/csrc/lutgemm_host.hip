@@ -23,7 +23,9 @@ constexpr int kMfmaWaves = 8;       // waves of a matrix-core workgroup: K-steps
 constexpr int kMfmaTileCols = 64;   // outputs per matrix-core workgroup
 constexpr int kMfmaStepK = 128;
 constexpr int kMaxDevices = 64;
+constexpr int kTileMaxSlices = 16;
 constexpr size_t kTileSumBytes = 64u << 20;   // GEMM kernel: sums of the K-slices of a launch, at most
+constexpr size_t kTileGapBytes = kTileMaxSlices * tile_slice_stride(0, 0) * 4;   // what lies between them
 
 thread_local int g_last_hip_error = 0;
 
@@ -148,7 +150,8 @@ int stream_split_buffer(hipStream_t stream, size_t bytes, void **out)
         if (ws.split) ws.retired_split.push_back(ws.split);
         ws.split = nullptr;
         ws.split_bytes = 0;
-        const size_t want = grown(bytes, 1u << 20);
+        // (the gaps between slices on top of a power of two: sums that fill one would otherwise take the next)
+        const size_t want = grown(bytes > kTileGapBytes ? bytes - kTileGapBytes : bytes, 1u << 20) + kTileGapBytes;
         e = hipMalloc(&ws.split, want);
         if (e != hipSuccess) {
             g_last_hip_error = (int)e;
@@ -674,12 +677,12 @@ double plan_tile(TileProblem &t)
     const long tiles = (long)t.n_tiles * t.m_tiles;
     const double alone = t.tile_rows == 128 ? 1.2 : 0.9, beside = t.tile_rows == 128 ? 2.1 : 1.6;
     double best_cost = 0.0;
-    for (int ks = 1; ks <= 16 && (ks == 1 || 2 * ks <= t.steps); ++ks) {
+    for (int ks = 1; ks <= kTileMaxSlices && (ks == 1 || 2 * ks <= t.steps); ++ks) {
         const int steps = ((t.steps + ks - 1) / ks + 1) & ~1;
         const int slices = (t.steps + steps - 1) / steps;
         if (slices != ks) continue;
         const long wgs = tiles * slices;
-        if (ks > 1 && (wgs > 2 * kCUs || (size_t)ks * t.M * t.N * 4 > kTileSumBytes)) break;
+        if (ks > 1 && (wgs > 2 * kCUs || ks * tile_slice_stride(t.M, t.N) * 4 > kTileSumBytes)) break;
         const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;
         double cost = (double)rounds * (steps * beside + 5.0);
         if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 5.0;
@@ -747,7 +750,7 @@ int run_tile(const Problem &p, int mode, const Accum &acc)
     if (t.ksplit > 1 && !acc.fixed) {
         void *sums = nullptr;
         lock.lock();
-        const int rc = stream_split_buffer(acc.stream, (size_t)t.ksplit * t.M * t.N * 4, &sums);
+        const int rc = stream_split_buffer(acc.stream, t.ksplit * tile_slice_stride(t.M, t.N) * 4, &sums);
         if (rc != LUTGEMM_OK && rc != LUTGEMM_ECAPTURE) return rc;
         t.partial = (float *)sums;
     }
@@ -1563,9 +1566,9 @@ int lutgemm_reserve_workspace(void *stream, size_t words)
     unsigned long long *unused = nullptr;
     const int rc = stream_workspace((hipStream_t)stream, words, &unused);
     if (rc != LUTGEMM_OK) return rc;
-    // the sums of the GEMM kernel's K-slices: at most sixteen per output, 64 MB in all (plan_tile)
+    // the sums of the GEMM kernel's K-slices: at most sixteen per output and what lies between them, 64 MB in all (plan_tile)
     void *sums = nullptr;
-    return stream_split_buffer((hipStream_t)stream, words < kTileSumBytes / 64 ? words * 64 : kTileSumBytes, &sums);
+    return stream_split_buffer((hipStream_t)stream, words < (kTileSumBytes - kTileGapBytes) / 64 ? words * 64 + kTileGapBytes : kTileSumBytes, &sums);
 }
 
 int lutgemm_copy_bytes(void *dst, const void *src, size_t bytes, void *stream)
