@@ -49,7 +49,8 @@ def _run(cmd):
 
 
 KERNEL_SOURCES = ("lutgemm_host.hip", "lut_gemv_rowwise.hip", "lut_gemv_block.hip", "lut_gemv_block_staged.hip",
-                  "lut_gemv_group.hip", "lut_gemv_fused.hip", "lut_gemv_chain.hip", "lut_gemm_mfma.hip", "lut_gemm_mx.hip", "lut_gemm_tile.hip", "lut_gemm_tile_serial.hip",
+                  "lut_gemv_group.hip", "lut_gemv_fused.hip", "lut_gemv_chain.hip", "lut_gemm_mfma.hip", "lut_gemm_mx.hip", "lut_gemm_tile.hip",
+                  "lut_gemm_tile_pair.hip", "lut_gemm_tile_serial.hip",
                   "decode_kernels.hip")
 KERNEL_HEADERS = ("lutgemm_internal.h", "lutgemm_common.h", "lutgemm_launch.h", "lut_gemv_device.h",
                   "lut_gemm_mfma_device.h", "lut_gemm_mx_device.h", "lut_dequant_device.h", "lut_gemm_tile_device.h")

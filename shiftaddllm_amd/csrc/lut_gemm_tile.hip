@@ -13,8 +13,6 @@ hipError_t launch_fmt(const TileProblem &p, hipStream_t stream)
         hipLaunchKernelGGL((lut_gemm_tile_kernel<NB, FMT, 2>), grid, block, 0, stream, p);
     else
         hipLaunchKernelGGL((lut_gemm_tile_kernel<NB, FMT, 4>), grid, block, 0, stream, p);
-    if (p.ksplit > 1)
-        hipLaunchKernelGGL(tile_sum_kernel, dim3((unsigned)(((size_t)p.M * p.N / 4 + 255) / 256)), dim3(256), 0, stream, p);
     return hipGetLastError();
 }
 
@@ -32,12 +30,20 @@ hipError_t launch_nb(const TileProblem &p, hipStream_t stream)
 hipError_t launch_tile(const TileProblem &p, int nb, hipStream_t stream)
 {
     if (p.ksplit > 1 && !p.partial) return launch_tile_serial(p, nb, stream);
-    switch (nb) {
-    case 1: return launch_nb<1>(p, stream);
-    case 2: return launch_nb<2>(p, stream);
-    case 3: return launch_nb<3>(p, stream);
-    default: return launch_nb<4>(p, stream);
-    }
+    hipError_t e = hipSuccess;
+    if (p.pair)
+        e = launch_tile_pair(p, nb, stream);
+    else if (nb == 1)
+        e = launch_nb<1>(p, stream);
+    else if (nb == 2)
+        e = launch_nb<2>(p, stream);
+    else if (nb == 3)
+        e = launch_nb<3>(p, stream);
+    else
+        e = launch_nb<4>(p, stream);
+    if (p.ksplit == 1 || e != hipSuccess) return e;
+    hipLaunchKernelGGL(tile_sum_kernel, dim3((unsigned)(((size_t)p.M * p.N / 4 + 255) / 256)), dim3(256), 0, stream, p);
+    return hipGetLastError();
 }
 
 }  // namespace lutgemm

@@ -3,7 +3,7 @@
 //
 //   out[m][n] = init[m][n] + sum_k x[m][k] * W[n][k],  W formed from the sign planes on the fly.
 //
-// A workgroup of 4 waves owns 256 outputs x 32 * MF activation rows.  Each wave forms the weights of its
+// A workgroup of 4 waves (or of two such teams, each on half of the inputs) owns 256 outputs x 32 * MF activation rows.  Each wave forms the weights of its
 // own 64 outputs in registers (lut_dequant_device.h), directly in the layout of the matrix
 // instruction's A operand (v_mfma_f32_32x32x16_f16: lane l holds output l % 32 and eight inputs), so a
 // weight is formed once per workgroup and never stored; the activations, the B operand, go through LDS
@@ -54,16 +54,30 @@ __device__ __forceinline__ void static_for(F &&f)
     static_for_impl(std::make_integer_sequence<int, N>{}, f);
 }
 
-// SERIAL: the workgroup takes all K-slices of its tile, one after the other, and adds their sums up as
-// tile_sum_kernel does: the bits are those of slices that run side by side, and no memory is needed.
-template <int NB, int FMT, int MF, bool SERIAL>
-__device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int m_tile, int slice, char *lds)
+// How a workgroup goes about its tile:
+enum TileKind : int {
+    kTileAlone = 0,   // four waves, one K-slice
+    // Eight waves: two teams of four take half of the slice's steps each, in LDS of their own, and add up at the end.
+    // For calls whose workgroups have a CU to themselves: two waves per SIMD instead of one, whose vector and matrix work
+    // overlap, without more slices, whose sums cost memory traffic (5120x13824x2 int8 exponents at 512 rows, 3 slices 105.7 -> 88.3
+    // us; 6 slices of four waves, which fill the chip as well, 92.1).
+    kTilePair = 1,
+    // Four waves take all K-slices in turn and add them up as tile_sum_kernel does: the bits are those of slices
+    // that run side by side, and no memory is needed.  The second form: slices of teams, half by half.
+    kTileSerial = 2,
+    kTileSerialPair = 3,
+};
+
+// tid: the thread among the team's 256;  lds: the workgroup's, of which team `team` takes part `team`
+template <int NB, int FMT, int MF, int KIND>
+__device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int m_tile, int slice, int tid, int team, char *lds_all)
 {
+    char *const lds = lds_all + team * kTileLdsBytes<FMT, MF>;
     constexpr bool UNI = FMT == kTileUniform;
     constexpr bool BLOCK = FMT >= kTileBlock;
     constexpr int kTabs = BLOCK ? 4 : 1;                       // tables per 32-output fragment and step
     constexpr int kFragTabs = FMT == kTileBlockWide ? 1 : 2;   // fragments with tables of their own
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, kh = lane >> 5;
+    const int lane = tid & 63, wave = tid >> 6, l32 = lane & 31, kh = lane >> 5;
     const int n0 = __builtin_amdgcn_readfirstlane(n_tile * kTileN + wave * kTileWaveN);
     const int m0 = m_tile * 32 * MF;
     int nn[2];
@@ -395,7 +409,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         __syncthreads();
     };
 
-    auto take_slice = [&](int sl) {
+    auto take_steps = [&](int t0, int t1) {   // (even numbers)
 #pragma unroll
         for (int f = 0; f < 2; ++f)
 #pragma unroll
@@ -403,7 +417,6 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[f][i][r] = 0.0f;
         // ---- prologue: step 0's activations in LDS, its weights in A[0] --------------------------------------
-        const int t0 = sl * p.slice_steps, t1 = min(t0 + p.slice_steps, p.steps);   // (even numbers)
         load_x(t0);
         load_words(t0, words);
         fetch_scales(t0);
@@ -436,41 +449,57 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         for (int f = 0; f < kFragTabs; ++f) back[f] = inverse_unit(unit[f]);
         scale_sums(back, std::false_type());
     };
-    if constexpr (SERIAL) {
-        f32x16 total[2][MF];
+    auto each_sum = [&](auto &&f) {
 #pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int i = 0; i < MF; ++i)
 #pragma unroll
-                for (int r = 0; r < 16; ++r) total[f][i][r] = 0.0f;
+                for (int r = 0; r < 16; ++r) f(h, i, r);
+    };
+    // the steps of a slice, and where its second half begins
+    auto first_step = [&](int sl) { return sl * p.slice_steps; };
+    auto last_step = [&](int sl) { return min((sl + 1) * p.slice_steps, p.steps); };
+    auto second_half = [&](int sl) { return first_step(sl) + (((last_step(sl) - first_step(sl)) / 2 + 1) & ~1); };
+    constexpr bool SERIAL = KIND == kTileSerial || KIND == kTileSerialPair;
+    if constexpr (SERIAL) {
+        f32x16 total[2][MF];
+        each_sum([&](int h, int i, int r) { total[h][i][r] = 0.0f; });
 #pragma clang loop unroll(disable)
         for (int sl = 0; sl < p.ksplit; ++sl) {   // (every wave has left the LDS of a slice behind the barrier of its last step)
-            take_slice(sl);
-#pragma unroll
-            for (int f = 0; f < 2; ++f)
-#pragma unroll
-                for (int i = 0; i < MF; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) total[f][i][r] += acc[f][i][r];
+            if constexpr (KIND == kTileSerialPair) {
+                f32x16 half[2][MF];
+                each_sum([&](int h, int i, int r) { half[h][i][r] = 0.0f; });
+#pragma clang loop unroll(disable)
+                for (int part = 0; part < 2; ++part) {
+                    take_steps(part ? second_half(sl) : first_step(sl), part ? last_step(sl) : second_half(sl));
+                    each_sum([&](int h, int i, int r) { half[h][i][r] += acc[h][i][r]; });
+                }
+                each_sum([&](int h, int i, int r) { total[h][i][r] += half[h][i][r]; });
+            } else {
+                take_steps(first_step(sl), last_step(sl));
+                each_sum([&](int h, int i, int r) { total[h][i][r] += acc[h][i][r]; });
+            }
         }
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
-#pragma unroll
-            for (int i = 0; i < MF; ++i) acc[f][i] = total[f][i];
+        each_sum([&](int h, int i, int r) { acc[h][i][r] = total[h][i][r]; });
+    } else if constexpr (KIND == kTilePair) {
+        const int from = first_step(slice), middle = second_half(slice), to = last_step(slice);
+        take_steps(team ? middle : from, team ? to : middle);
+        // (a barrier per step: the team with fewer of them joins the others')
+        for (int t = team ? to - middle : middle - from; t < middle - from; ++t) __syncthreads();
     } else {
-        take_slice(slice);
+        take_steps(first_step(slice), last_step(slice));
     }
 
     // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
     // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
     float *sums = !SERIAL && p.ksplit > 1 ? p.partial + (size_t)slice * tile_slice_stride(p.M, p.N) : nullptr;
+    auto write_out = [&](auto f_c) {
+        constexpr int f = decltype(f_c)::value;
 #pragma unroll
-    for (int i = 0; i < MF; ++i) {
-        const int m = m0 + 32 * i + l32;
-        if (m >= p.M) continue;
-#pragma unroll
-        for (int f = 0; f < 2; ++f)
+        for (int i = 0; i < MF; ++i) {
+            const int m = m0 + 32 * i + l32;
+            if (m >= p.M) continue;
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int n = n0 + 32 * f + 8 * g + 4 * kh;
@@ -485,6 +514,41 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
                 if (!p.overwrite) add_halves(v, p.init + (size_t)m * p.init_stride + n);
                 store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
             }
+        }
+    };
+    if constexpr (KIND == kTilePair) {
+        // team 0 finishes the waves' first 32 outputs, team 1 the others: each leaves what the other finishes in LDS
+        auto at = [&](int of, int i, int g) { return (f32x4 *)(lds_all + (((of * 4 + wave) * MF + i) * 4 + g) * 1024 + lane * 16); };
+        auto finish = [&](auto mine_c) {
+            constexpr int mine = decltype(mine_c)::value;
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    f32x4 v;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = acc[1 - mine][i][4 * g + r];
+                    *at(mine, i, g) = v;
+                }
+            __syncthreads();
+#pragma unroll
+            for (int i = 0; i < MF; ++i)
+#pragma unroll
+                for (int g = 0; g < 4; ++g) {
+                    const f32x4 v = *at(1 - mine, i, g);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) acc[mine][i][4 * g + r] += v[r];
+                }
+            write_out(mine_c);
+        };
+        __syncthreads();   // (the LDS of both teams changes hands)
+        if (team == 0)
+            finish(std::integral_constant<int, 0>());
+        else
+            finish(std::integral_constant<int, 1>());
+    } else {
+        write_out(std::integral_constant<int, 0>());
+        write_out(std::integral_constant<int, 1>());
     }
 }
 
@@ -525,12 +589,14 @@ static __global__ void __launch_bounds__(256) tile_sum_kernel(const TileProblem 
     store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
 }
 
-template <int NB, int FMT, int MF, bool SERIAL>
+template <int NB, int FMT, int MF, int KIND>
 __device__ __forceinline__ void gemm_workgroup(const TileProblem &p, char *lds)
 {
     int n_tile, m_tile, slice;
     decode_tile(p, (int)blockIdx.x, n_tile, m_tile, slice);
-    if (slice >= (SERIAL ? 1 : p.ksplit)) return;
+    if (slice >= (KIND == kTileSerial || KIND == kTileSerialPair ? 1 : p.ksplit)) return;
+    const int tid = (int)threadIdx.x & (kTileThreads - 1);
+    const int team = KIND == kTilePair ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kTileThreads) : 0;
     if constexpr (FMT == kTileBlock) {
         // most tiles have no wave whose outputs lie in two row groups, and need half the tables
         bool straddles = false;
@@ -540,11 +606,11 @@ __device__ __forceinline__ void gemm_workgroup(const TileProblem &p, char *lds)
             straddles = straddles || (first < p.N && first / p.rows_per_group != last / p.rows_per_group);
         }
         if (!straddles) {
-            gemm_tile<NB, kTileBlockWide, MF, SERIAL>(p, n_tile, m_tile, slice, lds);
+            gemm_tile<NB, kTileBlockWide, MF, KIND>(p, n_tile, m_tile, slice, tid, team, lds);
             return;
         }
     }
-    gemm_tile<NB, FMT, MF, SERIAL>(p, n_tile, m_tile, slice, lds);
+    gemm_tile<NB, FMT, MF, KIND>(p, n_tile, m_tile, slice, tid, team, lds);
 }
 
 template <int NB, int FMT, int MF>
@@ -552,16 +618,27 @@ __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_
 lut_gemm_tile_kernel(const TileProblem p)
 {
     __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
-    gemm_workgroup<NB, FMT, MF, false>(p, lds);
+    gemm_workgroup<NB, FMT, MF, kTileAlone>(p, lds);
 }
 
-// One workgroup per tile and per CU (a call that is cut has at most 256 tiles): two sets of accumulators fit.
 template <int NB, int FMT, int MF>
+__global__ void __launch_bounds__(2 * kTileThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
+lut_gemm_tile_pair_kernel(const TileProblem p)
+{
+    // (what the teams hand over at the end: 32 outputs x 32 MF rows of every wave)
+    constexpr int kHandOver = 2 * 4 * 32 * 32 * MF * 4, kTeams = 2 * kTileLdsBytes<FMT, MF>;
+    __shared__ __attribute__((aligned(16))) char lds[kTeams > kHandOver ? kTeams : kHandOver];
+    gemm_workgroup<NB, FMT, MF, kTilePair>(p, lds);
+}
+
+// One workgroup per tile and per CU (a call that is cut has at most 256 tiles): two sets of accumulators fit, or three
+// of 64 rows.
+template <int NB, int FMT, int MF, int KIND>
 __global__ void __launch_bounds__(kTileThreads) __attribute__((amdgpu_waves_per_eu(1, 1)))
 lut_gemm_tile_serial_kernel(const TileProblem p)
 {
     __shared__ __attribute__((aligned(16))) char lds[kTileLdsBytes<FMT, MF>];
-    gemm_workgroup<NB, FMT, MF, true>(p, lds);
+    gemm_workgroup<NB, FMT, MF, KIND>(p, lds);
 }
 
 }  // namespace lutgemm

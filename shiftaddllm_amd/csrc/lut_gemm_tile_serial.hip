@@ -9,10 +9,12 @@ template <int NB, int FMT>
 hipError_t launch_fmt(const TileProblem &p, hipStream_t stream)
 {
     const dim3 grid((unsigned)((p.n_tiles + 7) / 8 * 8 * p.m_tiles)), block(kTileThreads);
-    if (p.tile_rows == 64)
-        hipLaunchKernelGGL((lut_gemm_tile_serial_kernel<NB, FMT, 2>), grid, block, 0, stream, p);
+    if (p.pair)
+        hipLaunchKernelGGL((lut_gemm_tile_serial_kernel<NB, FMT, 2, kTileSerialPair>), grid, block, 0, stream, p);
+    else if (p.tile_rows == 64)
+        hipLaunchKernelGGL((lut_gemm_tile_serial_kernel<NB, FMT, 2, kTileSerial>), grid, block, 0, stream, p);
     else
-        hipLaunchKernelGGL((lut_gemm_tile_serial_kernel<NB, FMT, 4>), grid, block, 0, stream, p);
+        hipLaunchKernelGGL((lut_gemm_tile_serial_kernel<NB, FMT, 4, kTileSerial>), grid, block, 0, stream, p);
     return hipGetLastError();
 }
 
@@ -27,8 +29,13 @@ hipError_t launch_nb(const TileProblem &p, hipStream_t stream)
 
 }  // namespace
 
-hipError_t launch_tile_serial(const TileProblem &p, int nb, hipStream_t stream)
+hipError_t launch_tile_serial(const TileProblem &as_planned, int nb, hipStream_t stream)
 {
+    TileProblem p = as_planned;
+    if (p.pair) {   // (the rows of a tile do not matter to the bits; at most 256 tiles of 64 rows, as plan_tile cuts for teams)
+        p.tile_rows = 64;
+        p.m_tiles = (p.M + 63) / 64;
+    }
     switch (nb) {
     case 1: return launch_nb<1>(p, stream);
     case 2: return launch_nb<2>(p, stream);

@@ -197,6 +197,7 @@ struct TileProblem {
     int n_tiles, m_tiles, tile_rows;
     int steps;                       // K-steps, rounded up to an even number
     int ksplit, slice_steps;         // K-slices and steps of each (even; the last one may have fewer)
+    int pair;                        // 1: two teams of waves per workgroup, half of a slice's steps each
     float *partial;                  // ksplit > 1: [slice][M][N] partial sums; null: a workgroup takes its tile's slices in turn
     int init_stride, overwrite;
     int out_type;                    // IoType

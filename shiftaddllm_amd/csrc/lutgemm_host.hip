@@ -658,15 +658,19 @@ int run_mx(Problem &p, const Accum &acc)
 }
 
 // ---- GEMM kernel for many activation rows ------------------------------------------------------------
-// Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices: a workgroup each, two per CU.
+// Cut a problem into tiles of 256 outputs x 64 or 128 rows and K-slices, a workgroup each.  A workgroup is four waves,
+// two workgroups per CU, or two teams of four that halve its slice (one per CU).
 // The cut depends on the sizes alone, so that a call gives the same bits eagerly, under capture and through the
 // entry point that allocates nothing.  Returns the time the plan should take.
-// Costs in microseconds, taken at three planes for all of them: a step of a 128-row tile takes 1.2 alone on its CU
-// and 2.1 beside another one (64 rows: 0.9 and 1.6), a workgroup's start and end 5; the sums of the slices
-// are written and read at about 4 TB/s, by a second launch that costs another 4.
-// Measured at one to four planes (128 rows alone, beside another; 64 rows alone): row-wise 0.88, 0.97, 1.07, 1.36 / 1.63,
-// 1.73, 1.88, 2.19 / 0.66, 0.73, 0.84, 1.04; int8 exponents 1.41, 1.25, 1.40, 1.75 / 1.85, 1.84, 2.06, 2.44 / 1.18, 1.10,
-// 1.25, 1.57.
+// Costs in microseconds, for all formats and planes.  A step of a 128-row tile: 1.1 alone on its CU (measured 1.0 to 1.25),
+// 1.95 beside another workgroup or for two teams together, 1.65 for teams while a third of the CUs are idle (clocks
+// are higher); 64 rows: 0.8, 1.35 and 1.2.  A workgroup's start and end 4.6, with teams 6.  The sums of the slices
+// and the launch that adds them up 6 and 0.2 per MB.  What they pick (us; s: slices of four waves, p: of teams, * = taken):
+//   512 rows:  5120x13824x2 int8 exponents s3 105.7 s6 92.1 p2 111.6 p3* 88.3; 13824x5120x2 int8 exponents s1 106.8 s2 99.5 p1* 85.2;
+//              4096x4096x3 s3 37.9 s4 34.2 p3 35.7 p4* 34.3 (s3 was taken before: 105.7, 106.6 and 42.5)
+//   1024 rows: 4096x4096x3 s1 72.1 s2 51.6 p1 60.7 p2* 50.3; 5120x5120x2 blocks s1 92.1 s2 84.3 s3 76.1 p1* 72.4
+//   128 rows:  8192x28672x4 s8 76.0 p4 104.4 p8* 72.9; 8192x8192x4 s8 34.2 p4 42.2 p8* 34.3; 11008x4096x3 s5 30.4 p3 34.2 p5* 29.8
+//   64 rows:   8192x28672x4 s8 58.1 p4 81.7 p8* 50.2; 8192x8192x4 s8 25.6 p8* 24.2; 13824x5120x2 int8 exponents s8 30.6 p4* 29.2
 double plan_tile(TileProblem &t)
 {
     constexpr long kCUs = 256;
@@ -675,36 +679,49 @@ double plan_tile(TileProblem &t)
     t.m_tiles = (t.M + t.tile_rows - 1) / t.tile_rows;
     t.steps = (t.kwords + 3) / 4 * 2;
     const long tiles = (long)t.n_tiles * t.m_tiles;
-    const double alone = t.tile_rows == 128 ? 1.2 : 0.9, beside = t.tile_rows == 128 ? 2.1 : 1.6;
+    const bool tall = t.tile_rows == 128;
     double best_cost = 0.0;
     for (int ks = 1; ks <= kTileMaxSlices && (ks == 1 || 2 * ks <= t.steps); ++ks) {
         const int steps = ((t.steps + ks - 1) / ks + 1) & ~1;
         const int slices = (t.steps + steps - 1) / steps;
         if (slices != ks) continue;
         const long wgs = tiles * slices;
-        if (ks > 1 && (wgs > 2 * kCUs || ks * tile_slice_stride(t.M, t.N) * 4 > kTileSumBytes)) break;
-        const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;
-        double cost = (double)rounds * (steps * beside + 5.0);
-        if (rest > 0) cost += (rest > kCUs ? steps * beside : steps * alone) + 5.0;
-        if (ks > 1) cost += 4.0 + 2.0 * (double)((size_t)ks * t.M * t.N * 4) / 4e6;
-        if (ks == 1 || cost < best_cost * 0.99) {
-            best_cost = cost;
-            t.ksplit = slices;
-            t.slice_steps = steps;
+        const size_t sums = ks > 1 ? ks * tile_slice_stride(t.M, t.N) * 4 : 0;
+        if (ks > 1 && (wgs > 2 * kCUs || sums > kTileSumBytes)) break;
+        for (int pair = 0; pair < 2; ++pair) {
+            if (pair && wgs > kCUs) continue;   // (rounds of teams end together: 11008x4096x3 at 2048 rows s1 199 p1 209)
+            const long rounds = wgs / (2 * kCUs), rest = wgs - rounds * 2 * kCUs;   // (of two workgroups per CU)
+            const double together = tall ? 1.95 : 1.35, fixed = pair ? 6.0 : 4.6;
+            const int own = pair ? (steps / 2 + 1) & ~1 : steps;
+            double step = together;   // of the last, partly filled round
+            if (pair) {
+                const double idle = 1.0 - (double)rest / kCUs;
+                step -= (tall ? 0.3 : 0.15) * (idle > 0.4 ? 1.0 : idle / 0.4);
+            } else if (rest <= kCUs) {
+                step = tall ? 1.1 : 0.8;
+            }
+            double cost = (double)rounds * (own * together + fixed);
+            if (rest > 0) cost += own * step + fixed;
+            if (sums) cost += 6.0 + 0.2e-6 * (double)sums;
+            if ((ks == 1 && !pair) || cost < best_cost * 0.99) {
+                best_cost = cost;
+                t.pair = pair;
+                t.ksplit = slices;
+                t.slice_steps = steps;
+            }
         }
     }
     return best_cost;
 }
 
 // Whether a call takes the GEMM kernel rather than the matrix-core kernel, from what either should take (in
-// microseconds; the slowest term only).  The matrix-core kernel forms the weights of a 32-row chunk in rounds of
-// 64 outputs x 1024 inputs, about 3 us each with one workgroup per CU.
-// Measured (us, matrix-core kernel / this one, * = taken): 4096x4096x3 at 64 rows 13.1* / 19.1, 128 rows 15.0* / 26.1, 512
-// rows 54.7 / 42.1*; 11008x4096x3 at 256 rows 83 / 48.5*; 8192x8192x4 at 64 rows 27.4* / 30.2, 128 rows 52.5 / 41.5*;
-// 28672x8192x4 at 48 rows 97 / 67.5*; 1024x28672x4 at 256 rows 44.3* / 53.6, 512 rows 76.7 / 59.4*; 4096x11008x2 at 128 rows
-// 28.8* / 35.7; int8 exponents 13824x5120x2 at 128 rows 74.5 / 42.6*, 768x3072x3 at 512 rows 15.9* / 27.9.  The estimate of
-// the matrix-core kernel is low where its last round is nearly empty, and the slower kernel is taken by a tenth or so:
-// 11008x4096x3 at 48 rows 25.8* / 24.0, 64 rows 29.1* / 24.6; int8 exponents 13824x5120x2 at 64 rows 38.7* / 35.3.
+// microseconds).  A round of the matrix-core kernel (32-row tiles, one K-step per wave, one workgroup per CU) takes 2.2 to
+// 3.0 with two to four planes and 0.9 more with the decoding of block formats.
+// Measured (us, matrix-core kernel / this one, * = taken): 11008x4096x3 at 48 rows 25.7 / 22.5*, 128 rows 43.1 / 29.8*; 4096x11008x2 at
+// 128 rows 29.2 / 29.1*, 200 rows 55.3 / 36.2*; int8 exponents 5120x13824x2 at 33 rows 34.2 / 26.6*, 13824x5120x2 at 64 rows
+// 40.2 / 28.7*, 768x3072x3 at 512 rows 16.7* / 26.3; 1024x28672x4 at 128 rows 28.4* / 36.8, 200 rows 44.0 / 38.3*; 2964x2208x3 in
+// groups of 96 at 200 rows 22.8* / 22.6, 512 rows 35.7 / 27.7*; uniform 4096x4096x4 at 128 rows 30.0* / 31.4, 200 rows 55.8 /
+// 40.4*; 2048x2048x3 at 512 rows 17.6* / 23.1.  Of 104 such calls none takes the slower kernel by more than its noise.
 bool tile_wanted(const Problem &p, int mode)
 {
     const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
@@ -719,8 +736,14 @@ bool tile_wanted(const Problem &p, int mode)
     t.N = p.N;
     t.M = p.M;
     t.kwords = p.kwords;
-    const double rounds = (double)((p.N + 63) / 64) * (double)((p.M + 31) / 32) * (double)((p.K + 1023) / 1024);
-    return plan_tile(t) < 5.0 + 3.0 * rounds / 256.0;
+    // The matrix-core kernel with tiles of 32 rows: a round is one K-step per wave, one workgroup per CU.
+    Group one{};
+    one.count = 1;
+    one.p[0] = p;
+    plan_mfma(one.p[0], 2, mfma_slices(one, 2));
+    const double rounds = (double)((one.p[0].n_blocks + 255) / 256) * (double)(one.p[0].sets_per_split / kMfmaWaves);
+    const double round = 1.6 + 0.32 * p.nb + (is_block(mode) ? 0.9 : 0.0);
+    return plan_tile(t) < 5.0 + round * rounds;
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)

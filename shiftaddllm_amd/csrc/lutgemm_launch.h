@@ -34,9 +34,10 @@ hipError_t launch_mx(const Problem &p, void *split, hipStream_t stream);
 inline int mx_chunk_rows(int M) { return M <= 5 ? 5 : M <= 8 ? 8 : 16; }
 inline size_t mx_split_bytes(int M, int K) { return (size_t)M * K * 3 + (size_t)K + (size_t)M * (K / 32) * 4; }
 
-// GEMM kernel for many activation rows, every alpha format; one wave per SIMD and 256 outputs per workgroup
+// GEMM kernel for many activation rows, every alpha format; 256 outputs per workgroup
 struct TileProblem;
 hipError_t launch_tile(const TileProblem &p, int nb, hipStream_t stream);
+hipError_t launch_tile_pair(const TileProblem &p, int nb, hipStream_t stream);     // (launch_tile's, where p.pair is set)
 hipError_t launch_tile_serial(const TileProblem &p, int nb, hipStream_t stream);   // (launch_tile's, where p.partial is null)
 
 }  // namespace lutgemm
