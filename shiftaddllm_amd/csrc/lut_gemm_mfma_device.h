@@ -28,10 +28,16 @@ namespace lutgemm {
 // base + 4*li + kb, or of chunk li and row group kb, and the lanes hand them round by ds_bpermute.
 // Shorter groups (OWN) leave every lane with four tables of its own.
 //
-// Nothing is staged through LDS in the main loop and there is no barrier in it: a lane's B operands of a
-// step are the 32 activations of row li under its word kb, 64 contiguous bytes that it loads itself
-// (L2 hits).  Each wave runs its own two-deep pipeline of (signs, scales, activations) and the waves of
-// a workgroup drift freely until the final reduction.
+// Activations: a lane's B operands of a step are the 32 activations of row li under its word kb, 64 contiguous
+// bytes.  With 16 rows a lane loads them itself.  A request's 64 lanes then touch 32 cache lines, 32 bytes of each, and
+// every line is asked for four times; at 32 rows that bounded the kernel (8192x28672x4 46.4 us, 36.3 with the activations
+// left out, 45.0 with the weights left unformed).  So with 32 rows a request takes four rows' 256 contiguous bytes and the
+// wave turns them round in LDS of its own: 42.4 us; 28672x8192x4 54.9 -> 49.4, 11008x4096x3 15.4 -> 14.2.  (With 16 rows
+// the detour costs more than it gives, registers above all: 8192x8192x4 at 4 rows 12.0 -> 16.2; nor does it where weights come in two pieces and forming
+// them bounds the kernel: uniform 8192x8192x4 at 17 rows 30.3 -> 31.3.)
+//
+// There is no barrier in the main loop: each wave runs its own two-deep pipeline of (signs, scales, activations) and
+// the waves of a workgroup drift freely until the final reduction.
 // ---------------------------------------------------------------------------
 constexpr int kMfmaThreads = 512;
 constexpr int kMfmaWaves = kMfmaThreads / 64;
@@ -41,12 +47,19 @@ constexpr int kMfmaMaxRowGroups = 4;  // alpha row groups 64 outputs may touch (
 constexpr int kRedRow = 65;           // the final reduction's LDS rows, padded against bank conflicts
 template <int MT>
 constexpr int kMfmaRedBytes = kMfmaWaves * 16 * MT * kRedRow * 4;
-// the rows' reciprocal RMS sit behind the final reduction
+// a wave's activations on their way to operands: 16 rows of 128 inputs, 16 bytes apart, so that the 16 rows of a
+// read spread over all banks
+constexpr int kTurnRow = 256 + 16;
 template <int MT>
-constexpr int kMfmaLdsBytes = kMfmaRedBytes<MT> + 16 * MT * 4;
+constexpr int kMfmaTurnBytes = MT > 1 ? kMfmaWaves * MT * 16 * kTurnRow : 0;
+// the rows' reciprocal RMS sit behind both
+template <int MT>
+constexpr int kMfmaScaleAt = kMfmaTurnBytes<MT> > kMfmaRedBytes<MT> ? kMfmaTurnBytes<MT> : kMfmaRedBytes<MT>;
+template <int MT>
+constexpr int kMfmaLdsBytes = kMfmaScaleAt<MT> + 16 * MT * 4;
 
-// Operands of one K-step of a wave: per bit plane word kb of 4 outputs; per 16-row tile the lane's 32
-// activations; the scales of the lane's table(s), as they lie in memory.
+// Operands of one K-step of a wave: per bit plane word kb of 4 outputs; per 16-row tile the lane's 32 activations (to
+// be turned round: chunk li of rows kb, kb + 4, ...); the scales of the lane's table(s), as they lie in memory.
 template <int NB, int MT, int FMT, bool OWN>
 struct MfmaOperands {
     static constexpr int kScales = FMT == kWeightUniform ? (OWN ? 4 : 2) : (OWN ? 2 * NB : NB);
@@ -86,11 +99,14 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     const int step_begin = kslice * p.sets_per_split;
     const int step_end = min(step_begin + p.sets_per_split, p.nsets);
 
-    // the lane's activations: row li of each 16-row tile (rows beyond M are clamped to
-    // the last one: computed twice, written once)
-    uint32_t xlane[MT];   // (byte offsets: the host keeps M * K * 2 below 2^32)
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) xlane[mt] = (uint32_t)min(m0 + 16 * mt + li, p.M - 1) * (uint32_t)p.K * 2u;
+    // the lane's activations: row li of each 16-row tile, or rows kb + 4 c (rows beyond M are clamped to the last one:
+    // computed twice, written once; byte offsets: the host keeps M * K * 2 below 2^32, and what wraps beyond it belongs
+    // to no row)
+    constexpr bool TURN = MT > 1 && !UNI;
+    const uint32_t row_bytes_x = (uint32_t)p.K * 2u, xlast = (uint32_t)(p.M - 1) * row_bytes_x;
+    const uint32_t xfirst = (uint32_t)(TURN ? m0 + kb : min(m0 + li, p.M - 1)) * row_bytes_x;
+    [[maybe_unused]] char *const turn_in = xs + wave * (MT * 16 * kTurnRow) + kb * kTurnRow + li * 16;
+    [[maybe_unused]] const char *const turn_out = xs + wave * (MT * 16 * kTurnRow) + li * kTurnRow + kb * 64;
 
     // block formats: the tile's row groups; this lane forms tables of group rg and looks its own outputs up
     // among those of lane group rg_of
@@ -145,11 +161,14 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
                     r.s[b] = *(const unsigned short *)((const char *)p.alpha + (size_t)(g * NB + b) * (p.N * 2u) + col2);
             }
         }
+        // (beyond K: the last chunk, for weights of zero)
+        [[maybe_unused]] const uint32_t xchunk = (uint32_t)min(16 * step + li, p.K / 8 - 1) * 16u;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                r.x[mt][c] = *(const u32x4 *)((const char *)p.x + (xlane[mt] + (uint32_t)(4 * step + kbc) * 64u) + 16 * c);
+                r.x[mt][c] = TURN ? *(const u32x4 *)((const char *)p.x + (min(xfirst + (uint32_t)(16 * mt + 4 * c) * row_bytes_x, xlast) + xchunk))
+                                  : *(const u32x4 *)((const char *)p.x + (xfirst + (uint32_t)(4 * step + kbc) * 64u) + 16 * c);
     };
 
     // split RMSNorm, consuming side: wave w sums the slots of rows w, w + 8, ... and leaves
@@ -157,7 +176,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // The slots are requested here, ahead of everything else, and summed once the first
     // step's operands have been requested behind them (see the main loop): loads return in
     // order, so that wait is for the slots alone.
-    float *row_scale = (float *)(xs + kMfmaRedBytes<MT>);
+    float *row_scale = (float *)(xs + kMfmaScaleAt<MT>);
     constexpr int kScaleRows = 2 * MT;  // rows per wave
     bool scaled = false;
     [[maybe_unused]] f32x4 slot4[kScaleRows];
@@ -316,6 +335,16 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         }
         return r;
     };
+    [[maybe_unused]] auto turn_round = [&](Operands &ops) {   // to inputs 8 c .. 8 c + 7 of the lane's word
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) *(u32x4 *)(turn_in + (16 * mt + 4 * c) * kTurnRow) = ops.x[mt][c];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) ops.x[mt][c] = *(const u32x4 *)(turn_out + 16 * mt * kTurnRow + 16 * c);
+    };
     auto multiply = [&](const Operands &ops, const Table (&tab)[kTables]) {
         Table t4[4];   // per output, or (block formats) per byte of the word
 #pragma unroll
@@ -355,6 +384,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
 #pragma unroll
                         for (int j = 0; j < 4; ++j) ops.x[mt][c][j] = halves_of_bf16(ops.x[mt][c][j]);
             }
+        if constexpr (TURN) turn_round(ops);
         if (!chosen) {
             chosen = true;
             if constexpr (OWN) {
@@ -450,6 +480,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // red[wave][j = (e*MT + mt)*4 + r][lane], rows padded to 65 words so that the
     // read-out below (consecutive threads = consecutive outputs) spreads over the banks
     float *red = (float *)xs;
+    if constexpr (TURN) __syncthreads();   // (the waves' activations lie there)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
 #pragma unroll
