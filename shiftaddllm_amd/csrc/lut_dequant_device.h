@@ -182,11 +182,11 @@ __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const 
     return !(sum <= least * 2048.0f) || sum > 32768.0f || least < 0x1p-24f;
 }
 
-// The sign words of 32 inputs of one output, one per plane -> y[c]: byte i of it holds the table indices
-// of inputs 8 c + i (low nibble) and 8 c + 4 + i (high nibble).  Bits above the index are garbage, except
-// bit 3 at four planes (plane 3 itself).
+// The sign words of 32 inputs of one output, one per plane -> z: bytes 0, 1 of z[2 h + p] hold the table indices of
+// inputs 16 h + 2 p, 16 h + 2 p + 1 (low nibbles) and of the inputs 4 further on (high nibbles), bytes 2, 3 those of the
+// inputs 8 further on.  Bits above the index are garbage, except bit 3 at four planes (plane 3 itself).
 template <int NB, bool UNI>
-__device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (&y)[4])
+__device__ __forceinline__ void sign_pairs(const uint32_t (&w)[NB], uint32_t (&z)[4])
 {
     // (as one three-input bit operation, truth table (m & a) | (~m & b): the compiler takes a chain of them apart)
     auto bfi = [](uint32_t m, uint32_t a, uint32_t b) { return __builtin_amdgcn_bitop3_b32(m, a, b, 0xca); };
@@ -221,45 +221,71 @@ __device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (
             n[3] = bfi(0x33333333u, n[3], odd2);
         }
     }
-    const uint32_t z01a = __builtin_amdgcn_perm(n[1], n[0], 0x05010400u), z01b = __builtin_amdgcn_perm(n[1], n[0], 0x07030602u);
-    const uint32_t z23a = __builtin_amdgcn_perm(n[3], n[2], 0x05010400u), z23b = __builtin_amdgcn_perm(n[3], n[2], 0x07030602u);
-    y[0] = __builtin_amdgcn_perm(z23a, z01a, 0x05040100u);
-    y[1] = __builtin_amdgcn_perm(z23a, z01a, 0x07060302u);
-    y[2] = __builtin_amdgcn_perm(z23b, z01b, 0x05040100u);
-    y[3] = __builtin_amdgcn_perm(z23b, z01b, 0x07060302u);
+    z[0] = __builtin_amdgcn_perm(n[1], n[0], 0x05010400u);
+    z[1] = __builtin_amdgcn_perm(n[3], n[2], 0x05010400u);
+    z[2] = __builtin_amdgcn_perm(n[1], n[0], 0x07030602u);
+    z[3] = __builtin_amdgcn_perm(n[3], n[2], 0x07030602u);
 }
 
-// Eight weights (inputs 8 c .. 8 c + 7, in order) as a matrix operand.
+// The same in the order of one operand at a time (tables that change every 8 inputs) -> y[c]: byte i of it holds the
+// indices of inputs 8 c + i (low nibble) and 8 c + 4 + i (high nibble).
+template <int NB, bool UNI>
+__device__ __forceinline__ void sign_indices(const uint32_t (&w)[NB], uint32_t (&y)[4])
+{
+    uint32_t z[4];
+    sign_pairs<NB, UNI>(w, z);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        y[2 * h] = __builtin_amdgcn_perm(z[2 * h + 1], z[2 * h], 0x05040100u);
+        y[2 * h + 1] = __builtin_amdgcn_perm(z[2 * h + 1], z[2 * h], 0x07060302u);
+    }
+}
+
+// The four weights of the bytes' low (HALF 0) or high nibbles: the first two and the last two, packed.
+template <int NB, bool UNI, int HALF>
+__device__ __forceinline__ u32x2 pick_four(uint32_t y, const WeightTable<NB, UNI> &t)
+{
+    constexpr uint32_t kMask = NB == 1 ? 0x01010101u : NB == 2 ? 0x03030303u : 0x07070707u;
+    constexpr bool half = HALF != 0;
+    const uint32_t sel = (half ? y >> 4 : y) & kMask;
+    uint32_t h, l;
+    if constexpr (NB <= 2) {
+        h = __builtin_amdgcn_perm(t.hi[0], t.hi[0], sel);
+        l = __builtin_amdgcn_perm(t.lo[0], t.lo[0], sel);
+    } else {
+        h = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
+        l = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel);
+        if constexpr (NB == 4 && !UNI) {
+            // plane 3 positive: the other sign (h ^ (bits & mask))
+            h = __builtin_amdgcn_bitop3_b32(half ? y : y << 4, 0x80808080u, h, 0x6a);
+        } else if constexpr (NB == 4) {
+            const uint32_t top = ((half ? y >> 7 : y >> 3) & 0x01010101u);
+            const uint32_t mask = (top << 8) - top;       // bytes of 0xff where plane 3 is positive
+            const uint32_t h1 = __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel), l1 = __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel);
+            h = (h & ~mask) | (h1 & mask);
+            l = (l & ~mask) | (l1 & mask);
+        }
+    }
+    return (u32x2){__builtin_amdgcn_perm(h, l, 0x05010400u), __builtin_amdgcn_perm(h, l, 0x07030602u)};
+}
+
+// Eight weights (inputs 8 c .. 8 c + 7, in order) as a matrix operand, from sign_indices' y[c].
 template <int NB, bool UNI>
 __device__ __forceinline__ u32x4 pick_weights(uint32_t y, const WeightTable<NB, UNI> &t)
 {
-    constexpr uint32_t kMask = NB == 1 ? 0x01010101u : NB == 2 ? 0x03030303u : 0x07070707u;
-    uint32_t out[4];
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-        const uint32_t sel = (half ? y >> 4 : y) & kMask;
-        uint32_t h, l;
-        if constexpr (NB <= 2) {
-            h = __builtin_amdgcn_perm(t.hi[0], t.hi[0], sel);
-            l = __builtin_amdgcn_perm(t.lo[0], t.lo[0], sel);
-        } else {
-            h = __builtin_amdgcn_perm(t.hi[1], t.hi[0], sel);
-            l = __builtin_amdgcn_perm(t.lo[1], t.lo[0], sel);
-            if constexpr (NB == 4 && !UNI) {
-                // plane 3 positive: the other sign (h ^ (bits & mask))
-                h = __builtin_amdgcn_bitop3_b32(half ? y : y << 4, 0x80808080u, h, 0x6a);
-            } else if constexpr (NB == 4) {
-                const uint32_t top = ((half ? y >> 7 : y >> 3) & 0x01010101u);
-                const uint32_t mask = (top << 8) - top;       // bytes of 0xff where plane 3 is positive
-                const uint32_t h1 = __builtin_amdgcn_perm(t.hi[3], t.hi[2], sel), l1 = __builtin_amdgcn_perm(t.lo[3], t.lo[2], sel);
-                h = (h & ~mask) | (h1 & mask);
-                l = (l & ~mask) | (l1 & mask);
-            }
-        }
-        out[2 * half] = __builtin_amdgcn_perm(h, l, 0x05010400u);
-        out[2 * half + 1] = __builtin_amdgcn_perm(h, l, 0x07030602u);
-    }
-    return (u32x4){out[0], out[1], out[2], out[3]};
+    const u32x2 a = pick_four<NB, UNI, 0>(y, t), b = pick_four<NB, UNI, 1>(y, t);
+    return (u32x4){a.x, a.y, b.x, b.y};
+}
+
+// Sixteen weights of one table as two operands, from sign_pairs' z[2 h], z[2 h + 1]: four instructions fewer per
+// output and sign word than through sign_indices.
+template <int NB, bool UNI>
+__device__ __forceinline__ void pick_pair(uint32_t z0, uint32_t z1, const WeightTable<NB, UNI> &t, u32x4 (&out)[2])
+{
+    const u32x2 a = pick_four<NB, UNI, 0>(z0, t), b = pick_four<NB, UNI, 0>(z1, t);
+    const u32x2 c = pick_four<NB, UNI, 1>(z0, t), d = pick_four<NB, UNI, 1>(z1, t);
+    out[0] = (u32x4){a.x, b.x, c.x, d.x};
+    out[1] = (u32x4){a.y, b.y, c.y, d.y};
 }
 
 // ---- block formats: one multiplier, as it lies in memory and decoded --------------------------------------

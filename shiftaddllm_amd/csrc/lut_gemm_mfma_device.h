@@ -364,13 +364,29 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
                 w[b] = ops.w[b][e];
                 asm volatile("" : "+v"(w[b]));   // (opaque: or the indices are kept for a second piece)
             }
-            sign_indices<NB, UNI>(w, y);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const f16x8 a = __builtin_bit_cast(f16x8, pick_weights<NB, UNI>(y[c], t4[FMT == kWeightBlock ? c : e]));
+            auto product = [&](int c, const u32x4 &a) {
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[e][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, __builtin_bit_cast(f16x8, ops.x[mt][c]), acc[e][mt], 0, 0, 0);
+                    acc[e][mt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, ops.x[mt][c]),
+                                                                        acc[e][mt], 0, 0, 0);
+            };
+            // Two operands at a time save four instructions, but hold four registers more: 16-row tiles of four planes
+            // and the grouped kernel, which have none left, spill more (8192x8192x4 at 4 rows 12.2 -> 12.6 us, decoding
+            // a token for eight sequences 2391 -> 2470); 32-row tiles gain (8192x28672x4 42.4 -> 41.6, 11008x4096x3 14.2 ->
+            // 13.7), three planes a little (4096x4096x3 at 8 rows 6.96 -> 6.81).
+            if constexpr (FMT == kWeightBlock || (MT == 1 && (NB == 4 || EXTRA))) {
+                sign_indices<NB, UNI>(w, y);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) product(c, pick_weights<NB, UNI>(y[c], t4[FMT == kWeightBlock ? c : e]));
+            } else {
+                sign_pairs<NB, UNI>(w, y);
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    u32x4 a[2];
+                    pick_pair<NB, UNI>(y[2 * h], y[2 * h + 1], t4[e], a);
+                    product(2 * h, a[0]);
+                    product(2 * h + 1, a[1]);
+                }
             }
         }
     };
