@@ -107,6 +107,15 @@ __device__ __forceinline__ int fast_div(int n, const Divisor &d)
     return (int)__umulhi((uint32_t)(2 * n) >> d.shift, d.magic);
 }
 
+// Division of any n by d with reciprocal_of(d) = floor(2^32 / d): the multiply-high is at most one below the quotient.
+inline uint32_t reciprocal_of(int d) { return d == 1 ? 0xffffffffu : (uint32_t)((1ull << 32) / (uint32_t)d); }
+
+__device__ __forceinline__ int quotient(int n, int d, uint32_t reciprocal)
+{
+    const int q = (int)__umulhi((uint32_t)n, reciprocal);
+    return q + (n - q * d >= d ? 1 : 0);
+}
+
 // Field order: a kernel fetches its arguments a cache line at a time, on demand, and
 // each line touched for the first time before the sign words are requested is a round
 // trip on the start-up path.  What the kernels need to issue their first loads comes
@@ -149,8 +158,16 @@ struct Problem {
                            // one bias row for all of them: stride 0)
     __half *out;
     unsigned long long *accum;  // [M][N] fixed-point words, zero between launches
-    Divisor by_items;        // item / items_per_wg
-    Divisor by_short_items;  // item / short_items
+    union {
+        struct {
+            Divisor by_items;        // look-up kernel: item / items_per_wg
+            Divisor by_short_items;  // item / short_items
+        };
+        struct {
+            uint32_t tiles_reciprocal;    // matrix-core kernel: reciprocal_of(n_tiles)
+            uint32_t ksplit_reciprocal;   // reciprocal_of(ksplit)
+        };
+    };
     // Matrix-core kernel: K-steps per K-slice and slices per tile.
     int sets_per_split;
     int ksplit;

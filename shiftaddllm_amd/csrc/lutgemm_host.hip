@@ -394,6 +394,8 @@ void plan_mfma(Problem &p, int mt, long want)
     p.sets_per_split = (p.sets_per_split + kMfmaWaves - 1) / kMfmaWaves * kMfmaWaves;  // whole rounds
     p.ksplit = (p.nsets + p.sets_per_split - 1) / p.sets_per_split;
     p.n_blocks = p.n_tiles * p.ksplit * p.mchunks;
+    p.tiles_reciprocal = reciprocal_of(p.n_tiles);
+    p.ksplit_reciprocal = reciprocal_of(p.ksplit);
 }
 
 // LUTGEMM_OPTION_MFMA_BLOCKS: workgroups a matrix-core launch aims for instead of the rules below.
