@@ -68,14 +68,6 @@ struct MfmaOperands {
     uint32_t s[kScales];
 };
 
-// The arguments' cache lines, asked for together: each is a round trip of its own where it is first needed otherwise.
-// (With the index divided by prepared reciprocals as well, decoding a token for eight sequences, 128 launches of this
-// kernel, 2391 -> 2334 us; 8192x28672x4 at 32 rows, two rounds of workgroups, 41.8 -> 40.2; 4096x4096x3 at 16 7.25 -> 6.95.)
-__device__ __forceinline__ void touch_arguments(const Problem &p)
-{
-    asm volatile("" :: "s"(p.N), "s"(p.n_blocks), "s"(p.ksplit), "s"(p.norm_eps), "s"(p.out_type));
-}
-
 // xs: kMfmaLdsBytes<MT> bytes of LDS for the final reduction (and, behind them, the reciprocal RMS of the
 // tile's rows).
 // OWN: every lane forms its own four tables (per-column alphas with groups that are no multiple of 128

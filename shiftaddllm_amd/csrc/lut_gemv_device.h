@@ -1380,6 +1380,7 @@ lut_gemv_group_kernel(const Group g)
     // (through the constant address space, which the kernel arguments live in: the fields are
     // then scalar loads that may be repeated at will instead of values to keep in registers)
     const Problem &p = *(const Problem *)((const __attribute__((address_space(4))) Problem *)&g.p[0] + blockIdx.y);
+    touch_arguments(p);
     if ((int)blockIdx.x >= p.n_blocks) return;
     auto run = [&](auto planes) {
         constexpr int NB = decltype(planes)::value;

@@ -200,6 +200,16 @@ struct Problem {
 static_assert(offsetof(Problem, by_group_words) == 64 && offsetof(Problem, gate) == 128 && offsetof(Problem, norm_eps) == 192,
               "Problem: fields are grouped by cache line");
 
+// The arguments' cache lines, asked for together: each is a round trip of its own where it is first needed otherwise.
+// Matrix-core kernel, with the index divided by prepared reciprocals as well: decoding a token for eight sequences, 128
+// launches, 2391 -> 2334 us; 8192x28672x4 at 32 rows, two rounds of workgroups, 41.8 -> 40.2; 4096x4096x3 at 16 7.25 ->
+// 6.95.  Grouped look-up kernel: a token for one sequence, 64 such launches, 1437 -> 1400 us.  The lone look-up
+// kernels ask for theirs in two batches by themselves and gain nothing.
+__device__ __forceinline__ void touch_arguments(const Problem &p)
+{
+    asm volatile("" :: "s"(p.N), "s"(p.n_blocks), "s"(p.ksplit), "s"(p.norm_eps), "s"(p.out_type));
+}
+
 // One problem of the GEMM kernel for many activation rows (lut_gemm_tile_device.h).
 struct TileProblem {
     const uint32_t *W;
