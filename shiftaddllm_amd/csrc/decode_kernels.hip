@@ -17,6 +17,7 @@
 #include <type_traits>
 
 #include "lutgemm_gfx950.h"
+#include "lutgemm_common.h"
 #include "lutgemm_internal.h"
 
 namespace {
@@ -239,6 +240,12 @@ attention_kernel(const __half *__restrict__ q, const __half *__restrict__ k, con
     }
 }
 
+// The query heads of a kv head and how workgroups are given to them: 1 << spread (sequence, kv head) pairs side by side.
+struct HeadLayout {
+    int rep, KV, spread;
+    uint32_t rep_reciprocal, KV_reciprocal;
+};
+
 // The same for head_dim HD in {64, 128}.  Bound by the stream of cached keys and values, and with a short
 // context by the memory round trips in front of it.
 //
@@ -256,12 +263,15 @@ attention_kernel(const __half *__restrict__ q, const __half *__restrict__ k, con
 // Eight sequences of 32 heads at position 700 (92 MB): 23.1 -> 20.0 us, of which 3.3 are what position 0 takes;
 // one sequence at position 255: 7.1 -> 6.4.  Before, whole blocks were fetched and then worked on, and the rotated
 // query went through LDS and a barrier.
+// The start is a chain of round trips: the arguments (asked for at once), the position, the first rows.  Off it since: the
+// software divisions that found a workgroup's head, and, in wave 0, the new position's rows being asked for behind the
+// earlier ones' (eight sequences at position 700 17.3 -> 16.6 us on the device, a token for one sequence 1402 -> 1394).
 template <int HD, int T>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4)))
 attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, const __half *__restrict__ v,
                     const __half *__restrict__ cos_t, const __half *__restrict__ sin_t,
                     __half *__restrict__ k_cache, __half *__restrict__ v_cache,
-                    const long long *__restrict__ pos_ptr, __half *__restrict__ out, int H, int KV, int max_pos)
+                    const long long *__restrict__ pos_ptr, __half *__restrict__ out, const HeadLayout layout, int max_pos)
 {
     constexpr int kChunks = HD / 8;             // 16-byte chunks of a row
     constexpr int kPosGroups = T / kChunks;     // rows that the workgroup's threads cover side by side
@@ -271,22 +281,27 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     __shared__ float part[kWaves][HD], wave_mx[kWaves], wave_total[kWaves];
 
     const int tid = threadIdx.x;
-    const int rep = H / KV;
-    int group = blockIdx.x / rep, member = blockIdx.x % rep;   // (sequence, kv head) and the query head within it
-    if (rep > 1 && (gridDim.x / rep) % 8 == 0) {
-        const int at = blockIdx.x >> 3;
-        group = at / rep * 8 + (blockIdx.x & 7);
-        member = at % rep;
-    }
-    const int b = group / KV, kvh = group % KV, h = kvh * rep + member;
+    const int rep = layout.rep, KV = layout.KV, H = KV * rep;
+    int pos = (int)*pos_ptr;
+    asm volatile("" :: "s"(layout.spread), "s"(q), "s"(cos_t), "s"(out));   // (all of the arguments' cache lines at once)
+    const int at = blockIdx.x >> layout.spread;
+    int group = lutgemm::quotient(at, rep, layout.rep_reciprocal);      // (sequence, kv head) and the query head within it
+    const int member = at - group * rep;
+    group = (group << layout.spread) + (blockIdx.x & ((1 << layout.spread) - 1));
+    const int b = lutgemm::quotient(group, KV, layout.KV_reciprocal), kvh = group - b * KV, h = kvh * rep + member;
     const int jg = tid / kChunks, ch = tid % kChunks;
     const int other = ch < kChunks / 2 ? ch + kChunks / 2 : ch - kChunks / 2;   // the chunk ch is rotated with
     const u32x4 *qh = (const u32x4 *)(q + ((size_t)b * H + h) * HD);
     const u32x4 *kh = (const u32x4 *)(k + ((size_t)b * KV + kvh) * HD);
     const u32x4 *vh = (const u32x4 *)(v + ((size_t)b * KV + kvh) * HD);
     const u32x4 q_own = qh[ch], q_other = qh[other];
-
-    int pos = (int)*pos_ptr;
+    // (the new position's rows, ahead of the earlier ones': wave 0 needs them first)
+    u32x4 k_own = {}, k_other = {}, v_own = {};
+    if (jg == 0) {
+        k_own = kh[ch];
+        k_other = kh[other];
+        v_own = vh[ch];
+    }
     pos = min(max(pos, 0), max_pos - 1);
     const size_t cache_row0 = ((size_t)b * KV + kvh) * max_pos;
     const u32x4 cos_c = ((const u32x4 *)(cos_t + (size_t)pos * HD))[ch], sin_c = ((const u32x4 *)(sin_t + (size_t)pos * HD))[ch];
@@ -331,8 +346,7 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     if (jg == 0) {
         // the new position: one row of lanes takes it, and one head of the kv head's appends it
         float kr[8], vv[8];
-        rotate(kh[ch], kh[other], kr);
-        const u32x4 v_own = vh[ch];
+        rotate(k_own, k_other, kr);
         unpack8(v_own, vv);
         float dot = 0.0f;
 #pragma unroll
@@ -483,11 +497,14 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
     if (!aligned16(k_cache) || !aligned16(v_cache)) return LUTGEMM_EALIGN;
     // (16-byte loads of every operand: others go to the general kernel)
     if ((head_dim == 64 || head_dim == 128) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
+        const int rep = heads / kv_heads;
+        const HeadLayout layout{rep, kv_heads, rep > 1 && (long)batch * kv_heads % 8 == 0 ? 3 : 0, lutgemm::reciprocal_of(rep),
+                                lutgemm::reciprocal_of(kv_heads)};
         auto launch = [&](auto kernel, int threads) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)(batch * heads)), dim3(threads), 0, (hipStream_t)stream,
                                (const __half *)q, (const __half *)k, (const __half *)v, (const __half *)cos_table,
                                (const __half *)sin_table, (__half *)k_cache, (__half *)v_cache,
-                               (const long long *)position, (__half *)out, heads, kv_heads, max_positions);
+                               (const long long *)position, (__half *)out, layout, max_positions);
             return launch_status();
         };
         // With fewer workgroups than CUs eight waves each instead of four: 32 heads at position 255 6.4 us against
