@@ -483,6 +483,17 @@ typedef struct lutgemm_fused_problem {
 int lutgemm_gemv_rowwise_f16_fused(int count, const lutgemm_fused_problem *problems, void *stream);
 
 /*
+ * The first half of a gated MLP: act = fp16(fp16(silu(gate)) * up), [M][N], where gate_up[0] and
+ * gate_up[1] describe the two products (same M and N, M * N a multiple of 8, overwrite = 1, no
+ * next_input / sumsq_out; otherwise as for lutgemm_gemv_rowwise_f16_fused).  Where the matrix-core
+ * kernel takes both, one launch forms act and leaves the two out_f16 alone (it needs up to
+ * 2 * M * N + M * N / 2 workspace words); otherwise, and where the stream has no memory for
+ * that, they hold the sums that lutgemm_decode_silu_mul_f16 then reads.  The values of act are the
+ * same either way.  act and the outputs are 16-byte aligned and overlap nothing else of the call.
+ */
+int lutgemm_gemv_rowwise_f16_gated(const lutgemm_fused_problem *gate_up, void *act_f16, void *stream);
+
+/*
  * Row-wise GEMVs that DEPEND on each other in ONE launch (no counterpart in the
  * reference, which launches every linear layer separately and waits for each).
  * Of a GEMV's bytes all but the activation row are independent of the GEMV in

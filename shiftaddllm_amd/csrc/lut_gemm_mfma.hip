@@ -78,4 +78,14 @@ hipError_t launch_mfma_group(const Group &g, int mt, int blocks, hipStream_t str
     return hipGetLastError();
 }
 
+hipError_t launch_mfma_gated(const GatedProblems &g, int mt, int blocks, hipStream_t stream)
+{
+    const dim3 grid((unsigned)blocks, 2u), block(kMfmaThreads);
+    if (mt == 2)
+        hipLaunchKernelGGL((lut_gemm_mfma_gated_kernel<2>), grid, block, 0, stream, g);
+    else
+        hipLaunchKernelGGL((lut_gemm_mfma_gated_kernel<1>), grid, block, 0, stream, g);
+    return hipGetLastError();
+}
+
 }  // namespace lutgemm

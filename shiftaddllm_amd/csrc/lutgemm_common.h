@@ -235,6 +235,17 @@ struct TileProblem {
 // (4096x4096x3, 512 rows in 4 slices 42.6 -> 34.2 us, 1024 rows in 2 slices 60.0 -> 51.6).
 __host__ __device__ constexpr size_t tile_slice_stride(int M, int N) { return (size_t)M * N + 17 * 64; }
 
+// The product of a gate and an up projection, act = fp16(fp16(silu(gate)) * up), formed by the launch of both.
+struct GatedPair {
+    uint32_t *words;   // [M][N]: the first sum of an output that is complete, fp16 bits | 1 << 16; zero between launches
+    __half *act;       // [M][N]
+};
+
+struct GatedProblems {
+    Problem p[2];
+    GatedPair pair;
+};
+
 struct Group {
     int count;
     Problem p[kMaxGroup];

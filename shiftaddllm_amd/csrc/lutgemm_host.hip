@@ -489,9 +489,15 @@ int run_mfma(Problem &p, const Accum &acc)
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
+// Where the product of a gate and an up projection goes, and whether it went there.
+struct Gated {
+    __half *out;
+    bool done;
+};
+
 // All problems of a group on the matrix-core kernel in one launch (they share the
 // row-tile height: all M <= 16 or all M > 16).
-int run_mfma_group(Group &g, const Accum &acc)
+int run_mfma_group(Group &g, const Accum &acc, Gated *gated)
 {
     const int mt = g.p[0].M > 16 ? 2 : 1;
     size_t words = 0;
@@ -505,15 +511,29 @@ int run_mfma_group(Group &g, const Accum &acc)
         if (p.n_blocks > begin) begin = p.n_blocks;  // grid.x: the largest problem's workgroups
         any_split = any_split || p.ksplit > 1;
     }
-    if (any_split) {
-        unsigned long long *base = nullptr;
-        int rc = accum_words(acc, words, &base);
+    // (behind the problems' words, where the launch forms a product, one 32-bit word per output)
+    const size_t pair_words = gated ? ((size_t)g.p[0].M * g.p[0].N + 1) / 2 : 0;
+    unsigned long long *base = nullptr;
+    if (any_split || gated) {
+        int rc = accum_words(acc, words + pair_words, &base);
+        if (rc != LUTGEMM_OK && gated) {   // (no memory for them: the sums alone)
+            gated = nullptr;
+            rc = any_split ? accum_words(acc, words, &base) : LUTGEMM_OK;
+        }
         if (rc != LUTGEMM_OK) return rc;
+    }
+    if (any_split) {
         size_t off = 0;
         for (int i = 0; i < g.count; ++i) {
             g.p[i].accum = base + off;
             off += (size_t)g.p[i].M * g.p[i].N;
         }
+    }
+    if (gated) {
+        const GatedProblems pair{{g.p[0], g.p[1]}, {(uint32_t *)(base + words), gated->out}};
+        gated->done = true;
+        const hipError_t e = launch_mfma_gated(pair, mt, begin, acc.stream);
+        return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
     }
     const hipError_t e = g.count == 1 ? launch_mfma_fused(g.p[0], mt, acc.stream) : launch_mfma_group(g, mt, begin, acc.stream);
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
@@ -886,7 +906,7 @@ int share_workgroups(Problem *const *ps, int count, long budget, int *most, bool
 // Up to kMaxGroup row-wise problems in one launch of the look-up kernel.  Problems
 // with enough rows for the matrix-core kernel (and no fused transform) are launched
 // on that path instead.
-int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc)
+int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc, Gated *gated = nullptr)
 {
     Group g{};
     g.count = count;
@@ -941,7 +961,7 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
             const char *lo, *hi;
             bool written;
         };
-        Span spans[6 * kMaxGroup];
+        Span spans[6 * kMaxGroup + 1];
         int n = 0;
         auto add = [&](const void *ptr, size_t bytes, bool written) {
             if (ptr) spans[n++] = Span{(const char *)ptr, (const char *)ptr + bytes, written};
@@ -956,6 +976,7 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
             add(p.gate, mk * 2, false);
             add(p.sumsq_in, (size_t)p.M * p.sumsq_slots * 4, false);
         }
+        if (gated) add(gated->out, (size_t)g.p[0].M * g.p[0].N * 2, true);
         for (int i = 0; i < n; ++i)
             for (int j = i + 1; j < n; ++j)
                 if ((spans[i].written || spans[j].written) && spans[i].lo < spans[j].hi && spans[j].lo < spans[i].hi)
@@ -967,7 +988,7 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
     // would redo the transform of all rows (measured slower than a separate kernel).
     bool same_height = true;
     for (int i = 1; i < count; ++i) same_height = same_height && ((g.p[i].M > 16) == (g.p[0].M > 16));
-    if (all_mfma && xform == kXNone && same_height && (count > 1 || !plain)) return run_mfma_group(g, acc);
+    if (all_mfma && xform == kXNone && same_height && (count > 1 || !plain)) return run_mfma_group(g, acc, gated);
     if (plain && all_mfma) {
         for (int i = 0; i < count; ++i) {
             int rc = run_mfma(g.p[i], acc);
@@ -1361,6 +1382,20 @@ int lutgemm_gemv_rowwise_f16_fused(int count, const lutgemm_fused_problem *probl
 {
     if (!problems || count < 1 || count > kMaxGroup) return LUTGEMM_EINVAL;
     return run_group(count, problems, Accum{(hipStream_t)stream_v});
+}
+
+int lutgemm_gemv_rowwise_f16_gated(const lutgemm_fused_problem *gate_up, void *act_f16, void *stream)
+{
+    if (!gate_up || !act_f16) return LUTGEMM_EINVAL;
+    const lutgemm_fused_problem &gate = gate_up[0], &up = gate_up[1];
+    if (gate.M != up.M || gate.N != up.N || (long long)gate.M * gate.N % 8 != 0) return LUTGEMM_EINVAL;
+    for (const lutgemm_fused_problem *p : {&gate, &up})
+        if (p->overwrite != 1 || p->next_input_f16 || p->sumsq_out_f32) return LUTGEMM_EINVAL;
+    if (!aligned(act_f16, 16) || !aligned(gate.out_f16, 16) || !aligned(up.out_f16, 16)) return LUTGEMM_EALIGN;
+    Gated gated{(__half *)act_f16, false};
+    const int rc = run_group(2, gate_up, Accum{(hipStream_t)stream}, &gated);
+    if (rc != LUTGEMM_OK || gated.done) return rc;
+    return lutgemm_decode_silu_mul_f16(gate.out_f16, up.out_f16, act_f16, (size_t)gate.M * gate.N, stream);
 }
 
 int lutgemm_gemv_rowwise_f16_chain(int count, const lutgemm_chain_problem *problems,

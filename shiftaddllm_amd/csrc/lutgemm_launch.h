@@ -27,6 +27,7 @@ hipError_t chain_resident_workgroups(int *count);
 hipError_t launch_mfma(const Problem &p, int mt, hipStream_t stream);
 hipError_t launch_mfma_fused(const Problem &p, int mt, hipStream_t stream);  // one problem with fused extras
 hipError_t launch_mfma_group(const Group &g, int mt, int blocks, hipStream_t stream);
+hipError_t launch_mfma_gated(const GatedProblems &g, int mt, int blocks, hipStream_t stream);  // gate, up and their product
 // block-scaled matrix-core kernel (alphas are powers of two): splits p.x into `split` (mx_split_bytes:
 // three pieces per value, a row of zeros, a scale word per block of 32), then runs the problem; grid =
 // p.n_blocks, row chunks of mx_chunk_rows(p.M) rows

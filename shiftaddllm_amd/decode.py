@@ -18,7 +18,7 @@ HIP graph; q/k/v and gate/up can be issued as one fused launch each.
 Two implementations of everything between the linears exist: glue="hip" (the
 default) runs this library's fused kernels -- RMSNorm, rotary + KV append +
 attention, SiLU*up -- and lets o_proj / down_proj accumulate straight into the
-residual stream, eight launches per block; glue="torch" spells the same step in
+residual stream, eight launches per block (five with grouped launches); glue="torch" spells the same step in
 framework operations and is what the parity test's dense model is built from.
 """
 from __future__ import annotations
@@ -221,11 +221,12 @@ class LutDecoder(nn.Module):
                 raise RuntimeError(lib.lutgemm_strerror(rc).decode())
 
     def _fused_gemv(self, lins, x, outs, sp, norm=None, gate=None, overwrite=False, next_norm=None, next_in=None,
-                    sumsq_out=None, sumsq_in=None):
+                    sumsq_out=None, sumsq_in=None, act=None):
         """One launch: outs[i] (+)= lins[i](t(x)), t = RMSNorm with weight `norm`, or
         silu(gate) * x, or identity.  next_norm / next_in / sumsq_out: the outputs complete
         a residual row whose norm-weighted copy and sums of squares are left for the next
-        GEMV; sumsq_in: x is such a copy and the sums are scaled by its reciprocal RMS."""
+        GEMV; sumsq_in: x is such a copy and the sums are scaled by its reciprocal RMS.
+        act: lins are a gate and an up projection, act = silu(gate) * up (outs are scratch)."""
         lib, B = native.cabi(), x.shape[0]
         ptr = lambda t: t.data_ptr() if t is not None else None
         arr = (native.FusedProblem * len(lins))()
@@ -234,7 +235,8 @@ class LutDecoder(nn.Module):
                                          l.N, l.K, l.wbit, l.num_groups, B, int(overwrite), ptr(norm), ptr(gate),
                                          self.cfg.rms_eps, ptr(next_norm), ptr(next_in), ptr(sumsq_out),
                                          ptr(sumsq_in), sumsq_in.shape[-1] if sumsq_in is not None else 0)
-        rc = lib.lutgemm_gemv_rowwise_f16_fused(len(lins), arr, sp)
+        rc = lib.lutgemm_gemv_rowwise_f16_gated(arr, act.data_ptr(), sp) if act is not None else \
+            lib.lutgemm_gemv_rowwise_f16_fused(len(lins), arr, sp)
         if rc:
             raise RuntimeError(lib.lutgemm_strerror(rc).decode())
 
@@ -305,10 +307,10 @@ class LutDecoder(nn.Module):
         q, k, v = self.qkv[:nq], self.qkv[nq:nq + nkv], self.qkv[nq + nkv:]
         g, u = self.gate_up[:B * I].view(B, I), self.gate_up[B * I:].view(B, I)
         x, h = self.x_res, self.h_norm
-        # With grouped launches on, q,k,v and gate,up overwrite their outputs and, with one
-        # or two rows (look-up kernel), SiLU*up rides inside the down_proj kernel: seven
-        # launches per block, eight with more rows.  Without grouped launches the glue
-        # kernels also clear the accumulate-into outputs.
+        # With grouped launches on, q,k,v and gate,up overwrite their outputs and SiLU*up costs no
+        # launch: with one or two rows (look-up kernel) it rides inside the down_proj kernel, with more
+        # the gate,up launch forms it.  Without grouped launches the glue kernels also clear
+        # the accumulate-into outputs.
         fold = self.fuse
         fold_gate = fold and B <= 2                         # input transforms live in the look-up kernel
         fold_norm = fold_gate and self.fold_norm
@@ -335,18 +337,18 @@ class LutDecoder(nn.Module):
                                                    self.sin.data_ptr(), self.k_cache[li].data_ptr(),
                                                    self.v_cache[li].data_ptr(), self.pos.data_ptr(),
                                                    self.att.data_ptr(), B, H, KV, hd, cfg.max_positions, sp))
-            gate_up = [blk.gate_proj, blk.up_proj]
+            gate_up, act = [blk.gate_proj, blk.up_proj], None if fold_gate else self.act
             if split:                                                   # x += o_proj(att); h = x * post_norm
                 self._fused_gemv([blk.o_proj], self.att, [x], sp, next_norm=blk.post_norm, next_in=h,
                                  sumsq_out=self.sumsq[2 * li])
-                self._fused_gemv(gate_up, h, [g, u], sp, overwrite=True, sumsq_in=self.sumsq[2 * li])
+                self._fused_gemv(gate_up, h, [g, u], sp, overwrite=True, sumsq_in=self.sumsq[2 * li], act=act)
             else:
                 self._gemv_into([blk.o_proj], self.att, [x], sp)        # x += o_proj(att)
                 if fold_norm:
                     self._fused_gemv(gate_up, x, [g, u], sp, norm=blk.post_norm, overwrite=True)
                 elif fold:
                     rmsnorm(blk.post_norm)
-                    self._fused_gemv(gate_up, h, [g, u], sp, overwrite=True)
+                    self._fused_gemv(gate_up, h, [g, u], sp, overwrite=True, act=act)
                 else:
                     rmsnorm(blk.post_norm, self.gate_up)
                     self._gemv_into(gate_up, h, [g, u], sp)
@@ -356,7 +358,8 @@ class LutDecoder(nn.Module):
             if fold_gate:
                 self._fused_gemv([blk.down_proj], u, [x], sp, gate=g, **nxt)
             else:
-                check(lib.lutgemm_decode_silu_mul_f16(g.data_ptr(), u.data_ptr(), self.act.data_ptr(), B * I, sp))
+                if not fold:
+                    check(lib.lutgemm_decode_silu_mul_f16(g.data_ptr(), u.data_ptr(), self.act.data_ptr(), B * I, sp))
                 if nxt:
                     self._fused_gemv([blk.down_proj], self.act, [x], sp, **nxt)
                 else:

@@ -53,6 +53,7 @@ C_ABI_SYMBOLS = (
     "lutgemm_decode_rmsnorm_f16",
     "lutgemm_decode_attention_f16",
     "lutgemm_decode_silu_mul_f16",
+    "lutgemm_gemv_rowwise_f16_gated",
 )
 
 
@@ -208,6 +209,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.lutgemm_decode_attention_f16.restype = ci
     lib.lutgemm_decode_silu_mul_f16.argtypes = [vp, vp, vp, sz, vp]
     lib.lutgemm_decode_silu_mul_f16.restype = ci
+    lib.lutgemm_gemv_rowwise_f16_gated.argtypes = [ctypes.POINTER(FusedProblem), vp, vp]
+    lib.lutgemm_gemv_rowwise_f16_gated.restype = ci
     lib.lutgemm_set_timestamp_buffer.argtypes = [vp, sz]
     lib.lutgemm_set_timestamp_buffer.restype = ci
     return lib
