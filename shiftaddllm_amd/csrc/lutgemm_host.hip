@@ -407,9 +407,9 @@ int mfma_blocks_override()
 // K-slices per tile for the problems of one launch (all get the same number, each up to
 // its own limit).
 //   32-row tile: as many as reach one workgroup per CU (its register count allows no second one).  Measured at 32 rows (us, slices -> time):
-//   8192x28672x4: 1 -> 79.6, 2 -> 47.7, 4 -> 55.0; 8192x8192x4: 1 -> 27.4, 2 -> 20.6, 4 -> 24.2; 5120x13824x2: 1 -> 34.5,
-//   3 -> 19.7, 4 -> 24.0; 11008x4096x3: 1 -> 15.5, 2 -> 23.0; 28672x8192x4, whose 448 tiles leave a second round a
-//   quarter empty: 1 -> 55.6, 2 -> 72.3, 4 -> 75.9.
+//   8192x28672x3: 1 -> 57.5, 2 -> 37.4, 4 -> 42.8; 8192x8192x4: 1 -> 24.1, 2 -> 19.7, 4 -> 24.0; int8 exponents 5120x13824x2: 1 -> 37.0,
+//   3 -> 21.2, 4 -> 26.5; 11008x4096x3: 1 -> 13.6, 2 -> 22.1; 28672x8192x4, whose 448 tiles leave a second round a
+//   quarter empty: 1 -> 48.3, 2 -> 63.8, 4 -> 71.4.
 //   16-row tile: the launch ends when the busiest CU does, two workgroups share a CU.  With w =
 //   ceil(workgroups / 256) workgroups on that CU and R rounds (one K-step per wave) per workgroup, the slice
 //   count that minimises
@@ -460,27 +460,86 @@ int mfma_slices(const Group &g, int mt)
     return best;
 }
 
-// 16-row tiles per workgroup of a lone problem.  Two of them form each weight once for 32 rows; a call that fits
-// the chip as single rounds of 16-row tiles, two workgroups per CU, is bound by latencies and better spread
-// (us, one against two, 32 rows: 4096x4096x3 8.9 / 10.6, 768x3072x3 6.3 / 8.7, 3072x768x3 4.8 / 6.3; 64 rows:
-// 768x3072x3 7.7 / 9.8; 11008x4096x3 at 32 rows, which does not fit, 17.5 / 15.6).  Beyond 64 rows two are taken
-// whatever the size, which the same measurements do not bear out everywhere: 768x3072x3 at 96 rows 8.0 / 9.9, at 128
-// rows 10.9 / 10.3, 2048x2048x3 at 128 rows 7.0 / 10.6, 1024x1024x3 at 256 rows 4.8 / 6.3, 1024x8192x4 at 96 rows
-// 13.4 / 13.2.
-int mfma_row_tiles(const Problem &p)
+// How a lone problem of more than 16 rows is cut up: the height of its tiles (mt 16-row tiles) and its K-slices, by
+// the estimate in us
+//     start + w * (rounds * (round + plane * nb) + wg), with several slices + cut + words * M * N * slices / 1e6,
+// where w = ceil(workgroups / 256), rounds = K-steps per wave of a slice, fitted to 1100 launches timed in graphs (17 to
+// 256 rows, 768 to 28672 inputs and outputs, 1 to 4 planes; 3 to 12 % rms).  32-row tiles form each weight once for twice the rows but
+// pay more per round and, one workgroup per CU, wait for every accumulator word; small calls are better off with twice
+// as many workgroups, large ones with few slices.  The choice is within 1 % of the best of all tried on
+// average, the former one (16-row tiles only where 64 rows at most fit the chip as single rounds, slices up to a
+// workgroup per CU for the rest) was 4 to 7 % off: us before / now 2048x2048x3 at 128 rows 10.5 / 7.3,
+// 4096x4096x3 at 64 13.2 / 11.2, 1024x1024x3 at 256 6.3 / 5.0, int8 exponents 768x3072x3 at 96 9.4 / 7.8, 4096x4096x4 at 17 13.5 / 10.9,
+// at 96 27.1 / 19.7, uniform 4096x4096x4 at 32 24.1 / 15.9, 8192x8192x4 at 64 29.3 / 27.0; of 177 calls the worst loses 4 %.
+struct MfmaCost {
+    double start, round, plane, wg, cut, words;
+};
+constexpr MfmaCost kMfmaCost[3][2] = {   // row-wise, uniform (q_bias makes every weight two pieces), block formats
+    {{3.3, 0.70, 0.35, 0.00, 1.15, 3.0}, {2.05, 0.92, 0.39, 2.10, 1.6, 4.9}},
+    {{4.6, 0.00, 1.71, 0.00, 0.85, 0.0}, {4.70, 0.43, 1.29, 1.43, 0.9, 6.5}},
+    {{2.75, 0.30, 0.84, 0.00, 1.6, 3.1}, {1.60, 0.64, 0.88, 1.67, 2.05, 5.6}},
+};
+
+struct MfmaPlan {
+    int mt, slices;
+    double us;
+    bool gemm;   // the GEMM kernel is expected to be faster than 5 us + a round's worst time per round of the widest cut
+};
+
+MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
 {
-    if (p.M <= 16) return 1;
-    const long tiles = (p.N + kMfmaTileCols - 1) / kMfmaTileCols, steps = (p.K + kMfmaStepK - 1) / kMfmaStepK;
-    return p.M <= 64 && tiles * ((p.M + 15) / 16) * ((steps + kMfmaWaves - 1) / kMfmaWaves) <= 512 ? 1 : 2;
+    const MfmaCost *const cost = kMfmaCost[p.alpha_mode == kRowF16 ? 0 : p.alpha_mode == kUniformF16 ? 1 : 2];
+    const int rounds = ((p.K + kMfmaStepK - 1) / kMfmaStepK + kMfmaWaves - 1) / kMfmaWaves;
+    const int most = !may_cut ? 1 : rounds < kMaxSlices ? rounds : kMaxSlices;
+    MfmaPlan best{0, 0, 0.0, false};
+    for (int mt = 1; mt <= 2; ++mt) {
+        const MfmaCost &c = cost[mt - 1];
+        const long tiles = (long)((p.N + kMfmaTileCols - 1) / kMfmaTileCols) * ((p.M + 16 * mt - 1) / (16 * mt));
+        for (int ks = must_cut ? 2 : 1; ks <= most; ++ks) {
+            const int own = (rounds + ks - 1) / ks;
+            if ((rounds + own - 1) / own != ks) continue;
+            const double us = c.start + (double)((tiles * ks + 255) / 256) * (own * (c.round + c.plane * p.nb) + c.wg) +
+                              (ks > 1 ? c.cut + c.words * 1e-6 * ((double)p.M * p.N * ks) : 0.0);
+            if (best.mt == 0 || us < best.us) best = MfmaPlan{mt, ks, us, false};
+        }
+    }
+    return best;
+}
+
+double gemm_estimate(const Problem &p);
+
+// The plan of a lone problem.  Which calls may take accumulator words, and so need a reservation under capture, does not
+// follow the estimate: those that a cut up to a workgroup per CU makes K-slices of, unless the GEMM kernel, which needs none,
+// is the other choice.  Up to 32 rows these calls always have slices (uncut, the few that are faster gain under 8 %:
+// 5120x2048x4 at 32 rows 8.1 / 8.7).
+MfmaPlan mfma_plan(const Problem &p)
+{
+    Group one{};
+    one.count = 1;
+    one.p[0] = p;
+    const long tiles = (p.N + kMfmaTileCols - 1) / kMfmaTileCols, rounds = ((p.K + kMfmaStepK - 1) / kMfmaStepK + kMfmaWaves - 1) / kMfmaWaves;
+    const int mt = p.M <= 16 || (p.M <= 64 && tiles * ((p.M + 15) / 16) * rounds <= 512) ? 1 : 2;
+    const int slices = mfma_slices(one, mt);
+    bool gemm = false;
+    if (p.M > 32) {
+        Problem wide = p;
+        plan_mfma(wide, 2, mt == 2 ? slices : mfma_slices(one, 2));
+        const double round = 1.6 + 0.32 * p.nb + (is_block(p.alpha_mode) ? 0.9 : 0.0);
+        gemm = gemm_estimate(p) < 5.0 + round * (double)((wide.n_blocks + 255) / 256) * (double)(wide.sets_per_split / kMfmaWaves);
+    }
+    if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm};
+    plan_mfma(one.p[0], mt, slices);
+    const bool cut = one.p[0].ksplit > 1 && !gemm;
+    MfmaPlan plan = pick_mfma(p, cut, cut && p.M <= 32);
+    plan.gemm = gemm;
+    return plan;
 }
 
 int run_mfma(Problem &p, const Accum &acc)
 {
-    const int mt = mfma_row_tiles(p);
-    Group one{};
-    one.count = 1;
-    one.p[0] = p;
-    plan_mfma(p, mt, mfma_slices(one, mt));
+    const MfmaPlan plan = mfma_plan(p);
+    const int mt = plan.mt;
+    plan_mfma(p, mt, plan.slices);
     if (p.ksplit > 1) {
         int rc = accum_words(acc, (size_t)p.M * p.N, &p.accum);
         if (rc != LUTGEMM_OK) return rc;
@@ -567,13 +626,10 @@ bool mfma_any(const Problem &p, int mode)
 int plan_single(Problem &p, int mode, int *kernel, int *mrows)
 {
     if (mfma_eligible(p, mode) || mfma_any(p, mode)) {
-        const int mt = mfma_row_tiles(p);
-        Group one{};
-        one.count = 1;
-        one.p[0] = p;
-        plan_mfma(p, mt, mfma_slices(one, mt));
+        const MfmaPlan plan = mfma_plan(p);
+        plan_mfma(p, plan.mt, plan.slices);
         *kernel = kMatrixCore;
-        *mrows = 16 * mt;
+        *mrows = 16 * plan.mt;
         return LUTGEMM_OK;
     }
     *kernel = kLookup;
@@ -736,14 +792,23 @@ double plan_tile(TileProblem &t)
     return best_cost;
 }
 
-// Whether a call takes the GEMM kernel rather than the matrix-core kernel, from what either should take (in
-// microseconds).  A round of the matrix-core kernel (32-row tiles, one K-step per wave, one workgroup per CU) takes 2.2 to
-// 3.0 with two to four planes and 0.9 more with the decoding of block formats.
-// Measured (us, matrix-core kernel / this one, * = taken): 11008x4096x3 at 48 rows 25.7 / 22.5*, 128 rows 43.1 / 29.8*; 4096x11008x2 at
-// 128 rows 29.2 / 29.1*, 200 rows 55.3 / 36.2*; int8 exponents 5120x13824x2 at 33 rows 34.2 / 26.6*, 13824x5120x2 at 64 rows
-// 40.2 / 28.7*, 768x3072x3 at 512 rows 16.7* / 26.3; 1024x28672x4 at 128 rows 28.4* / 36.8, 200 rows 44.0 / 38.3*; 2964x2208x3 in
-// groups of 96 at 200 rows 22.8* / 22.6, 512 rows 35.7 / 27.7*; uniform 4096x4096x4 at 128 rows 30.0* / 31.4, 200 rows 55.8 /
-// 40.4*; 2048x2048x3 at 512 rows 17.6* / 23.1.  Of 104 such calls none takes the slower kernel by more than its noise.
+double gemm_estimate(const Problem &p)
+{
+    TileProblem t{};
+    t.N = p.N;
+    t.M = p.M;
+    t.kwords = p.kwords;
+    return plan_tile(t);
+}
+
+// Whether a call takes the GEMM kernel rather than the matrix-core kernel: where that is expected to take less than the
+// latter's widest cut (see mfma_plan) and its best one is not 15 % faster still.  plan_tile's costs are those of two planes; for
+// that comparison they are scaled to what the planes and the format were measured to take (17 to 256 rows): 1.04 to 1.16
+// row-wise, 1.06 to 1.32 with the decoding of block formats, 1.4 to 1.8 uniform.
+// Measured (us, matrix-core kernel / this one, * = taken): 11008x4096x3 at 48 rows 24.1 / 24.1*, 128 rows 39.5 / 32.1*; 4096x11008x2 at
+// 128 rows 24.6* / 29.8, 192 rows 44.7 / 37.5*; 8192x8192x4 at 64 rows 25.1* / 29.0, 96 rows 46.0 / 38.8*; int8 exponents
+// 5120x13824x2 at 48 rows 30.5 / 28.7*, 4096x4096x4 at 96 rows 19.4* / 26.7; 1024x28672x4 at 128 rows 25.7* / 44.3; uniform
+// 4096x4096x4 at 128 rows 28.3* / 38.5.
 bool tile_wanted(const Problem &p, int mode)
 {
     const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
@@ -754,18 +819,9 @@ bool tile_wanted(const Problem &p, int mode)
     if (least > 0) return p.M >= least;
     if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
     if (p.M <= 32) return false;
-    TileProblem t{};
-    t.N = p.N;
-    t.M = p.M;
-    t.kwords = p.kwords;
-    // The matrix-core kernel with tiles of 32 rows: a round is one K-step per wave, one workgroup per CU.
-    Group one{};
-    one.count = 1;
-    one.p[0] = p;
-    plan_mfma(one.p[0], 2, mfma_slices(one, 2));
-    const double rounds = (double)((one.p[0].n_blocks + 255) / 256) * (double)(one.p[0].sets_per_split / kMfmaWaves);
-    const double round = 1.6 + 0.32 * p.nb + (is_block(mode) ? 0.9 : 0.0);
-    return plan_tile(t) < 5.0 + round * rounds;
+    const double planes = mode == kRowF16 ? 0.92 + 0.06 * p.nb : is_block(mode) ? 0.80 + 0.13 * p.nb : 1.05 + 0.19 * p.nb;
+    const MfmaPlan plan = mfma_plan(p);
+    return plan.gemm && (plan.us == 0.0 || plan.us > 0.85 * planes * gemm_estimate(p));
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)

@@ -22,6 +22,13 @@ CASES = [   # sizes that are cut for teams
 ]
 
 
+@pytest.fixture(autouse=True)
+def _gemm_kernel():
+    assert native.cabi().lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 33) == 0
+    yield
+    native.cabi().lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+
+
 @pytest.mark.parametrize("fmt,K,N,nb,M,groups,kind,slices", CASES)
 def test_teams_against_a_dense_product_and_in_turn(gpu_device, fmt, K, N, nb, M, groups, kind, slices):
     dev, lib = gpu_device, native.cabi()
