@@ -910,11 +910,13 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
 }
 
 // Share a workgroup budget between look-up problems that run side by side so that the longest
-// range of every problem takes about the same time.  An item costs a table build plus look-ups in
-// proportion to its bit planes (0.45 + 0.13 * nb us measured), whatever the problem; the problems
-// end with their slowest workgroup, so the items per workgroup of problem i are floor(T / cost_i)
-// for the smallest T whose workgroups fit the budget.  (Sharing in proportion to the sign bytes
-// gave q,k,v of 2, 4 and 3 bits 5, 3 and 4 items per workgroup: 3.6, 2.9 and 3.4 us of work.)
+// range of every problem takes about the same time.  An item costs a table build plus look-ups in proportion to its bit
+// planes: 0.10 + 0.38 * nb us where two workgroups share the CU (one row to two of gate,up adds 5.4 items to each: of 2, 3 and 4
+// bits 4.65, 6.5 and 8.7 us); the problems end with their slowest workgroup, so the items per workgroup of problem i
+// are floor(T / cost_i) for the smallest T whose workgroups fit the budget.  (With 0.45 + 0.13 * nb, a lone item's, gate,up of
+// 2 and 4 bits took 23.9 us at two rows, now 19.7, of 2 and 3 bits 20.4, now 18.4; q,k,v of 1, 4 and 3 bits went
+// from 12.5 to 14.7.  Inputs shorter than 4096 keep the lone item's: on them it depends which launches have ranges that
+// end inside a K-row, and so need accumulator words.)
 // With equal bit widths this is a share in proportion to the items, rounded down: a few
 // workgroups more than can be resident run as a second, mostly empty round, and fewer
 // workgroups with more items each are the better trade anyway (q,k,v of 4096x4096 as 3 x 64
@@ -926,10 +928,12 @@ int share_workgroups(Problem *const *ps, int count, long budget, int *most, bool
     long items[kMaxGroup];
     double cost[kMaxGroup];
     double lo = 0.0, hi = 0.0;
+    bool long_rows = true;
+    for (int i = 0; i < count; ++i) long_rows = long_rows && ps[i]->K >= 4096;
     for (int i = 0; i < count; ++i) {
         const Problem &p = *ps[i];
         items[i] = (long)((p.N + kTileCols - 1) / kTileCols) * p.nsets;
-        cost[i] = 0.45 + 0.13 * p.nb;
+        cost[i] = long_rows ? 0.10 + 0.38 * p.nb : 0.45 + 0.13 * p.nb;
         const double all = (double)items[i] * cost[i];
         if (all > hi) hi = all;
     }
@@ -968,7 +972,7 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
     g.count = count;
     size_t words = 0;
     long total_bytes = 0;
-    bool plain = true, all_mfma = true;
+    bool plain = true, all_mfma = true, mixed = false, long_rows = true;
     int xform = kXNone;
     for (int i = 0; i < count; ++i) {
         const lutgemm_fused_problem &q = problems[i];
@@ -1006,6 +1010,8 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
         xform = mine;
         plain = plain && !p.norm_w && !p.gate && !p.overwrite && !p.next_in && !p.sumsq_out && !p.sumsq_in;
         all_mfma = all_mfma && mfma_eligible(p, kRowF16);
+        mixed = mixed || p.nb != g.p[0].nb;
+        long_rows = long_rows && q.K >= 4096;
         words += (size_t)q.M * q.N;
         total_bytes += (long)q.N * (q.K / 8) * q.nb * q.M;
     }
@@ -1057,7 +1063,14 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
     int begin = 0;
     bool any_split = false;
     {
-        int rc = share_workgroups(ps, count, (long)target_blocks(total_bytes), &begin, &any_split);
+        // Two workgroups per CU also on short streams where a workgroup begins with an RMSNorm (it hides one's start behind
+        // the other's) or widths differ (finer shares): us, budget of 256 against 512, one row, 4096 inputs with RMSNorm: q,k,v of
+        // 2, 3 and 4 bits 10.7 / 8.9, of 3 bits 9.0 / 8.8, grouped heads (4096 + 2 x 1024 outputs) 7.8 / 7.2, two rows 10.9 / 7.9;
+        // without it q,k,v of 2, 3 and 4 bits 9.9 / 8.0, of 3 bits 7.65 / 8.2.  2048 inputs: 8 MB 6.3 / 6.9, two rows 9 MB
+        // 6.25 / 6.55.
+        const bool pairs = count > 1 && (xform == kXNorm || mixed) && long_rows && total_bytes >= (9l << 20) &&
+                           option(LUTGEMM_OPTION_TARGET_BLOCKS) <= 0;
+        int rc = share_workgroups(ps, count, pairs ? 512 : (long)target_blocks(total_bytes), &begin, &any_split);
         if (rc != LUTGEMM_OK) return rc;
     }
     if (any_split) {
