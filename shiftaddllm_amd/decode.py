@@ -109,7 +109,7 @@ class LutDecoder(nn.Module):
         self.chain = bool(chain) and fuse_launches and glue == "hip" and batch <= 2 and cfg.hidden <= 8192
         # One or two sequences: RMSNorm inside the q,k,v and gate,up GEMVs (every workgroup re-reads
         # the row to form its RMS and scales its finished sums; the look-up kernel only).  Measured
-        # against the split below on the 7B decoder at one sequence: 1.535 vs 1.572 ms per token.
+        # against the split below on the 7B decoder at one sequence: 1.39 vs 1.43 ms per token.
         self.fold_norm = fuse_launches and batch <= 2
         # RMSNorm split over the GEMV that completes the residual row (it leaves x * norm weight and
         # the row's sums of squares) and the GEMVs that read it (they scale their sums): no norm
