@@ -881,8 +881,8 @@ def main():
                                 "HIP kernel; batch 1: look-up kernel, RMSNorm folded into the q/k/v and gate/up "
                                 "launches, SiLU*up folded into the down_proj GEMV (5 launches per block); "
                                 "batch 8: matrix-core kernel, RMSNorm split over the GEMV that completes the "
-                                "residual row and the GEMVs that read it, SiLU*up as a HIP kernel "
-                                "(6 launches per block); embedding gather and fp16 lm_head in torch; "
+                                "residual row and the GEMVs that read it, SiLU*up formed by the gate/up launch "
+                                "(5 launches per block); embedding gather and fp16 lm_head in torch; "
                                 "batch1_chained: o_proj, gate/up, down_proj and the next block's q,k,v as ONE chained "
                                 "launch per block (activations handed over through tagged rows), 2 launches per block")
 

@@ -265,7 +265,7 @@ struct HeadLayout {
 // query went through LDS and a barrier.
 // The start is a chain of round trips: the arguments (asked for at once), the position, the first rows.  Off it since: the
 // software divisions that found a workgroup's head, and, in wave 0, the new position's rows being asked for behind the
-// earlier ones' (eight sequences at position 700 17.3 -> 16.6 us on the device, a token for one sequence 1402 -> 1394).
+// earlier ones' (eight sequences at position 700 20.3 -> 19.4 us on the device, a token for one sequence 1402 -> 1394).
 template <int HD, int T>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4)))
 attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, const __half *__restrict__ v,

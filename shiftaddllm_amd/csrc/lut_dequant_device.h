@@ -4,8 +4,8 @@
 // row tile instead of once per bit plane: W = sum_b +-alpha_b takes 2^nb values per alpha group, so a
 // lane keeps those values as a byte-wise table in registers and picks four weights at a time with
 // v_perm_b32 by the nb sign bits of each:
-//   * 13 shift / bit-field-insert instructions merge the nb sign words of 32 inputs into nibbles, 8
-//     byte permutes put the nibbles of four consecutive inputs into the bytes of one register;
+//   * 13 shift / bit-field-insert instructions merge the nb sign words of 32 inputs into nibbles, four byte
+//     permutes (eight for one operand at a time) put the nibbles of four inputs into the bytes of one register;
 //   * per four weights: mask, one v_perm_b32 for the high bytes, one for the low bytes, two that
 //     interleave them into two packed fp16 pairs.
 // About two vector instructions per weight at three planes, where expanding every plane to +-alpha
