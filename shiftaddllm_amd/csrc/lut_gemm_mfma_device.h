@@ -107,7 +107,10 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // to no row)
     constexpr bool TURN = MT > 1 && !UNI;
     const uint32_t row_bytes_x = (uint32_t)p.K * 2u, xlast = (uint32_t)(p.M - 1) * row_bytes_x;
-    const uint32_t xfirst = (uint32_t)(TURN ? m0 + kb : min(m0 + li, p.M - 1)) * row_bytes_x;
+    uint32_t xfirst[TURN ? 1 : MT];
+#pragma unroll
+    for (int mt = 0; mt < (TURN ? 1 : MT); ++mt)
+        xfirst[mt] = (uint32_t)(TURN ? m0 + kb : min(m0 + 16 * mt + li, p.M - 1)) * row_bytes_x;
     [[maybe_unused]] char *const turn_in = xs + wave * (MT * 16 * kTurnRow) + kb * kTurnRow + li * 16;
     [[maybe_unused]] const char *const turn_out = xs + wave * (MT * 16 * kTurnRow) + li * kTurnRow + kb * 64;
 
@@ -170,8 +173,8 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int c = 0; c < 4; ++c)
-                r.x[mt][c] = TURN ? *(const u32x4 *)((const char *)p.x + (min(xfirst + (uint32_t)(16 * mt + 4 * c) * row_bytes_x, xlast) + xchunk))
-                                  : *(const u32x4 *)((const char *)p.x + (xfirst + (uint32_t)(4 * step + kbc) * 64u) + 16 * c);
+                r.x[mt][c] = TURN ? *(const u32x4 *)((const char *)p.x + (min(xfirst[0] + (uint32_t)(16 * mt + 4 * c) * row_bytes_x, xlast) + xchunk))
+                                  : *(const u32x4 *)((const char *)p.x + (xfirst[TURN ? 0 : mt] + (uint32_t)(4 * step + kbc) * 64u) + 16 * c);
     };
 
     // split RMSNorm, consuming side: wave w sums the slots of rows w, w + 8, ... and leaves
