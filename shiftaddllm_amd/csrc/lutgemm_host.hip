@@ -470,7 +470,7 @@ int mfma_slices(const Group &g, int mt)
 // average, the former one (16-row tiles only where 64 rows at most fit the chip as single rounds, slices up to a
 // workgroup per CU for the rest) was 4 to 7 % off: us before / now 2048x2048x3 at 128 rows 10.5 / 7.3,
 // 4096x4096x3 at 64 13.2 / 11.2, 1024x1024x3 at 256 6.3 / 5.0, int8 exponents 768x3072x3 at 96 9.4 / 7.8, 4096x4096x4 at 17 13.5 / 10.9,
-// at 96 27.1 / 19.7, uniform 4096x4096x4 at 32 24.1 / 15.9, 8192x8192x4 at 64 29.3 / 27.0; of 177 calls the worst loses 4 %.
+// at 96 27.1 / 19.7, uniform 4096x4096x4 at 32 24.6 / 17.0, 8192x8192x4 at 64 29.3 / 27.0; of 177 calls the worst loses 4 %.
 struct MfmaCost {
     double start, round, plane, wg, cut, words;
 };
@@ -808,7 +808,7 @@ double gemm_estimate(const Problem &p)
 // Measured (us, matrix-core kernel / this one, * = taken): 11008x4096x3 at 48 rows 24.1 / 24.1*, 128 rows 39.5 / 32.1*; 4096x11008x2 at
 // 128 rows 24.6* / 29.8, 192 rows 44.7 / 37.5*; 8192x8192x4 at 64 rows 25.1* / 29.0, 96 rows 46.0 / 38.8*; int8 exponents
 // 5120x13824x2 at 48 rows 30.5 / 28.7*, 4096x4096x4 at 96 rows 19.4* / 26.7; 1024x28672x4 at 128 rows 25.7* / 44.3; uniform
-// 4096x4096x4 at 128 rows 28.3* / 38.5.
+// 4096x4096x4 at 128 rows 29.5* / 37.8.
 bool tile_wanted(const Problem &p, int mode)
 {
     const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
