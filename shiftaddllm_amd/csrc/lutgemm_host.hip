@@ -483,7 +483,7 @@ constexpr MfmaCost kMfmaCost[3][2] = {   // row-wise, uniform (q_bias makes ever
 struct MfmaPlan {
     int mt, slices;
     double us;
-    bool gemm;   // the GEMM kernel is expected to be faster than 5 us + a round's worst time per round of the widest cut
+    bool gemm;   // the GEMM kernel is the other choice: faster than 5 us + a round's worst time per round of the widest cut, or never_cut
 };
 
 MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
@@ -508,10 +508,35 @@ MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
 
 double gemm_estimate(const Problem &p);
 
-// The plan of a lone problem.  Which calls may take accumulator words, and so need a reservation under capture, does not
-// follow the estimate: those that a cut up to a workgroup per CU makes K-slices of, unless the GEMM kernel, which needs none,
-// is the other choice.  Up to 32 rows these calls always have slices (uncut, the few that are faster gain under 8 %:
-// 5120x2048x4 at 32 rows 8.1 / 8.7).
+// Whether a call of more than 32 rows that a cut up to a workgroup per CU makes K-slices of takes none: callers that
+// reserve nothing before a capture rely on which calls need accumulator words, so this line is fixed in the sizes and follows neither
+// the costs above nor those of plan_tile.  It was drawn where the GEMM kernel, which needs none, was the faster choice:
+// slices of four waves and steps of 1.2 us (128 rows) or 0.9 (64) alone on a CU, 2.1 or 1.6 beside another, against rounds of 3 us.
+bool never_cut(const Problem &p)
+{
+    const int rows = p.M <= 64 ? 64 : 128;
+    const long tiles = (long)((p.N + 255) / 256) * ((p.M + rows - 1) / rows), all = (p.kwords + 3) / 4 * 2;
+    const double alone = rows == 128 ? 1.2 : 0.9, beside = rows == 128 ? 2.1 : 1.6;
+    double best = 0.0;
+    for (int ks = 1; ks <= kTileMaxSlices && (ks == 1 || 2 * ks <= all); ++ks) {
+        const long steps = ((all + ks - 1) / ks + 1) & ~1l, wgs = tiles * ks, rounds = wgs / 512, rest = wgs - rounds * 512;
+        const size_t sums = ks > 1 ? (size_t)ks * p.M * p.N * 4 : 0;
+        if ((all + steps - 1) / steps != ks) continue;
+        if (ks > 1 && (wgs > 512 || sums > kTileSumBytes)) break;
+        double us = (double)rounds * (steps * beside + 5.0) + (sums ? 4.0 + 0.5e-6 * (double)sums : 0.0);
+        if (rest > 0) us += steps * (rest > 256 ? beside : alone) + 5.0;
+        if (ks == 1 || us < best * 0.99) best = us;
+    }
+    const double rounds = (double)((p.N + 63) / 64) * (double)((p.M + 31) / 32) * (double)((p.K + 1023) / 1024);
+    return best < 5.0 + 3.0 * rounds / 256.0;
+}
+
+double gemm_estimate(const Problem &p);
+
+// The plan of a lone problem.  Which calls take accumulator words, and so need a reservation under capture: those that a
+// cut up to a workgroup per CU makes K-slices of, beyond 32 rows less those of never_cut and less those that the GEMM kernel is
+// expected to be faster for (a refit of the costs may only take calls out).  Up to 32 rows these calls keep their slices
+// (uncut, the few that are faster gain under 8 %: 5120x2048x4 at 32 rows 8.1 / 8.7).
 MfmaPlan mfma_plan(const Problem &p)
 {
     Group one{};
@@ -520,16 +545,18 @@ MfmaPlan mfma_plan(const Problem &p)
     const long tiles = (p.N + kMfmaTileCols - 1) / kMfmaTileCols, rounds = ((p.K + kMfmaStepK - 1) / kMfmaStepK + kMfmaWaves - 1) / kMfmaWaves;
     const int mt = p.M <= 16 || (p.M <= 64 && tiles * ((p.M + 15) / 16) * rounds <= 512) ? 1 : 2;
     const int slices = mfma_slices(one, mt);
-    bool gemm = false;
+    plan_mfma(one.p[0], mt, slices);
+    bool cut = one.p[0].ksplit > 1, gemm = false;
     if (p.M > 32) {
         Problem wide = p;
         plan_mfma(wide, 2, mt == 2 ? slices : mfma_slices(one, 2));
         const double round = 1.6 + 0.32 * p.nb + (is_block(p.alpha_mode) ? 0.9 : 0.0);
         gemm = gemm_estimate(p) < 5.0 + round * (double)((wide.n_blocks + 255) / 256) * (double)(wide.sets_per_split / kMfmaWaves);
+        // (uncut, the GEMM kernel is the other choice for these)
+        if (cut && !gemm) gemm = never_cut(p);
+        cut = cut && !gemm;
     }
     if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm};
-    plan_mfma(one.p[0], mt, slices);
-    const bool cut = one.p[0].ksplit > 1 && !gemm;
     MfmaPlan plan = pick_mfma(p, cut, cut && p.M <= 32);
     plan.gemm = gemm;
     return plan;

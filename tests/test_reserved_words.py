@@ -1,0 +1,51 @@
+"""Which calls need accumulator words, and so a reservation before a capture, is fixed in the sizes: it does not move with
+the costs that choose between kernels and cuts.  Checked on the host through the described plans."""
+import random
+
+import pytest
+
+from test_launch_plans import BLOCK_I8, GEMM, MATRIX_CORE, ROWWISE, UNIFORM, describe, lib  # noqa: F401
+
+
+def never_cut(N, K, M):
+    """Whether the GEMM kernel, which needs no words, was the choice for a call of more than 32 rows when the line was
+    drawn: its time with slices of four waves against rounds of 3 us of the matrix-core kernel."""
+    rows = 64 if M <= 64 else 128
+    alone, beside = (0.9, 1.6) if rows == 64 else (1.2, 2.1)
+    tiles, steps = -(-N // 256) * -(-M // rows), -(-K // 128) * 2
+    best = None
+    for ks in range(1, 17):
+        if ks > 1 and 2 * ks > steps:
+            break
+        own = (-(-steps // ks) + 1) // 2 * 2
+        if -(-steps // own) != ks:
+            continue
+        if ks > 1 and (tiles * ks > 512 or ks * M * N * 4 > 64 << 20):
+            break
+        full, rest = divmod(tiles * ks, 512)
+        us = full * (own * beside + 5) + (4 + 2 * ks * M * N / 1e6 if ks > 1 else 0)
+        us += own * (beside if rest > 256 else alone) + 5 if rest else 0
+        if best is None or us < 0.99 * best:
+            best = us
+    return best < 5 + 3 * -(-N // 64) * -(-M // 32) * -(-K // 1024) / 256
+
+
+@pytest.mark.parametrize("fmt,N,K,nb,M", [(ROWWISE, 4096, 14336, 1, 33), (ROWWISE, 3904, 17536, 2, 33), (UNIFORM, 3536, 26240, 1, 40),
+                                          (ROWWISE, 512, 49152, 1, 512), (UNIFORM, 3860, 25984, 1, 64)])
+def test_calls_that_once_needed_a_reservation_by_mistake(lib, fmt, N, K, nb, M):  # noqa: F811
+    rc, p = describe(lib, fmt, N, K, nb, K // 128, M)
+    assert rc == 0 and not p.needs_workspace and never_cut(N, K, M)
+
+
+def test_calls_of_many_rows_that_need_words(lib):  # noqa: F811
+    rng = random.Random(7)
+    needed = 0
+    for i in range(20000):
+        K, N = (128 * rng.randint(1, 400), 16 * rng.randint(4, 600)) if i % 2 else (32 * rng.randint(4, 1400), 4 * rng.randint(16, 2400))
+        M, nb, fmt = rng.randint(33, 600) if i % 3 else rng.randint(33, 64), rng.randint(1, 4), rng.choice((ROWWISE, UNIFORM, BLOCK_I8))
+        rc, p = describe(lib, fmt, N, K, nb, 1 if fmt == BLOCK_I8 else K // 32, M)
+        assert rc == 0 and p.kernel in (MATRIX_CORE, GEMM)
+        if p.needs_workspace:
+            needed += 1
+            assert not never_cut(N, K, M), (fmt, N, K, nb, M)
+    assert needed > 500
