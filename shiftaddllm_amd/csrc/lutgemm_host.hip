@@ -537,7 +537,9 @@ double gemm_estimate(const Problem &p);
 // cut up to a workgroup per CU makes K-slices of, beyond 32 rows less those of never_cut and less those that the GEMM kernel is
 // expected to be faster for (a refit of the costs may only take calls out).  Up to 32 rows these calls keep their slices
 // (uncut, the few that are faster gain under 8 %: 5120x2048x4 at 32 rows 8.1 / 8.7).
-MfmaPlan mfma_plan(const Problem &p)
+// `or_gemm`: the GEMM kernel may take the call instead; without it slices are all there is to spread a call with (4096x28672x4 at
+// 64 rows, uncut 100.9 us, in two slices 65.9).
+MfmaPlan mfma_plan(const Problem &p, bool or_gemm)
 {
     Group one{};
     one.count = 1;
@@ -547,7 +549,7 @@ MfmaPlan mfma_plan(const Problem &p)
     const int slices = mfma_slices(one, mt);
     plan_mfma(one.p[0], mt, slices);
     bool cut = one.p[0].ksplit > 1, gemm = false;
-    if (p.M > 32) {
+    if (or_gemm && p.M > 32) {
         Problem wide = p;
         plan_mfma(wide, 2, mt == 2 ? slices : mfma_slices(one, 2));
         const double round = 1.6 + 0.32 * p.nb + (is_block(p.alpha_mode) ? 0.9 : 0.0);
@@ -562,9 +564,10 @@ MfmaPlan mfma_plan(const Problem &p)
     return plan;
 }
 
+// (the grouped entry points' problems: the GEMM kernel is none of their kernels)
 int run_mfma(Problem &p, const Accum &acc)
 {
-    const MfmaPlan plan = mfma_plan(p);
+    const MfmaPlan plan = mfma_plan(p, false);
     const int mt = plan.mt;
     plan_mfma(p, mt, plan.slices);
     if (p.ksplit > 1) {
@@ -650,10 +653,12 @@ bool mfma_any(const Problem &p, int mode)
     return (unsigned long long)p.kwords * p.nb * p.N * 2 < (1ull << 32);
 }
 
+bool tile_possible(const Problem &p, int mode);
+
 int plan_single(Problem &p, int mode, int *kernel, int *mrows)
 {
     if (mfma_eligible(p, mode) || mfma_any(p, mode)) {
-        const MfmaPlan plan = mfma_plan(p);
+        const MfmaPlan plan = mfma_plan(p, tile_possible(p, mode));
         plan_mfma(p, plan.mt, plan.slices);
         *kernel = kMatrixCore;
         *mrows = 16 * plan.mt;
@@ -828,6 +833,17 @@ double gemm_estimate(const Problem &p)
     return plan_tile(t);
 }
 
+// What the GEMM kernel can take.
+bool tile_possible(const Problem &p, int mode)
+{
+    // (32-bit byte offsets into the operands)
+    const unsigned long long limit = 1ull << 32;
+    if ((unsigned long long)p.kwords * p.nb * p.N * 4 >= limit || (unsigned long long)p.M * p.K * 2 >= limit) return false;
+    if (is_block(mode) && (unsigned long long)p.K / 8 * p.nb * p.R * 3 >= limit) return false;
+    const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
+    return least <= 0 || p.M >= least;
+}
+
 // Whether a call takes the GEMM kernel rather than the matrix-core kernel: where that is expected to take less than the
 // latter's widest cut (see mfma_plan) and its best one is not 15 % faster still.  plan_tile's costs are those of two planes; for
 // that comparison they are scaled to what the planes and the format were measured to take (17 to 256 rows): 1.04 to 1.16
@@ -838,16 +854,12 @@ double gemm_estimate(const Problem &p)
 // 4096x4096x4 at 128 rows 29.5* / 37.8.
 bool tile_wanted(const Problem &p, int mode)
 {
-    const int least = option(LUTGEMM_OPTION_TILE_MIN_M);
-    // (32-bit byte offsets into the operands)
-    const unsigned long long limit = 1ull << 32;
-    if ((unsigned long long)p.kwords * p.nb * p.N * 4 >= limit || (unsigned long long)p.M * p.K * 2 >= limit) return false;
-    if (is_block(mode) && (unsigned long long)p.K / 8 * p.nb * p.R * 3 >= limit) return false;
-    if (least > 0) return p.M >= least;
+    if (!tile_possible(p, mode)) return false;
+    if (option(LUTGEMM_OPTION_TILE_MIN_M) > 0) return true;
     if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
     if (p.M <= 32) return false;
     const double planes = mode == kRowF16 ? 0.92 + 0.06 * p.nb : is_block(mode) ? 0.80 + 0.13 * p.nb : 1.05 + 0.19 * p.nb;
-    const MfmaPlan plan = mfma_plan(p);
+    const MfmaPlan plan = mfma_plan(p, true);
     return plan.gemm && (plan.us == 0.0 || plan.us > 0.85 * planes * gemm_estimate(p));
 }
 

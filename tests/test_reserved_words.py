@@ -49,3 +49,15 @@ def test_calls_of_many_rows_that_need_words(lib):  # noqa: F811
             needed += 1
             assert not never_cut(N, K, M), (fmt, N, K, nb, M)
     assert needed > 500
+
+
+@pytest.mark.parametrize("fmt,N,K,nb,M,rows,slices", [(ROWWISE, 4096, 28672, 4, 64, 32, 2), (ROWWISE, 512, 49152, 1, 512, 32, 2),
+                                                      (BLOCK_I8, 5120, 13824, 2, 48, 16, 1), (UNIFORM, 2048, 16384, 3, 40, 32, 4)])
+def test_without_the_gemm_kernel_calls_are_cut(lib, fmt, N, K, nb, M, rows, slices):  # noqa: F811
+    from shiftaddllm_amd import native
+    assert lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], 1 << 20) == 0
+    try:
+        rc, p = describe(lib, fmt, N, K, nb, 8 if fmt == BLOCK_I8 else K // 128, M)
+    finally:
+        lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
+    assert rc == 0 and (p.kernel, p.rows_per_pass, p.k_slices) == (MATRIX_CORE, rows, slices)
