@@ -844,23 +844,32 @@ bool tile_possible(const Problem &p, int mode)
     return least <= 0 || p.M >= least;
 }
 
-// Whether a call takes the GEMM kernel rather than the matrix-core kernel: where that is expected to take less than the
-// latter's widest cut (see mfma_plan) and its best one is not 15 % faster still.  plan_tile's costs are those of two planes; for
-// that comparison they are scaled to what the planes and the format were measured to take (17 to 256 rows): 1.04 to 1.16
-// row-wise, 1.06 to 1.32 with the decoding of block formats, 1.4 to 1.8 uniform.
-// Measured (us, matrix-core kernel / this one, * = taken): 11008x4096x3 at 48 rows 24.1 / 24.1*, 128 rows 39.5 / 32.1*; 4096x11008x2 at
-// 128 rows 24.6* / 29.8, 192 rows 44.7 / 37.5*; 8192x8192x4 at 64 rows 25.1* / 29.0, 96 rows 46.0 / 38.8*; int8 exponents
-// 5120x13824x2 at 48 rows 30.5 / 28.7*, 4096x4096x4 at 96 rows 19.4* / 26.7; 1024x28672x4 at 128 rows 25.7* / 44.3; uniform
-// 4096x4096x4 at 128 rows 29.5* / 37.8.
+// What the GEMM kernel is expected to take beside the matrix-core kernel's estimate: plan_tile's costs, which know neither
+// planes nor formats, scaled to what both kernels were measured to take, and 3 us that they are short of for few inputs.
+double gemm_us(const Problem &p)
+{
+    const double planes = p.alpha_mode == kRowF16 ? 0.55 + 0.13 * p.nb : is_block(p.alpha_mode) ? 0.62 + 0.22 * p.nb : 0.60 + 0.40 * p.nb;
+    return 3.0 + planes * gemm_estimate(p);
+}
+
+// Whether a call takes the GEMM kernel rather than the matrix-core kernel, by the two estimates (see mfma_plan for the
+// calls that may).  Drawn with 900 calls and checked on 3000 others near the line, timed on both (33 to 2048 rows, 512 to 28672
+// inputs and outputs): the kernel taken is within 1.0 % of the better one on average, 6 % of the calls lose more than 5 %.
+// Measured (us, matrix-core kernel / this one, * = taken):
+//   row-wise: 6464x4096x3 at 65 rows 18.0* / 22.8, 10944x5120x3 at 64 30.3 / 24.1*, 6144x5120x2 at 72 18.6* / 24.4, 7680x8192x3 at 112
+//   40.0 / 33.1*, 3072x3328x3 at 256 22.3* / 24.3, 24128x3072x2 at 80 45.1 / 33.5*; scales that are no powers of two 3392x6144x3 at
+//   72 24.6* / 31.3, 15360x3328x3 at 33 30.0* / 37.2, 20096x1024x2 at 160 34.5 / 37.7*
+//   fp16 blocks: 5056x4096x4 at 64 17.9* / 27.6, 10240x7040x3 at 56 39.7 / 28.6*, 4800x8192x2 at 512 99.5 / 62.1*, 19008x3072x3 at 72 46.1 / 35.9*
+//   int8 exponents: 6144x3584x4 at 56 17.8* / 25.3, 13312x5760x3 at 36 41.5 / 29.8*, 7168x5120x3 at 128 38.6* / 32.1
+//   uniform: 21888x1024x4 at 72 39.9* / 53.0, 5312x7168x3 at 112 52.7 / 40.9*, 12864x2048x3 at 128 43.4* / 38.1
 bool tile_wanted(const Problem &p, int mode)
 {
     if (!tile_possible(p, mode)) return false;
     if (option(LUTGEMM_OPTION_TILE_MIN_M) > 0) return true;
     if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
     if (p.M <= 32) return false;
-    const double planes = mode == kRowF16 ? 0.92 + 0.06 * p.nb : is_block(mode) ? 0.80 + 0.13 * p.nb : 1.05 + 0.19 * p.nb;
     const MfmaPlan plan = mfma_plan(p, true);
-    return plan.gemm && (plan.us == 0.0 || plan.us > 0.85 * planes * gemm_estimate(p));
+    return plan.gemm && (plan.us == 0.0 || plan.us > gemm_us(p));
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)

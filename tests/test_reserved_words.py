@@ -4,7 +4,7 @@ import random
 
 import pytest
 
-from test_launch_plans import BLOCK_I8, GEMM, MATRIX_CORE, ROWWISE, UNIFORM, describe, lib  # noqa: F401
+from test_launch_plans import BLOCK_F16, BLOCK_I8, GEMM, MATRIX_CORE, ROWWISE, UNIFORM, describe, lib  # noqa: F401
 
 
 def never_cut(N, K, M):
@@ -61,3 +61,19 @@ def test_without_the_gemm_kernel_calls_are_cut(lib, fmt, N, K, nb, M, rows, slic
     finally:
         lib.lutgemm_set_option(native.OPTIONS["TILE_MIN_M"], -1)
     assert rc == 0 and (p.kernel, p.rows_per_pass, p.k_slices) == (MATRIX_CORE, rows, slices)
+
+
+@pytest.mark.parametrize("fmt,N,K,nb,groups,M,kernel", [
+    # (us measured, matrix-core / GEMM kernel)
+    (BLOCK_F16, 20864, 1408, 3, 8, 64, MATRIX_CORE),   # 32.5 / 51.6
+    (BLOCK_F16, 7360, 4864, 4, 8, 48, MATRIX_CORE),    # 34.3 / 53.6
+    (BLOCK_I8, 4480, 4608, 4, 8, 72, MATRIX_CORE),     # 24.5 / 33.0
+    (UNIFORM, 21888, 1024, 4, 8, 72, MATRIX_CORE),     # 39.9 / 53.0
+    (ROWWISE, 6464, 4096, 3, 32, 65, MATRIX_CORE),     # 18.0 / 22.8
+    (BLOCK_I8, 10688, 1792, 4, 8, 256, GEMM),          # 78.6 / 42.7
+    (ROWWISE, 4352, 17408, 4, 136, 64, GEMM),          # 75.4 / 48.3
+    (UNIFORM, 5312, 7168, 3, 56, 112, GEMM),           # 52.7 / 40.9
+])
+def test_the_faster_kernel_where_they_differ_much(lib, fmt, N, K, nb, groups, M, kernel):  # noqa: F811
+    rc, p = describe(lib, fmt, N, K, nb, groups, M)
+    assert rc == 0 and p.kernel == kernel
