@@ -273,7 +273,9 @@ int lutgemm_copy_bytes(void *dst, const void *src, size_t bytes, void *stream);
  * lutgemm_reserve_workspace(stream, w) no call on `stream` whose sizes need at
  * most w words synchronises or allocates, so such calls can be captured into a
  * HIP graph without a warm-up call.  For a grouped or fused call add up the
- * words of its problems.  The reservation also covers the sums of K-slices of
+ * words of its problems; for lutgemm_gemv_rowwise_f16_gated M * N / 2 more (a captured
+ * call without these takes two launches).  Where the memory is not there (LUTGEMM_ENOMEM)
+ * the stream keeps what it had.  The reservation also covers the sums of K-slices of
  * calls of many rows (up to 64 bytes per word, 64 MB in all), but not the split
  * activations of lutgemm_gemv_rowwise_pow2_f16, whose size depends on K.
  * Reserving synchronises `stream` and may not be done while it is being captured

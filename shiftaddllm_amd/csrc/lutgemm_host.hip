@@ -93,11 +93,23 @@ size_t grown(size_t wanted, size_t least)
     return least;
 }
 
+// Device memory, or ENOMEM.  Callers go on without it (a smaller buffer, another kernel): the error that the runtime
+// would report to their next check of a launch is taken back.
+template <typename T>
+int allocate(T **out, size_t bytes)
+{
+    const hipError_t e = hipMalloc((void **)out, bytes);
+    if (e == hipSuccess) return LUTGEMM_OK;
+    (void)hipGetLastError();
+    g_last_hip_error = (int)e;
+    return LUTGEMM_ENOMEM;
+}
+
 // Grow-only, zero-initialised accumulator words per (device, stream).  Growing
 // synchronises the stream and allocates, which a stream under capture cannot do: that
-// case is refused before anything is touched (reserve the words beforehand).  An
-// outgrown buffer is kept (zero, unused by new launches) until
-// lutgemm_release_workspaces(): a graph captured earlier still points at it.
+// case is refused before anything is touched (reserve the words beforehand).  Without
+// memory for it the buffer stays as it is.  An outgrown buffer is kept (zero, unused by
+// new launches) until lutgemm_release_workspaces(): a graph captured earlier still points at it.
 int stream_workspace(hipStream_t stream, size_t words, unsigned long long **out)
 {
     int dev = 0;
@@ -110,21 +122,19 @@ int stream_workspace(hipStream_t stream, size_t words, unsigned long long **out)
         e = hipStreamIsCapturing(stream, &cap);
         if (e != hipSuccess) return hip_fail(e);
         if (cap != hipStreamCaptureStatusNone) return LUTGEMM_ECAPTURE;
-        e = hipStreamSynchronize(stream);  // queued work may still use the old buffer
-        if (e != hipSuccess) return hip_fail(e);
-        if (ws.accum) ws.retired.push_back(ws.accum);
-        ws.accum = nullptr;
-        ws.words = 0;
         const size_t want = grown(words, 1u << 18);
-        e = hipMalloc((void **)&ws.accum, want * sizeof(unsigned long long));
+        unsigned long long *grown_words = nullptr;
+        const int rc = allocate(&grown_words, want * sizeof(unsigned long long));
+        if (rc != LUTGEMM_OK) return rc;
+        e = hipStreamSynchronize(stream);  // queued work may still use the old buffer
+        if (e == hipSuccess) e = hipMemsetAsync(grown_words, 0, want * sizeof(unsigned long long), stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(stream);
         if (e != hipSuccess) {
-            g_last_hip_error = (int)e;
-            return LUTGEMM_ENOMEM;
+            (void)hipFree(grown_words);
+            return hip_fail(e);
         }
-        e = hipMemsetAsync(ws.accum, 0, want * sizeof(unsigned long long), stream);
-        if (e != hipSuccess) return hip_fail(e);
-        e = hipStreamSynchronize(stream);
-        if (e != hipSuccess) return hip_fail(e);
+        if (ws.accum) ws.retired.push_back(ws.accum);
+        ws.accum = grown_words;
         ws.words = want;
     }
     *out = ws.accum;
@@ -145,18 +155,18 @@ int stream_split_buffer(hipStream_t stream, size_t bytes, void **out)
         e = hipStreamIsCapturing(stream, &cap);
         if (e != hipSuccess) return hip_fail(e);
         if (cap != hipStreamCaptureStatusNone) return LUTGEMM_ECAPTURE;
-        e = hipStreamSynchronize(stream);
-        if (e != hipSuccess) return hip_fail(e);
-        if (ws.split) ws.retired_split.push_back(ws.split);
-        ws.split = nullptr;
-        ws.split_bytes = 0;
         // (the gaps between slices on top of a power of two: sums that fill one would otherwise take the next)
         const size_t want = grown(bytes > kTileGapBytes ? bytes - kTileGapBytes : bytes, 1u << 20) + kTileGapBytes;
-        e = hipMalloc(&ws.split, want);
+        void *grown_split = nullptr;
+        const int rc = allocate(&grown_split, want);
+        if (rc != LUTGEMM_OK) return rc;
+        e = hipStreamSynchronize(stream);
         if (e != hipSuccess) {
-            g_last_hip_error = (int)e;
-            return LUTGEMM_ENOMEM;
+            (void)hipFree(grown_split);
+            return hip_fail(e);
         }
+        if (ws.split) ws.retired_split.push_back(ws.split);
+        ws.split = grown_split;
         ws.split_bytes = want;
     }
     *out = ws.split;
