@@ -516,8 +516,6 @@ MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
     return best;
 }
 
-double gemm_estimate(const Problem &p);
-
 // Whether a call of more than 32 rows that a cut up to a workgroup per CU makes K-slices of takes none: callers that
 // reserve nothing before a capture rely on which calls need accumulator words, so this line is fixed in the sizes and follows neither
 // the costs above nor those of plan_tile.  It was drawn where the GEMM kernel, which needs none, was the faster choice:
@@ -856,8 +854,12 @@ bool tile_possible(const Problem &p, int mode)
 
 // What the GEMM kernel is expected to take beside the matrix-core kernel's estimate: plan_tile's costs, which know neither
 // planes nor formats, scaled to what both kernels were measured to take, and 3 us that they are short of for few inputs.
+// Up to 64 inputs, a single step of either kernel and outside what the estimates were fitted to, calls keep the line they had
+// (us, matrix-core kernel / this one, * = taken: 6028x64x4 at 33 rows 6.4 / 8.6*, 3100x64x3 at 200 7.0* / 9.6, 13800x64x3 at 128
+// 15.5 / 10.9*).
 double gemm_us(const Problem &p)
 {
+    if (p.K <= 64) return 0.95 * gemm_estimate(p);
     const double planes = p.alpha_mode == kRowF16 ? 0.55 + 0.13 * p.nb : is_block(p.alpha_mode) ? 0.62 + 0.22 * p.nb : 0.60 + 0.40 * p.nb;
     return 3.0 + planes * gemm_estimate(p);
 }

@@ -73,6 +73,9 @@ def test_without_the_gemm_kernel_calls_are_cut(lib, fmt, N, K, nb, M, rows, slic
     (BLOCK_I8, 10688, 1792, 4, 8, 256, GEMM),          # 78.6 / 42.7
     (ROWWISE, 4352, 17408, 4, 136, 64, GEMM),          # 75.4 / 48.3
     (UNIFORM, 5312, 7168, 3, 56, 112, GEMM),           # 52.7 / 40.9
+    (ROWWISE, 13800, 64, 3, 2, 128, GEMM),             # 15.5 / 10.9
+    (ROWWISE, 1820, 64, 3, 1, 100, MATRIX_CORE),       # 4.1 / 9.6
+    (ROWWISE, 6028, 64, 4, 1, 33, GEMM),               # 6.4 / 8.6: calls of up to 64 inputs keep the line they had
 ])
 def test_the_faster_kernel_where_they_differ_much(lib, fmt, N, K, nb, groups, M, kernel):  # noqa: F811
     rc, p = describe(lib, fmt, N, K, nb, groups, M)
