@@ -485,6 +485,21 @@ typedef struct lutgemm_fused_problem {
 int lutgemm_gemv_rowwise_f16_fused(int count, const lutgemm_fused_problem *problems, void *stream);
 
 /*
+ * How these problems would be launched by lutgemm_gemv_rowwise_f16_fused (or _grouped: all optional fields null), as
+ * lutgemm_describe_plan describes a lone call: host arithmetic on sizes, options and the addresses' alignment and overlap; nothing
+ * is read through them.  Returns what that call would return for them without launching anything.
+ */
+typedef struct lutgemm_group_plan {
+    int kernel;                                  /* 0: table look-up kernel, 1: matrix-core kernel */
+    int launches;                                /* 1, or one per problem */
+    int needs_workspace;                         /* 1: accumulator words, lutgemm_workspace_words(N, M) of every problem */
+    int workgroups[LUTGEMM_MAX_GROUP];
+    int units_per_workgroup[LUTGEMM_MAX_GROUP]; /* items of 256 inputs x 256 outputs (look-up), K-steps per slice (matrix cores) */
+} lutgemm_group_plan;
+
+int lutgemm_describe_group_plan(int count, const lutgemm_fused_problem *problems, lutgemm_group_plan *plan);
+
+/*
  * The first half of a gated MLP: act = fp16(fp16(silu(gate)) * up), [M][N], where gate_up[0] and
  * gate_up[1] describe the two products (same M and N, M * N a multiple of 8, overwrite = 1, no
  * next_input / sumsq_out; otherwise as for lutgemm_gemv_rowwise_f16_fused).  Where the matrix-core

@@ -592,6 +592,20 @@ struct Gated {
     bool done;
 };
 
+// (returns whether some problem needs accumulator words)
+bool plan_mfma_group(Group &g, int mt, int *most)
+{
+    const int slices = mfma_slices(g, mt);
+    bool any_split = false;
+    for (int i = 0; i < g.count; ++i) {
+        Problem &p = g.p[i];
+        plan_mfma(p, mt, slices);
+        if (p.n_blocks > *most) *most = p.n_blocks;
+        any_split = any_split || p.ksplit > 1;
+    }
+    return any_split;
+}
+
 // All problems of a group on the matrix-core kernel in one launch (they share the
 // row-tile height: all M <= 16 or all M > 16).
 int run_mfma_group(Group &g, const Accum &acc, Gated *gated)
@@ -599,15 +613,8 @@ int run_mfma_group(Group &g, const Accum &acc, Gated *gated)
     const int mt = g.p[0].M > 16 ? 2 : 1;
     size_t words = 0;
     for (int i = 0; i < g.count; ++i) words += (size_t)g.p[i].M * g.p[i].N;
-    const int slices = mfma_slices(g, mt);
-    int begin = 0;
-    bool any_split = false;
-    for (int i = 0; i < g.count; ++i) {
-        Problem &p = g.p[i];
-        plan_mfma(p, mt, slices);
-        if (p.n_blocks > begin) begin = p.n_blocks;  // grid.x: the largest problem's workgroups
-        any_split = any_split || p.ksplit > 1;
-    }
+    int begin = 0;   // grid.x: the largest problem's workgroups
+    const bool any_split = plan_mfma_group(g, mt, &begin);
     // (behind the problems' words, where the launch forms a product, one 32-bit word per output)
     const size_t pair_words = gated ? ((size_t)g.p[0].M * g.p[0].N + 1) / 2 : 0;
     unsigned long long *base = nullptr;
@@ -969,71 +976,159 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
-// Share a workgroup budget between look-up problems that run side by side so that the longest
-// range of every problem takes about the same time.  An item costs a table build plus look-ups in proportion to its bit
-// planes: 0.10 + 0.38 * nb us where two workgroups share the CU (one row to two of gate,up adds 5.4 items to each: of 2, 3 and 4
-// bits 4.65, 6.5 and 8.7 us); the problems end with their slowest workgroup, so the items per workgroup of problem i
-// are floor(T / cost_i) for the smallest T whose workgroups fit the budget.  (With 0.45 + 0.13 * nb, a lone item's, gate,up of
-// 2 and 4 bits took 23.9 us at two rows, now 19.7, of 2 and 3 bits 20.4, now 18.4; q,k,v of 1, 4 and 3 bits went
-// from 12.5 to 14.7.  Inputs shorter than 4096 keep the lone item's: on them it depends which launches have ranges that
-// end inside a K-row, and so need accumulator words.)
+// What a workgroup of a grouped look-up launch takes, in us: an item is a table build plus look-ups in proportion to its bit
+// planes.  With a workgroup per CU 0.45 + 0.13 * nb (measured).  Where two share a CU 0.10 + 0.38 * nb (one row to two of
+// gate,up adds 5.4 items to each: of 2, 3 and 4 bits 4.65, 6.5 and 8.7 us), and a range that ends inside a second tile has
+// another tile's sums to hand over (1.05, fitted with 100 launches of unlike widths, one and two rows, 4096 to 8192 inputs: 1.5 %
+// behind the best of four sharings on average, with 0.75 to 1.5 much the same, without 4 %).  us, RMSNorm in front, with the first
+// costs / with the second ones without the hand-over and kEngines below / as they are:
+//   one row: gate,up 4096 -> 11008 of 1 and 3 bits 13.4 / 10.8 / 10.8; q,k,v 5120 -> 5120 of 2, 4 and 3 bits 12.3 / 11.3 / 11.1
+//   two rows: q,k,v 4096 -> 4096 of 1, 4 and 3 bits 12.9 / 14.8 / 11.5, of 2, 1 and 4 bits 10.3 / 13.7 / 10.2; 5120 -> 5120 of 3, 2 and 2 bits
+//   13.3 / 15.3 / 13.2; gate,up 4096 -> 11008 of 2 and 4 bits 25.0 / 21.4 / 20.8, of 3 and 4 bits 27.1 / 26.8 / 23.3, of 1 and 4 bits 20.6 / 18.3 /
+//   18.2; slower: 4096 -> 14336 of 4 and 3 bits 23.0 / 26.9 / 26.6, q,k,v 5120 -> 5120 of 4, 1 and 1 bits 14.5 / 16.1 / 16.2
+struct ItemCost {
+    double fixed, plane, hand_over;
+};
+constexpr ItemCost kItemAlone{0.45, 0.13, 0.0}, kItemBeside{0.10, 0.38, 1.05};
+// Workgroups are dealt to the chip's 32 shader engines in turn, the empty ones of a problem narrower than the grid as well, and
+// an engine holds 16 of this kernel's; what is dealt to a full engine waits for a range to end (gate,up 4096 -> 11008 of 3 and 4
+// bits at two rows: 230 + 276 workgroups, 17 on the first engines, 26.6 us; 198 + 276 23.0).
+constexpr long kEngines = 32;
+
+// Share a workgroup budget between look-up problems that run side by side so that the longest range of every problem takes
+// about the same time: the problems end with their slowest workgroup, so the items per workgroup of each are what it
+// takes in T, for the smallest T whose workgroups fit the budget (`by_engine`: fit every engine's part of it).
 // With equal bit widths this is a share in proportion to the items, rounded down: a few
 // workgroups more than can be resident run as a second, mostly empty round, and fewer
 // workgroups with more items each are the better trade anyway (q,k,v of 4096x4096 as 3 x 64
 // workgroups of 4 items 5.31 us per GEMV of the four-launch block, as 3 x 86 of 3 items 5.54).
-// *most: the largest workgroup count of a problem (raised only); *any_split: some problem needs
-// accumulator words (set only).
-int share_workgroups(Problem *const *ps, int count, long budget, int *most, bool *any_split)
-{
-    long items[kMaxGroup];
-    double cost[kMaxGroup];
-    double lo = 0.0, hi = 0.0;
-    bool long_rows = true;
-    for (int i = 0; i < count; ++i) long_rows = long_rows && ps[i]->K >= 4096;
-    for (int i = 0; i < count; ++i) {
-        const Problem &p = *ps[i];
-        items[i] = (long)((p.N + kTileCols - 1) / kTileCols) * p.nsets;
-        cost[i] = long_rows ? 0.10 + 0.38 * p.nb : 0.45 + 0.13 * p.nb;
-        const double all = (double)items[i] * cost[i];
-        if (all > hi) hi = all;
+struct Shares {
+    int most;         // the largest workgroup count of a problem
+    bool any_split;   // some problem needs accumulator words
+};
+
+struct Sharing {
+    Problem *const *ps;
+    int count;
+    ItemCost item;
+    long budget;
+    bool by_engine;
+
+    double cost(int i) const { return item.fixed + item.plane * ps[i]->nb; }
+    long items(int i) const { return (long)((ps[i]->N + kTileCols - 1) / kTileCols) * ps[i]->nsets; }
+
+    // the items of a range of problem i that takes `us`: within one tile (or of whole ones), or across two
+    long within(int i, double us) const
+    {
+        const long across = us > 2.0 * item.hand_over ? (long)((us - 2.0 * item.hand_over) / cost(i)) : 0;
+        long whole = us > item.hand_over ? (long)((us - item.hand_over) / cost(i)) : 0;
+        const int nsets = ps[i]->nsets;
+        if (whole >= nsets)
+            whole -= whole % nsets;
+        else
+            while (whole > across && nsets % whole) --whole;
+        return across > whole ? across : whole;
     }
-    auto workgroups = [&](double t) {
-        long n = 0;
+
+    bool fits(double us) const
+    {
+        long wgs[kMaxGroup], all = 0, widest = 0;
         for (int i = 0; i < count; ++i) {
-            long ipw = (long)(t / cost[i]);
-            if (ipw < 1) return (long)1 << 40;
-            n += ((items[i] + ipw - 1) / ipw) * ps[i]->M;
+            const long ipw = within(i, us);
+            if (ipw < 1) return false;
+            wgs[i] = (items(i) + ipw - 1) / ipw * ps[i]->M;
+            all += wgs[i];
+            widest = wgs[i] > widest ? wgs[i] : widest;
         }
-        return n;
-    };
-    for (int it = 0; it < 50; ++it) {
-        const double mid = 0.5 * (lo + hi);
-        if (workgroups(mid) <= budget) hi = mid; else lo = mid;
+        if (!by_engine) return all <= budget;
+        for (int at = 0; at < count; ++at) {   // (an engine with most of them is one that a problem begins on)
+            long here = 0;
+            for (int i = 0; i < count; ++i) {
+                const long from = ((at - i) * widest % kEngines + kEngines) % kEngines;
+                here += wgs[i] / kEngines + (from < wgs[i] % kEngines ? 1 : 0);
+            }
+            if (here > budget / kEngines) return false;
+        }
+        return true;
     }
+
+    int plan(Shares *out) const
+    {
+        double lo = 0.0, hi = 0.0;
+        for (int i = 0; i < count; ++i) {
+            const double all = (double)items(i) * cost(i) + 2.0 * item.hand_over;
+            if (all > hi) hi = all;
+        }
+        for (int it = 0; it < 50; ++it) {
+            const double mid = 0.5 * (lo + hi);
+            if (fits(mid)) hi = mid; else lo = mid;
+        }
+        *out = Shares{0, false};
+        for (int i = 0; i < count; ++i) {
+            Problem &p = *ps[i];
+            long ipw = within(i, hi);
+            if (ipw < 1) ipw = 1;
+            const int rc = plan_lookup(p, 1, (items(i) + ipw - 1) / ipw * p.M);
+            if (rc != LUTGEMM_OK) return rc;
+            if (p.n_blocks > out->most) out->most = p.n_blocks;   // grid.x: the largest problem's workgroups
+            out->any_split = out->any_split || lookup_splits_k(p);
+        }
+        return LUTGEMM_OK;
+    }
+};
+
+// The shares of a grouped look-up launch.
+int share_group(Problem *const *ps, int count, int xform, Shares *out)
+{
+    long bytes = 0;
+    bool mixed = false, long_rows = true;
     for (int i = 0; i < count; ++i) {
-        Problem &p = *ps[i];
-        long ipw = (long)(hi / cost[i]);
-        if (ipw < 1) ipw = 1;
-        const long want = ((items[i] + ipw - 1) / ipw) * p.M;
-        int rc = plan_lookup(p, 1, want);
-        if (rc != LUTGEMM_OK) return rc;
-        if (p.n_blocks > *most) *most = p.n_blocks;  // grid.x: the largest problem's workgroups
-        *any_split = *any_split || lookup_splits_k(p);
+        bytes += (long)ps[i]->N * (ps[i]->K / 8) * ps[i]->nb * ps[i]->M;
+        mixed = mixed || ps[i]->nb != ps[0]->nb;
+        long_rows = long_rows && ps[i]->K >= 4096;
     }
-    return LUTGEMM_OK;
+    // Two workgroups per CU also on short streams where a workgroup begins with an RMSNorm (it hides one's start behind
+    // the other's) or widths differ (finer shares): us, budget of 256 against 512, one row, 4096 inputs with RMSNorm: q,k,v of
+    // 2, 3 and 4 bits 10.7 / 8.9, of 3 bits 9.0 / 8.8, grouped heads (4096 + 2 x 1024 outputs) 7.8 / 7.2, two rows 10.9 / 7.9;
+    // without it q,k,v of 2, 3 and 4 bits 9.9 / 8.0, of 3 bits 7.65 / 8.2.  2048 inputs: 8 MB 6.3 / 6.9, two rows 9 MB
+    // 6.25 / 6.55.
+    const bool pairs = count > 1 && (xform == kXNorm || mixed) && long_rows && bytes >= (9l << 20) &&
+                       option(LUTGEMM_OPTION_TARGET_BLOCKS) <= 0;
+    const long usual = target_blocks(bytes), budget = pairs ? 512 : usual;
+    // Callers that reserve nothing before a capture rely on which launches need accumulator words: none with the usual
+    // budget and the costs of a workgroup alone, none now.  (They do wherever every range of that share is of whole rows of
+    // items, which it is not if ranges that are all shorter than that of some problem fit.)
+    const Sharing alone{ps, count, kItemAlone, usual, false};
+    double whole = 0.0;
+    for (int i = 0; i < count; ++i) {
+        const double us = alone.cost(i) * ps[i]->nsets;
+        whole = us > whole ? us : whole;
+    }
+    if (!alone.fits(whole * (1.0 - 1e-9))) {
+        const int rc = alone.plan(out);
+        if (rc == LUTGEMM_OK && !out->any_split) return rc;
+    }
+    // (inputs shorter than 4096 keep the first costs: 3072 -> 8192 of 2 and 4 bits at two rows 11.3, with the second ones 12.5)
+    return Sharing{ps, count, budget == 512 && mixed && long_rows ? kItemBeside : kItemAlone, budget, budget == 512}.plan(out);
 }
 
 // Up to kMaxGroup row-wise problems in one launch of the look-up kernel.  Problems
 // with enough rows for the matrix-core kernel (and no fused transform) are launched
 // on that path instead.
-int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc, Gated *gated = nullptr)
+struct GroupPlan {
+    Group g;
+    int xform;
+    bool one_mfma, each_mfma;   // one launch of the matrix-core kernel, one per problem; neither: the look-up kernel, with
+    Shares shares;
+};
+
+int plan_group(int count, const lutgemm_fused_problem *problems, const Gated *gated, GroupPlan &plan)
 {
-    Group g{};
+    Group &g = plan.g;
     g.count = count;
-    size_t words = 0;
-    long total_bytes = 0;
-    bool plain = true, all_mfma = true, mixed = false, long_rows = true;
-    int xform = kXNone;
+    bool plain = true, all_mfma = true;
+    int &xform = plan.xform;
+    xform = kXNone;
     for (int i = 0; i < count; ++i) {
         const lutgemm_fused_problem &q = problems[i];
         Problem &p = g.p[i];
@@ -1070,10 +1165,6 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
         xform = mine;
         plain = plain && !p.norm_w && !p.gate && !p.overwrite && !p.next_in && !p.sumsq_out && !p.sumsq_in;
         all_mfma = all_mfma && mfma_eligible(p, kRowF16);
-        mixed = mixed || p.nb != g.p[0].nb;
-        long_rows = long_rows && q.K >= 4096;
-        words += (size_t)q.M * q.N;
-        total_bytes += (long)q.N * (q.K / 8) * q.nb * q.M;
     }
     // Every problem finishes its outputs with a plain read-modify-write, and the outputs are
     // requested early: nothing a problem of the launch writes (out, next_input, sumsq_out) may
@@ -1110,30 +1201,31 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
     // would redo the transform of all rows (measured slower than a separate kernel).
     bool same_height = true;
     for (int i = 1; i < count; ++i) same_height = same_height && ((g.p[i].M > 16) == (g.p[0].M > 16));
-    if (all_mfma && xform == kXNone && same_height && (count > 1 || !plain)) return run_mfma_group(g, acc, gated);
-    if (plain && all_mfma) {
+    plan.one_mfma = all_mfma && xform == kXNone && same_height && (count > 1 || !plain);
+    plan.each_mfma = !plan.one_mfma && plain && all_mfma;
+    if (plan.one_mfma || plan.each_mfma) return LUTGEMM_OK;
+    Problem *ps[kMaxGroup];
+    for (int i = 0; i < count; ++i) ps[i] = &g.p[i];
+    return share_group(ps, count, xform, &plan.shares);
+}
+
+int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc, Gated *gated = nullptr)
+{
+    GroupPlan plan{};
+    const int rc = plan_group(count, problems, gated, plan);
+    if (rc != LUTGEMM_OK) return rc;
+    Group &g = plan.g;
+    if (plan.one_mfma) return run_mfma_group(g, acc, gated);
+    if (plan.each_mfma) {
         for (int i = 0; i < count; ++i) {
             int rc = run_mfma(g.p[i], acc);
             if (rc != LUTGEMM_OK) return rc;
         }
         return LUTGEMM_OK;
     }
-    Problem *ps[kMaxGroup];
-    for (int i = 0; i < count; ++i) ps[i] = &g.p[i];
-    int begin = 0;
-    bool any_split = false;
-    {
-        // Two workgroups per CU also on short streams where a workgroup begins with an RMSNorm (it hides one's start behind
-        // the other's) or widths differ (finer shares): us, budget of 256 against 512, one row, 4096 inputs with RMSNorm: q,k,v of
-        // 2, 3 and 4 bits 10.7 / 8.9, of 3 bits 9.0 / 8.8, grouped heads (4096 + 2 x 1024 outputs) 7.8 / 7.2, two rows 10.9 / 7.9;
-        // without it q,k,v of 2, 3 and 4 bits 9.9 / 8.0, of 3 bits 7.65 / 8.2.  2048 inputs: 8 MB 6.3 / 6.9, two rows 9 MB
-        // 6.25 / 6.55.
-        const bool pairs = count > 1 && (xform == kXNorm || mixed) && long_rows && total_bytes >= (9l << 20) &&
-                           option(LUTGEMM_OPTION_TARGET_BLOCKS) <= 0;
-        int rc = share_workgroups(ps, count, pairs ? 512 : (long)target_blocks(total_bytes), &begin, &any_split);
-        if (rc != LUTGEMM_OK) return rc;
-    }
-    if (any_split) {
+    if (plan.shares.any_split) {
+        size_t words = 0;
+        for (int i = 0; i < count; ++i) words += (size_t)g.p[i].M * g.p[i].N;
         unsigned long long *base = nullptr;
         int rc = accum_words(acc, words, &base);
         if (rc != LUTGEMM_OK) return rc;
@@ -1143,7 +1235,7 @@ int run_group(int count, const lutgemm_fused_problem *problems, const Accum &acc
             off += (size_t)g.p[i].M * g.p[i].N;
         }
     }
-    const hipError_t e = count == 1 ? launch_gemv_fused(g.p[0], xform, acc.stream) : launch_gemv_group(g, xform, begin, acc.stream);
+    const hipError_t e = count == 1 ? launch_gemv_fused(g.p[0], plan.xform, acc.stream) : launch_gemv_group(g, plan.xform, plan.shares.most, acc.stream);
     return e == hipSuccess ? LUTGEMM_OK : hip_fail(e);
 }
 
@@ -1270,7 +1362,6 @@ int plan_chain(int count, const lutgemm_chain_problem *problems, int grid_in, Ch
         if (rc != LUTGEMM_OK) return rc;
     }
     const int stage_blocks = option(LUTGEMM_OPTION_CHAIN_BLOCKS) > 0 ? option(LUTGEMM_OPTION_CHAIN_BLOCKS) : grid;
-    int begin = 0;
     bool any_split = false;
     for (int first = 0; first < count;) {
         int last = first;
@@ -1285,13 +1376,13 @@ int plan_chain(int count, const lutgemm_chain_problem *problems, int grid_in, Ch
         // would hold more takes further rounds of the grid
         constexpr int kWindowItems = kThreads / kTables;
         for (long rounds = 1;; ++rounds) {
-            bool split = false;
-            int rc = share_workgroups(ps, last - first, rounds * (long)stage_blocks, &begin, &split);
+            Shares shares;
+            const int rc = Sharing{ps, last - first, kItemAlone, rounds * (long)stage_blocks, false}.plan(&shares);
             if (rc != LUTGEMM_OK) return rc;
             bool fits = true;
             for (int i = first; i < last; ++i) fits = fits && g.p[i].items_per_wg <= kWindowItems;
             if (fits) {
-                any_split = any_split || split;
+                any_split = any_split || shares.any_split;
                 break;
             }
             if (rounds >= 4096) return LUTGEMM_EUNSUP;
@@ -1305,7 +1396,6 @@ int plan_chain(int count, const lutgemm_chain_problem *problems, int grid_in, Ch
     *grid_out = total_units < grid ? total_units : grid;
     *any_split_out = any_split;
     *words_out = words;
-    (void)begin;
     return LUTGEMM_OK;
 }
 
@@ -1511,6 +1601,34 @@ int lutgemm_gemv_rowwise_f16_fused(int count, const lutgemm_fused_problem *probl
 {
     if (!problems || count < 1 || count > kMaxGroup) return LUTGEMM_EINVAL;
     return run_group(count, problems, Accum{(hipStream_t)stream_v});
+}
+
+int lutgemm_describe_group_plan(int count, const lutgemm_fused_problem *problems, lutgemm_group_plan *plan)
+{
+    if (!problems || !plan || count < 1 || count > kMaxGroup) return LUTGEMM_EINVAL;
+    GroupPlan group{};
+    const int rc = plan_group(count, problems, nullptr, group);
+    if (rc != LUTGEMM_OK) return rc;
+    *plan = lutgemm_group_plan{};
+    plan->kernel = group.one_mfma || group.each_mfma ? kMatrixCore : kLookup;
+    plan->launches = group.each_mfma ? count : 1;
+    if (group.one_mfma) {
+        int most = 0;
+        plan->needs_workspace = plan_mfma_group(group.g, group.g.p[0].M > 16 ? 2 : 1, &most);
+    } else if (!group.each_mfma) {
+        plan->needs_workspace = group.shares.any_split;
+    }
+    for (int i = 0; i < count; ++i) {
+        Problem &p = group.g.p[i];
+        if (group.each_mfma) {
+            const MfmaPlan mfma = mfma_plan(p, false);
+            plan_mfma(p, mfma.mt, mfma.slices);
+            plan->needs_workspace |= p.ksplit > 1;
+        }
+        plan->workgroups[i] = p.n_blocks;
+        plan->units_per_workgroup[i] = plan->kernel == kMatrixCore ? p.sets_per_split : p.items_per_wg;
+    }
+    return LUTGEMM_OK;
 }
 
 int lutgemm_gemv_rowwise_f16_gated(const lutgemm_fused_problem *gate_up, void *act_f16, void *stream)

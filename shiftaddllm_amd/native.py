@@ -54,6 +54,7 @@ C_ABI_SYMBOLS = (
     "lutgemm_decode_attention_f16",
     "lutgemm_decode_silu_mul_f16",
     "lutgemm_gemv_rowwise_f16_gated",
+    "lutgemm_describe_group_plan",
 )
 
 
@@ -115,6 +116,12 @@ class ChainPlan(ctypes.Structure):
     _fields_ = [("workgroups", ctypes.c_int), ("units", ctypes.c_int), ("needs_workspace", ctypes.c_int),
                 ("stage", ctypes.c_int * MAX_GROUP), ("first_unit", ctypes.c_int * MAX_GROUP),
                 ("unit_count", ctypes.c_int * MAX_GROUP), ("items_per_unit", ctypes.c_int * MAX_GROUP)]
+
+
+class GroupPlan(ctypes.Structure):
+    """struct lutgemm_group_plan of include/lutgemm_gfx950.h."""
+    _fields_ = [("kernel", ctypes.c_int), ("launches", ctypes.c_int), ("needs_workspace", ctypes.c_int),
+                ("workgroups", ctypes.c_int * MAX_GROUP), ("units_per_workgroup", ctypes.c_int * MAX_GROUP)]
 
 
 class NativeLibraryMissing(ImportError):
@@ -211,6 +218,8 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.lutgemm_decode_silu_mul_f16.restype = ci
     lib.lutgemm_gemv_rowwise_f16_gated.argtypes = [ctypes.POINTER(FusedProblem), vp, vp]
     lib.lutgemm_gemv_rowwise_f16_gated.restype = ci
+    lib.lutgemm_describe_group_plan.argtypes = [ci, ctypes.POINTER(FusedProblem), ctypes.POINTER(GroupPlan)]
+    lib.lutgemm_describe_group_plan.restype = ci
     lib.lutgemm_set_timestamp_buffer.argtypes = [vp, sz]
     lib.lutgemm_set_timestamp_buffer.restype = ci
     return lib
