@@ -341,15 +341,24 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         }
         return r;
     };
+    // LDS that the lanes of a wave hand each other: the hardware takes a wave's LDS requests in order, but one lane's loads
+    // depend on none of its own stores, so the compiler is told to keep the order.  (No instruction of its own.)
+    [[maybe_unused]] auto wave_handover = []() {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    };
     [[maybe_unused]] auto turn_round = [&](Operands &ops) {   // to inputs 8 c .. 8 c + 7 of the lane's word
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int c = 0; c < 4; ++c) *(u32x4 *)(turn_in + (16 * mt + 4 * c) * kTurnRow) = ops.x[mt][c];
+        wave_handover();
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
             for (int c = 0; c < 4; ++c) ops.x[mt][c] = *(const u32x4 *)(turn_out + 16 * mt * kTurnRow + 16 * c);
+        wave_handover();   // (the next step's stores)
     };
     auto multiply = [&](const Operands &ops, const Table (&tab)[kTables]) {
         Table t4[4];   // per output, or (block formats) per byte of the word
