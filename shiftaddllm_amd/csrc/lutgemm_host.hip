@@ -888,7 +888,13 @@ bool tile_wanted(const Problem &p, int mode)
     if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
     if (p.M <= 32) return false;
     const MfmaPlan plan = mfma_plan(p, true);
-    return plan.gemm && (plan.us == 0.0 || plan.us > gemm_us(p));
+    if (!plan.gemm || plan.us == 0.0) return plan.gemm;
+    // bf16 activations: the matrix-core kernel converts them on the way, 6 % (four planes) to 15 % (one) of its time; in front of the
+    // GEMM kernel that is a launch of 4.2 us and 1.3 per million.  us, fp16 and bf16 of either kernel (* = taken): 13184 -> 2944
+    // of 3 bits at 128 rows 31.7, 35.0* / 29.6*, 35.9; 4096 -> 4096 of 3 bits at 384 rows 34.7, 37.7* / 31.2*, 36.6; 13824 -> 5120 of 2 bits
+    // at 56 rows 26.8, 31.1 / 23.7*, 29.0*, of 3 bits at 1024 rows 307.9, 334.1 / 165.9*, 188.7*.
+    const double on_the_way = 1.18 - 0.03 * p.nb;
+    return p.x_type == kIoBF16 ? on_the_way * plan.us > gemm_us(p) + 4.2 + 1.3e-6 * ((double)p.M * p.K) : plan.us > gemm_us(p);
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)

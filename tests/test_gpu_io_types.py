@@ -1,9 +1,12 @@
 """LutLinear on bf16 and fp32 activations: the kernels that convert them themselves (one and two rows on the
 look-up kernel, few rows on the matrix-core kernels) and those that only write the caller's type, against the
 dense fp64 product of the activations as fp16."""
+import ctypes
+
 import pytest
 import torch
 
+from shiftaddllm_amd import native
 from shiftaddllm_amd.lut_gemm.quant import LutLinear, encode_apot_int8
 from test_gpu_tile import BLOCK_F16, BLOCK_I8, ROW, _dense, _scales
 
@@ -39,3 +42,27 @@ def test_activation_types_against_a_dense_product(gpu_device, fmt, K, N, nb, M, 
     off = torch.empty(M * K + 1, dtype=dtype, device=dev)[1:].view(M, K).copy_(x)
     with torch.no_grad():
         assert (lin(off).double() - want).norm().item() <= (3e-3 if dtype == torch.bfloat16 else 6e-4) * want.norm().item()
+
+
+@pytest.mark.parametrize("K,N,nb,M,one_launch", [(13184, 2944, 3, 100, True), (8192, 2432, 1, 300, True), (4096, 11008, 3, 48, True),
+                                                 (13824, 5120, 2, 56, False), (8192, 8192, 4, 96, False)])
+def test_bf16_calls_near_the_line_between_two_kernels(gpu_device, K, N, nb, M, one_launch):
+    """A conversion ahead of the GEMM kernel is part of its price: where the matrix-core kernel, which converts on the way, is
+    within that, a bf16 call is one launch.  LUTGEMM_EUNSUP asks the caller to convert."""
+    dev, lib, EUNSUP = gpu_device, native.cabi(), -3
+    g = torch.Generator(device=dev).manual_seed(K + N + M)
+    bW = torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 32, nb, N), generator=g, device=dev, dtype=torch.int32)
+    alpha = _scales(g, dev, K // 128, nb, N, "pow2").half()
+    x = torch.randn((M, K), generator=g, device=dev).bfloat16()
+    out = torch.full((M, N), float("nan"), dtype=torch.float32, device=dev)
+    def call(rows, x_type):
+        layer = native.Linear(bW.data_ptr(), alpha.data_ptr(), None, rows.data_ptr(), None, out.data_ptr(), ROW, N, K, nb, K // 128, M, 0, x_type, 2)
+        rc = lib.lutgemm_linear_f16(ctypes.byref(layer), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return rc
+    assert call(x, 1) == (0 if one_launch else EUNSUP)
+    if not one_launch:
+        assert call(x.half(), 0) == 0
+    want = x.half().double() @ _dense(ROW, bW, alpha, None)
+    # fp32 sums of K products: sqrt(K) roundings of 2^-24
+    assert float((out.double() - want).norm() / want.norm()) <= 2.0 ** -24 * K ** 0.5
