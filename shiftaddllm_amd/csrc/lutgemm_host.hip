@@ -494,6 +494,7 @@ struct MfmaPlan {
     int mt, slices;
     double us;
     bool gemm;   // the GEMM kernel is the other choice: faster than 5 us + a round's worst time per round of the widest cut, or never_cut
+    double gemm_us;   // gemm_estimate, where it was asked for
 };
 
 MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
@@ -501,7 +502,7 @@ MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
     const MfmaCost *const cost = kMfmaCost[p.alpha_mode == kRowF16 ? 0 : p.alpha_mode == kUniformF16 ? 1 : 2];
     const int rounds = ((p.K + kMfmaStepK - 1) / kMfmaStepK + kMfmaWaves - 1) / kMfmaWaves;
     const int most = !may_cut ? 1 : rounds < kMaxSlices ? rounds : kMaxSlices;
-    MfmaPlan best{0, 0, 0.0, false};
+    MfmaPlan best{};
     for (int mt = 1; mt <= 2; ++mt) {
         const MfmaCost &c = cost[mt - 1];
         const long tiles = (long)((p.N + kMfmaTileCols - 1) / kMfmaTileCols) * ((p.M + 16 * mt - 1) / (16 * mt));
@@ -510,7 +511,7 @@ MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
             if ((rounds + own - 1) / own != ks) continue;
             const double us = c.start + (double)((tiles * ks + 255) / 256) * (own * (c.round + c.plane * p.nb) + c.wg) +
                               (ks > 1 ? c.cut + c.words * 1e-6 * ((double)p.M * p.N * ks) : 0.0);
-            if (best.mt == 0 || us < best.us) best = MfmaPlan{mt, ks, us, false};
+            if (best.mt == 0 || us < best.us) best = MfmaPlan{mt, ks, us, false, 0.0};
         }
     }
     return best;
@@ -557,18 +558,21 @@ MfmaPlan mfma_plan(const Problem &p, bool or_gemm)
     const int slices = mfma_slices(one, mt);
     plan_mfma(one.p[0], mt, slices);
     bool cut = one.p[0].ksplit > 1, gemm = false;
+    double gemm_us = 0.0;
     if (or_gemm && p.M > 32) {
         Problem wide = p;
         plan_mfma(wide, 2, mt == 2 ? slices : mfma_slices(one, 2));
         const double round = 1.6 + 0.32 * p.nb + (is_block(p.alpha_mode) ? 0.9 : 0.0);
-        gemm = gemm_estimate(p) < 5.0 + round * (double)((wide.n_blocks + 255) / 256) * (double)(wide.sets_per_split / kMfmaWaves);
+        gemm_us = gemm_estimate(p);
+        gemm = gemm_us < 5.0 + round * (double)((wide.n_blocks + 255) / 256) * (double)(wide.sets_per_split / kMfmaWaves);
         // (uncut, the GEMM kernel is the other choice for these)
         if (cut && !gemm) gemm = never_cut(p);
         cut = cut && !gemm;
     }
-    if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm};
+    if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm, gemm_us};
     MfmaPlan plan = pick_mfma(p, cut, cut && p.M <= 32);
     plan.gemm = gemm;
+    plan.gemm_us = gemm_us;
     return plan;
 }
 
@@ -670,10 +674,11 @@ bool mfma_any(const Problem &p, int mode)
 
 bool tile_possible(const Problem &p, int mode);
 
-int plan_single(Problem &p, int mode, int *kernel, int *mrows)
+// `known`: tile_wanted's plan, where it made one
+int plan_single(Problem &p, int mode, const MfmaPlan &known, int *kernel, int *mrows)
 {
-    if (mfma_eligible(p, mode) || mfma_any(p, mode)) {
-        const MfmaPlan plan = mfma_plan(p, tile_possible(p, mode));
+    if (known.mt || mfma_eligible(p, mode) || mfma_any(p, mode)) {
+        const MfmaPlan plan = known.mt ? known : mfma_plan(p, tile_possible(p, mode));
         plan_mfma(p, plan.mt, plan.slices);
         *kernel = kMatrixCore;
         *mrows = 16 * plan.mt;
@@ -864,11 +869,11 @@ bool tile_possible(const Problem &p, int mode)
 // Up to 64 inputs, a single step of either kernel and outside what the estimates were fitted to, calls keep the line they had
 // (us, matrix-core kernel / this one, * = taken: 6028x64x4 at 33 rows 6.4 / 8.6*, 3100x64x3 at 200 7.0* / 9.6, 13800x64x3 at 128
 // 15.5 / 10.9*).
-double gemm_us(const Problem &p)
+double gemm_us(const Problem &p, double estimate)
 {
-    if (p.K <= 64) return 0.95 * gemm_estimate(p);
+    if (p.K <= 64) return 0.95 * estimate;
     const double planes = p.alpha_mode == kRowF16 ? 0.55 + 0.13 * p.nb : is_block(p.alpha_mode) ? 0.62 + 0.22 * p.nb : 0.60 + 0.40 * p.nb;
-    return 3.0 + planes * gemm_estimate(p);
+    return 3.0 + planes * estimate;
 }
 
 // Whether a call takes the GEMM kernel rather than the matrix-core kernel, by the two estimates (see mfma_plan for the
@@ -881,20 +886,24 @@ double gemm_us(const Problem &p)
 //   fp16 blocks: 5056x4096x4 at 64 17.9* / 27.6, 10240x7040x3 at 56 39.7 / 28.6*, 4800x8192x2 at 512 99.5 / 62.1*, 19008x3072x3 at 72 46.1 / 35.9*
 //   int8 exponents: 6144x3584x4 at 56 17.8* / 25.3, 13312x5760x3 at 36 41.5 / 29.8*, 7168x5120x3 at 128 38.6* / 32.1
 //   uniform: 21888x1024x4 at 72 39.9* / 53.0, 5312x7168x3 at 112 52.7 / 40.9*, 12864x2048x3 at 128 43.4* / 38.1
-bool tile_wanted(const Problem &p, int mode)
+// `planned`: the matrix-core kernel's plan, where one was made (mt = 0 otherwise).
+bool tile_wanted(const Problem &p, int mode, MfmaPlan *planned)
 {
+    MfmaPlan &plan = *planned;
+    plan = MfmaPlan{};
     if (!tile_possible(p, mode)) return false;
     if (option(LUTGEMM_OPTION_TILE_MIN_M) > 0) return true;
     if (!mfma_any(p, mode)) return p.M > 8;   // (the look-up kernel, four rows at a time, is the other choice)
     if (p.M <= 32) return false;
-    const MfmaPlan plan = mfma_plan(p, true);
+    plan = mfma_plan(p, true);
     if (!plan.gemm || plan.us == 0.0) return plan.gemm;
     // bf16 activations: the matrix-core kernel converts them on the way, 6 % (four planes) to 15 % (one) of its time; in front of the
     // GEMM kernel that is a launch of 4.2 us and 1.3 per million.  us, fp16 and bf16 of either kernel (* = taken): 13184 -> 2944
     // of 3 bits at 128 rows 31.7, 35.0* / 29.6*, 35.9; 4096 -> 4096 of 3 bits at 384 rows 34.7, 37.7* / 31.2*, 36.6; 13824 -> 5120 of 2 bits
     // at 56 rows 26.8, 31.1 / 23.7*, 29.0*, of 3 bits at 1024 rows 307.9, 334.1 / 165.9*, 188.7*.
     const double on_the_way = 1.18 - 0.03 * p.nb;
-    return p.x_type == kIoBF16 ? on_the_way * plan.us > gemm_us(p) + 4.2 + 1.3e-6 * ((double)p.M * p.K) : plan.us > gemm_us(p);
+    return p.x_type == kIoBF16 ? on_the_way * plan.us > gemm_us(p, plan.gemm_us) + 4.2 + 1.3e-6 * ((double)p.M * p.K)
+                                 : plan.us > gemm_us(p, plan.gemm_us);
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)
@@ -954,9 +963,10 @@ int run(int mode, const uint32_t *bW, const void *alpha, const void *qbias, cons
     p.out_type = out_type;
     // (ahead of the GEMM kernel: LUTGEMM_OPTION_BLOCK_SCALED = 2 means any number of rows)
     if (alpha_pow2 && mode == kRowF16 && mfma_eligible(p, mode) && p.M >= mfma_min_rows() && mx_wanted(p)) return run_mx(p, acc);
-    if (tile_wanted(p, mode)) return x_type == kIoF16 ? run_tile(p, mode, acc) : LUTGEMM_EUNSUP;
+    MfmaPlan planned;
+    if (tile_wanted(p, mode, &planned)) return x_type == kIoF16 ? run_tile(p, mode, acc) : LUTGEMM_EUNSUP;
     int kernel = kLookup, mrows = 1;
-    rc = plan_single(p, mode, &kernel, &mrows);
+    rc = plan_single(p, mode, planned, &kernel, &mrows);
     if (rc != LUTGEMM_OK) return rc;
     if (kernel == kMatrixCore) {
         if (x_type == kIoF32) return LUTGEMM_EUNSUP;   // (a step's operands would not fit the registers)
@@ -1798,7 +1808,8 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
     int rc = fill_described(p, format, N, K, nb, groups, M);
     if (rc != LUTGEMM_OK) return rc;
     *plan = lutgemm_plan{};
-    if (tile_wanted(p, format)) {
+    MfmaPlan planned;
+    if (tile_wanted(p, format, &planned)) {
         TileProblem t{};
         t.N = N;
         t.M = M;
@@ -1816,7 +1827,7 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
         return LUTGEMM_OK;
     }
     int kernel = kLookup, mrows = 1;
-    rc = plan_single(p, format, &kernel, &mrows);
+    rc = plan_single(p, format, planned, &kernel, &mrows);
     if (rc != LUTGEMM_OK) return rc;
     plan->kernel = kernel;
     plan->workgroups = p.n_blocks;
