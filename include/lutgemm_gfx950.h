@@ -316,7 +316,8 @@ typedef struct lutgemm_plan {
     int k_units;         /* sets of 256 inputs (look-up), steps of 128 (matrix cores), of 64 (GEMM; an even number) */
     /* look-up kernel: the tiles x k_units items of a row chunk, tile-major, are cut into
      * `ranges` contiguous ranges: the first `long_ranges` of `items_per_long_range`
-     * items, the others of `items_per_short_range` (the last one may be shorter) */
+     * items, the others of `items_per_short_range` (the last one may be shorter).
+     * GEMM kernel: `ranges` is the teams of waves that share the steps of a slice, 1 or 2. */
     int ranges, long_ranges, items_per_long_range, items_per_short_range;
     /* matrix-core and GEMM kernels: every tile is cut into `k_slices` slices of
      * `units_per_slice` steps (the last one may be shorter) */

@@ -1824,6 +1824,7 @@ int lutgemm_describe_plan(int format, int N, int K, int nb, int groups, int M, l
         plan->k_units = t.steps;
         plan->k_slices = t.ksplit;
         plan->units_per_slice = t.slice_steps;
+        plan->ranges = t.pair ? 2 : 1;
         return LUTGEMM_OK;
     }
     int kernel = kLookup, mrows = 1;

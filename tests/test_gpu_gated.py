@@ -55,6 +55,38 @@ def test_same_bits_as_two_launches(gpu_device, M, N, K, gate_bits, up_bits, grou
         torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("M,N,K", [(8, 1024, 1024), (16, 8192, 8192), (24, 1024, 4096)])   # one K-slice, several, 32-row tiles
+def test_special_activations_and_sums(gpu_device, M, N, K):
+    """Infinite and NaN sums (the exchanged word of an output is never taken for an empty one), sums beyond fp16, zeros of
+    either sign: the bits of two launches, NaN as NaN."""
+    dev, lib, nb = gpu_device, native.cabi(), 2
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    x = torch.randn((M, K), generator=g, device=dev).half()
+    x[0, 3], x[1, K - 1], x[2, K // 2] = float("nan"), float("inf"), -float("inf")
+    x[3] = 0.0
+    x[4] = 30000.0
+    outs = [torch.empty((M, N), dtype=torch.float16, device=dev) for _ in range(2)]
+    weights = [(torch.randint(-2 ** 31, 2 ** 31 - 1, (K // 32, nb, N), generator=g, device=dev, dtype=torch.int32),
+                (0.02 * torch.randn((8, nb, N), generator=g, device=dev)).half()) for _ in range(2)]
+    pair = (native.FusedProblem * 2)()
+    for i, (bW, alpha) in enumerate(weights):
+        pair[i] = native.FusedProblem(bW.data_ptr(), alpha.data_ptr(), x.data_ptr(), outs[i].data_ptr(), N, K, nb, 8, M, 1, None, None,
+                                      1e-5, None, None, None, None, 0)
+    want, act = torch.empty_like(outs[0]), torch.empty_like(outs[0])
+    sp = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    assert lib.lutgemm_gemv_rowwise_f16_fused(2, pair, sp) == 0
+    assert lib.lutgemm_decode_silu_mul_f16(outs[0].data_ptr(), outs[1].data_ptr(), want.data_ptr(), M * N, sp) == 0
+    torch.cuda.synchronize()
+    assert torch.isnan(want[0]).all() and not torch.isfinite(want[4]).all() and (want[3] == 0).all()
+    for _ in range(2):
+        act.fill_(7.0)
+        assert lib.lutgemm_gemv_rowwise_f16_gated(pair, act.data_ptr(), sp) == 0
+        torch.cuda.synchronize()
+        nan = torch.isnan(want)
+        assert torch.equal(torch.isnan(act), nan)
+        assert torch.equal(act[~nan].view(torch.int16), want[~nan].view(torch.int16))
+
+
 def test_what_is_refused(gpu_device):
     lib = native.cabi()
     t = torch.zeros(1 << 16, dtype=torch.float16, device=gpu_device)

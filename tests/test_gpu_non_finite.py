@@ -68,6 +68,30 @@ def test_special_activations_stay_in_their_rows(gpu_device, kernel, M, fmt, K, N
             assert not torch.isfinite(got[row]).any(), row
 
 
+@pytest.mark.parametrize("kernel,M,fmt,K,N,nb,groups,kind", [
+    # 32-row tiles, whose activations pass through LDS; K that fills no step; K-slices
+    (MFMA, 31, ROW, 1056, 33024, 4, 33, "any"), (MFMA, 32, BLOCK_F16, 4096, 8192, 4, 8, "any"), (MFMA, 20, ROW, 8192, 6144, 2, 64, "pow2"),
+    # two teams of waves per workgroup, of which one holds the value; several slices
+    (TILE, 129, ROW, 896, 20480, 3, 7, "pow2"), (TILE, 207, ROW, 9312, 256, 3, 97, "any"), (TILE, 39, BLOCK_F16, 7712, 940, 2, 5, "any"),
+    (TILE, 207, UNIFORM, 9312, 256, 2, 97, ""),
+])
+def test_special_activations_in_tall_tiles_and_teams(gpu_device, kernel, M, fmt, K, N, nb, groups, kind):
+    bW, alpha, q_bias, x = _problem(fmt, K, N, nb, groups, M, kind, gpu_device)
+    clean, plan = _call(kernel, fmt, bW, alpha, q_bias, x, groups, F32)
+    assert (plan.rows_per_pass == 32) if kernel == MFMA else plan.ranges == 2
+    special = {1: (float("nan"), 5), 3: (float("inf"), K - 1), 4: (-float("inf"), K // 2), 17: (float("inf"), K - 9), M - 1: (float("nan"), K - 1)}
+    for row, (value, k) in special.items():
+        x[row, k] = value
+    got, _ = _call(kernel, fmt, bW, alpha, q_bias, x, groups, F32)
+    for row in range(M):
+        if row not in special:
+            assert torch.equal(got[row], clean[row]), row
+        elif special[row][0] != special[row][0]:
+            assert torch.isnan(got[row]).all(), row
+        else:
+            assert not torch.isfinite(got[row]).any(), row
+
+
 @pytest.mark.parametrize("special", [float("inf"), float("nan")])
 @pytest.mark.parametrize("fmt,groups", [(ROW, 8), (UNIFORM, 8), (BLOCK_F16, 8)])
 @pytest.mark.parametrize("kernel,M", [(MFMA, 7), (TILE, 45)])

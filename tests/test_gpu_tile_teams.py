@@ -1,6 +1,7 @@
-"""GEMM kernel with two teams of waves per workgroup, each on half of a slice's steps: halves of unequal length, K that
-fills no step, tiles of 64 and 128 rows, several slices; against the dense fp64 product and, bit for bit, against the
-kernel that takes halves and slices in turn (a capture on a stream that holds no memory)."""
+"""GEMM kernel with two teams of waves per workgroup, each on half of a slice's steps: halves of unequal length, a slice of
+two steps, which leaves the second team none, K that fills no step, tiles of 64 and 128 rows; against the dense fp64
+product and, where there are several slices, bit for bit against the kernel that takes halves and slices in turn (a capture
+on a stream that holds no memory; calls of one slice are captured as they are)."""
 import ctypes
 
 import pytest
@@ -19,6 +20,12 @@ CASES = [   # sizes that are cut for teams
     (UNIFORM, 896, 20476, 3, 129, 7, "", 1),        # N off the tile
     (BLOCK_I8, 8192, 2560, 2, 256, 8, "pow2", 11),  # 12 steps a slice, the last one shorter
     (ROW, 8224, 8192, 4, 64, 257, "any", 7),        # 64-row tiles
+    (ROW, 9312, 256, 3, 207, 97, "any", 13),        # 12 steps a slice, the last one two
+    (UNIFORM, 9312, 256, 3, 207, 97, "", 13),
+    (BLOCK_F16, 10080, 1160, 4, 197, 5, "wide", 14),  # as above; row groups of 232 outputs, in two of which some waves' 64 lie
+    (UNIFORM, 4096, 4100, 2, 500, 32, "", 3),       # N off the tile
+    (BLOCK_F16, 4096, 4000, 3, 500, 5, "any", 4),
+    (BLOCK_I8, 7712, 940, 2, 39, 5, "pow2", 16),    # 64-row tiles
 ]
 
 
@@ -45,7 +52,7 @@ def test_teams_against_a_dense_product_and_in_turn(gpu_device, fmt, K, N, nb, M,
         alpha = _scales(g, dev, groups if fmt == ROW else K // 8, nb, N if fmt == ROW else groups, kind).half()
     plan = native.Plan()
     assert lib.lutgemm_describe_plan(fmt, N, K, nb, groups, M, ctypes.byref(plan)) == 0
-    assert plan.kernel == 3 and plan.k_slices == slices, (plan.kernel, plan.k_slices)
+    assert (plan.kernel, plan.k_slices, plan.ranges) == (3, slices, 2), (plan.kernel, plan.k_slices, plan.ranges, plan.units_per_slice, plan.k_units)
     out = torch.empty((M, N), dtype=torch.float32, device=dev)
     ptr = lambda t: t.data_ptr() if t is not None else None
     layer = native.Linear(ptr(bW), ptr(alpha), ptr(q_bias), ptr(x), None, ptr(out), fmt, N, K, nb, groups, M, 0, 0, 2)
