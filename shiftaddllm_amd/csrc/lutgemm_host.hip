@@ -1107,13 +1107,14 @@ int share_group(Problem *const *ps, int count, int xform, Shares *out)
     // the other's) or widths differ (finer shares): us, budget of 256 against 512, one row, 4096 inputs with RMSNorm: q,k,v of
     // 2, 3 and 4 bits 10.7 / 8.9, of 3 bits 9.0 / 8.8, grouped heads (4096 + 2 x 1024 outputs) 7.8 / 7.2, two rows 10.9 / 7.9;
     // without it q,k,v of 2, 3 and 4 bits 9.9 / 8.0, of 3 bits 7.65 / 8.2.  2048 inputs: 8 MB 6.3 / 6.9, two rows 9 MB
-    // 6.25 / 6.55.
+    // 6.25 / 6.55; 3072 inputs: one row, q,k,v of 2, 4 and 3 bits 7.4 / 7.7, of 3 bits 6.8 / 7.6, gate,up of 2 and 4 bits 9.6 / 9.1, of
+    // 3 bits 8.6 / 8.9 (two rows would gain there: 11.0 / 8.7, 9.2 / 8.3, 13.2 / 9.5 of 1 and 3 bits).
     const bool pairs = count > 1 && (xform == kXNorm || mixed) && long_rows && bytes >= (9l << 20) &&
                        option(LUTGEMM_OPTION_TARGET_BLOCKS) <= 0;
     const long usual = target_blocks(bytes), budget = pairs ? 512 : usual;
     // Callers that reserve nothing before a capture rely on which launches need accumulator words: none with the usual
-    // budget and the costs of a workgroup alone, none now.  (They do wherever every range of that share is of whole rows of
-    // items, which it is not if ranges that are all shorter than that of some problem fit.)
+    // budget and the costs of a workgroup alone, none now.  (That is where all its ranges are whole rows of items, nsets of
+    // them or a multiple; they are not if times too short for one row of the dearest problem already fit.)
     const Sharing alone{ps, count, kItemAlone, usual, false};
     double whole = 0.0;
     for (int i = 0; i < count; ++i) {
