@@ -495,6 +495,7 @@ struct MfmaPlan {
     double us;
     bool gemm;   // the GEMM kernel is the other choice: faster than 5 us + a round's worst time per round of the widest cut, or never_cut
     double gemm_us;   // gemm_estimate, where it was asked for
+    bool one_launch;  // no memory here, slices there
 };
 
 MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
@@ -511,7 +512,7 @@ MfmaPlan pick_mfma(const Problem &p, bool may_cut, bool must_cut)
             if ((rounds + own - 1) / own != ks) continue;
             const double us = c.start + (double)((tiles * ks + 255) / 256) * (own * (c.round + c.plane * p.nb) + c.wg) +
                               (ks > 1 ? c.cut + c.words * 1e-6 * ((double)p.M * p.N * ks) : 0.0);
-            if (best.mt == 0 || us < best.us) best = MfmaPlan{mt, ks, us, false, 0.0};
+            if (best.mt == 0 || us < best.us) best = MfmaPlan{mt, ks, us, false, 0.0, false};
         }
     }
     return best;
@@ -540,7 +541,7 @@ bool never_cut(const Problem &p)
     return best < 5.0 + 3.0 * rounds / 256.0;
 }
 
-double gemm_estimate(const Problem &p);
+double gemm_estimate(const Problem &p, bool *sliced);
 
 // The plan of a lone problem.  Which calls take accumulator words, and so need a reservation under capture: those that a
 // cut up to a workgroup per CU makes K-slices of, beyond 32 rows less those of never_cut and less those that the GEMM kernel is
@@ -557,22 +558,24 @@ MfmaPlan mfma_plan(const Problem &p, bool or_gemm)
     const int mt = p.M <= 16 || (p.M <= 64 && tiles * ((p.M + 15) / 16) * rounds <= 512) ? 1 : 2;
     const int slices = mfma_slices(one, mt);
     plan_mfma(one.p[0], mt, slices);
-    bool cut = one.p[0].ksplit > 1, gemm = false;
+    bool cut = one.p[0].ksplit > 1, gemm = false, one_launch = false;
     double gemm_us = 0.0;
     if (or_gemm && p.M > 32) {
         Problem wide = p;
         plan_mfma(wide, 2, mt == 2 ? slices : mfma_slices(one, 2));
         const double round = 1.6 + 0.32 * p.nb + (is_block(p.alpha_mode) ? 0.9 : 0.0);
-        gemm_us = gemm_estimate(p);
+        bool sliced = false;
+        gemm_us = gemm_estimate(p, &sliced);
         gemm = gemm_us < 5.0 + round * (double)((wide.n_blocks + 255) / 256) * (double)(wide.sets_per_split / kMfmaWaves);
-        // (uncut, the GEMM kernel is the other choice for these)
-        if (cut && !gemm) gemm = never_cut(p);
+        if (cut && !gemm) gemm = never_cut(p);   // (uncut, the GEMM kernel is the other choice for these)
+        one_launch = !cut && sliced;
         cut = cut && !gemm;
     }
-    if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm, gemm_us};
+    if (p.M <= 16 || mfma_blocks_override()) return MfmaPlan{mt, slices, 0.0, gemm, gemm_us, one_launch};
     MfmaPlan plan = pick_mfma(p, cut, cut && p.M <= 32);
     plan.gemm = gemm;
     plan.gemm_us = gemm_us;
+    plan.one_launch = one_launch;
     return plan;
 }
 
@@ -844,13 +847,15 @@ double plan_tile(TileProblem &t)
     return best_cost;
 }
 
-double gemm_estimate(const Problem &p)
+double gemm_estimate(const Problem &p, bool *sliced)
 {
     TileProblem t{};
     t.N = p.N;
     t.M = p.M;
     t.kwords = p.kwords;
-    return plan_tile(t);
+    const double us = plan_tile(t);
+    *sliced = t.ksplit > 1;
+    return us;
 }
 
 // What the GEMM kernel can take.
@@ -880,7 +885,7 @@ double gemm_us(const Problem &p, double estimate)
 // calls that may).  Drawn with 900 calls and checked on 3000 others near the line, timed on both (33 to 2048 rows, 512 to 28672
 // inputs and outputs): the kernel taken is within 1.0 % of the better one on average, 6 % of the calls lose more than 5 %.
 // Measured (us, matrix-core kernel / this one, * = taken):
-//   row-wise: 6464x4096x3 at 65 rows 18.0* / 22.8, 10944x5120x3 at 64 30.3 / 24.1*, 6144x5120x2 at 72 18.6* / 24.4, 7680x8192x3 at 112
+//   row-wise: 6464x4096x3 at 65 rows 18.0* / 22.8, 10944x5120x3 at 64 30.3* / 24.1, 6144x5120x2 at 72 18.6* / 24.4, 7680x8192x3 at 112
 //   40.0 / 33.1*, 3072x3328x3 at 256 22.3* / 24.3, 24128x3072x2 at 80 45.1 / 33.5*; scales that are no powers of two 3392x6144x3 at
 //   72 24.6* / 31.3, 15360x3328x3 at 33 30.0* / 37.2, 20096x1024x2 at 160 34.5 / 37.7*
 //   fp16 blocks: 5056x4096x4 at 64 17.9* / 27.6, 10240x7040x3 at 56 39.7 / 28.6*, 4800x8192x2 at 512 99.5 / 62.1*, 19008x3072x3 at 72 46.1 / 35.9*
@@ -899,11 +904,19 @@ bool tile_wanted(const Problem &p, int mode, MfmaPlan *planned)
     if (!plan.gemm || plan.us == 0.0) return plan.gemm;
     // bf16 activations: the matrix-core kernel converts them on the way, 6 % (four planes) to 15 % (one) of its time; in front of the
     // GEMM kernel that is a launch of 4.2 us and 1.3 per million.  us, fp16 and bf16 of either kernel (* = taken): 13184 -> 2944
-    // of 3 bits at 128 rows 31.7, 35.0* / 29.6*, 35.9; 4096 -> 4096 of 3 bits at 384 rows 34.7, 37.7* / 31.2*, 36.6; 13824 -> 5120 of 2 bits
-    // at 56 rows 26.8, 31.1 / 23.7*, 29.0*, of 3 bits at 1024 rows 307.9, 334.1 / 165.9*, 188.7*.
+    // of 3 bits at 128 rows 31.7, 35.0* / 29.6*, 35.9; 4096 -> 4096 of 3 bits at 384 rows 34.7, 37.7* / 31.2*, 36.6; 13824 -> 5120 of 3
+    // bits at 128 rows 58.8, 65.7 / 36.2*, 41.2*, at 1024 307.9, 334.1 / 165.9*, 188.7*.
     const double on_the_way = 1.18 - 0.03 * p.nb;
-    return p.x_type == kIoBF16 ? on_the_way * plan.us > gemm_us(p, plan.gemm_us) + 4.2 + 1.3e-6 * ((double)p.M * p.K)
-                                 : plan.us > gemm_us(p, plan.gemm_us);
+    const bool bf16 = p.x_type == kIoBF16;
+    const double here = bf16 ? on_the_way * plan.us : plan.us;
+    const double there = gemm_us(p, plan.gemm_us) + (bf16 ? 4.2 + 1.3e-6 * ((double)p.M * p.K) : 0.0);
+    // One launch without memory is given up for slices only where these are expected to save an eighth, or were the choice before the
+    // estimates: where their sums have no place (a capture with nothing reserved) they are taken in turn.  Of 70 calls that either rule
+    // would move, those kept in one launch took 4 % more with slices, the others 12 % less, and five times as long in turn (us,
+    // this kernel / slices / in turn: 13920x2560x2 at 75 rows 26.3* / 35.2 / 93, 4480x12800x3 at 34 27.1* / 29.1 / 261, 9120x9984x3 at 64 49.8 /
+    // 37.6* / 194).
+    if (here <= there || !plan.one_launch || here > 1.13 * there) return here > there;
+    return never_cut(p);
 }
 
 int run_tile(const Problem &p, int mode, const Accum &acc)

@@ -45,7 +45,7 @@ def test_activation_types_against_a_dense_product(gpu_device, fmt, K, N, nb, M, 
 
 
 @pytest.mark.parametrize("K,N,nb,M,one_launch", [(13184, 2944, 3, 100, True), (8192, 2432, 1, 300, True), (4096, 11008, 3, 48, True),
-                                                 (13824, 5120, 2, 56, False), (8192, 8192, 4, 96, False)])
+                                                 (13824, 5120, 3, 128, False), (8192, 8192, 4, 96, False)])
 def test_bf16_calls_near_the_line_between_two_kernels(gpu_device, K, N, nb, M, one_launch):
     """A conversion ahead of the GEMM kernel is part of its price: where the matrix-core kernel, which converts on the way, is
     within that, a bf16 call is one launch.  LUTGEMM_EUNSUP asks the caller to convert."""

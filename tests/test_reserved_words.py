@@ -80,3 +80,17 @@ def test_without_the_gemm_kernel_calls_are_cut(lib, fmt, N, K, nb, M, rows, slic
 def test_the_faster_kernel_where_they_differ_much(lib, fmt, N, K, nb, groups, M, kernel):  # noqa: F811
     rc, p = describe(lib, fmt, N, K, nb, groups, M)
     assert rc == 0 and p.kernel == kernel
+
+
+@pytest.mark.parametrize("N,K,nb,M,kernel", [
+    # us measured, one launch of the matrix-core kernel / the GEMM kernel's slices / those in turn
+    (13920, 2560, 2, 75, MATRIX_CORE),    # 26.3 / 35.2 / 93
+    (4480, 12800, 3, 34, MATRIX_CORE),    # 27.1 / 29.1 / 261
+    (10848, 3200, 4, 50, MATRIX_CORE),    # 26.6 / 32.4 / 110
+    (9120, 9984, 3, 64, GEMM),            # 49.8 / 37.6 / 194
+    (12816, 3072, 3, 123, GEMM),          # 47.4 / 34.2 / 74
+])
+def test_one_launch_is_given_up_for_slices_only_for_a_gain(lib, N, K, nb, M, kernel):  # noqa: F811
+    """Slices are taken in turn where their sums have no place, as under a capture with nothing reserved."""
+    rc, p = describe(lib, ROWWISE, N, K, nb, K // 128, M)
+    assert rc == 0 and p.kernel == kernel and not p.needs_workspace and (p.k_slices > 1) == (kernel == GEMM) and not never_cut(N, K, M)
