@@ -511,6 +511,28 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     // red[wave][j = (e*MT + mt)*4 + r][lane], rows padded to 65 words so that the
     // read-out below (consecutive threads = consecutive outputs) spreads over the banks
     float *red = (float *)xs;
+    // Thread t finishes output column t & 63 of rows (t >> 6) + 8*i: a wave covers 64
+    // consecutive outputs of one row, so its atomics and its fp16 read-modify-write
+    // fall into whole cache lines.
+    const int nl = tid & 63;
+    const int n = n_base + nl;
+    // What the caller had in those outputs is requested here, not where the sums are complete: the request then runs beside
+    // the reduction and the atomics instead of behind them (128 rows of int8 exponents 3072x768 11.3 -> 10.6 us, 4096x11008x3
+    // with a bias at 4 rows 10.0 -> 9.6).  Ahead of the main loop it costs registers that the operands need (8 sequences'
+    // down_proj of 4 planes 13.7 -> 14.7).  Whoever completes an output has read it before any contribution of its own, and
+    // nobody writes it before all contributions are there.
+    [[maybe_unused]] uint16_t init_bits[2 * MT];
+    [[maybe_unused]] uint16_t next_w_bits = 0;
+    if constexpr (!GATE) {
+#pragma unroll
+        for (int i = 0; i < 2 * MT; ++i) init_bits[i] = 0;
+        if (!p.overwrite)
+#pragma unroll
+            for (int i = 0; i < 2 * MT; ++i)
+                init_bits[i] = *(const uint16_t *)(p.init + (size_t)min(m0 + (tid >> 6) + 8 * i, p.M - 1) * p.init_stride + min(n, p.N - 1));
+        if constexpr (EXTRA)
+            if (p.next_w) next_w_bits = *(const uint16_t *)(p.next_w + min(n, p.N - 1));
+    }
     if constexpr (TURN) __syncthreads();   // (the waves' activations lie there)
 #pragma unroll
     for (int e = 0; e < 4; ++e)
@@ -520,16 +542,9 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             for (int r = 0; r < 4; ++r)
                 red[(wave * (16 * MT) + (e * MT + mt) * 4 + r) * kRedRow + lane] = acc[e][mt][r];
     __syncthreads();
-    // Thread t finishes output column t & 63 of rows (t >> 6) + 8*i: a wave covers 64
-    // consecutive outputs of one row, so its atomics and its fp16 read-modify-write
-    // fall into whole cache lines.
-    const int nl = tid & 63;
-    const int n = n_base + nl;
     const int src_lane = (nl >> 4) * 16;            // kb of the column; + li of the row below
     const int src_j = (nl & 3) * MT * 4 + ((nl >> 2) & 3);  // e and r of the column; + mt*4 of the row
-    [[maybe_unused]] float next_w = 0.0f;
-    if constexpr (EXTRA)
-        if (p.next_w) next_w = __half2float(p.next_w[min(n, p.N - 1)]);
+    [[maybe_unused]] const float next_w = half_bits_to_float(next_w_bits);
     float val[2 * MT];
     Contribution contrib[2 * MT];
     unsigned long long old[2 * MT];
@@ -583,7 +598,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         [[maybe_unused]] float sq = 0.0f;  // square of the output this thread completed
         if (m < p.M && n < p.N && (p.ksplit == 1 || (int)(old[i] >> 56) == p.ksplit - 1)) {
             const float y = p.ksplit == 1 ? val[i] : fixed_total((old[i] | contrib[i].flags) + contrib[i].add, p.ksplit);
-            const float sum = (p.overwrite ? 0.0f : __half2float(p.init[(size_t)m * p.init_stride + n])) + y;
+            const float sum = half_bits_to_float(init_bits[i]) + y;
             const __half y16 = __float2half_rn(sum);
             if constexpr (EXTRA)
                 p.out[(size_t)m * p.N + n] = y16;
