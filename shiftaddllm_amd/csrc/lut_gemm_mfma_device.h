@@ -341,13 +341,6 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
         }
         return r;
     };
-    // LDS that the lanes of a wave hand each other: the hardware takes a wave's LDS requests in order, but one lane's loads
-    // depend on none of its own stores, so the compiler is told to keep the order.  (No instruction of its own.)
-    [[maybe_unused]] auto wave_handover = []() {
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
-    };
     [[maybe_unused]] auto turn_round = [&](Operands &ops) {   // to inputs 8 c .. 8 c + 7 of the lane's word
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
@@ -517,12 +510,12 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     const int nl = tid & 63;
     const int n = n_base + nl;
     // What the caller had in those outputs is requested here, not where the sums are complete: the request then runs beside
-    // the reduction and the atomics instead of behind them (128 rows of int8 exponents 3072x768 11.3 -> 10.6 us, 4096x11008x3
-    // with a bias at 4 rows 10.0 -> 9.6).  Ahead of the main loop it costs registers that the operands need (8 sequences'
+    // the reduction and the atomics instead of behind them (128 rows of int8 exponents 3072x768 11.2 -> 10.4 us, 4096x4096x3
+    // with a bias at 16 rows 7.5 -> 6.9).  Ahead of the main loop it costs registers that the operands need (8 sequences'
     // down_proj of 4 planes 13.7 -> 14.7).  Whoever completes an output has read it before any contribution of its own, and
     // nobody writes it before all contributions are there.
-    [[maybe_unused]] uint16_t init_bits[2 * MT];
-    [[maybe_unused]] uint16_t next_w_bits = 0;
+    [[maybe_unused]] uint32_t init_bits[2 * MT];
+    [[maybe_unused]] uint32_t next_w_bits = 0;
     if constexpr (!GATE) {
 #pragma unroll
         for (int i = 0; i < 2 * MT; ++i) init_bits[i] = 0;
@@ -544,7 +537,6 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     __syncthreads();
     const int src_lane = (nl >> 4) * 16;            // kb of the column; + li of the row below
     const int src_j = (nl & 3) * MT * 4 + ((nl >> 2) & 3);  // e and r of the column; + mt*4 of the row
-    [[maybe_unused]] const float next_w = half_bits_to_float(next_w_bits);
     float val[2 * MT];
     Contribution contrib[2 * MT];
     unsigned long long old[2 * MT];
@@ -592,6 +584,11 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             }
         return;
     }
+    // (as new values: or they are converted, and waited for, where they were requested)
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) asm volatile("" : "+v"(init_bits[i]));
+    if constexpr (EXTRA) asm volatile("" : "+v"(next_w_bits));
+    [[maybe_unused]] const float next_w = half_bits_to_float(next_w_bits);
 #pragma unroll
     for (int i = 0; i < 2 * MT; ++i) {
         const int m = m0 + (tid >> 6) + 8 * i;

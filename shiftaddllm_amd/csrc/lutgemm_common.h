@@ -347,13 +347,22 @@ __device__ __forceinline__ void store_result(void *out, size_t i, float v, int t
 // Four consecutive fp16 values of any alignment (a bias row may begin on any of them) added to v.  The vector type
 // says so: the compiler then takes one 8-byte load, which this hardware allows at any address, because it may.
 typedef u32x2 u32x2_of_halves __attribute__((aligned(2)));
-__device__ __forceinline__ void add_halves(float (&v)[4], const __half *from)
+__device__ __forceinline__ void add_halves(float (&v)[4], const u32x2 old)
 {
-    const u32x2 old = *(const u32x2_of_halves *)from;
     v[0] += half_bits_to_float(old.x & 0xffffu);
     v[1] += half_bits_to_float(old.x >> 16);
     v[2] += half_bits_to_float(old.y & 0xffffu);
     v[3] += half_bits_to_float(old.y >> 16);
+}
+__device__ __forceinline__ void add_halves(float (&v)[4], const __half *from) { add_halves(v, *(const u32x2_of_halves *)from); }
+
+// LDS that the lanes of a wave hand each other: the hardware takes a wave's LDS requests in order, but one lane's loads
+// depend on none of its own stores, so the compiler is told to keep the order.  (No instruction of its own.)
+__device__ __forceinline__ void wave_handover()
+{
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
 }
 
 // four consecutive results
