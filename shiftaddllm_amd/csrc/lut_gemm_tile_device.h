@@ -160,28 +160,28 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     [[maybe_unused]] auto put_scale = [&](int t, const ScaleSlot &z, uint32_t u) {
         ((float *)stage_at(t))[z.dst] = decode_multiplier(u, p.mode);
     };
-    auto fetch_scales = [&](int t) {
+    auto fetch_scales = [&](int t, uint32_t (&to)[kFetched]) {
         if constexpr (BLOCK) {
-            fetched[0] = raw_scale(t, own);
+            to[0] = raw_scale(t, own);
         } else {
             // threads 0..127: two outputs each for the step's first word, the others for its second
             const uint32_t n = (uint32_t)min(n_tile * kTileN + 2 * (tid & 127), p.N - 2);
             const uint32_t g = (uint32_t)fast_div(min(2 * t + (tid >> 7), p.kwords - 1), p.by_group_words);
             if constexpr (UNI) {
                 const uint32_t at = (g * (uint32_t)p.N + n) * 2u;
-                fetched[0] = *(const uint32_t *)((const char *)p.alpha + at);
-                fetched[1] = *(const uint32_t *)((const char *)p.qbias + at);
+                to[0] = *(const uint32_t *)((const char *)p.alpha + at);
+                to[1] = *(const uint32_t *)((const char *)p.qbias + at);
             } else {
 #pragma unroll
                 for (int b = 0; b < NB; ++b)
-                    fetched[b] = *(const uint32_t *)((const char *)p.alpha + ((g * NB + (uint32_t)b) * (uint32_t)p.N + n) * 2u);
+                    to[b] = *(const uint32_t *)((const char *)p.alpha + ((g * NB + (uint32_t)b) * (uint32_t)p.N + n) * 2u);
             }
         }
     };
-    auto store_scales = [&](int t) {
+    auto store_scales = [&](int t, const uint32_t (&from)[kFetched]) {
         if constexpr (BLOCK) {
             const int all = 8 * NB * n_rg;
-            if (tid < all) put_scale(t, own, fetched[0]);
+            if (tid < all) put_scale(t, own, from[0]);
             for (int i = tid + kTileThreads; i < all; i += kTileThreads) {   // (row groups of a few outputs)
                 const ScaleSlot z = scale_slot(i);
                 put_scale(t, z, raw_scale(t, z));
@@ -191,8 +191,8 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
             unsigned short *dst = (unsigned short *)stage_at(t) + 2 * tid * kEach;
 #pragma unroll
             for (int b = 0; b < kFetched; ++b) {
-                dst[b] = (unsigned short)fetched[b];
-                dst[kEach + b] = (unsigned short)(fetched[b] >> 16);
+                dst[b] = (unsigned short)from[b];
+                dst[kEach + b] = (unsigned short)(from[b] >> 16);
             }
         }
     };
@@ -335,7 +335,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
     auto step = [&](int t, auto parity) {
         constexpr int P = decltype(parity)::value;
         store_x(P ^ 1);
-        fetch_scales(t + 2);
+        fetch_scales(t + 2, fetched);
         load_x(t + 2);
         if (lo_cur) {
             uint32_t y[2][4];
@@ -405,7 +405,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         });
         lo_cur = __builtin_amdgcn_ballot_w64(inexact) != 0ull;
         if (lo_cur) second_piece(t + 1, P ^ 1);
-        store_scales(t + 2);
+        store_scales(t + 2, fetched);
         __syncthreads();
     };
 
@@ -419,10 +419,12 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         // ---- prologue: step 0's activations in LDS, its weights in A[0] --------------------------------------
         load_x(t0);
         load_words(t0, words);
-        fetch_scales(t0);
-        store_scales(t0);
-        fetch_scales(t0 + 1);
-        store_scales(t0 + 1);
+        uint32_t of_first[kFetched];
+        fetch_scales(t0, of_first);
+        fetch_scales(t0 + 1, fetched);
+        __builtin_amdgcn_sched_barrier(0);
+        store_scales(t0, of_first);
+        store_scales(t0 + 1, fetched);
         store_x(0);
         load_x(t0 + 1);
         __syncthreads();
@@ -493,27 +495,73 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 
     // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
     // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
+    // What the sums are added to is requested a 32-row fragment ahead of its use (1024x16384x3 at 512 rows with a bias 30.4 -> 27.2 us,
+    // 256x15360x3 at 330 rows 19.4 -> 14.4).
+    // `turn`: Stored from the accumulators, an instruction touches 32 rows' lines.  Teams, whose sums pass through LDS anyway, turn
+    // them round there (16-byte chunk c of row r in slot c ^ r), so that an instruction stores 32 outputs of eight rows: 4096x4096x4 at
+    // 512 rows, two slices, 37.7 -> 36.3 us.  A lone team's two more passes through LDS cost more than it gives: 640x5376x3 at
+    // 759 rows 19.1 -> 20.3.
     float *sums = !SERIAL && p.ksplit > 1 ? p.partial + (size_t)slice * tile_slice_stride(p.M, p.N) : nullptr;
-    auto write_out = [&](auto f_c) {
+    const bool add = !sums && !p.overwrite;
+    auto write_out = [&](auto f_c, auto &&turn) {
         constexpr int f = decltype(f_c)::value;
+        constexpr bool TURN = KIND == kTilePair;
+        const int here = opaque(lane);   // (nothing formed from it is worth a register of the main loop)
+        // piece u of a fragment: the lane's row and output in it
+        auto row = [&](int u) { return TURN ? here / 8 + 8 * u : here & 31; };
+        auto output = [&](int u) { return n0 + 32 * f + (TURN ? 4 * (here & 7) : 8 * u + 4 * (here / 32)); };
+        u32x2 init[2][4];
+        auto request = [&](int i) {
+            if (add)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    init[i & 1][u] = *(const u32x2_of_halves *)(p.init + (size_t)min(m0 + 32 * i + row(u), p.M - 1) * p.init_stride + min(output(u), p.N - 4));
+        };
+        request(0);
 #pragma unroll
         for (int i = 0; i < MF; ++i) {
-            const int m = m0 + 32 * i + l32;
-            if (m >= p.M) continue;
+            if (i + 1 < MF) request(i + 1);
+            f32x4 v4[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-                const int n = n0 + 32 * f + 8 * g + 4 * kh;
-                if (n >= p.N) continue;
-                float v[4];
+            for (int u = 0; u < 4; ++u)
 #pragma unroll
-                for (int r = 0; r < 4; ++r) v[r] = acc[f][i][4 * g + r];
-                if (sums) {
-                    *(f32x4 *)(sums + (size_t)m * p.N + n) = (f32x4){v[0], v[1], v[2], v[3]};
-                    continue;
-                }
-                if (!p.overwrite) add_halves(v, p.init + (size_t)m * p.init_stride + n);
-                store_results(p.out, (size_t)m * p.N + n, v, p.out_type);
+                for (int r = 0; r < 4; ++r) v4[u][r] = acc[f][i][4 * u + r];
+            if constexpr (TURN) {
+                char *const at = turn(i);
+#pragma unroll
+                for (int u = 0; u < 4; ++u) *(f32x4 *)(at + (here & 31) * 128 + (((2 * u + here / 32) ^ (here & 7)) * 16)) = v4[u];
+                wave_handover();
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v4[u] = *(const f32x4 *)(at + row(u) * 128 + (((here & 7) ^ (row(u) & 7)) * 16));
             }
+            auto store_all = [&](auto &&store) {
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const int m = m0 + 32 * i + row(u), n = output(u);
+                    if (m < p.M && n < p.N) store((size_t)m * p.N + n, v4[u]);
+                }
+            };
+            if (sums) {
+                store_all([&](size_t at, const f32x4 &v) { *(f32x4 *)(sums + at) = v; });
+                continue;
+            }
+            if (add)
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    asm volatile("" : "+v"(init[i & 1][u]));   // (as new values: or they are converted, and waited for, where they were requested)
+                    float v[4] = {v4[u][0], v4[u][1], v4[u][2], v4[u][3]};
+                    add_halves(v, init[i & 1][u]);
+                    v4[u] = (f32x4){v[0], v[1], v[2], v[3]};
+                }
+            auto results = [&](int type) {
+                store_all([&](size_t at, const f32x4 &v4) {
+                    const float v[4] = {v4[0], v4[1], v4[2], v4[3]};
+                    store_results(p.out, at, v, type);
+                });
+            };
+            if (p.out_type == kIoF32) results(kIoF32);
+            else if (p.out_type == kIoBF16) results(kIoBF16);
+            else results(kIoF16);
         }
     };
     if constexpr (KIND == kTilePair) {
@@ -539,7 +587,8 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 #pragma unroll
                     for (int r = 0; r < 4; ++r) acc[mine][i][4 * g + r] += v[r];
                 }
-            write_out(mine_c);
+            wave_handover();   // (the lanes' pieces have been read: the wave turns its sums round where they lay)
+            write_out(mine_c, [&](int i) { return lds_all + ((1 - mine) * 4 + wave) * MF * 4096 + i * 4096; });
         };
         __syncthreads();   // (the LDS of both teams changes hands)
         if (team == 0)
@@ -547,8 +596,8 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         else
             finish(std::integral_constant<int, 1>());
     } else {
-        write_out(std::integral_constant<int, 0>());
-        write_out(std::integral_constant<int, 1>());
+        write_out(std::integral_constant<int, 0>(), nullptr);
+        write_out(std::integral_constant<int, 1>(), nullptr);
     }
 }
 
