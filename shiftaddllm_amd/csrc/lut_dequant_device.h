@@ -153,12 +153,14 @@ __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntri
 }
 
 // Whether some entry may be no fp16 number.  The entries of up to three planes are looked at themselves.
-// More of them are bounded by the multipliers: all are multiples of u, the smallest of the multipliers' lowest
-// set bits, and at most the sum of magnitudes, so they are fp16 numbers where that is at most 2048 u (eleven
-// bits) and u is no less than 2^-24 (the smallest fp16 number): a third of the instructions.  (bits & bits - 1
-// clears the lowest mantissa bit; on a power of two it clears an exponent bit instead, which halves u at
-// worst.)  A zero multiplier counts for nothing; NaN and infinity are inexact.
-template <int NB, bool UNI>
+// More of them are bounded by the multipliers, a third of the instructions: all are sums of these, so they are fp16 numbers where
+// every multiplier is a multiple of u, their sum of magnitudes at most 2048 u (eleven bits) and u no less than 2^-24 (the
+// smallest fp16 number).  NaN and infinity are inexact.  LOWEST: u is the smallest of the multipliers' lowest set bits.  (bits & bits
+// - 1 clears the lowest mantissa bit; on a power of two it clears an exponent bit instead, which halves u at worst.  A zero
+// multiplier counts for nothing.)  Otherwise u follows from the sum, and adding and taking away 1.5 * 2^23 u rounds a multiplier to
+// a multiple of it: half the instructions (4096x11008x4 at 1024 rows 137.4 -> 134.3 us, 18016x432x4 at 407 36.2 -> 33.5, 8192x28672x4 at 32
+// 47.7 -> 47.0), but 16-row tiles, which have no registers for it, lose (8192x8192x4 in groups of 32 at 8 rows 21.9 -> 28.8).
+template <int NB, bool UNI, bool LOWEST>
 __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const float (&a)[NB], float q)
 {
     if constexpr (TableEntries<NB, UNI>::kCount <= 4) {
@@ -167,6 +169,19 @@ __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const 
 #pragma unroll
         for (int i = 0; i < t.kCount; ++i) bits |= __builtin_bit_cast(uint32_t, r.e[i]);
         return (bits << 1) != 0u;
+    }
+    if constexpr (!LOWEST) {
+        float sum = UNI ? fabsf(q) : 0.0f;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) sum += fabsf(a[b]);
+        const float below = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, sum) & 0x7f800000u);   // 2^10 u
+        const float magic = fmaxf(below, 0x1p-14f) * 0x1.8p13f;
+        auto off = [&](float v) { return !((v + magic) - magic == v); };
+        bool rounds = !(sum <= 32768.0f);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) rounds = off(a[b]) || rounds;
+        if constexpr (UNI) rounds = off(q) || rounds;
+        return rounds;
     }
     float sum = 0.0f, least = 3.0e38f;
     auto take = [&](float v) {

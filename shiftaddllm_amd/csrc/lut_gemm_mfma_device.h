@@ -326,7 +326,7 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
             if (lo) {
                 pack_table(table_residual(e), tab[i]);
             } else {
-                inexact = may_round<NB, UNI>(e, a, q * u) || inexact;
+                inexact = may_round<NB, UNI, MT == 1>(e, a, q * u) || inexact;
                 pack_table(e, tab[i]);
             }
         }

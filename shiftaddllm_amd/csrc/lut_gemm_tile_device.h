@@ -254,7 +254,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
             return false;
         }
         pack_table(e, tab[f][c]);
-        return may_round<NB, UNI>(e, a, q * u);
+        return may_round<NB, UNI, FMT == kTileBlock>(e, a, q * u);
     };
     auto make_tables = [&](int t, bool lo) {
         bool inexact = false;
@@ -362,32 +362,62 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         // indices are live at a time; where both fragments share their tables, chunk after chunk.  The loop needs every
         // register there is: with both fragments' at once it reloaded spilled values behind all loads in flight,
         // 8192x8192x4 at 128 rows 51 us instead of 41.5, 11008x4096x4 at 2048 rows 294 instead of 242.)
+        // Items, in order, and about how many vector instructions each takes; an item goes to the slot in which its share
+        // of all of them lies, so that the matrix instructions have as even a load beside them as may be (against items of whole
+        // operands, as many in each slot: 640x5376x3 at 759 rows 19.5 -> 19.1 us, int8 exponents 28.0 -> 25.9).
         constexpr bool WIDE = FMT == kTileBlockWide;
-        constexpr int kFragment = BLOCK ? 10 : 7, kItems = WIDE ? 3 + 4 * 3 : 2 * kFragment, kSlots = 4 * MF;
+        constexpr int kSigns = NB == 4 ? 23 : 5 + 4 * NB, kLoad = 2 * NB, kTable = 8 << (NB - 1), kQuarter = NB == 4 ? 7 : 6;
+        constexpr int kFragment = BLOCK ? 2 + 4 * 2 : 3 + 8, kItems = WIDE ? 3 + 4 * 5 : 2 * kFragment, kSlots = 4 * MF;
+        auto weight = [](int k) constexpr {
+            if (WIDE) return k < 2 ? kSigns + 4 : k == 2 ? 2 * kLoad : (k - 3) % 5 == 0 ? kTable : kQuarter;
+            const int r = k % kFragment - 2;
+            return r == -2 ? +kSigns : r == -1 ? +kLoad : r == 0 ? +kTable : +kQuarter;
+        };
+        auto first_item = [weight](int slot) constexpr {
+            if (BLOCK && !WIDE) return slot * kItems / kSlots;   // (finer items cost registers it does not have: 4096x4160x4 at 700 rows 68 -> 78 us)
+            int all = 0, before = 0, k = 0;
+            for (int i = 0; i < kItems; ++i) all += weight(i);
+            while (k < kItems && (2 * before + weight(k)) * kSlots < 2 * all * slot) before += weight(k++);
+            return k;
+        };
         auto item = [&](auto k_c) {
             constexpr int k = decltype(k_c)::value;
             if constexpr (WIDE) {
-                constexpr int r = k - 3, c = r / 3, f = r % 3 - 1;
+                constexpr int r = k - 3, c = r / 5, q = r % 5 - 1;
                 if constexpr (k < 2)
                     sign_indices<NB, UNI>(words[k], y[k]);
                 else if constexpr (k == 2)
                     load_words(t + 2, words);
-                else if constexpr (f < 0)
+                else if constexpr (q < 0)
                     inexact = make_table(t + 1, false, 0, c) || inexact;
-                else
-                    A[P ^ 1][c][f] = pick(f, c, y[f]);
+                else {   // half of an operand
+                    constexpr int f = q / 2, half = q % 2;
+                    const u32x2 v = pick_four<NB, UNI, half>(y[f][c], tab[0][c]);
+                    A[P ^ 1][c][f][2 * half] = v.x;
+                    A[P ^ 1][c][f][2 * half + 1] = v.y;
+                }
             } else {
                 constexpr int f = k / kFragment, r = k % kFragment - 2;
-                constexpr bool table = BLOCK ? r % 2 == 0 : r == 0;
-                constexpr int c = BLOCK ? r / 2 : table ? 0 : r - 1;
-                if constexpr (r == -2)
+                if constexpr (r == -2 && BLOCK)
                     sign_indices<NB, UNI>(words[f], y[f]);
+                else if constexpr (r == -2)
+                    sign_pairs<NB, UNI>(words[f], y[f]);
                 else if constexpr (r == -1)
                     load_fragment(t + 2, f, words[f]);
-                else if constexpr (table)
-                    inexact = make_table(t + 1, false, f, c) || inexact;
-                else
-                    A[P ^ 1][c][f] = pick(f, c, y[f]);
+                else if constexpr (BLOCK) {
+                    constexpr int c = r / 2;
+                    if constexpr (r % 2 == 0)
+                        inexact = make_table(t + 1, false, f, c) || inexact;
+                    else
+                        A[P ^ 1][c][f] = pick(f, c, y[f]);
+                } else if constexpr (r == 0) {
+                    inexact = make_table(t + 1, false, f, 0) || inexact;
+                } else {   // a quarter of a pair of operands
+                    constexpr int q = r - 1, h = q / 4, z = q % 2, half = q / 2 % 2;
+                    const u32x2 v = pick_four<NB, UNI, half>(y[f][2 * h + z], tab[f][0]);
+                    A[P ^ 1][2 * h][f][z + 2 * half] = v.x;
+                    A[P ^ 1][2 * h + 1][f][z + 2 * half] = v.y;
+                }
             }
         };
         f16x8 b = activations(P, 0, 0);
@@ -398,7 +428,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 #pragma unroll
             for (int f = 0; f < 2; ++f)
                 acc[f][i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, A[P][j][f]), b, acc[f][i], 0, 0, 0);
-            constexpr int first = s * kItems / kSlots, count = (s + 1) * kItems / kSlots - first;
+            constexpr int first = first_item(s), count = (s + 1 < kSlots ? first_item(s + 1) : kItems) - first;
             static_for<count>([&](auto c_c) { item(std::integral_constant<int, first + decltype(c_c)::value>()); });
             b = next;
             __builtin_amdgcn_sched_barrier(0);
