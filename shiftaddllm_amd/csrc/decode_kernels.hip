@@ -240,9 +240,9 @@ attention_kernel(const __half *__restrict__ q, const __half *__restrict__ k, con
     }
 }
 
-// The query heads of a kv head and how workgroups are given to them: 1 << spread (sequence, kv head) pairs side by side.
+// The query heads of a kv head and how workgroups are given to them: 1 << spread (sequence, kv head) pairs, of `pairs`, side by side.
 struct HeadLayout {
-    int rep, KV, spread;
+    int rep, KV, spread, pairs;
     uint32_t rep_reciprocal, KV_reciprocal;
 };
 
@@ -258,7 +258,13 @@ struct HeadLayout {
 // exponentials and weighted value sum (the "online" form of softmax); the rows of a wave are merged by lane
 // exchanges, the waves through LDS.
 //
-// Heads of one kv head sit on one XCD, behind one L2, where the count of kv heads allows it.
+// Heads of one kv head sit on one XCD, behind one L2: eight (sequence, kv head) pairs lie side by side, one to an XCD, and
+// workgroups beyond the last pair leave at once (with places only where eight divides the pairs, 14 sequences of 40 heads on 10 kv
+// heads at position 1887 lost the sharing: a step of three blocks 524 -> 449 us).
+// Cached rows are read non-temporally: no launch behind this one finds them in a cache (256 MB hold less than three
+// blocks' 92 MB), and kept there they push out what is found, the activations and norms of the step.  A token for eight
+// sequences at position 700 2258 -> 2166 us, four blocks of eight sequences of 32 heads on 8 kv heads at position 1000 318 -> 306.
+// (Heads that share rows have to sit behind one L2 for it: spread over the XCDs 524 -> 564 us in the first example.)
 //
 // Eight sequences of 32 heads at position 700 (92 MB): 23.1 -> 20.0 us, of which 3.3 are what position 0 takes;
 // one sequence at position 255: 7.1 -> 6.4.  Before, whole blocks were fetched and then worked on, and the rotated
@@ -278,6 +284,7 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     constexpr int kRows = 8;
     constexpr int kBlock = kRows * kPosGroups;  // positions
     constexpr int kWaves = T / 64;
+    constexpr int kNonTemporal = 2;   // (of a buffer load's cache policy)
     __shared__ float part[kWaves][HD], wave_mx[kWaves], wave_total[kWaves];
 
     const int tid = threadIdx.x;
@@ -288,6 +295,7 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     int group = lutgemm::quotient(at, rep, layout.rep_reciprocal);      // (sequence, kv head) and the query head within it
     const int member = at - group * rep;
     group = (group << layout.spread) + (blockIdx.x & ((1 << layout.spread) - 1));
+    if (group >= layout.pairs) return;
     const int b = lutgemm::quotient(group, KV, layout.KV_reciprocal), kvh = group - b * KV, h = kvh * rep + member;
     const int jg = tid / kChunks, ch = tid % kChunks;
     const int other = ch < kChunks / 2 ? ch + kChunks / 2 : ch - kChunks / 2;   // the chunk ch is rotated with
@@ -313,7 +321,7 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     auto fetch = [&](auto rsrc, u32x4 (&row)[kRows], int j0) {
 #pragma unroll
         for (int u = 0; u < kRows; ++u)
-            row[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16 + (j0 + u * kPosGroups) * (HD * 2), 0, 0);   // (scalar offsets escape the range check)
+            row[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16 + (j0 + u * kPosGroups) * (HD * 2), 0, kNonTemporal);   // (scalar offsets escape the range check)
     };
     fetch(krsrc, krow, 0);
     fetch(vrsrc, vrow, 0);
@@ -498,10 +506,10 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
     // (16-byte loads of every operand: others go to the general kernel)
     if ((head_dim == 64 || head_dim == 128) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
         const int rep = heads / kv_heads;
-        const HeadLayout layout{rep, kv_heads, rep > 1 && (long)batch * kv_heads % 8 == 0 ? 3 : 0, lutgemm::reciprocal_of(rep),
-                                lutgemm::reciprocal_of(kv_heads)};
+        const int pairs = batch * kv_heads, spread = rep > 1 ? 3 : 0;
+        const HeadLayout layout{rep, kv_heads, spread, pairs, lutgemm::reciprocal_of(rep), lutgemm::reciprocal_of(kv_heads)};
         auto launch = [&](auto kernel, int threads) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(batch * heads)), dim3(threads), 0, (hipStream_t)stream,
+            hipLaunchKernelGGL(kernel, dim3((unsigned)(((((pairs - 1) >> spread) + 1) << spread) * rep)), dim3(threads), 0, (hipStream_t)stream,
                                (const __half *)q, (const __half *)k, (const __half *)v, (const __half *)cos_table,
                                (const __half *)sin_table, (__half *)k_cache, (__half *)v_cache,
                                (const long long *)position, (__half *)out, layout, max_positions);
