@@ -261,9 +261,9 @@ struct HeadLayout {
 // Heads of one kv head sit on one XCD, behind one L2: eight (sequence, kv head) pairs lie side by side, one to an XCD, and
 // workgroups beyond the last pair leave at once (with places only where eight divides the pairs, 14 sequences of 40 heads on 10 kv
 // heads at position 1887 lost the sharing: a step of three blocks 524 -> 449 us).
-// Cached rows are read non-temporally: no launch behind this one finds them in a cache (256 MB hold less than three
-// blocks' 92 MB), and kept there they push out what is found, the activations and norms of the step.  A token for eight
-// sequences at position 700 2258 -> 2166 us, four blocks of eight sequences of 32 heads on 8 kv heads at position 1000 318 -> 306.
+// ONCE: cached rows are read non-temporally: no launch behind this one finds them in a cache (256 MB hold less than three
+// blocks' 92 MB), and kept there they push out what is found, the activations and norms of the step.  A launch for eight
+// sequences at position 700 19.4 -> 17.3 us, a token 2258 -> 2166, four blocks of eight sequences of 32 heads on 8 kv heads at position 1000 318 -> 306.
 // (Heads that share rows have to sit behind one L2 for it: spread over the XCDs 524 -> 564 us in the first example.)
 //
 // Eight sequences of 32 heads at position 700 (92 MB): 23.1 -> 20.0 us, of which 3.3 are what position 0 takes;
@@ -272,7 +272,7 @@ struct HeadLayout {
 // The start is a chain of round trips: the arguments (asked for at once), the position, the first rows.  Off it since: the
 // software divisions that found a workgroup's head, and, in wave 0, the new position's rows being asked for behind the
 // earlier ones' (eight sequences at position 700 20.3 -> 19.4 us on the device, a token for one sequence 1402 -> 1394).
-template <int HD, int T>
+template <int HD, int T, bool ONCE>
 __global__ void __launch_bounds__(T) __attribute__((amdgpu_waves_per_eu(4, 4)))
 attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, const __half *__restrict__ v,
                     const __half *__restrict__ cos_t, const __half *__restrict__ sin_t,
@@ -321,7 +321,7 @@ attention_hd_kernel(const __half *__restrict__ q, const __half *__restrict__ k, 
     auto fetch = [&](auto rsrc, u32x4 (&row)[kRows], int j0) {
 #pragma unroll
         for (int u = 0; u < kRows; ++u)
-            row[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16 + (j0 + u * kPosGroups) * (HD * 2), 0, kNonTemporal);   // (scalar offsets escape the range check)
+            row[u] = __builtin_amdgcn_raw_buffer_load_b128(rsrc, tid * 16 + (j0 + u * kPosGroups) * (HD * 2), 0, ONCE ? kNonTemporal : 0);   // (scalar offsets escape the range check)
     };
     fetch(krsrc, krow, 0);
     fetch(vrsrc, vrow, 0);
@@ -506,7 +506,11 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
     // (16-byte loads of every operand: others go to the general kernel)
     if ((head_dim == 64 || head_dim == 128) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
         const int rep = heads / kv_heads;
-        const int pairs = batch * kv_heads, spread = rep > 1 ? 3 : 0;
+        // Caches of less than 8 MB a block (small networks, short contexts) may still lie in the memory-side cache at the next
+        // token: read as usual (3 sequences of 8 heads on 2 kv heads, 2048 positions, 6 MB: a step 121.5 us, 122.8 otherwise).
+        const int pairs = batch * kv_heads;
+        const bool once = (long)pairs * max_positions * head_dim * 4 >= 8l << 20;
+        const int spread = rep > 1 && (once || pairs % 8 == 0) ? 3 : 0;
         const HeadLayout layout{rep, kv_heads, spread, pairs, lutgemm::reciprocal_of(rep), lutgemm::reciprocal_of(kv_heads)};
         auto launch = [&](auto kernel, int threads) {
             hipLaunchKernelGGL(kernel, dim3((unsigned)(((((pairs - 1) >> spread) + 1) << spread) * rep)), dim3(threads), 0, (hipStream_t)stream,
@@ -518,8 +522,12 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
         // With fewer workgroups than CUs eight waves each instead of four: 32 heads at position 255 6.4 us against
         // 6.7; 256 workgroups at position 700 20.4 against 20.0, where the memory is what they wait for.
         const bool wide = (long)batch * heads < 256;
-        if (head_dim == 128) return wide ? launch(attention_hd_kernel<128, 512>, 512) : launch(attention_hd_kernel<128, 256>, 256);
-        return wide ? launch(attention_hd_kernel<64, 512>, 512) : launch(attention_hd_kernel<64, 256>, 256);
+        auto launch_as = [&](auto once_c) {
+            constexpr bool ONCE = decltype(once_c)::value;
+            if (head_dim == 128) return wide ? launch(attention_hd_kernel<128, 512, ONCE>, 512) : launch(attention_hd_kernel<128, 256, ONCE>, 256);
+            return wide ? launch(attention_hd_kernel<64, 512, ONCE>, 512) : launch(attention_hd_kernel<64, 256, ONCE>, 256);
+        };
+        return once ? launch_as(std::true_type()) : launch_as(std::false_type());
     }
     const int groups = kThreads / head_dim;
     const size_t lds = sizeof(float) * ((size_t)3 * head_dim + max_positions + 4 + (size_t)groups * head_dim);
