@@ -646,6 +646,24 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
                                  void *out, int batch, int heads, int kv_heads, int head_dim, int max_positions,
                                  void *stream);
 
+/* The same for a caller that knows how many bytes of weights and the like a token reads besides cached keys and values
+ * (`step_bytes`; 0 = not known, as the call above).  Results are the same, bit for bit; where so much passes between two
+ * tokens that cached rows cannot be found again, they are read past the caches (lutgemm_describe_attention_plan). */
+int lutgemm_decode_attention_step_f16(const void *q, const void *k, const void *v, const void *cos_table,
+                                      const void *sin_table, void *k_cache, void *v_cache, const int64_t *position,
+                                      void *out, int batch, int heads, int kv_heads, int head_dim, int max_positions,
+                                      size_t step_bytes, void *stream);
+
+/* How an attention call would be launched (host arithmetic): by the kernel for any head size (`general`; so are operands
+ * off 16-byte alignment), how many workgroups of how many threads, whether (sequence, kv head) pairs are placed one to
+ * an XCD (the grid is then filled up to eight of them), and whether cached rows are read past the caches (`once`).
+ * Returns what the call would return for these sizes. */
+typedef struct lutgemm_attention_plan {
+    int general, workgroups, threads, placed, once;
+} lutgemm_attention_plan;
+int lutgemm_describe_attention_plan(int batch, int heads, int kv_heads, int head_dim, int max_positions, size_t step_bytes,
+                                    lutgemm_attention_plan *plan);
+
 /* out = fp16(fp16(silu(gate)) * up) over `count` values (multiple of 8);
  * pointers 16-byte aligned. */
 int lutgemm_decode_silu_mul_f16(const void *gate, const void *up, void *out, size_t count, void *stream);

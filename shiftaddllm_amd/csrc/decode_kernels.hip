@@ -261,10 +261,9 @@ struct HeadLayout {
 // Heads of one kv head sit on one XCD, behind one L2: eight (sequence, kv head) pairs lie side by side, one to an XCD, and
 // workgroups beyond the last pair leave at once (with places only where eight divides the pairs, 14 sequences of 40 heads on 10 kv
 // heads at position 1887 lost the sharing: a step of three blocks 524 -> 449 us).
-// ONCE: cached rows are read non-temporally: no launch behind this one finds them in a cache (256 MB hold less than three
-// blocks' 92 MB), and kept there they push out what is found, the activations and norms of the step.  A launch for eight
-// sequences at position 700 19.4 -> 17.3 us, a token 2258 -> 2166, four blocks of eight sequences of 32 heads on 8 kv heads at position 1000 318 -> 306.
-// (Heads that share rows have to sit behind one L2 for it: spread over the XCDs 524 -> 564 us in the first example.)
+// ONCE: cached rows are read non-temporally (read_once says for which steps, and what it gives).  A launch for eight sequences at
+// position 700 19.4 -> 17.3 us.  (Heads that share rows have to sit behind one L2 for it: spread over the XCDs 524 -> 564 us in the
+// first example.)
 //
 // Eight sequences of 32 heads at position 700 (92 MB): 23.1 -> 20.0 us, of which 3.3 are what position 0 takes;
 // one sequence at position 255: 7.1 -> 6.4.  Before, whole blocks were fetched and then worked on, and the rotated
@@ -464,6 +463,21 @@ silu_mul_kernel(const u32x4 *__restrict__ gate, const u32x4 *__restrict__ up, u3
     out[u] = o;
 }
 
+// Whether a step's cached rows are read non-temporally: where no later launch finds them in a cache, and kept there they push out what
+// is found.  That is a matter of all that a token reads against the 256 MB of the memory-side cache, not of one block's rows: where
+// weights and rows in use together come to less than about 400 MB, some of the rows are still there at the next token, and read so they
+// are not (8 heads of 128, 8 blocks, 109 MB besides the caches, one sequence at position 2000 283 -> 341 us, eight of 2 kv heads 331 -> 382;
+// four blocks, 88 MB, four sequences 182 -> 212).  The weights alone decide, since the position is the device's: from 402 MB on
+// (two blocks of 32 heads, 434 MB, two sequences at positions 60, 200, 1000, 2000 167.1 -> 167.1, 167.8 -> 167.1, 186 -> 182, 215 -> 202; below
+// it the early positions lose: 16 heads, 306 MB, two sequences at positions 30, 300, 1000 284 -> 287, 295 -> 306, 346 -> 349).  Caches under
+// 8 MB are not worth it.  Query heads that share rows, over long contexts, drift apart and miss rows that leave L2 first: up to 64 MB
+// (32 heads on 8 kv heads, 2048 positions: eight sequences, four blocks at positions 400 and 2000 297 -> 286 and 358 -> 347, sixteen
+// sequences, eight blocks at position 2000 832 -> 882).
+bool read_once(long cache_bytes, int rep, size_t step_bytes)
+{
+    return step_bytes >= (size_t)384 << 20 && cache_bytes >= 8l << 20 && (rep == 1 || cache_bytes <= 64l << 20);
+}
+
 bool aligned16(const void *p) { return ((uintptr_t)p & 15u) == 0; }
 
 int launch_status()
@@ -492,42 +506,55 @@ int lutgemm_decode_rmsnorm_f16(const void *x, const void *weight, void *y, int r
     return launch_status();
 }
 
-int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, const void *cos_table,
-                                 const void *sin_table, void *k_cache, void *v_cache, const int64_t *position,
-                                 void *out, int batch, int heads, int kv_heads, int head_dim, int max_positions,
-                                 void *stream)
+int lutgemm_describe_attention_plan(int batch, int heads, int kv_heads, int head_dim, int max_positions, size_t step_bytes,
+                                    lutgemm_attention_plan *plan)
+{
+    if (!plan || batch < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0) return LUTGEMM_EINVAL;
+    if (head_dim < 8 || head_dim > kThreads || head_dim % 8 != 0) return LUTGEMM_EINVAL;
+    if (max_positions < 1 || max_positions > 8192) return LUTGEMM_EINVAL;
+    *plan = {head_dim != 64 && head_dim != 128, batch * heads, kThreads, 0, 0};
+    if (plan->general) return LUTGEMM_OK;
+    const int rep = heads / kv_heads, pairs = batch * kv_heads;
+    const long cache_bytes = (long)pairs * max_positions * head_dim * 4;
+    plan->placed = rep > 1 && (cache_bytes >= 8l << 20 || pairs % 8 == 0);
+    if (plan->placed) plan->workgroups = (pairs + 7) / 8 * 8 * rep;
+    // With fewer workgroups than CUs eight waves each instead of four: 32 heads at position 255 6.4 us against
+    // 6.7; 256 workgroups at position 700 20.4 against 20.0, where the memory is what they wait for.
+    plan->threads = (long)batch * heads < 256 ? 512 : 256;
+    plan->once = read_once(cache_bytes, rep, step_bytes);
+    return LUTGEMM_OK;
+}
+
+int lutgemm_decode_attention_step_f16(const void *q, const void *k, const void *v, const void *cos_table,
+                                      const void *sin_table, void *k_cache, void *v_cache, const int64_t *position,
+                                      void *out, int batch, int heads, int kv_heads, int head_dim, int max_positions,
+                                      size_t step_bytes, void *stream)
 {
     if (!q || !k || !v || !cos_table || !sin_table || !k_cache || !v_cache || !position || !out)
         return LUTGEMM_EINVAL;
-    if (batch < 1 || heads < 1 || kv_heads < 1 || heads % kv_heads != 0) return LUTGEMM_EINVAL;
-    if (head_dim < 8 || head_dim > kThreads || head_dim % 8 != 0) return LUTGEMM_EINVAL;
-    if (max_positions < 1 || max_positions > 8192) return LUTGEMM_EINVAL;
+    lutgemm_attention_plan plan;
+    const int rc = lutgemm_describe_attention_plan(batch, heads, kv_heads, head_dim, max_positions, step_bytes, &plan);
+    if (rc != LUTGEMM_OK) return rc;
     if (!aligned16(k_cache) || !aligned16(v_cache)) return LUTGEMM_EALIGN;
     // (16-byte loads of every operand: others go to the general kernel)
-    if ((head_dim == 64 || head_dim == 128) && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
+    if (!plan.general && aligned16(q) && aligned16(k) && aligned16(v) && aligned16(cos_table) && aligned16(sin_table)) {
         const int rep = heads / kv_heads;
-        // Caches of less than 8 MB a block (small networks, short contexts) may still lie in the memory-side cache at the next
-        // token: read as usual (3 sequences of 8 heads on 2 kv heads, 2048 positions, 6 MB: a step 121.5 us, 122.8 otherwise).
-        const int pairs = batch * kv_heads;
-        const bool once = (long)pairs * max_positions * head_dim * 4 >= 8l << 20;
-        const int spread = rep > 1 && (once || pairs % 8 == 0) ? 3 : 0;
-        const HeadLayout layout{rep, kv_heads, spread, pairs, lutgemm::reciprocal_of(rep), lutgemm::reciprocal_of(kv_heads)};
-        auto launch = [&](auto kernel, int threads) {
-            hipLaunchKernelGGL(kernel, dim3((unsigned)(((((pairs - 1) >> spread) + 1) << spread) * rep)), dim3(threads), 0, (hipStream_t)stream,
+        const HeadLayout layout{rep, kv_heads, plan.placed ? 3 : 0, batch * kv_heads, lutgemm::reciprocal_of(rep),
+                                lutgemm::reciprocal_of(kv_heads)};
+        auto launch = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3((unsigned)plan.workgroups), dim3(plan.threads), 0, (hipStream_t)stream,
                                (const __half *)q, (const __half *)k, (const __half *)v, (const __half *)cos_table,
                                (const __half *)sin_table, (__half *)k_cache, (__half *)v_cache,
                                (const long long *)position, (__half *)out, layout, max_positions);
             return launch_status();
         };
-        // With fewer workgroups than CUs eight waves each instead of four: 32 heads at position 255 6.4 us against
-        // 6.7; 256 workgroups at position 700 20.4 against 20.0, where the memory is what they wait for.
-        const bool wide = (long)batch * heads < 256;
         auto launch_as = [&](auto once_c) {
             constexpr bool ONCE = decltype(once_c)::value;
-            if (head_dim == 128) return wide ? launch(attention_hd_kernel<128, 512, ONCE>, 512) : launch(attention_hd_kernel<128, 256, ONCE>, 256);
-            return wide ? launch(attention_hd_kernel<64, 512, ONCE>, 512) : launch(attention_hd_kernel<64, 256, ONCE>, 256);
+            const bool wide = plan.threads == 512;
+            if (head_dim == 128) return wide ? launch(attention_hd_kernel<128, 512, ONCE>) : launch(attention_hd_kernel<128, 256, ONCE>);
+            return wide ? launch(attention_hd_kernel<64, 512, ONCE>) : launch(attention_hd_kernel<64, 256, ONCE>);
         };
-        return once ? launch_as(std::true_type()) : launch_as(std::false_type());
+        return plan.once ? launch_as(std::true_type()) : launch_as(std::false_type());
     }
     const int groups = kThreads / head_dim;
     const size_t lds = sizeof(float) * ((size_t)3 * head_dim + max_positions + 4 + (size_t)groups * head_dim);
@@ -536,6 +563,15 @@ int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, co
                        (const __half *)sin_table, (__half *)k_cache, (__half *)v_cache,
                        (const long long *)position, (__half *)out, heads, kv_heads, head_dim, max_positions);
     return launch_status();
+}
+
+int lutgemm_decode_attention_f16(const void *q, const void *k, const void *v, const void *cos_table,
+                                 const void *sin_table, void *k_cache, void *v_cache, const int64_t *position,
+                                 void *out, int batch, int heads, int kv_heads, int head_dim, int max_positions,
+                                 void *stream)
+{
+    return lutgemm_decode_attention_step_f16(q, k, v, cos_table, sin_table, k_cache, v_cache, position, out, batch, heads, kv_heads,
+                                             head_dim, max_positions, 0, stream);
 }
 
 int lutgemm_decode_silu_mul_f16(const void *gate, const void *up, void *out, size_t count, void *stream)

@@ -159,6 +159,8 @@ class LutDecoder(nn.Module):
             self.register_buffer("gate_tagged", torch.zeros((batch, I), **i32), persistent=False)
             self.register_buffer("up_tagged", torch.zeros((batch, I), **i32), persistent=False)
             self.register_buffer("chain_words", torch.zeros((2,), **i32), persistent=False)   # epoch, status
+        # what a step reads besides the KV cache: the attention kernel reads past the caches where it is much
+        self.step_bytes = sum(t.nbytes for t in self.blocks.buffers()) + self.lm_head.nbytes
         self._graph = None
         self._stream = None
 
@@ -270,10 +272,11 @@ class LutDecoder(nn.Module):
         first = self.blocks[0]
         self._fused_gemv([first.q_proj, first.k_proj, first.v_proj], x, [q, k, v], sp, norm=first.input_norm, overwrite=True)
         for li, blk in enumerate(self.blocks):
-            check(lib.lutgemm_decode_attention_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), self.cos.data_ptr(),
-                                                   self.sin.data_ptr(), self.k_cache[li].data_ptr(),
-                                                   self.v_cache[li].data_ptr(), self.pos.data_ptr(),
-                                                   self.att.data_ptr(), B, H, KV, hd, cfg.max_positions, sp))
+            check(lib.lutgemm_decode_attention_step_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), self.cos.data_ptr(),
+                                                        self.sin.data_ptr(), self.k_cache[li].data_ptr(),
+                                                        self.v_cache[li].data_ptr(), self.pos.data_ptr(),
+                                                        self.att.data_ptr(), B, H, KV, hd, cfg.max_positions,
+                                                        self.step_bytes, sp))
             t = 4 * li                                     # tag bases of this block: t+1 .. t+4
             ps = [problem(blk.o_proj, self.att, xt, out_tag=t + 1),                                     # x += o_proj(att)
                   problem(blk.gate_proj, xt, gt, x_tag=t + 1, out_tag=t + 2, norm=blk.post_norm, overwrite=True),
@@ -333,10 +336,11 @@ class LutDecoder(nn.Module):
             else:
                 rmsnorm(blk.input_norm, self.qkv)
                 self._gemv_into(qkv_lins, h, [q, k, v], sp)
-            check(lib.lutgemm_decode_attention_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), self.cos.data_ptr(),
-                                                   self.sin.data_ptr(), self.k_cache[li].data_ptr(),
-                                                   self.v_cache[li].data_ptr(), self.pos.data_ptr(),
-                                                   self.att.data_ptr(), B, H, KV, hd, cfg.max_positions, sp))
+            check(lib.lutgemm_decode_attention_step_f16(q.data_ptr(), k.data_ptr(), v.data_ptr(), self.cos.data_ptr(),
+                                                        self.sin.data_ptr(), self.k_cache[li].data_ptr(),
+                                                        self.v_cache[li].data_ptr(), self.pos.data_ptr(),
+                                                        self.att.data_ptr(), B, H, KV, hd, cfg.max_positions,
+                                                        self.step_bytes, sp))
             gate_up, act = [blk.gate_proj, blk.up_proj], None if fold_gate else self.act
             if split:                                                   # x += o_proj(att); h = x * post_norm
                 self._fused_gemv([blk.o_proj], self.att, [x], sp, next_norm=blk.post_norm, next_in=h,

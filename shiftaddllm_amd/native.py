@@ -52,6 +52,8 @@ C_ABI_SYMBOLS = (
     "lutgemm_release_workspaces",
     "lutgemm_decode_rmsnorm_f16",
     "lutgemm_decode_attention_f16",
+    "lutgemm_decode_attention_step_f16",
+    "lutgemm_describe_attention_plan",
     "lutgemm_decode_silu_mul_f16",
     "lutgemm_gemv_rowwise_f16_gated",
     "lutgemm_describe_group_plan",
@@ -122,6 +124,11 @@ class GroupPlan(ctypes.Structure):
     """struct lutgemm_group_plan of include/lutgemm_gfx950.h."""
     _fields_ = [("kernel", ctypes.c_int), ("launches", ctypes.c_int), ("needs_workspace", ctypes.c_int),
                 ("workgroups", ctypes.c_int * MAX_GROUP), ("units_per_workgroup", ctypes.c_int * MAX_GROUP)]
+
+
+class AttentionPlan(ctypes.Structure):
+    """struct lutgemm_attention_plan of include/lutgemm_gfx950.h."""
+    _fields_ = [(n, ctypes.c_int) for n in ("general", "workgroups", "threads", "placed", "once")]
 
 
 class NativeLibraryMissing(ImportError):
@@ -214,6 +221,10 @@ def _bind(lib: ctypes.CDLL) -> ctypes.CDLL:
     lib.lutgemm_decode_rmsnorm_f16.restype = ci
     lib.lutgemm_decode_attention_f16.argtypes = [vp] * 9 + [ci] * 5 + [vp]
     lib.lutgemm_decode_attention_f16.restype = ci
+    lib.lutgemm_decode_attention_step_f16.argtypes = [vp] * 9 + [ci] * 5 + [sz, vp]
+    lib.lutgemm_decode_attention_step_f16.restype = ci
+    lib.lutgemm_describe_attention_plan.argtypes = [ci] * 5 + [sz, ctypes.POINTER(AttentionPlan)]
+    lib.lutgemm_describe_attention_plan.restype = ci
     lib.lutgemm_decode_silu_mul_f16.argtypes = [vp, vp, vp, sz, vp]
     lib.lutgemm_decode_silu_mul_f16.restype = ci
     lib.lutgemm_gemv_rowwise_f16_gated.argtypes = [ctypes.POINTER(FusedProblem), vp, vp]
