@@ -258,12 +258,11 @@ struct HeadLayout {
 // exponentials and weighted value sum (the "online" form of softmax); the rows of a wave are merged by lane
 // exchanges, the waves through LDS.
 //
-// Heads of one kv head sit on one XCD, behind one L2: eight (sequence, kv head) pairs lie side by side, one to an XCD, and
-// workgroups beyond the last pair leave at once (with places only where eight divides the pairs, 14 sequences of 40 heads on 10 kv
-// heads at position 1887 lost the sharing: a step of three blocks 524 -> 449 us).
+// Heads of one kv head sit on one XCD, behind one L2, where place_pairs finds that no CU gets more to do for it: eight (sequence,
+// kv head) pairs lie side by side, one to an XCD, and workgroups beyond the last pair leave at once.
 // ONCE: cached rows are read non-temporally (read_once says for which steps, and what it gives).  A launch for eight sequences at
-// position 700 19.4 -> 17.3 us.  (Heads that share rows have to sit behind one L2 for it: spread over the XCDs 524 -> 564 us in the
-// first example.)
+// position 700 19.4 -> 17.3 us.  (Heads that share rows have to sit behind one L2 for it: 14 sequences of 40 heads on 10 kv heads at
+// position 1887 spread over the XCDs, a step of three blocks 524 -> 564 us.)
 //
 // Eight sequences of 32 heads at position 700 (92 MB): 23.1 -> 20.0 us, of which 3.3 are what position 0 takes;
 // one sequence at position 255: 7.1 -> 6.4.  Before, whole blocks were fetched and then worked on, and the rotated
@@ -463,6 +462,18 @@ silu_mul_kernel(const u32x4 *__restrict__ gate, const u32x4 *__restrict__ up, u3
     out[u] = o;
 }
 
+// Whether the query heads of a (sequence, kv head) pair are placed on one XCD: where the fullest of its 32 CUs gets no more workgroups
+// than with all spread evenly.  Rows that heads share then come from memory once and are found in one L2 (20 pairs at position 1000, 4 and 8
+// query heads each, rows from memory 12.9 -> 11.4 and 18.3 -> 11.0 us, from the memory-side cache 11.6 -> 8.3 and 18.8 -> 8.5; 9 pairs of 12
+// 11.7 -> 10.3 and 11.1 -> 8.2); an XCD with two workgroups to a CU beside others with one takes up to twice as long (position 1000, one
+// pair of 64 8.2 -> 13.6, nine of 24 11.7 -> 14.8, nine of 48 16.4 -> 21.5).  One or two pairs of 32, which fill an XCD each and have but its
+// way to memory, lose as well (8.07 -> 8.33 and 8.15 -> 8.40); of 24 they are level.
+bool place_pairs(int pairs, int rep)
+{
+    auto rounds = [](int workgroups) { return (workgroups + 31) / 32; };
+    return rep > 1 && (pairs > 2 || rep <= 24) && rounds((pairs + 7) / 8 * rep) <= rounds((pairs * rep + 7) / 8);
+}
+
 // Whether a step's cached rows are read non-temporally: where no later launch finds them in a cache, and kept there they push out what
 // is found.  That is a matter of all that a token reads against the 256 MB of the memory-side cache, not of one block's rows: where
 // weights and rows in use together come to less than about 400 MB, some of the rows are still there at the next token, and read so they
@@ -516,7 +527,7 @@ int lutgemm_describe_attention_plan(int batch, int heads, int kv_heads, int head
     if (plan->general) return LUTGEMM_OK;
     const int rep = heads / kv_heads, pairs = batch * kv_heads;
     const long cache_bytes = (long)pairs * max_positions * head_dim * 4;
-    plan->placed = rep > 1 && (cache_bytes >= 8l << 20 || pairs % 8 == 0);
+    plan->placed = place_pairs(pairs, rep);
     if (plan->placed) plan->workgroups = (pairs + 7) / 8 * 8 * rep;
     // With fewer workgroups than CUs eight waves each instead of four: 32 heads at position 255 6.4 us against
     // 6.7; 256 workgroups at position 700 20.4 against 20.0, where the memory is what they wait for.

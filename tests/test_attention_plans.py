@@ -66,3 +66,25 @@ def test_the_decoder_says_what_a_token_reads():
     model = LutDecoder(cfg, None, device="cpu", default_bits=3)
     macs = 2 * (256 * 256 * 2 + 256 * 128 * 2 + 3 * 256 * 512)
     assert model.step_bytes == macs * 3 // 8 + macs // 128 * 3 * 2 + 2 * 96 * 256     # signs, one scale per 128 inputs, output matrix
+
+
+@pytest.mark.parametrize("max_positions", [64, 8192])
+def test_no_cu_gets_more_to_do_where_pairs_are_placed(lib, max_positions):
+    """32 CUs to an XCD: where query heads of a pair share one, its fullest CU holds no more workgroups than with all spread evenly, and
+    the grid has room for every pair and head."""
+    for pairs in range(1, 140):
+        for rep in (1, 2, 3, 4, 5, 7, 8, 12, 16, 24, 32, 33, 48, 64):
+            rc, plan = describe(lib, 1, pairs * rep, pairs, max_positions=max_positions)
+            assert rc == 0
+            if not plan.placed:
+                assert plan.workgroups == pairs * rep
+                continue
+            fullest, even = -(-pairs // 8) * rep, -(-pairs * rep // 8)
+            assert rep > 1 and plan.workgroups == 8 * fullest
+            assert -(-fullest // 32) <= -(-even // 32)
+
+
+def test_pairs_that_share_rows_are_placed_where_it_pays(lib):
+    placed = lambda pairs, rep: describe(lib, 1, pairs * rep, pairs)[1].placed == 1
+    assert all(placed(pairs, rep) for pairs in (1, 2, 3, 7, 9, 20) for rep in (2, 4, 8)) and placed(140, 4) and placed(64, 4) and placed(8, 64)
+    assert not any(placed(*few) for few in ((1, 64), (2, 64), (4, 64), (9, 64), (9, 24), (9, 48), (17, 24), (1, 32), (2, 32), (8, 1)))
