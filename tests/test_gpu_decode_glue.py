@@ -101,7 +101,7 @@ def test_attention_step(gpu_device, B, H, KV, hd, max_pos, positions):
 @pytest.mark.parametrize("B,H,KV,hd,max_pos,pos,offset", [
     (2, 16, 4, 128, 600, 255, 0),    # heads of a kv head placed together (8 kv heads); one row short of a block
     (2, 16, 4, 128, 600, 257, 0),    # a block and one row
-    (3, 9, 3, 64, 700, 640, 0),      # 9 kv heads: not placed
+    (3, 9, 3, 64, 700, 640, 0),      # 9 kv heads: two rounds of places, the last ones empty
     (16, 16, 16, 128, 300, 129, 0),  # 256 workgroups: four waves each, one row beyond their block
     (16, 32, 8, 64, 300, 256, 0),    # the same at the other head size, grouped
     (1, 4, 2, 128, 80, 70, 1),       # operands off 16-byte alignment: the general kernel
