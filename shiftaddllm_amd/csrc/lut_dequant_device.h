@@ -158,8 +158,8 @@ __device__ __forceinline__ TableEntries<NB, UNI> table_residual(const TableEntri
 // smallest fp16 number).  NaN and infinity are inexact.  LOWEST: u is the smallest of the multipliers' lowest set bits.  (bits & bits
 // - 1 clears the lowest mantissa bit; on a power of two it clears an exponent bit instead, which halves u at worst.  A zero
 // multiplier counts for nothing.)  Otherwise u follows from the sum, and adding and taking away 1.5 * 2^23 u rounds a multiplier to
-// a multiple of it: half the instructions (4096x11008x4 at 1024 rows 137.4 -> 134.3 us, 18016x432x4 at 407 36.2 -> 33.5, 8192x28672x4 at 32
-// 47.7 -> 47.0), but 16-row tiles, which have no registers for it, lose (8192x8192x4 in groups of 32 at 8 rows 21.9 -> 28.8).
+// a multiple of it: half the instructions (outputs x inputs x planes: 11008x4096x4 at 1024 rows 142 -> 136 us, 4096x4096x4 57.3 -> 54.4, 432x18016x4 at
+// 407 35.3 -> 32.6, 8192x28672x4 at 32 44.1 -> 43.4), but 16-row tiles, which have no registers for it, lose (8192x8192x4 in groups of 32 at 8 rows 21.9 -> 28.8).
 template <int NB, bool UNI, bool LOWEST>
 __device__ __forceinline__ bool may_round(const TableEntries<NB, UNI> &t, const float (&a)[NB], float q)
 {

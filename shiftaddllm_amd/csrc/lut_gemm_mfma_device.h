@@ -510,8 +510,8 @@ __device__ __forceinline__ void mfma_tile(const Problem &p, int local_block, cha
     const int nl = tid & 63;
     const int n = n_base + nl;
     // What the caller had in those outputs is requested here, not where the sums are complete: the request then runs beside
-    // the reduction and the atomics instead of behind them (128 rows of int8 exponents 3072x768 11.2 -> 10.4 us, 4096x4096x3
-    // with a bias at 16 rows 7.5 -> 6.9).  Ahead of the main loop it costs registers that the operands need (8 sequences'
+    // the reduction and the atomics instead of behind them (768x3072x3 int8 exponents at 128 rows 11.1 -> 10.3 us, 4096x4096x3
+    // with a bias at 16 rows 7.5 -> 6.8).  Ahead of the main loop it costs registers that the operands need (8 sequences'
     // down_proj of 4 planes 13.7 -> 14.7).  Whoever completes an output has read it before any contribution of its own, and
     // nobody writes it before all contributions are there.
     [[maybe_unused]] uint32_t init_bits[2 * MT];

@@ -363,8 +363,10 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
         // register there is: with both fragments' at once it reloaded spilled values behind all loads in flight,
         // 8192x8192x4 at 128 rows 51 us instead of 41.5, 11008x4096x4 at 2048 rows 294 instead of 242.)
         // Items, in order, and about how many vector instructions each takes; an item goes to the slot in which its share
-        // of all of them lies, so that the matrix instructions have as even a load beside them as may be (against items of whole
-        // operands, as many in each slot: 640x5376x3 at 759 rows 19.5 -> 19.1 us, int8 exponents 28.0 -> 25.9).
+        // of all of them lies, so that the matrix instructions have as even a load beside them as may be.  Against items of whole
+        // operands, as many in each slot, it is worth 1 % (outputs x inputs x planes: 4096x4096x4 at 1024 rows 53.0 -> 52.5 us,
+        // 11008x4096x4 134.8 -> 133.6, 11008x4096x3 at 2048 204.8 -> 203.7; 5376x640x3 at 759 and two planes level, 432x18016x4 at
+        // 407 rows 32.4 -> 32.6).
         constexpr bool WIDE = FMT == kTileBlockWide;
         constexpr int kSigns = NB == 4 ? 23 : 5 + 4 * NB, kLoad = 2 * NB, kTable = 8 << (NB - 1), kQuarter = NB == 4 ? 7 : 6;
         constexpr int kFragment = BLOCK ? 2 + 4 * 2 : 3 + 8, kItems = WIDE ? 3 + 4 * 5 : 2 * kFragment, kSlots = 4 * MF;
@@ -374,7 +376,7 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
             return r == -2 ? +kSigns : r == -1 ? +kLoad : r == 0 ? +kTable : +kQuarter;
         };
         auto first_item = [weight](int slot) constexpr {
-            if (BLOCK && !WIDE) return slot * kItems / kSlots;   // (finer items cost registers it does not have: 4096x4160x4 at 700 rows 68 -> 78 us)
+            if (BLOCK && !WIDE) return slot * kItems / kSlots;   // (finer items cost registers it does not have: 4160x4096x4 at 700 rows 68 -> 78 us)
             int all = 0, before = 0, k = 0;
             for (int i = 0; i < kItems; ++i) all += weight(i);
             while (k < kItems && (2 * before + weight(k)) * kSlots < 2 * all * slot) before += weight(k++);
@@ -525,12 +527,12 @@ __device__ __forceinline__ void gemm_tile(const TileProblem &p, int n_tile, int 
 
     // ---- write-out: lane l holds row l % 32 of a 32-row fragment and outputs 8 g + 4 (l / 32) + 0..3 ------
     // (K cut into slices: the sums of this slice, for tile_sum_kernel to add up)
-    // What the sums are added to is requested a 32-row fragment ahead of its use (1024x16384x3 at 512 rows with a bias 30.4 -> 27.2 us,
-    // 256x15360x3 at 330 rows 19.4 -> 14.4).
+    // (Sizes below: outputs x inputs x planes.)  What the sums are added to is requested a 32-row fragment ahead of its use (piece by piece
+    // where it is added 15360x256x3 at 330 rows with a bias 16.7 us, so 15.0; 2176x1024x3 int8 exponents at 1230 31.8 and 30.6).
     // `turn`: Stored from the accumulators, an instruction touches 32 rows' lines.  Teams, whose sums pass through LDS anyway, turn
     // them round there (16-byte chunk c of row r in slot c ^ r), so that an instruction stores 32 outputs of eight rows: 4096x4096x4 at
-    // 512 rows, two slices, 37.7 -> 36.3 us.  A lone team's two more passes through LDS cost more than it gives: 640x5376x3 at
-    // 759 rows 19.1 -> 20.3.
+    // 512 rows, two slices, 38.5 -> 37.0 us, 2176x1024x3 int8 exponents at 1230 rows with a bias 32.7 -> 30.6.  A lone team's two more
+    // passes through LDS cost more than it gives: 5376x640x3 at 759 rows 19.1 -> 20.3.
     float *sums = !SERIAL && p.ksplit > 1 ? p.partial + (size_t)slice * tile_slice_stride(p.M, p.N) : nullptr;
     const bool add = !sums && !p.overwrite;
     auto write_out = [&](auto f_c, auto &&turn) {

@@ -797,8 +797,9 @@ int run_mx(Problem &p, const Accum &acc)
 // entry point that allocates nothing.  Returns the time the plan should take.
 // Costs in microseconds, for all formats and planes.  A step of a 128-row tile: 1.1 alone on its CU (measured 1.0 to 1.25),
 // 1.95 beside another workgroup or for two teams together, 1.65 for teams while a third of the CUs are idle (clocks
-// are higher); 64 rows: 0.8, 1.35 and 1.2.  A workgroup's start and end 4.6, with teams 6.  The sums of the slices
-// and the launch that adds them up 6 and 0.2 per MB.  What they pick (us; s: slices of four waves, p: of teams, * = taken):
+// are higher); 64 rows: 0.8, 1.35 and 1.2.  A workgroup's start and end 4.6, with teams 6 (fitted when sums were added to a bias and
+// stored piece by piece, 2 more than now with teams or a bias).  The sums of the slices and the launch that adds them up 6 and 0.2 per
+// MB.  What they pick (us; s: slices of four waves, p: of teams, * = taken):
 //   512 rows:  5120x13824x2 int8 exponents s3 105.7 s6 92.1 p2 111.6 p3* 88.3; 13824x5120x2 int8 exponents s1 106.8 s2 99.5 p1* 85.2;
 //              4096x4096x3 s3 37.9 s4 34.2 p3 35.7 p4* 34.3 (s3 was taken before: 105.7, 106.6 and 42.5)
 //   1024 rows: 4096x4096x3 s1 72.1 s2 51.6 p1 60.7 p2* 50.3; 5120x5120x2 blocks s1 92.1 s2 84.3 s3 76.1 p1* 72.4
@@ -883,7 +884,10 @@ double gemm_us(const Problem &p, double estimate)
 
 // Whether a call takes the GEMM kernel rather than the matrix-core kernel, by the two estimates (see mfma_plan for the
 // calls that may).  Drawn with 900 calls and checked on 3000 others near the line, timed on both (33 to 2048 rows, 512 to 28672
-// inputs and outputs): the kernel taken is within 1.0 % of the better one on average, 6 % of the calls lose more than 5 %.
+// inputs and outputs), as both kernels then were: the kernel taken was within 1.0 % of the better one on average, 6 % of the calls lost
+// more than 5 %.  Closer to the line, 1000 calls that would change kernel at up to half as many rows again: 4.7 % and 22 % then,
+// 5.4 % and 24 % with the present kernels, five in six of those that lose by taking the
+// matrix-core kernel (most 768x17216x4 at 334 rows 72.8* / 32.8, 18192x1856x4 at 71 51.1* / 26.7).
 // Measured (us, matrix-core kernel / this one, * = taken):
 //   row-wise: 6464x4096x3 at 65 rows 18.0* / 22.8, 10944x5120x3 at 64 30.3* / 24.1, 6144x5120x2 at 72 18.6* / 24.4, 7680x8192x3 at 112
 //   40.0 / 33.1*, 3072x3328x3 at 256 22.3* / 24.3, 24128x3072x2 at 80 45.1 / 33.5*; scales that are no powers of two 3392x6144x3 at
